@@ -27,7 +27,7 @@ static int adjoint_impl(gs_ctx* c, const gs_params* p, const double* gN2, const 
 
     (void)hipEventRecord(v.ev[0], v.stream);
     double h;
-    if ((rc = ctx_build_grid(c, p->rmax, m, sx, &h))) return rc;
+    if ((rc = ctx_build_grid(c, p->rmax, m, sx, &h)) || (rc = ctx_row_chunks(c))) return rc;
     (void)hipEventRecord(v.ev[1], v.stream);
     v = view(c);
     const int mst = (int)std::ceil(p->rmax / h - 1e-12);

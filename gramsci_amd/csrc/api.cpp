@@ -75,6 +75,7 @@ template struct DevBuf<unsigned long long>;
 template struct DevBuf<unsigned char>;
 template struct DevBuf<int64_t>;
 template struct DevBuf<float>;
+template struct DevBuf<int4>;
 
 // ------------------------------------------------------------ thresholds
 // The reference's radial bin of a squared distance s (gramsci.F90:136-145,
@@ -240,6 +241,51 @@ int fill_bins(const gs_params& p, double rrel, double xmax, double wmax_d, doubl
     return GS_OK;
 }
 
+// fill_bins for the pair kernel.  A chunk's points lie within q.ext of its reference point per axis, so a
+// pair within rmax has coordinates (relative to that point) of at most q.ext and q.ext + rmax: rounding
+// both to FP32 and subtracting costs at most u (2 ext + 2 rmax) per component, u = 2^-24.
+//
+// mu guard.  With a = sqrt(3) ext and b = a + rmax bounding the two points' distances from the reference
+// point p, rho = |p|, u the rounding unit of the kernel's geometry and g(s) the error of s:
+//   D = 2(|xi|^2 - |xj|^2): both terms are rounded, |2(|x|^2 - rho^2)| <= 2 b (|x| + rho), which moves
+//     theta = (D/2) q by at most u (a + b)(2 rho + 3 (a + b)) q;
+//   S = |xi + xj|^2: relative error <= 5 u + (9 u b^2 + g) / S, and 1/S = s q^2 <= rmax^2 q^2;
+//   s: relative error g/s <= 4 sqrt(3) ew / |sep| + 6 ew^2 / s + 2^-21, 1/|sep| = q sqrt(S) <= q Sx with
+//     Sx = 2 rho + a + b;
+//   the reciprocal square root (half of the relative errors of s and S, plus 2^-22 in FP32 and less than
+//   2^-21 in FP64), the products and the FMA round by less than 2^-21 together.
+// k0, k1 and k2 q^2 carry factors of 2, 2 and 4 over these, so that a relative error of S s near one,
+// where the linearisation fails, gives a bound above 1/2 and hence a recheck.  Outside the range of
+// coordinates where S s neither overflows nor loses bits to underflow every pair is rechecked.
+int fill_pair_bins(const gs_params& p, const PairGrid& q, double xmax, double wmax_d, double wmax_r, BinDesc& B)
+{
+    int rc = fill_bins(p, q.ext + 0.5 * p.rmax, xmax, wmax_d, wmax_r, B);
+    if (rc) return rc;
+    const bool fp64 = p.precision == GS_FP64;
+    const double ms = B.mu_scale, r = p.rmax;
+    const double u = fp64 ? std::ldexp(1.0, -52) : std::ldexp(1.0, -24);
+    // FP64: the coordinates are exact, s is rounded three times
+    const double ew = fp64 ? 0.0 : std::ldexp(2.0 * q.ext + 2.0 * r, -24) * 1.01;
+    const double g = fp64 ? std::ldexp(r * r, -50) : s_guard(r * r, ew);
+    const double a = std::sqrt(3.0) * q.ext * 1.001, b = a + r * 1.001;
+    B.mu_ab = (float)((a + b) * 1.001);
+    B.mu_k0 = (float)(ms * 2.0 * std::ldexp(1.0, -20));
+    B.mu_k1a = (float)(ms * 2.0 * 2.0 * std::sqrt(3.0) * ew);
+    B.mu_k1b = (float)(ms * 2.0 * u * (a + b));
+    B.mu_k2a = (float)(ms * 4.0 * 0.5 * (9.0 * u * b * b + g) * r * r);
+    B.mu_k2b = (float)(ms * 4.0 * 3.0 * ew * ew);
+    const bool in_range = fp64 ? (r > 1e-30 && xmax < 1e30 && q.ext < 1e30)
+                               : (r > 1e-5 && r < 1e8 && xmax < 1e8 && q.ext < 1e8);
+    if (!in_range) B.mu_k0 = 1.0f;
+    // the kernel's bin table has one entry past the last bin: the estimate of a pair that is not yet
+    // rejected must not go beyond it
+    const double top = std::sqrt((double)B.rej_hi);
+    const double est = p.log_bins ? (std::log10(top) - std::log10(p.rmin)) / (std::log10(r) - std::log10(p.rmin)) * p.nbins
+                                  : (top - p.rmin) / (r - p.rmin) * p.nbins;
+    B.wide = !(est < p.nbins + 0.9) || r > 1e8 || q.ext > 1e8;
+    return GS_OK;
+}
+
 // Fixed-point scales 2^F of the weights and products.  Pairs: each weight is scaled by its
 // class's 2^F, below 2^26, so the largest pair product of every class stays below 2^52 (the
 // pair kernel rounds it to an integer with one FP64 addition of 2^52 and sums runs of up to
@@ -343,6 +389,8 @@ struct gs_ctx {
     DevBuf<uint32_t> flags;
     DevBuf<int32_t> orig;
     int32_t n_chunks = 0;
+    int chunk_group = 0;        // points per chunk of chunk_off (0: none built on this grid)
+    DevBuf<int4> chunks;        // descriptors of the pair kernel's chunks
     // launch scratch
     DevBuf<unsigned char> params;
     DevBuf<unsigned long long> out;
@@ -399,7 +447,7 @@ extern "C" int gs_destroy(gs_ctx* c)
     (void)hipStreamSynchronize(c->stream);
     c->xyz.release(); c->w.release(); c->buf.release();
     c->cell_of.release(); c->cell_start.release(); c->fill.release(); c->chunk_nc.release();
-    c->chunk_off.release(); c->scan_tmp.release(); c->pw.release(); c->ws.release(); c->pl.release(); c->flags.release();
+    c->chunk_off.release(); c->chunks.release(); c->scan_tmp.release(); c->pw.release(); c->ws.release(); c->pl.release(); c->flags.release();
     c->orig.release();
     c->params.release(); c->out.release(); c->queue.release(); c->part.release(); c->wpart.release();
     extra_release(c->extra);
@@ -618,7 +666,7 @@ static double choose_h(const gs_ctx* c, double rmax, int m, int sx)
 // chunks.
 int grid_build_raw(const double* xyz, const double* w, const int32_t* buf, int64_t n, int64_t n_data,
                    const double* bbox, double h, int sx, const GridBufs& b, int64_t max_cells, GridDesc* g_out,
-                   int32_t* nch, hipStream_t st)
+                   hipStream_t st)
 {
     GridDesc g{};
     g.h = h;
@@ -640,16 +688,26 @@ int grid_build_raw(const double* xyz, const double* w, const int32_t* buf, int64
     if (e == hipSuccess)
         e = launch_scatter(xyz, w, buf, n, n_data, g, b.cell_of, b.cell_start, b.fill, b.pw, b.ws, b.pl, b.flags, b.orig,
                            st);
-    const int nrow = g.dim[1] * g.dim[2];
-    if (e == hipSuccess) e = launch_row_chunks(b.cell_start, g.dim[0], nrow, b.chunk_nc, st);
-    if (e == hipSuccess) e = exclusive_scan(b.chunk_nc, b.chunk_off, nrow + 1, b.scan_tmp, st);
-    int32_t nc = 0;
-    if (e == hipSuccess) e = hipMemcpyAsync(&nc, b.chunk_off + nrow, sizeof(int32_t), hipMemcpyDeviceToHost, st);
-    if (e == hipSuccess) e = hipStreamSynchronize(st);
     if (e != hipSuccess) return hip_fail(e, "grid build");
     *g_out = g;
-    *nch = nc;
     return GS_OK;
+}
+
+hipError_t pair_chunks_raw(const GridDesc& g, int64_t n, int group, const GridBufs& b, hipStream_t st)
+{
+    const int nrow = g.dim[1] * g.dim[2];
+    hipError_t e = launch_row_chunks(b.cell_start, g.dim[0], nrow, group, b.chunk_nc, st);
+    if (e == hipSuccess) e = exclusive_scan(b.chunk_nc, b.chunk_off, nrow + 1, b.scan_tmp, st);
+    if (e == hipSuccess)
+        e = launch_chunks(b.chunk_off, nrow, b.cell_start, g.dim[0], nullptr, nullptr, 0, group,
+                          max_chunks(n, nrow, group), b.chunks, st);
+    return e;
+}
+
+static GridBufs grid_bufs(gs_ctx* c)
+{
+    return GridBufs{c->cell_of.ptr, c->cell_start.ptr, c->fill.ptr, c->chunk_nc.ptr, c->chunk_off.ptr, c->scan_tmp.ptr,
+                    c->pw.ptr, c->ws.ptr, c->pl.ptr, c->flags.ptr, c->orig.ptr, c->chunks.ptr};
 }
 
 int build_grid(gs_ctx* c, double h, int sx)
@@ -661,28 +719,51 @@ int build_grid(gs_ctx* c, double h, int sx)
     if (ncell > (1 << 26)) return fail(GS_ELIMIT, "grid too large (%lld cells)", (long long)ncell);
     int rc;
     if ((rc = c->cell_of.reserve(n)) || (rc = c->cell_start.reserve(ncell + 1)) || (rc = c->fill.reserve(ncell + 1)) ||
-        (rc = c->chunk_nc.reserve(ncell + 1)) || (rc = c->chunk_off.reserve(ncell + 1)) ||
         (rc = c->scan_tmp.reserve(scan_scratch_size(ncell + 1))) || (rc = c->pw.reserve(n)) || (rc = c->ws.reserve(n)) ||
         (rc = c->pl.reserve(n)) || (rc = c->flags.reserve(n)) || (rc = c->orig.reserve(n)))
         return rc;
-    GridBufs b{c->cell_of.ptr, c->cell_start.ptr, c->fill.ptr, c->chunk_nc.ptr, c->chunk_off.ptr, c->scan_tmp.ptr,
-               c->pw.ptr, c->ws.ptr, c->pl.ptr, c->flags.ptr, c->orig.ptr};
     GridDesc g;
-    int32_t nch = 0;
+    c->grid_valid = false;
     if ((rc = grid_build_raw(c->xyz.ptr, c->has_w ? c->w.ptr : nullptr, c->has_buf ? c->buf.ptr : nullptr, n,
-                             c->n_data, c->bbox, h, sx, b, (int64_t)1 << 26, &g, &nch, c->stream)))
+                             c->n_data, c->bbox, h, sx, grid_bufs(c), (int64_t)1 << 26, &g, c->stream)))
         return rc;
     c->g = g;
     c->grid_h = h;
     c->grid_sx = sx;
-    c->n_chunks = nch;
+    c->chunk_group = 0;
     c->grid_valid = true;
     return GS_OK;
 }
 
-// Cells per rmax of the pair kernel for n points in bounding box bbox: the finest grid (m <= 8)
+// the pair kernel's chunks of the current grid
+static int build_chunks(gs_ctx* c, int group)
+{
+    if (c->chunk_group == group) return GS_OK;
+    const int64_t n = c->n_data + c->n_rand, nrow = (int64_t)c->g.dim[1] * c->g.dim[2];
+    int rc;
+    if ((rc = c->chunk_nc.reserve(nrow + 1)) || (rc = c->chunk_off.reserve(nrow + 1)) ||
+        (rc = c->chunks.reserve(max_chunks(n, nrow, group))))
+        return rc;
+    c->chunk_group = 0;
+    hipError_t e = pair_chunks_raw(c->g, n, group, grid_bufs(c), c->stream);
+    if (e != hipSuccess) return hip_fail(e, "row chunks");
+    c->chunk_group = group;
+    return GS_OK;
+}
+
+int ctx_row_chunks(gs_ctx* c)
+{
+    int rc = build_chunks(c, kChunk);
+    if (rc) return rc;
+    const int64_t nrow = (int64_t)c->g.dim[1] * c->g.dim[2];
+    hipError_t e = hipMemcpyAsync(&c->n_chunks, c->chunk_off.ptr + nrow, sizeof(int32_t), hipMemcpyDeviceToHost, c->stream);
+    if (e == hipSuccess) e = hipStreamSynchronize(c->stream);
+    return e == hipSuccess ? GS_OK : hip_fail(e, "row chunks");
+}
+
+// Cells per rmax of the adjoint kernels for n points in bounding box bbox: the finest grid (m <= 8)
 // whose cells still hold ~32 points or more.
-int pair_cell_div(int64_t n, const double* bbox, double rmax)
+static int adjoint_cell_div(int64_t n, const double* bbox, double rmax)
 {
     double vol = 1.0;
     for (int k = 0; k < 3; ++k) vol *= std::max(bbox[3 + k] - bbox[k], rmax * 1e-3);
@@ -693,6 +774,83 @@ int pair_cell_div(int64_t n, const double* bbox, double rmax)
         if (dens * h * h * h >= 32.0) best = m;
     }
     return best;
+}
+
+static int env_int(const char* name)    // a tuning override, 0 if unset or empty
+{
+    const char* ev = getenv(name);
+    return ev && *ev ? atoi(ev) : 0;
+}
+
+// Modelled VALU cycles per point of the pair kernel with chunks of `group` points on cells h and h / sx.  A
+// chunk spans about group / (dens h^2) in x; its candidates are half the volume within rmax of its box
+// (grown by the neighbour rows' cell width), in tiles of 64 that cost group / 2 steps of two pairs.
+static double pair_cost(const PairGrid& q, int group, double dens, double len_x, double rmax, double* cap,
+                        double* tiles_out)
+{
+    const double lin = std::max(dens * q.h * q.h, 1e-30);       // points per unit length of a row
+    const double row = lin * len_x;
+    const double len = std::min(group / lin, len_x);
+    *cap = std::min(std::max(2.0 * len, 0.25 * rmax), rmax);    // a chunk's largest extent
+    const double pieces = std::max(1.0, len / *cap);
+    const double pts = std::max(1.0, row) / std::max(1.0, std::ceil(row / group)) / pieces;     // per chunk
+    const double ax = len / pieces + 1.5 * q.h / q.sx, ay = 2.0 * q.h;
+    const double vol = ax * ay * ay + 2.0 * (2.0 * ax * ay + ay * ay) * rmax + M_PI * (ax + 2.0 * ay) * rmax * rmax +
+                       4.0 / 3.0 * M_PI * rmax * rmax * rmax;
+    const double tiles = 0.5 * dens * vol / kWave + 0.5;
+    const double rows = 0.5 * M_PI * (q.mst + 1.0) * (q.mst + 1.0);
+    *tiles_out = tiles;
+    return (tiles * (47.0 * group + 150.0) + 1500.0 + rows * 250.0) / pts;
+}
+
+void pair_group(PairGrid& q, double dens, double len_x, double rmax)
+{
+    const int want = env_int("GS_PAIR_GROUP");
+    double cap = rmax, c, tiles;
+    q.cost = 1e300;
+    for (int group : {64, 32, 16}) {
+        if ((want == 16 || want == 32 || want == 64) && want != group) continue;
+        const double cost = pair_cost(q, group, dens, len_x, rmax, &c, &tiles);
+        if (cost < q.cost) { q.cost = cost; q.group = group; q.tiles = tiles; cap = c; }
+    }
+    const double hx = q.h / q.sx;
+    q.cap_cells = (int)std::min(std::floor(cap / hx), 1e6);
+    q.ext = std::max((q.cap_cells + 1) * hx, q.h) * 1.001;
+}
+
+PairGrid pair_grid(int64_t n, const double* bbox, double rmax, int cell_div, int64_t max_cells)
+{
+    double vol = 1.0;
+    for (int k = 0; k < 3; ++k) vol *= std::max(bbox[3 + k] - bbox[k], rmax * 1e-3);
+    const double dens = (double)n / vol;
+    PairGrid best;
+    for (int m = cell_div > 0 ? cell_div : 1; m <= (cell_div > 0 ? cell_div : 8); ++m) {
+        PairGrid q;
+        q.m = m;
+        q.sx = pair_cell_sx();
+        q.h = choose_h_bbox(bbox, rmax, m, max_cells, q.sx);
+        q.mst = (int)std::ceil(rmax / q.h - 1e-12);
+        pair_group(q, dens, std::max(bbox[3] - bbox[0], rmax * 1e-3), rmax);
+        if (best.h == 0 || q.cost < best.cost) best = q;
+    }
+    return best;
+}
+
+int pair_lg_parts(int64_t n, const PairGrid& q)
+{
+    const int want = env_int("GS_PAIR_PARTS");
+    const double chunks = std::max(1.0, (double)n / q.group);
+    int lg = 0;
+    if (want) {
+        while (lg < 6 && (2 << lg) <= want) ++lg;
+    } else {
+        // two items for every SIMD at least; beyond that, items of no less than 12 tiles' work with the
+        // smallest chunks, as long as a wave takes few of them (an item costs some 10 us of dependent loads)
+        while (lg < 6 && (chunks * (1 << lg) < 2048.0 ||
+                          (chunks * (1 << lg) < 131072.0 && q.tiles * q.group / 16.0 >= 12.0 * (2 << lg))))
+            ++lg;
+    }
+    return lg;
 }
 
 // x cells per y/z cell of the pair kernels' grid: finer x cells cut each stencil row to the x-range that
@@ -716,7 +874,7 @@ int apex_cell_sx() { return cell_sx_env("GS_T3_CELL_SX", 4); }
 int default_cell_div(const gs_ctx* c, double rmax, int mode)
 {
     if (mode != 2) return 1;
-    return pair_cell_div(c->n_data + c->n_rand, c->bbox, rmax);
+    return adjoint_cell_div(c->n_data + c->n_rand, c->bbox, rmax);
 }
 
 }  // namespace gs
@@ -725,50 +883,61 @@ int default_cell_div(const gs_ctx* c, double rmax, int mode)
 
 namespace gs {
 
-// Launch shape of the pair kernel: work-group size and LDS histogram replicas (spreading same-bin
-// atomics).  256-thread work-groups (four waves per shared histogram) are kept when they reach 16
-// resident waves per CU; otherwise larger work-groups share one histogram among more waves to raise
-// residency.  Among shapes with the same residency, more replicas win.  Cached per variant.
-int pair2_shape(int nb, int nm, bool fp64, bool weighted, bool logb, int* reps_out, int* wg_out, int* waves_out)
+// Launch shape of the pair kernel: work-group size, LDS histogram replicas (spreading same-bin atomics)
+// and, with buffer points, histogram planes.  256-thread work-groups (four waves per shared histogram)
+// are kept when they reach 16 resident waves per CU; otherwise larger work-groups share one histogram
+// among more waves to raise residency.  Among shapes with the same residency, more replicas win.  A
+// histogram that does not fit otherwise runs with one plane and, at last, one wave.  Cached per variant.
+int pair2_shape(const PairVariant& v, PairShape* out)
 {
-    const bool rsd = nm >= 2;
-    int reps = 1, wg = kWG, best_waves = 0;
-    const char* ev_reps = getenv("GS_PAIR_REPS");    // tuning overrides (unset or empty: automatic)
-    const char* ev_wg = getenv("GS_PAIR_WG");
-    if (ev_reps && !*ev_reps) ev_reps = nullptr;
-    if (ev_wg && !*ev_wg) ev_wg = nullptr;
+    const int ev_reps = env_int("GS_PAIR_REPS"), ev_wg = env_int("GS_PAIR_WG");     // tuning overrides
     char key[96];
-    snprintf(key, sizeof(key), "%d/%d/%d/%d/%d/%d/%s/%s", nb, nm, (int)fp64, (int)rsd, (int)weighted, (int)logb,
-             ev_reps ? ev_reps : "", ev_wg ? ev_wg : "");
+    snprintf(key, sizeof(key), "%d/%d/%d%d%d%d/%d/%d", v.nb, v.nm, (int)v.fp64, (int)v.weighted, (int)v.logb,
+             (int)v.buf, ev_reps, ev_wg);
     static std::mutex mu;
-    static std::map<std::string, std::array<int, 3>> shapes;
+    static std::map<std::string, PairShape> shapes;
     std::lock_guard<std::mutex> lock(mu);
     auto it = shapes.find(key);
     if (it != shapes.end()) {
-        reps = it->second[0]; wg = it->second[1]; best_waves = it->second[2];
-    } else {
-        for (int pass = 0; pass < 2 && (pass == 0 || best_waves < 16); ++pass) {
-            for (int r = 1; r <= 32; r *= 2) {
-                for (int w = pass == 0 ? 256 : 384; w <= (pass == 0 ? 256 : 1024); w += 128) {
-                    if (ev_reps && atoi(ev_reps) != r) continue;
-                    if (ev_wg && atoi(ev_wg) != w) continue;
-                    if (pair2_lds_bytes(nb, rsd ? nm : 1, r, fp64, weighted, false, w) > 160 * 1024) continue;
-                    const int waves = pair2_occupancy(nb, nm, r, fp64, rsd, weighted, logb, false, w) * (w / kWave);
-                    if (waves > best_waves || (waves == best_waves && r > reps && w == wg)) {
-                        best_waves = waves;
-                        reps = r;
-                        wg = w;
-                    }
-                }
-            }
-        }
-        shapes[key] = {reps, wg, best_waves};
+        *out = it->second;
+        return it->second.waves ? GS_OK : fail(GS_ELIMIT, "histogram of %d bins does not fit in LDS", 3 * v.nb * v.nm);
     }
-    if (best_waves == 0) return fail(GS_ELIMIT, "histogram of %d bins does not fit in LDS", 3 * nb * nm);
-    *reps_out = reps;
-    *wg_out = wg;
-    *waves_out = best_waves;
+    PairShape s;
+    auto consider = [&](int planes, int r, int w) {
+        if (ev_reps && ev_reps != r) return;
+        if (ev_wg && ev_wg != w) return;
+        if (pair2_lds_bytes(v.nb, v.nm, planes, r, v.weighted, false, w) > kPairLdsMax) return;
+        const int waves = pair2_occupancy(v, planes, r, false, w) * (w / kWave);
+        if (waves > s.waves || (waves == s.waves && planes == s.planes && r > s.reps && w == s.wg))
+            s = PairShape{planes, r, w, waves};
+    };
+    for (int planes = v.buf ? 2 : 1; planes >= 1 && s.waves == 0; --planes) {
+        for (int r = 1; r <= 32; r *= 2) consider(planes, r, 256);
+        if (s.waves < 16)
+            for (int r = 1; r <= 32; r *= 2)
+                for (int w = 320; w <= 1024; w += 64) consider(planes, r, w);
+    }
+    for (int w = 192; w >= 64 && s.waves == 0; w -= 64) consider(1, 1, w);
+    shapes[key] = s;
+    if (s.waves == 0) return fail(GS_ELIMIT, "histogram of %d bins does not fit in LDS", 3 * v.nb * v.nm);
+    *out = s;
     return GS_OK;
+}
+
+// Work split and launch of the pair kernel over one catalogue's chunks (a: the arrays and outputs).
+hipError_t pair_launch(PairArgs& a, const PairVariant& var, const PairShape& shape, const PairGrid& q, int64_t n,
+                       int n_cu, hipStream_t st)
+{
+    a.group = q.group;
+    a.cap_cells = (float)q.cap_cells;
+    a.reps = shape.reps;
+    a.planes = shape.planes;
+    a.lg_parts = pair_lg_parts(n, q);
+    // no more work-groups than items could fill, a multiple of 8 (the same number on each XCD)
+    const int64_t wpg = shape.wg / kWave;
+    const int64_t items = max_chunks(n, (int64_t)a.g.dim[1] * a.g.dim[2], q.group) << a.lg_parts;
+    const int64_t nblocks = std::min<int64_t>((int64_t)n_cu * shape.waves / wpg, (items + wpg - 1) / wpg);
+    return launch_pair2(a, var, (int)((nblocks + 7) / 8 * 8), shape.wg, st);
 }
 
 // Pair kernel outputs (counts [3][nb][nm], 128-bit class sums, statistics) -> the C ABI's outputs:
@@ -820,73 +989,71 @@ extern "C" int gs_count_2pcf(gs_ctx* c, const gs_params* p, uint64_t* cnt, doubl
     if (rc) return rc;
     if ((rc = set_device(c))) return rc;
     const int nb = p->nbins, nm = p->nmu;
-    const bool rsd = nm >= 2, fp64 = p->precision == GS_FP64, weighted = c->has_w;
     const int nbt = 3 * nb * nm;
-    const int m = p->cell_div > 0 ? p->cell_div : default_cell_div(c, p->rmax, 2);
-    const int sx = pair_cell_sx();
-    const double h = choose_h(c, p->rmax, m, sx);
-    const int mst = (int)std::ceil(p->rmax / h - 1e-12);
-    std::vector<Row> rows = half_stencil(h, h / sx, p->rmax, mst);
+    const bool weighted = c->has_w;
+    const int64_t n = c->n_data + c->n_rand;
+    const PairGrid q = pair_grid(n, c->bbox, p->rmax, p->cell_div, (int64_t)1 << 24);
+    std::vector<Row> rows = half_stencil(q.h, q.h / q.sx, p->rmax, q.mst);
     if ((int)rows.size() > kMaxRows) return fail(GS_ELIMIT, "stencil too large");
 
     (void)hipEventRecord(c->ev[0], c->stream);
-    if ((rc = build_grid(c, h, sx))) return rc;
+    if ((rc = build_grid(c, q.h, q.sx))) return rc;
+    if ((rc = build_chunks(c, q.group))) return rc;
     (void)hipEventRecord(c->ev[1], c->stream);
 
     double xmax = 0;
     for (int k = 0; k < 6; ++k) xmax = std::max(xmax, std::fabs(c->bbox[k]));
     BinDesc B;
-    if ((rc = fill_bins(*p, (mst + 1) * h, xmax, c->wmax_d, c->wmax_r, B))) return rc;
+    if ((rc = fill_pair_bins(*p, q, xmax, c->wmax_d, c->wmax_r, B))) return rc;
+    const PairVariant var{nb, nm, p->precision == GS_FP64 || B.wide, weighted, p->log_bins != 0, c->has_buf};
+    PairShape shape;
+    if ((rc = pair2_shape(var, &shape))) return rc;
 
-    int reps = 1, wg = kWG, best_waves = 0;
-    if ((rc = pair2_shape(nb, nm, fp64, weighted, p->log_bins != 0, &reps, &wg, &best_waves))) return rc;
-
-    const size_t nout = (size_t)nbt + 2 * (size_t)nbt + 4;
-    if ((rc = c->params.reserve(sizeof(BinDesc) + rows.size() * sizeof(Row) + 64)) || (rc = c->out.reserve(nout)) ||
-        (rc = c->queue.reserve(8)))
+    const int copies = pair_copies(1, nbt);
+    const size_t nwork = (size_t)copies * pair_copy_words(1, nbt), nout = 3 * (size_t)nbt + 4;
+    if ((rc = c->params.reserve(sizeof(BinDesc) + rows.size() * sizeof(Row) + 64)) || (rc = c->out.reserve(nwork + nout)) ||
+        (rc = c->queue.reserve(64 * kQueuePad)))
         return rc;
     unsigned char* dB = c->params.ptr;
     Row* dRows = (Row*)(c->params.ptr + ((sizeof(BinDesc) + 15) / 16) * 16);
     hipError_t e = hipMemcpyAsync(dB, &B, sizeof(B), hipMemcpyHostToDevice, c->stream);
     if (e == hipSuccess && !rows.empty())
         e = hipMemcpyAsync(dRows, rows.data(), rows.size() * sizeof(Row), hipMemcpyHostToDevice, c->stream);
-    if (e == hipSuccess) e = hipMemsetAsync(c->out.ptr, 0, nout * sizeof(unsigned long long), c->stream);
-    if (e == hipSuccess) e = hipMemsetAsync(c->queue.ptr, 0, 8 * sizeof(int32_t), c->stream);
+    if (e == hipSuccess) e = hipMemsetAsync(c->out.ptr, 0, nwork * sizeof(unsigned long long), c->stream);
+    if (e == hipSuccess) e = hipMemsetAsync(c->queue.ptr, 0, 64 * kQueuePad * sizeof(int32_t), c->stream);
     if (e != hipSuccess) return hip_fail(e, "parameter upload");
 
     PairArgs a{};
     a.pw = c->pw.ptr;
-    a.ws = c->ws.ptr;
     a.pl = c->pl.ptr;
     a.flags = c->flags.ptr;
     a.cell_start = c->cell_start.ptr;
-    a.row_chunk = c->chunk_off.ptr;
+    a.chunks = c->chunks.ptr;
     a.rows = dRows;
     a.bins = (const BinDesc*)dB;
     a.queue = c->queue.ptr;
     a.out_cnt = c->out.ptr;
-    a.out_w = c->out.ptr + nbt;
-    a.out_stats = c->out.ptr + 3 * nbt;
+    a.out_w = c->out.ptr + 2 * nbt;
+    a.out_stats = c->out.ptr + 6 * nbt;
+    a.copies = copies;
+    a.copy_stride = pair_copy_words(1, nbt);
     a.g = c->g;
-    a.g.m = mst;
+    a.g.m = q.mst;
     a.nrows = (int)rows.size();
-    a.n_chunks = c->n_chunks;
-    a.reps = reps;
-    a.mirror = (rsd && !c->has_buf) ? 1 : 0;
-    const int occ = best_waves / (wg / kWave);
-    int nblocks = c->n_cu * occ;
-    if (nblocks > c->n_chunks) nblocks = std::max(c->n_chunks, 1);
+    a.n_chunks_dev = c->chunk_off.ptr + (size_t)c->g.dim[1] * c->g.dim[2];
     (void)hipEventRecord(c->ev[2], c->stream);
-    if (c->n_chunks > 0) {
-        e = launch_pair2(a, nb, nm, fp64, rsd, weighted, p->log_bins != 0, nblocks, wg, c->stream);
+    if (n > 0) {
+        e = pair_launch(a, var, shape, q, n, c->n_cu, c->stream);
         if (e != hipSuccess) return hip_fail(e, "pair kernel launch");
     }
     (void)hipEventRecord(c->ev[3], c->stream);
+    e = launch_pair_reduce(c->out.ptr, copies, 1, nbt, nm, weighted, c->out.ptr + nwork, c->stream);
     std::vector<unsigned long long> h_out(nout);
-    e = hipMemcpyAsync(h_out.data(), c->out.ptr, nout * sizeof(unsigned long long), hipMemcpyDeviceToHost, c->stream);
+    if (e == hipSuccess)
+        e = hipMemcpyAsync(h_out.data(), c->out.ptr + nwork, nout * sizeof(unsigned long long), hipMemcpyDeviceToHost,
+                           c->stream);
     if (e == hipSuccess) e = hipStreamSynchronize(c->stream);
     if (e != hipSuccess) return hip_fail(e, "pair kernel");
-
     combine2(h_out.data(), nb, nm, B, weighted, c->wsum_d, c->wsum_r, cnt, wsum, n2, n3, st);
     if (st) {
         float ms_grid = 0, ms_count = 0;
@@ -895,7 +1062,7 @@ extern "C" int gs_count_2pcf(gs_ctx* c, const gs_params* p, uint64_t* cnt, doubl
         st->ms_grid = ms_grid;
         st->ms_count = ms_count;
         st->ms_kernel_avg = ms_count;
-        st->cell_div = mst;
+        st->cell_div = q.mst;
     }
     return GS_OK;
 }

@@ -38,6 +38,7 @@ void batch_release(GsBatch& b)
     b.d_off.release(); b.d_row_base.release(); b.cell_of.release(); b.count.release(); b.cell_start.release();
     b.nch.release(); b.row_chunk.release(); b.scan_tmp.release(); b.queue.release(); b.orig.release();
     b.d_regions.release(); b.params.release(); b.pw.release(); b.ws.release(); b.pl.release(); b.flags.release();
+    b.chunks.release();
     b.out.release();
     b.xyz.release(); b.w.release(); b.buf.release(); b.ovf.release(); b.big.release();
     b.valid = false;
@@ -73,7 +74,7 @@ static int get_plan(gs_ctx* c, const gs_params& p, const BatchTune& tu, int kind
     const int nreg = B.nreg;
     const int64_t n = B.off[nreg];   // the batch's own copy of its catalogue (input order)
     const int nb = p.nbins, nm = p.nmu;
-    const bool rsd = nm >= 2, fp64 = p.precision == GS_FP64, weighted = B.has_w;
+    const bool fp64 = p.precision == GS_FP64, weighted = B.has_w;
     const int nbt = 3 * nb * nm;
 
     // cell edges (x cut finer for the pair kernel) and per-region grids
@@ -110,7 +111,25 @@ static int get_plan(gs_ctx* c, const gs_params& p, const BatchTune& tu, int kind
     if ((int)rows.size() > kMaxRows) return fail(GS_ELIMIT, "stencil too large");
     BinDesc bins;
     int rc;
-    if ((rc = fill_bins(p, kind == 3 ? 1.5 * p.rmax : (mst + 1) * h, B.xmax, B.wmax_d, B.wmax_r, bins))) return rc;
+    // pair kernel: chunk size for the regions' mean density and row length
+    PairGrid q;
+    if (kind == 2) {
+        double vol = 0.0, len = 0.0;
+        for (int r = 0; r < nreg; ++r) {
+            double v3 = 1.0;
+            for (int k = 0; k < 3; ++k) v3 *= std::max(B.bbox[6 * r + 3 + k] - B.bbox[6 * r + k], p.rmax * 1e-3);
+            vol += v3;
+            len += v3 * std::max(B.bbox[6 * r + 3] - B.bbox[6 * r], p.rmax * 1e-3);
+        }
+        q.m = m;
+        q.sx = sx;
+        q.h = h;
+        q.mst = mst;
+        pair_group(q, (double)n / vol, len / vol, p.rmax);
+        if ((rc = fill_pair_bins(p, q, B.xmax, B.wmax_d, B.wmax_r, bins))) return rc;
+    } else if ((rc = fill_bins(p, 1.5 * p.rmax, B.xmax, B.wmax_d, B.wmax_r, bins))) {
+        return rc;
+    }
 
     // triplet kernel: configuration and find_normal tables, LDS plan
     std::vector<uint16_t> tab3;
@@ -128,14 +147,15 @@ static int get_plan(gs_ctx* c, const gs_params& p, const BatchTune& tu, int kind
         if ((rc = plan_triplet_lds(ta, nb, fp64, weighted))) return rc;
         nh = ta.ncfg * nm * 4;
     }
-    const size_t nout = kind == 3 ? (size_t)nreg * 3 * nh + 8 : (size_t)nreg * 3 * nbt + 4;
+    const size_t nout = kind == 3 ? (size_t)nreg * 3 * nh + 8 : (size_t)nreg * 3 * nbt + 4 + (size_t)pair_copies(nreg, nbt) * pair_copy_words(nreg, nbt);
+    const int64_t nchunk = kind == 2 ? max_chunks(n, rows_tot, q.group) : 0;
     const int64_t scan_n = std::max<int64_t>(cells + 1, rows_tot + 1);
     // captured graphs hold raw pointers to the shared work buffers: if any of
     // them has to grow, every existing plan is destroyed before reallocating
     const bool grow = (size_t)n > B.cell_of.cap || (size_t)(cells + 1) > B.count.cap ||
                       (size_t)(cells + 1) > B.cell_start.cap || (size_t)(rows_tot + 1) > B.nch.cap ||
                       (size_t)(rows_tot + 1) > B.row_chunk.cap || (size_t)scan_scratch_size(scan_n) > B.scan_tmp.cap ||
-                      nout > B.out.cap || (kind == 3 && (size_t)(2 * n + 3) > B.ovf.cap) || B.queue.cap < 32;
+                      nout > B.out.cap || (size_t)nchunk > B.chunks.cap || (kind == 3 && (size_t)(2 * n + 3) > B.ovf.cap) || B.queue.cap < 32 + 64 * kQueuePad;
     if (grow) {
         for (auto& pl : B.plans) {
             if (pl.exec) (void)hipGraphExecDestroy(pl.exec);
@@ -146,10 +166,10 @@ static int get_plan(gs_ctx* c, const gs_params& p, const BatchTune& tu, int kind
     }
     if ((rc = B.cell_of.reserve(n)) || (rc = B.count.reserve(cells + 1)) || (rc = B.cell_start.reserve(cells + 1)) ||
         (rc = B.nch.reserve(rows_tot + 1)) || (rc = B.row_chunk.reserve(rows_tot + 1)) ||
-        (rc = B.scan_tmp.reserve(scan_scratch_size(scan_n))) || (rc = B.queue.reserve(32)) ||
+        (rc = B.scan_tmp.reserve(scan_scratch_size(scan_n))) || (rc = B.queue.reserve(32 + 64 * kQueuePad)) ||
         (kind == 3 && (rc = B.ovf.reserve(2 * n + 3))) ||
         (rc = B.orig.reserve(n)) || (rc = B.pw.reserve(n)) || (rc = B.ws.reserve(n)) || (rc = B.pl.reserve(n)) ||
-        (rc = B.flags.reserve(n)) ||
+        (rc = B.flags.reserve(n)) || (rc = B.chunks.reserve(nchunk)) ||
         (rc = B.out.reserve(nout)))
         return rc;
     // per-plan parameter blob: regions, bins, stencil rows (kept for the plan's lifetime)
@@ -182,32 +202,48 @@ static int get_plan(gs_ctx* c, const gs_params& p, const BatchTune& tu, int kind
 
     PairArgs a{};
     a.pw = B.pw.ptr;
-    a.ws = B.ws.ptr;
     a.pl = B.pl.ptr;
     a.flags = B.flags.ptr;
     a.cell_start = B.cell_start.ptr;
-    a.row_chunk = B.row_chunk.ptr;
+    a.chunks = B.chunks.ptr;
     a.rows = (const Row*)(pblob->ptr + rows_off);
     a.bins = (const BinDesc*)(pblob->ptr + bin_off);
-    a.queue = B.queue.ptr;
-    a.out_cnt = B.out.ptr;
-    a.out_w = B.out.ptr + (size_t)nreg * nbt;
-    a.out_stats = B.out.ptr + (size_t)nreg * 3 * nbt;
+    // outputs: the sum ([nreg][nbt] counts, [nreg][nbt][2] sums, statistics), then the copies it is made of
+    const size_t nsum = (size_t)nreg * 3 * nbt + 4;
+    a.queue = B.queue.ptr + 32;
+    a.out_cnt = B.out.ptr + nsum;
+    a.out_w = a.out_cnt + (size_t)nreg * 2 * nbt;
+    a.out_stats = a.out_cnt + (size_t)nreg * 6 * nbt;
+    a.copies = pair_copies(nreg, nbt);
+    a.copy_stride = pair_copy_words(nreg, nbt);
     a.g.h = h;
     a.g.h32 = (float)h;
     a.g.hx = hx;
     a.g.hx32 = (float)hx;
     a.g.m = mst;
     a.nrows = (int)rows.size();
+    a.group = q.group;
+    a.cap_cells = (float)q.cap_cells;
     a.reps = 1;
-    a.mirror = (rsd && !B.has_buf) ? 1 : 0;
+    a.planes = 1;
     a.regions = d_reg;
-    a.row_base = (const int32_t*)(pblob->ptr + rb_off);
     a.n_chunks_dev = B.row_chunk.ptr + rows_tot;
     a.nreg = nreg;
-    if (kind == 2 && pair2_lds_bytes(nb, rsd ? nm : 1, 1, fp64, weighted, true) > 64 * 1024) {
-        pblob->release(); B.plans.pop_back();
-        return fail(GS_ELIMIT, "per-wave histograms of %d bins do not fit in LDS", nbt);
+    const int32_t* d_row_base = (const int32_t*)(pblob->ptr + rb_off);
+    // one histogram per wave: fewer planes and waves where it would not fit otherwise
+    const PairVariant var{nb, nm, fp64 || (kind == 2 && bins.wide), weighted, p.log_bins != 0, B.has_buf};
+    int pair_wg = kWG, pair_waves = 0;
+    if (kind == 2) {
+        for (a.planes = var.buf ? 2 : 1; a.planes >= 1 && pair_waves == 0; --a.planes)
+            for (pair_wg = kWG; pair_wg >= kWave && pair_waves == 0; pair_wg /= 2)
+                pair_waves = pair2_occupancy(var, a.planes, 1, true, pair_wg) * (pair_wg / kWave);
+        ++a.planes;             // the loops' last step
+        pair_wg *= 2;
+        if (pair_waves == 0) {
+            pblob->release(); B.plans.pop_back();
+            return fail(GS_ELIMIT, "per-wave histograms of %d bins do not fit in LDS", nbt);
+        }
+        a.lg_parts = pair_lg_parts(n, q);
     }
     if (kind == 3) {
         ta.pw = B.pw.ptr;
@@ -274,16 +310,15 @@ static int get_plan(gs_ctx* c, const gs_params& p, const BatchTune& tu, int kind
             nblocks2 = v.n_cu * triplet3_occupancy(ta2, nb, fp64, weighted);
         }
     }
-    const int occ = kind == 3 ? triplet3_occupancy(ta1, nb, fp64, weighted)
-                              : std::max(1, pair2_occupancy(nb, nm, 1, fp64, rsd, weighted, p.log_bins != 0, true));
+    const int occ = kind == 3 ? triplet3_occupancy(ta1, nb, fp64, weighted) : pair_waves / (pair_wg / kWave);
     const int nblocks = kind == 3 ? std::max(1, (int)std::min<int64_t>((int64_t)v.n_cu * occ, std::max<int64_t>(n, 1)))
-                                  : v.n_cu * occ;
+                                  : (v.n_cu * occ + 7) / 8 * 8;
     if (kind == 3) ta1.batch = triplet_batch(n, nblocks);
 
     // capture: clear, count sort into cells, scans, scatter, row chunks, pair or triplet kernel
     e = hipStreamBeginCapture(v.stream, hipStreamCaptureModeThreadLocal);
     if (e == hipSuccess) e = launch_fill_u32(B.count.ptr, cells + 1, 0, v.stream);
-    if (e == hipSuccess) e = launch_fill_u32(B.queue.ptr, 32, 0, v.stream);
+    if (e == hipSuccess) e = launch_fill_u32(B.queue.ptr, 32 + 64 * kQueuePad, 0, v.stream);
     if (e == hipSuccess && nblocks2 > 0) e = launch_fill_u32(B.ovf.ptr, 1, 0, v.stream);
     if (e == hipSuccess && kind == 3) e = launch_fill_u32(B.ovf.ptr + n + 1, 2, 0, v.stream);
     if (e == hipSuccess) e = launch_fill_u32(B.out.ptr, (int64_t)nout * 2, 0, v.stream);
@@ -297,9 +332,14 @@ static int get_plan(gs_ctx* c, const gs_params& p, const BatchTune& tu, int kind
                              B.count.ptr, B.pw.ptr, B.ws.ptr, B.pl.ptr, B.flags.ptr, B.orig.ptr, v.stream);
     if (kind == 2) {
         if (e == hipSuccess)
-            e = launch_row_chunks_b(B.cell_start.ptr, d_reg, a.row_base, nreg, (int)rows_tot, B.nch.ptr, v.stream);
+            e = launch_row_chunks_b(B.cell_start.ptr, d_reg, d_row_base, nreg, (int)rows_tot, q.group, B.nch.ptr, v.stream);
         if (e == hipSuccess) e = exclusive_scan(B.nch.ptr, B.row_chunk.ptr, rows_tot + 1, B.scan_tmp.ptr, v.stream);
-        if (e == hipSuccess) e = launch_pair2(a, nb, nm, fp64, rsd, weighted, p.log_bins != 0, nblocks, kWG, v.stream);
+        if (e == hipSuccess)
+            e = launch_chunks(B.row_chunk.ptr, (int)rows_tot, B.cell_start.ptr, 0, d_reg, d_row_base, nreg, q.group,
+                              nchunk, B.chunks.ptr, v.stream);
+        if (e == hipSuccess) e = launch_pair2(a, var, nblocks, pair_wg, v.stream);
+        if (e == hipSuccess)
+            e = launch_pair_reduce(a.out_cnt, a.copies, nreg, nbt, nm, weighted, B.out.ptr, v.stream);
     } else if (e == hipSuccess && n > 0) {
         e = launch_triplet3(ta1, nb, fp64, weighted, nblocks, v.stream);
         if (e == hipSuccess && nblocks2 > 0) e = launch_triplet3(ta2, nb, fp64, weighted, nblocks2, v.stream);

@@ -223,23 +223,23 @@ __global__ __launch_bounds__(256) void k_scatter(const double* __restrict__ xyz,
     }
 }
 
-// Work chunks of the pair kernel: kChunk consecutive points of one x-row of
+// Work chunks of the pair kernels: up to `group` consecutive points of one x-row of
 // cells (fixed cy, cz).  nch[r] = chunks of row r; nch[nrow] = 0.
-__global__ __launch_bounds__(256) void k_row_chunks(const int32_t* __restrict__ start, int nx, int nrow,
+__global__ __launch_bounds__(256) void k_row_chunks(const int32_t* __restrict__ start, int nx, int nrow, int group,
                                                     int32_t* __restrict__ nch)
 {
     for (int r = blockIdx.x * blockDim.x + threadIdx.x; r <= nrow; r += gridDim.x * blockDim.x) {
         int v = 0;
-        if (r < nrow) v = (start[(r + 1) * nx] - start[r * nx] + kChunk - 1) / kChunk;
+        if (r < nrow) v = (start[(r + 1) * nx] - start[r * nx] + group - 1) / group;
         nch[r] = v;
     }
 }
 
-hipError_t launch_row_chunks(const int32_t* start, int nx, int nrow, int32_t* nch, hipStream_t st)
+hipError_t launch_row_chunks(const int32_t* start, int nx, int nrow, int group, int32_t* nch, hipStream_t st)
 {
     int nblk = (nrow + 256) / 256;
     if (nblk > 65535) nblk = 65535;
-    hipLaunchKernelGGL(k_row_chunks, dim3(nblk), dim3(256), 0, st, start, nx, nrow, nch);
+    hipLaunchKernelGGL(k_row_chunks, dim3(nblk), dim3(256), 0, st, start, nx, nrow, group, nch);
     return hipGetLastError();
 }
 
@@ -349,7 +349,7 @@ __global__ __launch_bounds__(256) void k_scatter_b(const double* __restrict__ xy
 __global__ __launch_bounds__(256) void k_row_chunks_b(const int32_t* __restrict__ start,
                                                       const RegionDesc* __restrict__ reg,
                                                       const int32_t* __restrict__ row_base, int nreg, int nrow_tot,
-                                                      int32_t* __restrict__ nch)
+                                                      int group, int32_t* __restrict__ nch)
 {
     for (int r = blockIdx.x * blockDim.x + threadIdx.x; r <= nrow_tot; r += gridDim.x * blockDim.x) {
         int v = 0;
@@ -357,7 +357,7 @@ __global__ __launch_bounds__(256) void k_row_chunks_b(const int32_t* __restrict_
             const RegionDesc R = reg[region_of(row_base, nreg, r)];
             const int lr = r - R.row_base;
             const int c0 = R.cell_base + lr * R.dim[0];
-            v = (start[c0 + R.dim[0]] - start[c0] + kChunk - 1) / kChunk;
+            v = (start[c0 + R.dim[0]] - start[c0] + group - 1) / group;
         }
         nch[r] = v;
     }
@@ -404,10 +404,10 @@ hipError_t launch_scatter_b(const double* xyz, const double* w, const int32_t* b
 }
 
 hipError_t launch_row_chunks_b(const int32_t* start, const RegionDesc* reg, const int32_t* row_base, int nreg,
-                               int nrow_tot, int32_t* nch, hipStream_t st)
+                               int nrow_tot, int group, int32_t* nch, hipStream_t st)
 {
     hipLaunchKernelGGL(k_row_chunks_b, dim3(blocks_for(nrow_tot + 1)), dim3(256), 0, st, start, reg, row_base, nreg,
-                       nrow_tot, nch);
+                       nrow_tot, group, nch);
     return hipGetLastError();
 }
 

@@ -2,6 +2,7 @@
 // implement the C ABI (api.cpp, pcf3.cpp, pcf4.cpp, adjoint.cpp, batched.cpp).
 #pragma once
 
+#include <algorithm>
 #include <cstdarg>
 #include <string>
 #include <vector>
@@ -61,6 +62,7 @@ struct GsBatch {
     DevBuf<double4> pw;
     DevBuf<double> ws;                   // sorted raw weights
     DevBuf<float4> pl;
+    DevBuf<int4> chunks;                 // pair kernel: chunk descriptors
     DevBuf<uint32_t> flags;
     DevBuf<unsigned long long> out;
     DevBuf<double> xyz, w;               // the batch's catalogue, input order
@@ -125,8 +127,10 @@ int ctx_set_device(gs_ctx* c);
 int ctx_upload(gs_ctx* c, const double* xyz, const double* w, const int32_t* buf, int64_t n);
 double round11(double h);
 int ctx_build_grid(gs_ctx* c, double rmax, int m, int sx, double* h_out);
-// device buffers of a grid build (sizes: cell_of, pw, pl, flags, orig n; cell_start, fill, chunk_nc,
-// chunk_off ncell + 1; scan_tmp scan_scratch_size(ncell + 1))
+// row chunks of kChunk points of the context's grid for the adjoint kernels: view().row_chunk, view().n_chunks
+int ctx_row_chunks(gs_ctx* c);
+// device buffers of a grid build (sizes: cell_of, pw, ws, pl, flags, orig n; cell_start, fill ncell + 1;
+// scan_tmp scan_scratch_size(ncell + 1)) and of its chunks (chunk_nc, chunk_off rows + 1; chunks max_chunks)
 struct GridBufs {
     int32_t *cell_of, *cell_start, *fill, *chunk_nc, *chunk_off, *scan_tmp;
     double4* pw;
@@ -134,13 +138,41 @@ struct GridBufs {
     float4* pl;
     uint32_t* flags;
     int32_t* orig;
+    int4* chunks;
 };
 int grid_build_raw(const double* xyz, const double* w, const int32_t* buf, int64_t n, int64_t n_data,
                    const double* bbox, double h, int sx, const GridBufs& b, int64_t max_cells, GridDesc* g_out,
-                   int32_t* nch, hipStream_t st);
-int pair2_shape(int nb, int nm, bool fp64, bool weighted, bool logb, int* reps, int* wg, int* waves);
+                   hipStream_t st);
+// row chunks of `group` points and their descriptors; their number is left at b.chunk_off[rows]
+hipError_t pair_chunks_raw(const GridDesc& g, int64_t n, int group, const GridBufs& b, hipStream_t st);
+// most chunks of `group` points that n points in nrow x-rows can make
+inline int64_t max_chunks(int64_t n, int64_t nrow, int group) { return n / group + std::min(n, nrow) + 1; }
+
+// Grid and work decomposition of the pair kernel for a catalogue.
+struct PairGrid {
+    int m = 1, sx = 1, group = 64;      // cells per rmax (y/z), x cells per cell, points per chunk
+    double h = 0;                       // y/z cell edge
+    int mst = 1;                        // ceil(rmax / h)
+    int cap_cells = 0;                  // a chunk spans at most cap_cells + 1 cells in x
+    double ext = 0;                     // bound on a chunk point's distance from its reference point, per axis
+    double cost = 0, tiles = 0;         // modelled VALU cycles per point, candidate tiles per chunk
+};
+PairGrid pair_grid(int64_t n, const double* bbox, double rmax, int cell_div, int64_t max_cells);
+// the chunk size (and the fields that follow from it) for given cells h, h / sx, at `dens` points per unit
+// volume in rows of length len_x
+void pair_group(PairGrid& q, double dens, double len_x, double rmax);
+// binning constants of the pair kernel on that grid
+int fill_pair_bins(const gs_params& p, const PairGrid& q, double xmax, double wmax_d, double wmax_r, BinDesc& B);
+// Launch shape of the pair kernel.
+struct PairShape {
+    int planes = 1, reps = 1, wg = kWG, waves = 0;  // histogram planes and replicas, threads, waves per CU
+};
+int pair2_shape(const PairVariant& v, PairShape* out);
+// log2 of the work items per chunk for n points on that grid
+int pair_lg_parts(int64_t n, const PairGrid& q);
+hipError_t pair_launch(PairArgs& a, const PairVariant& var, const PairShape& shape, const PairGrid& q, int64_t n,
+                       int n_cu, hipStream_t st);
 double choose_h_bbox(const double* bbox, double rmax, int m, int64_t max_cells, int sx);
-int pair_cell_div(int64_t n, const double* bbox, double rmax);
 int pair_cell_sx();
 int apex_cell_sx();
 void combine2(const unsigned long long* h_out, int nb, int nm, const BinDesc& B, bool weighted, long double Wd,

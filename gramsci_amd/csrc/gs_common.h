@@ -10,7 +10,9 @@ namespace gs {
 constexpr int kMaxBins = 127;   // int8 bin storage in the reference (node_module.F90:7)
 constexpr int kWG = 256;        // work-group size of the counting kernels
 constexpr int kWave = 64;       // CDNA wavefront
-constexpr int kChunk = 64;      // points per work item of the pair kernel (one per lane)
+constexpr int kChunk = 64;      // points per work item of the adjoint kernels (one per lane)
+
+constexpr int kQueuePad = 64;   // ints between the pair kernel's work counters (a cache line or more each)
 
 // Cell grid over the catalogue's bounding box.  Points are stored sorted by
 // cell id = (cz*ny + cy)*nx + cx (x fastest), so one x-row of cells is one
@@ -43,6 +45,11 @@ struct BinDesc {
     float   ua, ub;                // approximate bin: u = f(s)*ua + ub, f = sqrt (linear) or log2 (log)
     float   ms32;                  // mu_scale in FP32
     float   mu_ew, mu_em, mu_c;    // mu guard: dt = ms*(mu_ew/|sep| + mu_em/|mid| + mu_c)
+    // mu guard of the pair kernel (fill_pair_bins): the error of t is at most k0 + k1 q + k2 q^2 with
+    // k1 = mu_k1a Sx + mu_k1b (2 rho + 3 mu_ab), k2 = mu_k2a + mu_k2b Sx^2, Sx = 2 rho + mu_ab and rho
+    // the distance of the chunk's reference point from the origin
+    float   mu_k0, mu_k1a, mu_k1b, mu_k2a, mu_k2b, mu_ab;
+    int32_t wide;                  // the FP32 guard bands are too wide for the bin table
     // weighted fixed point.  Pairs: each point's weight is scaled by 2^fx_sd (data) or 2^fx_sr
     // (randoms), so that every scaled weight of its class is below 2^26, and a pair contributes
     // q = rint(w_i' * w_j') < 2^52: the DD, DR and RR sums carry the scales 2^(2 fx_sd),

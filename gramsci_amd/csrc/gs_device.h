@@ -15,6 +15,14 @@ __device__ __forceinline__ void glb_add128(unsigned long long* slot, unsigned lo
     if (hi) atomicAdd(slot + 1, hi);
 }
 
+// (lo, hi) += (l, h) as 128-bit numbers
+__device__ __forceinline__ void add128(unsigned long long& lo, unsigned long long& hi, unsigned long long l,
+                                       unsigned long long h)
+{
+    lo += l;
+    hi += h + (lo < l ? 1ull : 0ull);
+}
+
 // s = (bx-ax)^2 + (by-ay)^2 + (bz-az)^2 in FP64, evaluated left to right with
 // no contraction, as the reference forms it (kdtree2.F90:1689, gramsci.F90:1532).
 __device__ __forceinline__ double exact_s(double ax, double ay, double az, double bx, double by, double bz)
@@ -178,6 +186,54 @@ __device__ __forceinline__ int next_item(int32_t* queue, int n, int xcd, int& tr
     }
     return -1;
 }
+
+// Work items [0, n) in 64 segments, 8 per XCD, each with a counter on a cache line of its own (device-wide
+// atomics on one line run one after another, about 40 ns each: measured).  A wave's first item is its own
+// slot of its home segment, taken without an atomic; later ones come from the segment's counter, and when
+// that is used up from the next segment that has items left, found with one load of all counters.
+struct ItemQueue {
+    int32_t* counters;      // [64], kQueuePad apart, zero before the launch
+    int n;                  // items
+    int nwv;                // waves per work-group
+    int seg;                // the segment this wave takes items from
+    bool first;
+
+    __device__ __forceinline__ ItemQueue(int32_t* c, int items, int waves)
+        : counters(c), n(items), nwv(waves), seg((int)(((blockIdx.x & 7) << 3) | ((blockIdx.x >> 3) & 7))), first(true)
+    {
+    }
+    __device__ __forceinline__ int lo(int s) const { return (int)(((long long)n * s) >> 6); }
+    // waves whose home is segment s: those of the work-groups b with b mod 64 = f
+    __device__ __forceinline__ int slots(int s) const
+    {
+        const int f = (s >> 3) | ((s & 7) << 3), g = (int)gridDim.x;
+        return f < g ? (((g - 1 - f) >> 6) + 1) * nwv : 0;
+    }
+    // the next item of wave wv (uniform), -1 at the end; called by the whole wave
+    __device__ __forceinline__ int next(int lane, int wv)
+    {
+        if (first) {
+            first = false;
+            const int k = lo(seg) + (int)(blockIdx.x >> 6) * nwv + wv;
+            if (k < lo(seg + 1)) return k;
+        }
+        while (true) {
+            if (lo(seg + 1) - lo(seg) > slots(seg)) {
+                int k = 0;
+                if (lane == 0) k = atomicAdd(&counters[seg * kQueuePad], 1);
+                k = lo(seg) + slots(seg) + __builtin_amdgcn_readfirstlane(k);
+                if (k < lo(seg + 1)) return k;
+            }
+            const int used = __hip_atomic_load(&counters[lane * kQueuePad], __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT);
+            const unsigned long long m = __ballot(used < lo(lane + 1) - lo(lane) - slots(lane));
+            if (!m) return -1;
+            // the first such segment after this one, cyclically: the own XCD's come first
+            const int sh = (seg + 1) & 63;
+            const unsigned long long rot = sh ? (m >> sh) | (m << (64 - sh)) : m;
+            seg = (sh + (int)__builtin_ctzll(rot)) & 63;
+        }
+    }
+};
 
 }  // namespace dev
 }  // namespace gs

@@ -21,7 +21,7 @@ int64_t scan_scratch_size(int64_t n);
 hipError_t launch_scatter(const double* xyz, const double* w, const int32_t* buf, int64_t n, int64_t n_data,
                           const GridDesc& g, const int32_t* cell_of, const int32_t* start, int32_t* fill,
                           double4* pw, double* ws, float4* pl, uint32_t* flags, int32_t* orig, hipStream_t st);
-hipError_t launch_row_chunks(const int32_t* start, int nx, int nrow, int32_t* nch, hipStream_t st);
+hipError_t launch_row_chunks(const int32_t* start, int nx, int nrow, int group, int32_t* nch, hipStream_t st);
 
 // batched regions (grid.hip)
 hipError_t launch_fill_u32(void* p, int64_t n, uint32_t v, hipStream_t st);
@@ -33,7 +33,7 @@ hipError_t launch_scatter_b(const double* xyz, const double* w, const int32_t* b
                             int32_t* fill, double4* pw, double* ws, float4* pl, uint32_t* flags, int32_t* orig,
                             hipStream_t st);
 hipError_t launch_row_chunks_b(const int32_t* start, const RegionDesc* reg, const int32_t* row_base, int nreg,
-                               int nrow_tot, int32_t* nch, hipStream_t st);
+                               int nrow_tot, int group, int32_t* nch, hipStream_t st);
 
 // domain decomposition (decompose.hip)
 hipError_t launch_region_box(const float* xyz, const int32_t* reg, int64_t n, int nreg, int32_t* keys, hipStream_t st);
@@ -44,29 +44,46 @@ hipError_t launch_region_scatter(const float* xyz, int64_t n, const float* box, 
 // Arguments of the persistent 2PCF pair kernel (pair2.hip).
 struct PairArgs {
     const double4* pw;          // sorted points: x, y, z, raw weight
-    const double* ws;           // sorted raw weights alone (the weighted register tile reads 8 B per entry)
-    const float4* pl;           // sorted: cell-local FP32 x, y, z and the cell x index
+    const float4* pl;           // sorted: .w the cell x index
     const uint32_t* flags;      // sorted: bit0 random, bit1 never-apex
     const int32_t* cell_start;  // ncell+1
-    const int32_t* row_chunk;   // nrow+1: first work chunk of each x-row of cells
+    const int4* chunks;         // chunk descriptors (launch_chunks)
     const Row* rows;            // half stencil
     const BinDesc* bins;        // device copy
-    int32_t* queue;             // 8 work counters (one per XCD segment), zeroed before launch
-    unsigned long long* out_cnt;    // [3][nb][nm]
-    unsigned long long* out_w;      // [3][nb][nm][2] 128-bit fixed point (lo, hi)
+    int32_t* queue;             // 64 work counters (dev::ItemQueue), zeroed before launch
+    unsigned long long* out_cnt;    // [2][3][nb][nm]: plane 0 counts for both directions, plane 1 for one
+    unsigned long long* out_w;      // [2][3][nb][nm][2] 128-bit fixed point (lo, hi)
     unsigned long long* out_stats;  // [0] candidates, [1] rechecks, [2] overflow pairs
-    GridDesc g;
+    int64_t copy_stride;        // words between the copies of the outputs (pair_copy_words)
+    int32_t copies;             // power of two <= 64; work-group b adds to copy b mod copies
     int32_t nrows;
-    int32_t n_chunks;
-    int32_t reps;               // LDS histogram replicas (power of two <= 32)
-    int32_t mirror;             // (r, mu) with no buffer points: one update per unordered pair
-    // batched regions (nreg > 0): per-region grids; each wave keeps a private
-    // histogram tagged with its current region; n_chunks is read from n_chunks_dev
-    const RegionDesc* regions;
-    const int32_t* row_base;    // nreg+1 first global x-row per region
+    GridDesc g;
     const int32_t* n_chunks_dev;
+    int32_t group;              // points per chunk: 16, 32 or 64
+    int32_t lg_parts;           // log2 of the work items per chunk
+    float cap_cells;            // largest extent of a chunk in x cells, less one
+    int32_t reps;               // LDS histogram replicas (power of two <= 32)
+    int32_t planes;             // with buffer points: 2 if the LDS histogram has a plane per direction count
+    // batched regions (nreg > 0): per-region grids and outputs; each wave keeps a private
+    // histogram of its current region
+    const RegionDesc* regions;
     int32_t nreg;
-    int32_t pad2;
+};
+
+// One copy of the pair kernel's outputs: [nreg][2][nbt] counts, [nreg][2][nbt][2] sums, 4 statistics.
+inline int64_t pair_copy_words(int64_t nreg, int64_t nbt) { return 6 * nreg * nbt + 4; }
+// Copies of the outputs: as many as fit 1 MiB, at most 64.
+inline int pair_copies(int64_t nreg, int64_t nbt)
+{
+    int c = 1;
+    while (c < 64 && 2 * c * pair_copy_words(nreg, nbt) <= 131072) c *= 2;
+    return c;
+}
+
+// The pair kernel's variant: histogram, precision, unit or given weights, bins, buffer points or none.
+struct PairVariant {
+    int nb, nm;
+    bool fp64, weighted, logb, buf;
 };
 
 // Arguments of the persistent 3PCF triplet kernel (triplet3.hip).
@@ -207,12 +224,20 @@ hipError_t launch_adj_partials(const double* G, const double* w, int64_t n, int6
 hipError_t launch_adj_finish(const double* G, int64_t n, int64_t n_data, double s_d, double s_r, double inv_wd,
                              double inv_wr, double* out, hipStream_t st);
 
+// largest dynamic LDS of the pair kernel (160 KiB less its static part)
+constexpr size_t kPairLdsMax = 160 * 1024 - 64;
 // Dynamic LDS bytes of the pair kernel for these parameters and work-group size wg (a multiple of 64, <= 1024).
-size_t pair2_lds_bytes(int nb, int nm, int reps, bool fp64, bool weighted, bool batched = false, int wg = kWG);
-hipError_t launch_pair2(const PairArgs& a, int nb, int nm, bool fp64, bool rsd, bool weighted, bool logb,
-                        int nblocks, int wg, hipStream_t st);
+size_t pair2_lds_bytes(int nb, int nm, int planes, int reps, bool weighted, bool batched, int wg);
+hipError_t launch_pair2(const PairArgs& a, const PairVariant& v, int nblocks, int wg, hipStream_t st);
+// copies -> [nreg][nbt] counts and [nreg][nbt][2] sums over ordered pairs, 4 statistics
+hipError_t launch_pair_reduce(const unsigned long long* in, int copies, int nreg, int nbt, int nm, bool weighted,
+                              unsigned long long* out, hipStream_t st);
 // Work-groups of wg threads per CU the pair kernel can keep resident (0 if it cannot run).
-int pair2_occupancy(int nb, int nm, int reps, bool fp64, bool rsd, bool weighted, bool logb, bool batched = false,
-                    int wg = kWG);
+int pair2_occupancy(const PairVariant& v, int planes, int reps, bool batched, int wg);
+// Chunk descriptors {first point, points, x-row in its region, region} of the row chunks row_chunk[nrow + 1]
+// (regions and row_base for a batch; else one grid with nx cells per row); at most max_chunks of them.
+hipError_t launch_chunks(const int32_t* row_chunk, int nrow, const int32_t* cell_start, int nx,
+                         const RegionDesc* regions, const int32_t* row_base, int nreg, int group, int64_t max_chunks,
+                         int4* out, hipStream_t st);
 
 }  // namespace gs

@@ -8,7 +8,7 @@
 //
 // Limits: at most kNoAllocMaxPoints points and kNoAllocMaxCells grid cells
 // (the cell edge is widened until the grid fits).  Each GPU that runs the
-// library holds the array (about 54 MB) until the process ends.  Every call on
+// library holds the array (about 66 MB) until the process ends.  Every call on
 // a GPU uses that GPU's one array: calls that overlap on one GPU race.
 #include <cmath>
 #include <cstring>
@@ -41,10 +41,13 @@ constexpr size_t kOffFill = kOffCellStart + al((kNoAllocMaxCells + 1) * 4);
 constexpr size_t kOffChunkNc = kOffFill + al((kNoAllocMaxCells + 1) * 4);
 constexpr size_t kOffChunkOff = kOffChunkNc + al((kNoAllocMaxCells + 1) * 4);
 constexpr size_t kOffScan = kOffChunkOff + al((kNoAllocMaxCells + 1) * 4);
-constexpr size_t kOffParams = kOffScan + al(kScanTmpInts * 4);
+constexpr size_t kOffChunks = kOffScan + al(kScanTmpInts * 4);
+// chunk descriptors: at most n / 16 + n + 1
+constexpr size_t kOffParams = kOffChunks + al((kNoAllocMaxPoints / 16 + kNoAllocMaxPoints + 1) * sizeof(int4));
 constexpr size_t kOffOut = kOffParams + al(sizeof(BinDesc) + 16 + kMaxRows * sizeof(Row));
-constexpr size_t kOffQueue = kOffOut + al((3 * kMaxHist + 4) * 8);
-constexpr size_t kOffPart = kOffQueue + al(8 * 4);
+// outputs: the copies (pair_copies: one, or at most 131,072 words) and their sum
+constexpr size_t kOffQueue = kOffOut + al((9 * kMaxHist + 8 + 131072) * 8);
+constexpr size_t kOffPart = kOffQueue + al(64 * kQueuePad * 4);
 constexpr size_t kOffWpart = kOffPart + al(kRedBlocks * 6 * 8);
 constexpr size_t kNoAllocBytes = kOffWpart + al((kRedBlocks * 4 + 2) * 8);
 
@@ -153,27 +156,25 @@ extern "C" int gs_count_2pcf_noalloc(gs_ctx* c, const gs_params* p, const double
 
     // ---- grid (as gs_count_2pcf, with the cell edge widened to fit kNoAllocMaxCells)
     const int nb = p->nbins, nm = p->nmu;
-    const bool rsd = nm >= 2, fp64 = p->precision == GS_FP64, weighted = d_w != nullptr;
+    const bool weighted = d_w != nullptr;
     const int nbt = 3 * nb * nm;
-    const int m = p->cell_div > 0 ? p->cell_div : pair_cell_div(n, bbox, p->rmax);
-    const int sx = pair_cell_sx();
-    const double h = choose_h_bbox(bbox, p->rmax, m, kNoAllocMaxCells, sx);
-    const int mst = (int)std::ceil(p->rmax / h - 1e-12);
-    std::vector<Row> rows = half_stencil(h, h / sx, p->rmax, mst);
+    const PairGrid q = pair_grid(n, bbox, p->rmax, p->cell_div, kNoAllocMaxCells);
+    std::vector<Row> rows = half_stencil(q.h, q.h / q.sx, p->rmax, q.mst);
     if ((int)rows.size() > kMaxRows) return fail(GS_ELIMIT, "stencil too large");
     GridBufs gb{(int32_t*)(base + kOffCellOf), (int32_t*)(base + kOffCellStart), (int32_t*)(base + kOffFill),
                 (int32_t*)(base + kOffChunkNc), (int32_t*)(base + kOffChunkOff), (int32_t*)(base + kOffScan),
                 (double4*)(base + kOffPw), (double*)(base + kOffWs), (float4*)(base + kOffPl),
-                (uint32_t*)(base + kOffFlags), (int32_t*)(base + kOffOrig)};
+                (uint32_t*)(base + kOffFlags), (int32_t*)(base + kOffOrig), (int4*)(base + kOffChunks)};
     (void)hipEventRecord(v.ev[0], s);
     GridDesc g{};
-    int32_t n_chunks = 0;
     if (n > 0) {
         int64_t ncell = 1;
-        for (int k = 0; k < 3; ++k) ncell *= (int64_t)std::floor((bbox[3 + k] - bbox[k]) / (k == 0 ? h / sx : h)) + 1;
+        for (int k = 0; k < 3; ++k) ncell *= (int64_t)std::floor((bbox[3 + k] - bbox[k]) / (k == 0 ? q.h / q.sx : q.h)) + 1;
         if (scan_scratch_size(ncell + 1) > kScanTmpInts) return fail(GS_ELIMIT, "scan scratch too small");
-        if ((rc = grid_build_raw(d_xyz, d_w, d_buf, n, n_data, bbox, h, sx, gb, kNoAllocMaxCells, &g, &n_chunks, s)))
+        if ((rc = grid_build_raw(d_xyz, d_w, d_buf, n, n_data, bbox, q.h, q.sx, gb, kNoAllocMaxCells, &g, s)))
             return rc;
+        e = pair_chunks_raw(g, n, q.group, gb, s);
+        if (e != hipSuccess) return hip_fail(e, "row chunks");
     }
     (void)hipEventRecord(v.ev[1], s);
 
@@ -181,52 +182,52 @@ extern "C" int gs_count_2pcf_noalloc(gs_ctx* c, const gs_params* p, const double
     double xmax = 0;
     for (int k = 0; k < 6; ++k) xmax = std::max(xmax, std::fabs(bbox[k]));
     BinDesc B;
-    if ((rc = fill_bins(*p, (mst + 1) * h, xmax, wmax_d, wmax_r, B))) return rc;
-    int reps = 1, wg = kWG, best_waves = 0;
-    if ((rc = pair2_shape(nb, nm, fp64, weighted, p->log_bins != 0, &reps, &wg, &best_waves))) return rc;
+    if ((rc = fill_pair_bins(*p, q, xmax, wmax_d, wmax_r, B))) return rc;
+    const PairVariant var{nb, nm, p->precision == GS_FP64 || B.wide, weighted, p->log_bins != 0, d_buf != nullptr};
+    PairShape shape;
+    if ((rc = pair2_shape(var, &shape))) return rc;
     unsigned char* dB = base + kOffParams;
     Row* dRows = (Row*)(dB + ((sizeof(BinDesc) + 15) / 16) * 16);
     unsigned long long* out = (unsigned long long*)(base + kOffOut);
     int32_t* queue = (int32_t*)(base + kOffQueue);
-    const size_t nout = (size_t)3 * nbt + 4;
+    const int copies = pair_copies(1, nbt);
+    const size_t nwork = (size_t)copies * pair_copy_words(1, nbt), nout = (size_t)3 * nbt + 4;
     e = hipMemcpyAsync(dB, &B, sizeof(B), hipMemcpyHostToDevice, s);
     if (e == hipSuccess && !rows.empty())
         e = hipMemcpyAsync(dRows, rows.data(), rows.size() * sizeof(Row), hipMemcpyHostToDevice, s);
     // the array keeps the previous call's contents: clear what starts at zero (with fill kernels)
-    if (e == hipSuccess) e = launch_fill_u32(out, (int64_t)nout * 2, 0u, s);
-    if (e == hipSuccess) e = launch_fill_u32(queue, 8, 0u, s);
+    if (e == hipSuccess) e = launch_fill_u32(out, (int64_t)nwork * 2, 0u, s);
+    if (e == hipSuccess) e = launch_fill_u32(queue, 64 * kQueuePad, 0u, s);
     if (e != hipSuccess) return hip_fail(e, "parameter upload");
 
     PairArgs a{};
     a.pw = gb.pw;
-    a.ws = gb.ws;
     a.pl = gb.pl;
     a.flags = gb.flags;
     a.cell_start = gb.cell_start;
-    a.row_chunk = gb.chunk_off;
+    a.chunks = gb.chunks;
     a.rows = dRows;
     a.bins = (const BinDesc*)dB;
     a.queue = queue;
     a.out_cnt = out;
-    a.out_w = out + nbt;
-    a.out_stats = out + 3 * nbt;
+    a.out_w = out + 2 * nbt;
+    a.out_stats = out + 6 * nbt;
+    a.copies = copies;
+    a.copy_stride = pair_copy_words(1, nbt);
     a.g = g;
-    a.g.m = mst;
+    a.g.m = q.mst;
     a.nrows = (int)rows.size();
-    a.n_chunks = n_chunks;
-    a.reps = reps;
-    a.mirror = (rsd && !d_buf) ? 1 : 0;
-    const int occ = best_waves / (wg / kWave);
-    int nblocks = v.n_cu * occ;
-    if (nblocks > n_chunks) nblocks = std::max(n_chunks, 1);
+    a.n_chunks_dev = gb.chunk_off + (size_t)g.dim[1] * g.dim[2];
     (void)hipEventRecord(v.ev[2], s);
-    if (n_chunks > 0) {
-        e = launch_pair2(a, nb, nm, fp64, rsd, weighted, p->log_bins != 0, nblocks, wg, s);
+    if (n > 0) {
+        e = pair_launch(a, var, shape, q, n, v.n_cu, s);
         if (e != hipSuccess) return hip_fail(e, "pair kernel launch");
     }
     (void)hipEventRecord(v.ev[3], s);
+    e = launch_pair_reduce(out, copies, 1, nbt, nm, weighted, out + nwork, s);
     std::vector<unsigned long long> h_out(nout);
-    e = hipMemcpyAsync(h_out.data(), out, nout * sizeof(unsigned long long), hipMemcpyDeviceToHost, s);
+    if (e == hipSuccess)
+        e = hipMemcpyAsync(h_out.data(), out + nwork, nout * sizeof(unsigned long long), hipMemcpyDeviceToHost, s);
     if (e == hipSuccess) e = hipStreamSynchronize(s);
     if (e != hipSuccess) return hip_fail(e, "pair kernel");
     combine2(h_out.data(), nb, nm, B, weighted, Wd, Wr, cnt, wsum, n2, n3, st);
@@ -237,7 +238,7 @@ extern "C" int gs_count_2pcf_noalloc(gs_ctx* c, const gs_params* p, const double
         st->ms_grid = ms_grid;
         st->ms_count = ms_count;
         st->ms_kernel_avg = ms_count;
-        st->cell_div = mst;
+        st->cell_div = q.mst;
     }
     return GS_OK;
 }

@@ -7,41 +7,73 @@
 // (theta(j->i) = -theta(i->j) exactly).
 //
 // Work decomposition.  Points are sorted by cell with x fastest, so an x-row
-// of cells (fixed cy, cz) is one contiguous range.  A work item is a chunk of
-// 64 consecutive points of one x-row, one point per lane of a wavefront.  The
-// wave walks the half stencil of x-rows (dy, dz); for each it streams the
-// contiguous range of cells [cx_first + x0, cx_last + x1] in tiles of 64
-// points: in FP32 a register tile that rotates through the wave by DPP, in
-// FP64 a wave-private LDS tile read in a rotated order.
+// of cells (fixed cy, cz) is one contiguous range.  A chunk is up to `group`
+// (16, 32 or 64) consecutive points of one x-row; a work item is one of
+// `parts` equal shares of a chunk's candidates.  The wave reads the point
+// ranges of 64 stencil rows at once (one row per lane), numbers their points
+// by a prefix sum, and takes them in tiles of 64 that run across rows, so no
+// tile but the last is partial.  Every lane holds two apexes and one tile
+// entry; the entries rotate through the wave one lane per step (DPP), and
+// group / 2 steps bring every entry to every apex: lane L holds apexes
+// a = L mod group and a ^ (group / 2) and meets entries L .. L + group/2 - 1;
+// the other lanes that hold apex a cover the remaining entries.  The pairs
+// inside the chunk are a tile of their own (steps 1 .. group/2, half the lanes
+// in the last), and the own row's candidates start after the chunk, so no pair
+// needs an index test; missing apexes and entries are points far away.
 // Waves are persistent and independent (no work-group barriers in the main
-// loop); they pull items from 8 queues, one per XCD, each covering a
+// loop); they pull items from 64 queues, 8 per XCD, each covering a
 // contiguous z-slab of the grid so that an XCD's L2 sees one slab, and steal
 // from the other queues when their own is empty.
 //
+// What bounds it: VALU issue.  The vector ALUs issue adds, multiplies, moves
+// and 32-bit logic at about 1.55 wave-instructions per CU-cycle and everything
+// else (FMA, compares, DPP moves, conversions, 3-operand integer operations) at
+// about 0.95, transcendentals at 0.49 (measured), so the pair loop is written
+// for few operations of the second kind.
+//
+// Measured (kernel time; before: one apex-tile pair of 64 points per item, a tile per stencil row, mu
+// from the midpoint with two reciprocal square roots, a u32 and two u64 atomics per update):
+//   4M points, 1.90e11 binned pairs, (r, mu), weighted:  FP32 252 -> 183 ms
+//   800k points, same bins, FP64 geometry:               142 -> 46 ms
+//   60k points, 10 linear bins, unweighted:              0.51 -> 0.08 ms
+//   9k points, (r, mu), weighted:                        0.38 -> 0.04 ms
+// The small ones were bound by the few items (150 chunks of 64 points, each walking the whole stencil) and
+// by device-wide atomics on shared lines: the queue's end, the drains and the statistics.
+//
 // Precision variants (identical counts):
-//   FP64        s = |xj-xi|^2 in FP64 exactly as the reference; bins from the
-//               exact thresholds; mu with IEEE sqrt/div.
-//   FP32 guard  d = (xj_l - xi_l) + (cx_j - cx_i) * h from cell-local FP32
-//               coordinates (h has <= 11 significant bits, so the cell offset
-//               is exact).  A pair is binned directly only when s32 lies in the
-//               bin's certain interval [ok_lo, ok_hi) and its mu is farther
-//               than a rigorous error bound from a mu edge; otherwise it is
-//               re-evaluated with the FP64 path.
+//   FP64        s = |xj-xi|^2 in FP64 exactly as the reference, bins from the
+//               exact thresholds; the mu bin from a FP64 estimate that is
+//               taken only when it is farther from a mu edge than its error
+//               bound, else with the reference's IEEE sqrt and division.
+//   FP32 guard  coordinates relative to a point of the chunk, rounded to FP32.
+//               A pair is binned directly only when s32 lies in the bin's
+//               certain interval [ok_lo, ok_hi) and its mu is farther than a
+//               rigorous error bound from a mu edge; otherwise it is
+//               queued in LDS and re-evaluated in FP64, 64 at a time.
 //
-// (r, mu) without buffer points: every pair is counted in both directions and
-// theta(j->i) = -theta(i->j) exactly, so one update at mu bin m stands for
-// both ordered pairs (m and nm-1-m) and the drain adds it to both bins.  Only
-// pairs exactly on a mu edge (where the two directions are not mirror images)
-// are added explicitly.
+// mu from squared radii: with D = 2(|xi|^2 - |xj|^2) and
+// S = |xi + xj|^2 = 2|xi|^2 + 2|xj|^2 - s, theta = mid.sep / (|mid| |sep|)
+// = (D/2) rsq(S s): one transcendental and no midpoint.  The squared radii are
+// taken relative to the chunk's reference point p (formed in FP64 as
+// (x - p).(x + p)), so that D keeps its precision far from the origin.  The
+// error bound of t = (theta + 1) mu_scale is k0 + k1 q + k2 q^2 with
+// q = rsq(S s) = 1 / (2 |mid| |sep|); see fill_bins.
 //
-// Histograms live in LDS, shared by the work-group's waves: u32 counts
-// replicated `reps` times (replica = lane % reps, one plane of nbt counts per
-// replica) to spread same-bin atomics,
-// and per bin two u64 sums of the weight product's fixed-point value split at
-// bit 32 (no carries, so no returning atomics).  A wave that has issued 2^29
-// increments drains the histogram with atomic exchanges into the global
-// 128-bit accumulators; the rest is drained when the work-group ends.
-#include <cstdlib>
+// Histograms live in LDS, shared by the work-group's waves and replicated
+// `reps` times (replica = lane % reps).  Unweighted: u32 counts.  Weighted:
+// per bin two u64 planes, lo += q mod 2^32 and hi += (q >> 32) + 2^42, where
+// q < 2^52 is the weight product in fixed point: the sum is lo + 2^32 (hi mod
+// 2^42) and the count hi >> 42 -- two LDS atomics per update, no carries and
+// no returning atomics.  A bin overflows after 2^22 increments: a wave that may
+// have issued 2^20 / (waves of the work-group) increments since it last looked
+// scans the histogram and drains the bins that hold 2^20 or more.
+//
+// Without buffer points every pair counts in both directions, so one update at
+// mu bin m stands for both ordered pairs; k_pair_reduce adds entry m to m and
+// nm-1-m (plane 0 of the outputs).  Pairs exactly on a mu edge, where the two
+// directions are not mirror images, are added explicitly (plane 1).  With
+// buffer points a pair with one apex goes to plane 1 in the apex's direction.
+#include <type_traits>
 
 #include "gs_device.h"
 #include "gs_kernels.h"
@@ -52,659 +84,681 @@ namespace {
 
 using namespace dev;
 
-struct Stats {
-    unsigned long long cand, rechk, over;
+constexpr int kOkBytes = (kMaxBins + 1) * 8;    // certain intervals, at the start of the LDS
+constexpr int kListBytes = kWave * 12;          // per wave: queue of pairs to re-evaluate, tile index list
+constexpr uint32_t kCountOne = 1u << 10;        // one count in the high word of the hi plane (bit 42)
+constexpr unsigned kRunMax = 256;               // increments after which a run ends with its tile
+
+template <class R> struct Real4;                // point in the kernel's geometry precision
+template <> struct Real4<float> { static constexpr float far = 1e18f; };
+template <> struct Real4<double> { static constexpr double far = 1e150; };
+
+// one apex of a lane
+template <class R>
+struct Apex {
+    R x, y, z;      // FP32: relative to the chunk's reference point; FP64: absolute
+    R d;            // 2 (|x|^2 - |p|^2), p the reference point
+    R c;            // 2 (|x|^2 + |p|^2)
+    double w;       // weight scaled by its class's 2^F
+    int cb;         // LDS offset of the pair's class with a data neighbour, with the lane's replica
 };
 
-// One pair's histogram update.  base = class offset + b*nm (flat bin index
-// without the mu bin); counts live at hcr[base + m], hcr = this lane's replica plane.  mirrored:
-// mr == nm-1-m (always so for the FP32 mu bins; tested after an FP64 recheck).
-// Returns the number of LDS bin increments made.
-template <bool RSD, bool W>
-__device__ __forceinline__ int accumulate(uint32_t* hcr, unsigned long long* hw, int nm,
-                                          bool mirror, int base, int m, int mr, bool mirrored, int ci, int cj,
-                                          double x, unsigned long long* out_cnt, unsigned long long* out_w)
+// a lane's run of histogram increments to one bin, merged in registers
+struct Run {
+    int k;                  // LDS offset of the bin
+    uint32_t lo, hi, cn;    // sum of q (split at bit 32), count * kCountOne
+};
+
+__device__ __forceinline__ float rsq(float x) { return __builtin_amdgcn_rsqf(x); }
+__device__ __forceinline__ double rsq(double x) { return __builtin_amdgcn_rsq(x); }
+__device__ __forceinline__ float fract(float x) { return __builtin_amdgcn_fractf(x); }
+__device__ __forceinline__ double fract(double x) { return __builtin_amdgcn_fract(x); }
+
+// v truncated to an unsigned integer, 0 for a negative v (the conversion saturates)
+__device__ __forceinline__ int cvt_sat(float v)
 {
-    uint32_t qlo = 0, qhi = 0;
-    if constexpr (W) {
-        const unsigned long long q = quantise_rn(x);
-        qlo = (uint32_t)q;
-        qhi = (uint32_t)(q >> 32);
-    }
-    auto add = [&](int k, uint32_t c) {
-        atomicAdd(&hcr[k], c);
-        if constexpr (W) {
-            atomicAdd(&hw[2 * k], (unsigned long long)qlo * c);
-            atomicAdd(&hw[2 * k + 1], (unsigned long long)qhi * c);
-        }
-    };
-    if constexpr (!RSD) {
-        const int c = ci + cj;
-        if (c) add(base, (uint32_t)c);
-        return c;
-    } else if (mirror && mirrored) {
-        add(base + m, 1u);    // mirror-implied: stands for i->j at m and j->i at nm-1-m
-        return 1;
-    } else if (mirror) {
-        // a pair exactly on a mu edge: both ordered pairs explicitly, straight to global memory (rare)
-        const unsigned long long L = ((unsigned long long)qhi << 32) + qlo;
-        atomicAdd(&out_cnt[base + m], 1ull);
-        atomicAdd(&out_cnt[base + mr], 1ull);
-        if constexpr (W) {
-            glb_add128(&out_w[2 * (base + m)], L, 0ull);
-            glb_add128(&out_w[2 * (base + mr)], L, 0ull);
-        }
-        return 0;
-    } else {
-        if (ci) add(base + m, 1u);
-        if (cj) add(base + mr, 1u);
-        return ci + cj;
-    }
+    int r;
+    asm("v_cvt_u32_f32 %0, %1" : "=v"(r) : "v"(v));
+    return r;
 }
 
-// Drains the LDS histogram into the global accumulators with atomic
-// exchanges, so any wave may do it while the others keep adding.  Called by
-// all lanes of one wave (stride 64) or of the whole work-group.
-// With `mirror`, entry (cls, b, m) also stands for (cls, b, nm-1-m).
-__device__ void drain(uint32_t* hc, unsigned long long* hw, int nbt, int nm, int reps, bool weighted, bool mirror,
-                      int t0, int stride, unsigned long long* out_cnt, unsigned long long* out_w)
+__device__ __forceinline__ int lane_int(int v, int l) { return __builtin_amdgcn_readlane(v, l); }
+__device__ __forceinline__ double lane_double(double v, int l)
 {
-    for (int k = t0; k < nbt; k += stride) {
-        const int km = mirror ? (k - k % nm) + (nm - 1 - k % nm) : k;
-        unsigned long long s = 0;
-        for (int r = 0; r < reps; ++r) s += atomicExch(&hc[k + r * nbt], 0u);
-        if (s) {
-            atomicAdd(&out_cnt[k], s);
-            if (mirror) atomicAdd(&out_cnt[km], s);
-        }
-        if (weighted) {
-            const unsigned long long lo = atomicExch(&hw[2 * k], 0ull);
-            const unsigned long long hi = atomicExch(&hw[2 * k + 1], 0ull);
-            if (lo | hi) {
-                // value = hi * 2^32 + lo as a 128-bit number
-                const unsigned long long L = (hi << 32) + lo;
-                const unsigned long long H = (hi >> 32) + (L < lo ? 1ull : 0ull);
-                glb_add128(&out_w[2 * k], L, H);
-                if (mirror) glb_add128(&out_w[2 * km], L, H);
-            }
-        }
-    }
+    const long long b = __double_as_longlong(v);
+    const int lo = lane_int((int)(b & 0xffffffffll), l), hi = lane_int((int)(b >> 32), l);
+    return __longlong_as_double(((long long)hi << 32) | (long long)(uint32_t)lo);
 }
-
 
 }  // namespace
 
-size_t pair2_lds_bytes(int nb, int nm, int reps, bool fp64, bool weighted, bool batched, int wg)
+// LDS of one histogram: bins (with a plane per direction where `planes` is 2) times replicas
+static size_t hist_bytes(size_t nbt, int planes, int reps, bool weighted)
 {
-    const size_t nbt = (size_t)3 * nb * nm;
-    const size_t copies = batched ? (size_t)(wg / kWave) : 1;   // batched: one histogram per wave
-    size_t b = 0;
-    b += ((nbt * reps * 4 * copies + 15) / 16) * 16;          // counts
-    if (weighted) b += nbt * 16 * copies;                     // split fixed-point sums
-    b += ((size_t)(kMaxBins + 1) * 8);                        // ok_lo/ok_hi as float2
-    b += ((size_t)(kMaxBins + 2) * 8 + 15) / 16 * 16;         // t64
-    const int waves = wg / kWave;
-    if (fp64) b += (size_t)waves * kWave * (24 + 8 + 4 + 4);  // LDS tile: x, y, z, w, flags, pad
-    return b;
+    return ((size_t)planes * nbt * reps * (weighted ? 16 : 4) + 15) / 16 * 16;
 }
 
-// a lane's run of histogram increments to one bin, merged in registers
-struct RunCache {
-    int ck;
-    uint32_t cc;
-    unsigned long long cq;
-};
-
-// The unweighted FP32 kernels are compiled for six waves per SIMD (at most 80 VGPRs), the occupancy
-// their LDS use allows; the weighted ones are held to fewer waves by their LDS sums anyway.
-// DUAL (weighted FP32 only): each lane also holds the chunk point 32 lanes away, and a full tile is
-// done in 32 steps of two pairs each (below).  It needs about 127 VGPRs, so it is launched only where
-// that costs no resident waves.
-template <bool FP64, bool RSD, bool W, bool LOGB, bool DUAL>
-__global__ __launch_bounds__(1024) __attribute__((amdgpu_waves_per_eu((!FP64 && !W) ? 6 : 1))) void k_pair2(PairArgs a)
+size_t pair2_lds_bytes(int nb, int nm, int planes, int reps, bool weighted, bool batched, int wg)
 {
+    const size_t nbt = (size_t)3 * nb * nm;
+    const size_t waves = (size_t)(wg / kWave);
+    return kOkBytes + hist_bytes(nbt, planes, reps, weighted) * (batched ? waves : 1) + waves * kListBytes;
+}
+
+template <bool FP64, bool RSD, bool W, bool LOGB, bool BUF>
+__global__ __launch_bounds__(1024) void k_pair2(PairArgs a)
+{
+    using R = std::conditional_t<FP64, double, float>;
     extern __shared__ __align__(16) unsigned char smem[];
     const BinDesc& B = *a.bins;
     const int nb = B.nb;
     const int nm = RSD ? B.nm : 1;
     const int nbt = 3 * nb * nm;
     const bool batched = a.nreg > 0;
-    const int reps = batched ? 1 : a.reps;
+    const int reps = a.reps;
+    const int planes = BUF ? a.planes : 1;
     const int tid = threadIdx.x;
     const int lane = tid & (kWave - 1);
-    const int wv = tid / kWave;
-    const int rep = lane & (reps - 1);
-    const bool mirror = RSD && a.mirror;
+    const int wv = __builtin_amdgcn_readfirstlane(tid / kWave);
     const int nthr = blockDim.x;        // a multiple of 64, at most 1024
-    const int copies = batched ? nthr / kWave : 1;
+    const int nwv = nthr / kWave;
 
-    unsigned char* p = smem;
-    uint32_t* hc0 = (uint32_t*)p;
-    p += ((size_t)nbt * reps * 4 * copies + 15) / 16 * 16;
-    unsigned long long* hw0 = (unsigned long long*)p;
-    if (W) p += (size_t)nbt * 16 * copies;
-    // the histogram this wave adds to: shared by the work-group, or wave-private in batched mode
-    uint32_t* hc = batched ? hc0 + (size_t)wv * nbt : hc0;
-    unsigned long long* hw = batched ? hw0 + (size_t)wv * 2 * nbt : hw0;
-    uint32_t* hcr = hc + rep * nbt;      // this lane's replica plane of the counts
-    float2* okb = (float2*)p;
-    p += (size_t)(kMaxBins + 1) * 8;
-    double* t64 = (double*)p;
-    p += ((size_t)(kMaxBins + 2) * 8 + 15) / 16 * 16;
-    // FP64: wave-private LDS tile x[64], y[64], z[64], w[64], flags[64]
-    unsigned char* tb = p + (size_t)wv * kWave * 40;
-    double* tx = (double*)tb;
-    double* ty = tx + kWave;
-    double* tz = ty + kWave;
-    double* tw = tz + kWave;
-    uint32_t* tf = (uint32_t*)(tw + kWave);
-
-    for (int k = tid; k < nbt * reps * copies; k += nthr) hc0[k] = 0;
-    if (W)
-        for (int k = tid; k < 2 * nbt * copies; k += nthr) hw0[k] = 0;
-    for (int k = tid; k < nb; k += nthr) okb[k] = make_float2(B.ok_lo[k], B.ok_hi[k]);
-    for (int k = tid; k < nb + 2; k += nthr) t64[k] = B.t64[k];
+    // LDS: certain intervals (FP64: exact thresholds), histogram (one, or one per wave in batched mode),
+    // tile index lists
+    constexpr int kB = W ? 8 : 4;       // bytes of a histogram word
+    const int nent = planes * nbt * reps;                       // words of one plane of the histogram
+    const int hsize = (int)((nent * (W ? 16 : 4) + 15) / 16 * 16);
+    unsigned char* const hist = smem + kOkBytes + (batched ? wv * hsize : 0);   // this wave's histogram
+    const int hi_off = nent * 8;        // W: the hi plane's offset from the lo plane
+    unsigned char* const lists = smem + kOkBytes + (size_t)hsize * (batched ? nwv : 1) + wv * kListBytes;
+    int2* const queue = (int2*)lists;                   // pairs to re-evaluate
+    int* const jlist = (int*)(lists + kWave * 8);       // point of each tile entry
+    {
+        uint32_t* h0 = (uint32_t*)(smem + kOkBytes);
+        const int nw = hsize / 4 * (batched ? nwv : 1);
+        for (int k = tid; k < nw; k += nthr) h0[k] = 0;
+        if constexpr (FP64) {
+            for (int k = tid; k <= nb && k <= kMaxBins; k += nthr) ((double*)smem)[k] = B.t64[k];
+        } else {
+            // entry nb (an estimate just past the last bin) is never certain
+            for (int k = tid; k <= nb; k += nthr)
+                ((float2*)smem)[k] = k < nb ? make_float2(B.ok_lo[k], B.ok_hi[k]) : make_float2(INFINITY, -INFINITY);
+        }
+    }
     __syncthreads();
 
-    const float rej_lo = B.rej_lo, rej_hi = B.rej_hi, ua = B.ua, ub = B.ub;
+    const float ua = B.ua, ub = B.ub;
+    const R rej_lo = FP64 ? (R)B.t64[0] : (R)B.rej_lo, rej_hi = FP64 ? (R)B.t64[nb + 1] : (R)B.rej_hi;
     const double t_lo = B.t64[0], t_hi = B.t64[nb + 1];
     const double ms = B.mu_scale;
-    const int nbm = nb * nm;
-    const float ms32 = B.ms32, mu_ew = B.mu_ew, mu_em = B.mu_em, mu_c = B.mu_c;
-    const float nbm1f = (float)(nb - 1), nmm1f = (float)(nm - 1);
-    // mu edges are the integers 1..nm-1 of t; with nm = 127 also 0 and 127, where the reference's
-    // int8 store of floor(t)+1 wraps (gramsci.F90:326-328), so pairs there get the FP64 recheck
-    const float e_lo = nm == 127 ? 0.0f : 1.0f, e_hi = nm == 127 ? 127.0f : nmm1f;
-    // mu error bound dt = ms * (mu_ew / |sep| + mu_em / |mid| + mu_c), with ms folded into the
-    // constants (their 4x margin dwarfs the reassociation).  In the weighted kernel, whose
-    // residency LDS limits, dt_c and ub are kept in VGPRs so that each FMA of the loop reads at
-    // most one scalar operand; elsewhere the extra VGPRs would cost residency.
-    const float dt_ew = ms32 * mu_ew, dt_em = ms32 * mu_em;
-    float dt_c = ms32 * mu_c, ubv = ub;
-    if constexpr (W) asm volatile("" : "+v"(dt_c), "+v"(ubv));
+    const R msr = (R)ms, hms = (R)(0.5 * ms);
     // fixed-point scales of data and random weights (batched: the current region's)
     int sd = B.fx_sd, sr = B.fx_sr;
-    const int nrow_all = batched ? 0 : a.g.dim[1] * a.g.dim[2];
-    const int n_chunks = batched ? *a.n_chunks_dev : a.n_chunks;
-    const float h32 = a.g.h32, hx32 = a.g.hx32;    // cell edges in y/z and in x
-    int cur_r = -1;                 // region of this wave's private histogram (batched mode)
+    const int nbm = nb * nm;
+    const int n_chunks = *a.n_chunks_dev;
+    const int n_items = n_chunks << a.lg_parts;
+    const int group = a.group, half = group >> 1;
+    const int ai = lane & (group - 1), ai2 = ai ^ half;     // the lane's apexes in the chunk
+    const int rep_off = (lane & (reps - 1)) * planes * nbt * kB;
+    const float cap = a.cap_cells;
+    int nx = a.g.dim[0], ny = a.g.dim[1], nz = a.g.dim[2], cb = 0;
+    int cur_r = batched ? -1 : 0;   // region of this wave's histogram
 
-    Stats st{0, 0, 0};
-    // FP32 weighted path: per-lane run cache of the last histogram bin.  A lane's consecutive
-    // neighbours (adjacent points of one cell, data before randoms) often fall in the same
-    // bin; their updates are merged in registers and reach the LDS histogram with one set of
-    // atomics when the bin changes, which relieves same-address LDS atomic conflicts.
-    // The run's sum is one 64-bit integer: products are below 2^52 (fx_sd, fx_sr) and a run ends
-    // after at most 33 increments, so it cannot overflow; the flush splits it at bit 32 into
-    // the two LDS halves, which keeps value = hi * 2^32 + lo.  The update is written with
-    // selects, not branches, so that no register copies are needed where paths merge.  An empty
-    // run (cc = 0) stays attached to its last bin (bin 0 at the start): flushing it adds zeros, so
-    // the flush needs no test for a missing run.
-    static_assert(!DUAL || (W && !FP64), "two apexes per lane: weighted FP32 kernels only");
-    // with DUAL each lane's second apex has a run cache of its own
-    RunCache rc0{0, 0u, 0ull}, rc1{0, 0u, 0ull};
-    auto flush_one = [&](RunCache& c) {
-        atomicAdd(&hcr[c.ck], c.cc);
+    unsigned long long n_cand = 0;
+    unsigned long long n_rechk = 0;
+    unsigned int n_over = 0;
+
+    // the work-group's copy of the outputs: [2][nbt] counts and [2][nbt][2] sums of the current region
+    const size_t copy = (size_t)(blockIdx.x & (unsigned)(a.copies - 1)) * (size_t)a.copy_stride;
+    unsigned long long* out_cnt = a.out_cnt + copy;
+    unsigned long long* out_w = a.out_w + copy;
+
+    // adds word k (of this wave's histogram) to the outputs and clears it
+    auto drain_word = [&](int k) {
+        // with buffer points and a single plane every entry is one direction of a pair: plane 1
+        const int o = k % (planes * nbt) + (BUF && planes == 1 ? nbt : 0);
         if constexpr (W) {
-            atomicAdd(&hw[2 * c.ck], c.cq & 0xffffffffull);
-            atomicAdd(&hw[2 * c.ck + 1], c.cq >> 32);
-        }
-        c.cc = 0;
-        c.cq = 0;
-    };
-    auto flush = [&]() {
-        flush_one(rc0);
-        if constexpr (DUAL) flush_one(rc1);
-    };
-    auto put = [&](RunCache& rc, int k, uint32_t c, unsigned long long q) {   // c in {1, 2}
-        const bool nw = (k != rc.ck) || (rc.cc >= 32u);
-        if (nw) flush_one(rc);
-        rc.cc = (nw ? 0u : rc.cc) + c;
-        if constexpr (W) rc.cq = (nw ? 0ull : rc.cq) + (q << (c - 1));
-        rc.ck = k;
-    };
-    unsigned long long bound = 0;   // LDS increments issued by this wave since its last drain
-    // LDS bin increments between drains, over all waves sharing the histogram, stay below 2^31,
-    // which keeps every u32 count and every split sum from overflowing
-    const unsigned long long drain_at = (1ull << 31) / (unsigned long long)(batched ? 1 : nthr / kWave);
-    const int xcd = blockIdx.x & 7;
-    int tried = 0;
-
-    while (true) {
-        int item = -1;
-        if (lane == 0) item = next_item(a.queue, n_chunks, xcd, tried);
-        item = __builtin_amdgcn_readfirstlane(item);
-        if (item < 0) break;
-
-        int nx, ny, nz, cb, row;
-        const int grow = upper_index(a.row_chunk, batched ? a.row_base[a.nreg] : nrow_all, item);
-        const int q = item - a.row_chunk[grow];
-        if (batched) {
-            const int R = upper_index(a.row_base, a.nreg, grow);
-            const RegionDesc& rd = a.regions[R];
-            nx = rd.dim[0]; ny = rd.dim[1]; nz = rd.dim[2];
-            cb = rd.cell_base;
-            row = grow - rd.row_base;
-            sd = rd.fx_shift;
-            sr = rd.fx_shift_rand;
-            if (R != cur_r) {
-                if constexpr (W) flush();
-                if (cur_r >= 0)
-                    drain(hc, hw, nbt, nm, reps, W, mirror, lane, kWave, a.out_cnt + (size_t)cur_r * nbt,
-                          a.out_w + (size_t)cur_r * 2 * nbt);
-                cur_r = R;
-                bound = 0;
+            const unsigned long long h = atomicExch((unsigned long long*)(hist + hi_off) + k, 0ull);
+            const unsigned long long l = atomicExch((unsigned long long*)hist + k, 0ull);
+            if (h | l) {
+                const unsigned long long hs = h & ((1ull << 42) - 1);
+                const unsigned long long L = (hs << 32) + l;
+                const unsigned long long H = (hs >> 32) + (L < l ? 1ull : 0ull);
+                atomicAdd(&out_cnt[o], h >> 42);
+                glb_add128(&out_w[2 * o], L, H);
             }
         } else {
-            nx = a.g.dim[0]; ny = a.g.dim[1]; nz = a.g.dim[2];
-            cb = 0;
-            row = grow;
+            const uint32_t c = atomicExch((uint32_t*)hist + k, 0u);
+            if (c) atomicAdd(&out_cnt[o], (unsigned long long)c);
+        }
+    };
+    auto drain = [&](int t0, int stride) {
+        for (int k = t0; k < nent; k += stride) drain_word(k);
+    };
+
+    Run r1{rep_off, 0u, 0u, 0u}, r2{rep_off, 0u, 0u, 0u};
+    auto flush = [&](Run& r) {
+        atomicAdd((unsigned long long*)(hist + r.k), (unsigned long long)r.lo);
+        atomicAdd((unsigned long long*)(hist + r.k + hi_off), ((unsigned long long)r.cn << 32) | r.hi);
+        r.lo = 0; r.hi = 0; r.cn = 0;
+    };
+    // one increment of the bin at LDS offset k: merged with the lane's run of that bin (a lane's
+    // consecutive neighbours often share a bin), which is written out when the bin changes.  An empty
+    // run adds zeros.
+    auto put = [&](Run& r, int k, uint32_t qlo, uint32_t qhi) {
+        if (k != r.k) {
+            flush(r);
+            r.k = k;
+        }
+        const uint32_t s = r.lo + qlo;
+        r.hi += qhi + (s < qlo ? 1u : 0u);
+        r.lo = s;
+        r.cn += kCountOne;
+    };
+
+    // Pairs that are not certain wait in LDS (apex point, neighbour) and are re-evaluated together, with the
+    // reference's arithmetic, when 64 are full or the wave changes region or ends: the loop over the
+    // pairs keeps few registers, and a recheck fills a wave instead of one lane.
+    int nq = 0;
+    auto recheck = [&]() {
+        wave_sync();
+        if (lane < nq) {
+            const int2 pr = queue[lane];
+            const double4 Pi = a.pw[pr.x], Pj = a.pw[pr.y];
+            const uint32_t fi = a.flags[pr.x], fj = a.flags[pr.y];
+            const double se = exact_s(Pi.x, Pi.y, Pi.z, Pj.x, Pj.y, Pj.z);
+            if (se > t_lo && se < t_hi) {
+                const bool ci = !(fi & 2u), cj = !(fj & 2u);
+                const int b = adjust_bin(se, bin_estimate((float)se, LOGB, ua, ub), B.t64, nb);
+                if (b == nb) {
+                    n_over += (unsigned)ci + (unsigned)cj;
+                } else {
+                    int m = 0, mr = 0;
+                    if constexpr (RSD) exact_mu(Pi.x, Pi.y, Pi.z, Pj.x, Pj.y, Pj.z, ms, nm, m, mr);
+                    unsigned long long q = 0;
+                    if constexpr (W) q = quantise_rn(ldexp(Pi.w, (fi & 1u) ? sr : sd) * ldexp(Pj.w, (fj & 1u) ? sr : sd));
+                    const int k0 = (int)((fi & 1u) + (fj & 1u)) * nbm + b * nm;
+                    auto add = [&](int k) {
+                        if constexpr (W) {
+                            unsigned long long* h = (unsigned long long*)(hist + rep_off) + k;
+                            atomicAdd(h, q & 0xffffffffull);
+                            atomicAdd(h + nent, (q >> 32) + (1ull << 42));
+                        } else {
+                            atomicAdd((uint32_t*)(hist + rep_off) + k, 1u);
+                        }
+                    };
+                    auto add_global = [&](int k) {
+                        atomicAdd(&out_cnt[nbt + k], 1ull);
+                        if constexpr (W) glb_add128(&out_w[2 * (nbt + k)], q, 0ull);
+                    };
+                    if (ci && cj && mr == nm - 1 - m && !(BUF && planes == 1)) {
+                        add(k0 + m);
+                    } else if (BUF && planes == 2 && ci != cj) {
+                        add(k0 + (ci ? m : mr) + nbt);
+                    } else {        // exactly on a mu edge (or one plane): the ordered pairs one by one
+                        if (ci) add_global(k0 + m);
+                        if (cj) add_global(k0 + mr);
+                    }
+                }
+            }
+        }
+        n_rechk += (unsigned)nq;
+        nq = 0;
+        wave_sync();
+    };
+
+    // increments this wave may have issued since it last looked at its histogram
+    unsigned long long bound = 0;
+    const unsigned long long look_at = (W ? (1ull << 20) : (1ull << 31)) / (unsigned long long)(batched ? 1 : nwv);
+    auto look = [&]() {
+        if constexpr (W) {
+            flush(r1);
+            flush(r2);
+            for (int k = lane; k < nent; k += kWave)
+                if ((((unsigned long long*)(hist + hi_off))[k] >> 42) >= (1u << 20)) drain_word(k);
+        } else {
+            drain(lane, kWave);
+        }
+        bound = 0;
+    };
+
+    ItemQueue items(a.queue, n_items, nwv);
+    while (true) {
+        const int item = items.next(lane, wv);
+        if (item < 0) break;
+        const int part = item & ((1 << a.lg_parts) - 1);
+        const int4 ch = a.chunks[item >> a.lg_parts];
+        const int row = __builtin_amdgcn_readfirstlane(ch.z);
+        if (batched) {
+            const int rg = __builtin_amdgcn_readfirstlane(ch.w);
+            if (rg != cur_r) {
+                if (nq) recheck();
+                if constexpr (W) { flush(r1); flush(r2); }
+                if (cur_r >= 0) drain(lane, kWave);
+                cur_r = rg;
+                const RegionDesc& rd = a.regions[rg];
+                nx = rd.dim[0]; ny = rd.dim[1]; nz = rd.dim[2];
+                cb = rd.cell_base;
+                sd = rd.fx_shift;
+                sr = rd.fx_shift_rand;
+                out_cnt = a.out_cnt + copy + (size_t)rg * 2 * nbt;
+                out_w = a.out_w + copy + (size_t)rg * 4 * nbt;
+                bound = 0;
+            }
         }
         const int cy = row % ny, cz = row / ny;
-        const int rs = a.cell_start[cb + row * nx], re = a.cell_start[cb + (row + 1) * nx];
-        const int i0 = rs + q * kChunk;
-        const int n_i = min(kChunk, re - i0);
-        const int i = i0 + lane;
-        const bool vi = lane < n_i;
-        const int cx_first = (int)a.pl[i0].w;
-        const int cx_last = (int)a.pl[i0 + n_i - 1].w;
+        int ib = __builtin_amdgcn_readfirstlane(ch.x);
+        const int iend = ib + __builtin_amdgcn_readfirstlane(ch.y);
 
-        double4 Pi = make_double4(0, 0, 0, 0);
-        float4 Li = make_float4(0, 0, 0, 0);
-        uint32_t fi = 2u;
-        if (vi) {
-            Pi = a.pw[i];
-            Li = a.pl[i];
-            fi = a.flags[i];
-        }
-        const int ri = fi & 1, ci = (fi & 2) ? 0 : 1;
-        // the lane's second apex: the chunk point 32 lanes away
-        const int i2 = i0 + (lane ^ 32);
-        const bool vi2 = DUAL && (lane ^ 32) < n_i;
-        double4 Pi2 = make_double4(0, 0, 0, 0);
-        float4 Li2 = make_float4(0, 0, 0, 0);
-        uint32_t fi2 = 2u;
-        if (vi2) {
-            Pi2 = a.pw[i2];
-            Li2 = a.pl[i2];
-            fi2 = a.flags[i2];
-        }
-        const int ri2 = fi2 & 1, ci2 = (fi2 & 2) ? 0 : 1;
-        // a chunk of buffer points only (never apexes) gains nothing from a tile of buffer points only
-        const bool chunk_buf = __ballot(ci != 0) == 0;
-        // the apex weight scaled by its class's 2^F (exact): a pair's product w_i' w_j' then carries
-        // the scale of its class (DD, DR or RR)
-        const double wis = ldexp(Pi.w, ri ? sr : sd);
-        const float ax32 = (float)Pi.x, ay32 = (float)Pi.y, az32 = (float)Pi.z;   // absolute, for mu
-        const double wis2 = DUAL ? ldexp(Pi2.w, ri2 ? sr : sd) : 0.0;
-        const float ax2 = (float)Pi2.x, ay2 = (float)Pi2.y, az2 = (float)Pi2.z;
-        const int cb02 = ri2 ? nbm : 0;
-        // histogram class offsets of this lane's pairs with a data / a random neighbour
-        const int cb0 = ri ? nbm : 0, cb1 = cb0 + nbm;
+        // The FP32 error bounds hold for chunks of at most cap + 1 cells in x: a longer one (few points
+        // in a long row) is taken in pieces [ib, ib + n_i).
+        int n_i;
+        for (; ib < iend; ib += n_i) {
+            const float cxl = ib + ai < iend ? a.pl[ib + ai].w : INFINITY;
+            const int cx_first = (int)__int_as_float(lane_int(__float_as_int(cxl), 0));
+            n_i = __popcll(__ballot(lane < group && cxl - (float)cx_first <= cap));
+            const int cx_last = (int)__int_as_float(lane_int(__float_as_int(cxl), n_i - 1));
 
-        for (int r = 0; r < a.nrows; ++r) {
-            const Row rw = a.rows[r];
-            const int by = cy + rw.dy, bz = cz + rw.dz;
-            if (by < 0 || by >= ny || bz < 0 || bz >= nz) continue;
-            const int bx0 = max(cx_first + rw.x0, 0), bx1 = min(cx_last + rw.x1, nx - 1);
-            if (bx0 > bx1) continue;
-            const bool self = (rw.dy == 0 && rw.dz == 0);
-            const int rb = cb + (bz * ny + by) * nx;
-            int js = a.cell_start[rb + bx0];
-            const int je = a.cell_start[rb + bx1 + 1];
-            if (self) js = max(js, i0 + 1);
-            // lane position relative to the neighbour row's cell origin in y and z
-            const float yi_r = Li.y - (float)rw.dy * h32;
-            const float zi_r = Li.z - (float)rw.dz * h32;
-            const float yi_r2 = Li2.y - (float)rw.dy * h32;
-            const float zi_r2 = Li2.z - (float)rw.dz * h32;
-            for (int jt = js; jt < je; jt += kWave) {
-                const int nt = min(kWave, je - jt);
-                const int jmin = max(self ? i + 1 - jt : 0, 0);   // self row: only j > i
-                const int jmin2 = max(self ? i2 + 1 - jt : 0, 0);
-                if (vi) st.cand += (unsigned long long)(nt - min(jmin, nt));
-                bound += (unsigned long long)nt * 2ull * kWave;
-                // histogram update of one kept pair with neighbour flags fj, bin b, mu bins m / mr
-                auto finish = [&](uint32_t fj, double wj, int b, int m, int mr) {
-                    const int cj = (fj & 2) ? 0 : 1;
-                    const int base = ((fj & 1) ? cb1 : cb0) + __umul24(b, nm);
-                    double x = 0.0;
-                    if constexpr (W) x = wis * wj;
-                    accumulate<RSD, W>(hcr, hw, nm, mirror, base, m, mr, mr == nm - 1 - m, ci, cj, x,
-                                       a.out_cnt, a.out_w);
-                };
+            // ---- the lane's apexes, relative to the chunk's middle point
+            double4 P1 = make_double4(0, 0, 0, 0), P2 = P1;
+            uint32_t f1 = 2u, f2 = 2u;
+            const bool v1 = ai < n_i, v2 = ai2 < n_i;
+            if (v1) { P1 = a.pw[ib + ai]; f1 = a.flags[ib + ai]; }
+            if (v2) { P2 = a.pw[ib + ai2]; f2 = a.flags[ib + ai2]; }
+            const int mid = n_i >> 1;
+            const double px = lane_double(P1.x, mid), py = lane_double(P1.y, mid), pz = lane_double(P1.z, mid);
+            const double p2 = px * px + py * py + pz * pz;
+            // 2 (|x|^2 - |p|^2)
+            auto d_of = [&](const double4& P) {
+                return 2.0 * ((P.x - px) * (P.x + px) + (P.y - py) * (P.y + py) + (P.z - pz) * (P.z + pz));
+            };
+            auto apex = [&](const double4& P, uint32_t f, bool v) {
+                Apex<R> A;
+                if constexpr (FP64) { A.x = P.x; A.y = P.y; A.z = P.z; }
+                else { A.x = (float)(P.x - px); A.y = (float)(P.y - py); A.z = (float)(P.z - pz); }
+                const double d = d_of(P);
+                A.d = (R)d;
+                A.c = (R)(d + 4.0 * p2);
+                A.w = W ? ldexp(P.w, (f & 1u) ? sr : sd) : 0.0;
+                A.cb = rep_off + ((f & 1u) ? nbm * kB : 0);
+                if (!v) A.x = Real4<R>::far;
+                return A;
+            };
+            const Apex<R> A1 = apex(P1, f1, v1), A2 = apex(P2, f2, v2);
+            const bool c1 = !(f1 & 2u), c2 = !(f2 & 2u);        // may be an apex of the reference
+            const bool chunk_buf = BUF && __ballot(c1) == 0;
+            // error bound of t for this chunk (wave-uniform): k0 + k1 q + k2 q^2, and the distance from
+            // the nearest integer is tested as |fract(t) - 1/2| <= 1/2 - bound
+            R l0 = 0, l1 = 0, l2 = 0;
+            if constexpr (RSD) {
+                const float rho = (float)sqrt(p2) * 1.001f;
+                const float sx = 2.0f * rho + B.mu_ab;
+                l0 = (R)(0.5f - B.mu_k0);
+                l1 = (R)(-(B.mu_k1a * sx + B.mu_k1b * (2.0f * rho + 3.0f * B.mu_ab)));
+                l2 = (R)(-(B.mu_k2a + B.mu_k2b * sx * sx));
+            }
+
+            // ---- tile entry of the lane
+            R ex = 0, ey = 0, ez = 0, ed = 0;
+            double ew = 0.0;
+            int ec = 0;         // class offset of a random entry; BUF: times 2, plus the buffer flag
+
+            // pair of apex A with the lane's entry: binned, or true if it has to be re-evaluated
+            auto visit1 = [&](const Apex<R>& A, const bool ca, Run& run) __attribute__((always_inline)) -> bool {
+                R s;
                 if constexpr (FP64) {
-                    wave_sync();
-                    uint32_t fl = 2u;
-                    if (lane < nt) {
-                        const double4 Pj = a.pw[jt + lane];
-                        fl = a.flags[jt + lane];
-                        tx[lane] = Pj.x; ty[lane] = Pj.y; tz[lane] = Pj.z;
-                        if (W) tw[lane] = ldexp(Pj.w, (fl & 1u) ? sr : sd);
-                        tf[lane] = fl;
-                    }
-                    const bool skip = chunk_buf && __ballot((fl & 2u) == 0) == 0;
-                    wave_sync();
-                    // rotated schedule: at step k lane L takes tile entry (k + L) mod nt, so the
-                    // lanes of a wave pair with different neighbours (spreading their histogram
-                    // updates over many bins) while reading consecutive, conflict-free LDS words
-                    const int kend = (vi && !skip) ? nt : 0;
-                    const int lm = lane % nt;
-                    for (int k = 0; k < kend; ++k) {
-                        int kk = k + lm;
-                        kk = kk >= nt ? kk - nt : kk;
-                        if (kk < jmin) continue;
-                        const uint32_t fj = tf[kk];
-                        const double jx = tx[kk], jy = ty[kk], jz = tz[kk];
-                        const double s = exact_s(Pi.x, Pi.y, Pi.z, jx, jy, jz);
-                        if (!(s > t_lo && s < t_hi)) continue;
-                        const int b = adjust_bin(s, bin_estimate((float)s, LOGB, ua, ub), t64, nb);
-                        if (b == nb) { st.over += (uint64_t)(ci + ((fj & 2) ? 0 : 1)); continue; }
-                        int m = 0, mr = 0;
-                        if constexpr (RSD) exact_mu(Pi.x, Pi.y, Pi.z, jx, jy, jz, ms, nm, m, mr);
-                        finish(fj, W ? tw[kk] : 0.0, b, m, mr);
-                    }
+                    s = exact_s(A.x, A.y, A.z, ex, ey, ez);
                 } else {
-                    {
-                        // Register tile: lane L loads entry L; the entries then rotate through the
-                        // wave one lane per step (DPP), so after 64 steps every lane has met every
-                        // entry (after P steps for a tile of nt <= P entries, below).  Consecutive
-                        // lanes meet different neighbours at each step, which spreads their histogram
-                        // updates over many bins, and no LDS is read for the neighbours.
-                        // A partial tile is loaded with period P (the power of two >= nt): lane L
-                        // holds entry L mod P, a full-wave rotation keeps that pattern, and P steps
-                        // bring every entry to every lane.
-                        const int P = nt <= 1 ? 1 : 1 << (32 - __clz(nt - 1));
-                        const int le = lane & (P - 1);
-                        const bool has = le < nt;
-                        const int jl = jt + (has ? le : 0);
-                        uint32_t ef = a.flags[jl];
-                        const bool skip = chunk_buf && __ballot(has && (ef & 2u) == 0) == 0;
-                        float4 e = make_float4(0.f, 0.f, 0.f, 0.f);
-                        double ewj = 0.0;
-                        if (!skip) {
-                            e = a.pl[jl];
-                            if constexpr (W) ewj = ldexp(a.ws[jl], (ef & 1u) ? sr : sd);
+                    const float dx = ex - A.x, dy = ey - A.y, dz = ez - A.z;
+                    s = fmaf(dz, dz, fmaf(dy, dy, dx * dx));
+                }
+                if (!(s > rej_lo && s < rej_hi)) return false;
+                if (BUF && !ca && (ec & 1)) return false;     // two buffer points
+                int b;
+                bool safe;
+                if constexpr (FP64) {
+                    const float u = bin_estimate((float)s, LOGB, ua, ub);
+                    b = min(cvt_sat(u), nb - 1);
+                    const double* t = (const double*)smem;
+                    if (!(s >= t[b] && s < t[b + 1])) {
+                        while (b > 0 && s < t[b]) --b;
+                        while (b < nb && s >= t[b + 1]) ++b;
+                        if (b == nb) {
+                            n_over += (unsigned)ca + (BUF ? 1u - (unsigned)(ec & 1) : 1u);
+                            return false;
                         }
-                        // entry index, class and buffer flag in one rotated register (-1: no entry):
-                        // ep = eidx << 16 | (class offset of a random entry, nb*nm, or 0) << 1 | buffer,
-                        // so the self-row test eidx >= jmin is ep >= jmin << 16 and the pair's class
-                        // offset is cb0 + a field of ep (nb*nm <= 127*127 fits in 15 bits)
-                        int ep = has ? (le << 16) | ((ef & 1u) ? nbm << 1 : 0) | (int)((ef >> 1) & 1u) : -1;
-                        if constexpr (!DUAL) {
-                            const int jmin16 = jmin << 16;
-                            const int kend = __builtin_amdgcn_readfirstlane(skip ? 0 : P);
-                            for (int k = 0; k < kend; ++k) {
-                                if (vi && ep >= jmin16) do {
-                                    const float dx = fmaf(e.w - Li.w, hx32, e.x - Li.x);
-                                    const float dy = e.y - yi_r, dz = e.z - zi_r;
-                                    const float s = fmaf(dz, dz, fmaf(dy, dy, dx * dx));
-                                    if (!(s > rej_lo && s < rej_hi)) break;
-                                    int b = (int)__builtin_amdgcn_fmed3f(bin_estimate(s, LOGB, ua, ubv), 0.0f, nbm1f);
-                                    const float2 ok = okb[b];
-                                    bool safe = (s >= ok.x) && (s < ok.y);
-                                    int m = 0, mr;      // mr is read only after an FP64 recheck has set it
-                                    if constexpr (!RSD) mr = 0;
-                                    if constexpr (RSD) {
-                                        const float r = __builtin_amdgcn_rsqf(s);
-                                        // mid = x_i + d/2 (absolute), sep = x_i - x_j = -d
-                                        const float mx = fmaf(0.5f, dx, ax32), my = fmaf(0.5f, dy, ay32), mz = fmaf(0.5f, dz, az32);
-                                        const float D = -fmaf(mz, dz, fmaf(my, dy, mx * dx));
-                                        const float M2 = fmaf(mz, mz, fmaf(my, my, mx * mx));
-                                        const float rm = __builtin_amdgcn_rsqf(M2);
-                                        const float t = fmaf(D * rm * r, ms32, ms32);     // (theta + 1) * mu_scale
-                                        const float dt = fmaf(dt_ew, r, fmaf(dt_em, rm, dt_c));
-                                        // mu edges sit at the integers 1..nm-1 of t: the bin is certain when the
-                                        // nearest edge, clamp(rint(t), 1, nm-1), is farther than the error bound
-                                        // dt < 1/2 (a nearest integer of 0 or nm is more than 1/2 from any edge)
-                                        const float edge = __builtin_amdgcn_fmed3f(rintf(t), e_lo, e_hi);
-                                        safe = safe && (dt < 0.5f) && (fabsf(t - edge) >= dt);
-                                        m = min((int)t, nm - 1);       // t >= 0 up to rounding; truncation = floor there
-                                    }
-                                    bool mirrored = true;     // the FP32 mu bins are mirror images by construction
-                                    if (!safe) {
-                                        ++st.rechk;
-                                        const double4 Pj = a.pw[jt + (ep >> 16)];
-                                        Pi = a.pw[i];
-                                        const double se = exact_s(Pi.x, Pi.y, Pi.z, Pj.x, Pj.y, Pj.z);
-                                        if (!(se > t_lo && se < t_hi)) break;
-                                        b = exact_bin(se, t64, nb);
-                                        if (b == nb) { st.over += (uint64_t)(ci + (ep & 1 ? 0 : 1)); break; }
-                                        if constexpr (RSD) {
-                                            exact_mu(Pi.x, Pi.y, Pi.z, Pj.x, Pj.y, Pj.z, ms, nm, m, mr);
-                                            mirrored = mr == nm - 1 - m;
-                                        }
-                                    }
-                                    {
-                                        const int cj = (ep & 1) ? 0 : 1;
-                                        const int base = cb0 + ((ep >> 1) & 0x7fff) + __umul24(b, nm);
-                                        unsigned long long q = 0;
-                                        if constexpr (W) q = quantise_rn(wis * ewj);
-                                        if constexpr (W && !RSD) {
-                                            if (ci + cj) put(rc0, base, (uint32_t)(ci + cj), q);
-                                        } else if (W && mirror && mirrored) {
-                                            put(rc0, base + m, 1u, q);   // stands for i->j at m and j->i at nm-1-m
-                                        } else {
-                                            // mr: the mirror image of m unless the recheck found otherwise
-                                            accumulate<RSD, W>(hcr, hw, nm, mirror, base, m,
-                                                               mirrored ? nm - 1 - m : mr, mirrored, ci, cj,
-                                                               wis * ewj, a.out_cnt, a.out_w);
-                                        }
-                                    }
-                                } while (false);
-                                // rotate the register tile by one lane (all lanes active here)
-                                e.x = rot_lane(e.x); e.y = rot_lane(e.y); e.z = rot_lane(e.z); e.w = rot_lane(e.w);
-                                if constexpr (W) ewj = rot_lane(ewj);
-                                ep = rot_lane(ep);
-                            }
-                        } else {
-                            const int kend = __builtin_amdgcn_readfirstlane(skip ? 0 : P);
-                            // one apex's pair with the lane's current tile entry
-                            auto visit = [&](const bool va, const int ia, const float4 La, const float yr, const float zr,
-                                             const float axa, const float aya, const float aza, const int cia,
-                                             const int cba, const double wisa, const int jm16,
-                                             RunCache& rc) __attribute__((always_inline)) {
-                                if (va && ep >= jm16) do {
-                                    const float dx = fmaf(e.w - La.w, hx32, e.x - La.x);
-                                    const float dy = e.y - yr, dz = e.z - zr;
-                                    const float s = fmaf(dz, dz, fmaf(dy, dy, dx * dx));
-                                    if (!(s > rej_lo && s < rej_hi)) break;
-                                    int b = (int)__builtin_amdgcn_fmed3f(bin_estimate(s, LOGB, ua, ubv), 0.0f, nbm1f);
-                                    const float2 ok = okb[b];
-                                    bool safe = (s >= ok.x) && (s < ok.y);
-                                    int m = 0, mr;      // mr is read only after an FP64 recheck has set it
-                                    if constexpr (!RSD) mr = 0;
-                                    if constexpr (RSD) {
-                                        const float r = __builtin_amdgcn_rsqf(s);
-                                        // mid = x_i + d/2 (absolute), sep = x_i - x_j = -d
-                                        const float mx = fmaf(0.5f, dx, axa), my = fmaf(0.5f, dy, aya), mz = fmaf(0.5f, dz, aza);
-                                        const float D = -fmaf(mz, dz, fmaf(my, dy, mx * dx));
-                                        const float M2 = fmaf(mz, mz, fmaf(my, my, mx * mx));
-                                        const float rm = __builtin_amdgcn_rsqf(M2);
-                                        const float t = fmaf(D * rm * r, ms32, ms32);     // (theta + 1) * mu_scale
-                                        const float dt = fmaf(dt_ew, r, fmaf(dt_em, rm, dt_c));
-                                        // mu edges sit at the integers 1..nm-1 of t: the bin is certain when the
-                                        // nearest edge, clamp(rint(t), 1, nm-1), is farther than the error bound
-                                        // dt < 1/2 (a nearest integer of 0 or nm is more than 1/2 from any edge)
-                                        const float edge = __builtin_amdgcn_fmed3f(rintf(t), e_lo, e_hi);
-                                        safe = safe && (dt < 0.5f) && (fabsf(t - edge) >= dt);
-                                        m = min((int)t, nm - 1);       // t >= 0 up to rounding; truncation = floor there
-                                    }
-                                    bool mirrored = true;     // the FP32 mu bins are mirror images by construction
-                                    if (!safe) {
-                                        ++st.rechk;
-                                        const double4 Pj = a.pw[jt + (ep >> 16)];
-                                        const double4 Pa = a.pw[ia];
-                                        const double se = exact_s(Pa.x, Pa.y, Pa.z, Pj.x, Pj.y, Pj.z);
-                                        if (!(se > t_lo && se < t_hi)) break;
-                                        b = exact_bin(se, t64, nb);
-                                        if (b == nb) { st.over += (uint64_t)(cia + (ep & 1 ? 0 : 1)); break; }
-                                        if constexpr (RSD) {
-                                            exact_mu(Pa.x, Pa.y, Pa.z, Pj.x, Pj.y, Pj.z, ms, nm, m, mr);
-                                            mirrored = mr == nm - 1 - m;
-                                        }
-                                    }
-                                    {
-                                        const int cj = (ep & 1) ? 0 : 1;
-                                        const int base = cba + ((ep >> 1) & 0x7fff) + __umul24(b, nm);
-                                        unsigned long long q = 0;
-                                        if constexpr (W) q = quantise_rn(wisa * ewj);
-                                        if constexpr (W && !RSD) {
-                                            if (cia + cj) put(rc, base, (uint32_t)(cia + cj), q);
-                                        } else if (W && mirror && mirrored) {
-                                            put(rc, base + m, 1u, q);   // stands for i->j at m and j->i at nm-1-m
-                                        } else {
-                                            // mr: the mirror image of m unless the recheck found otherwise
-                                            accumulate<RSD, W>(hcr, hw, nm, mirror, base, m,
-                                                               mirrored ? nm - 1 - m : mr, mirrored, cia, cj,
-                                                               wisa * ewj, a.out_cnt, a.out_w);
-                                        }
-                                    }
-                                } while (false);
-                            };
-                            auto rotate = [&]() __attribute__((always_inline)) {
-                                // rotate the register tile by one lane (all lanes active here)
-                                e.x = rot_lane(e.x); e.y = rot_lane(e.y); e.z = rot_lane(e.z); e.w = rot_lane(e.w);
-                                if constexpr (W) ewj = rot_lane(ewj);
-                                ep = rot_lane(ep);
-                            };
-                            if (kend == kWave) {
-                                // a full tile in 32 steps: lane L meets 32 cyclically consecutive entries from
-                                // its own, lane L ^ 32 the other 32, and each pairs them with both apexes,
-                                // points L and L ^ 32, so every (apex, entry) pair is visited exactly once
-                                // and each rotation serves two pairs
-                                for (int k = 0; k < kWave / 2; ++k) {
-                                    visit(vi, i, Li, yi_r, zi_r, ax32, ay32, az32, ci, cb0, wis, jmin << 16, rc0);
-                                    visit(vi2, i2, Li2, yi_r2, zi_r2, ax2, ay2, az2, ci2, cb02, wis2, jmin2 << 16, rc1);
-                                    rotate();
-                                }
-                            } else {
-                                for (int k = 0; k < kend; ++k) {
-                                    visit(vi, i, Li, yi_r, zi_r, ax32, ay32, az32, ci, cb0, wis, jmin << 16, rc0);
-                                    rotate();
-                                }
-                            }
+                    }
+                    safe = true;
+                } else {
+                    b = cvt_sat(bin_estimate(s, LOGB, ua, ub));
+                    const float2 ok = ((const float2*)smem)[b];
+                    safe = s >= ok.x && s < ok.y;
+                }
+                int m = 0;
+                if constexpr (RSD) {
+                    const R S = (A.c + ed) - s;
+                    const R q = rsq(S * s);
+                    const R t = fma((A.d - ed) * q, hms, msr);
+                    const R lim = fma(fma(l2, q, l1), q, l0);
+                    // the negated form also leaves a NaN (mid-point at the origin) to the recheck
+                    safe = safe && fabs(fract(t) - (R)0.5) <= lim;
+                    m = (int)t;
+                }
+                if (!safe) return true;
+                const int k0 = A.cb + (BUF ? ec >> 1 : ec) + (int)__umul24(b, (unsigned)(nm * kB));
+                uint32_t qlo = 0, qhi = 0;
+                if constexpr (W) {
+                    const unsigned long long q = quantise_rn(A.w * ew);
+                    qlo = (uint32_t)q;
+                    qhi = (uint32_t)(q >> 32);
+                }
+                if constexpr (!BUF) {
+                    const int kk = k0 + m * kB;
+                    if constexpr (W) put(run, kk, qlo, qhi);
+                    else atomicAdd((uint32_t*)(hist + kk), 1u);
+                } else {
+                    // both ends apexes: plane 0; one: plane 1 in its direction
+                    const bool cj = !(ec & 1);
+                    const int mr = nm - 1 - m;
+                    if (planes == 2) {
+                        const int kk = k0 + (ca ? m : mr) * kB + (ca && cj ? 0 : nbt * kB);
+                        if constexpr (W) put(run, kk, qlo, qhi);
+                        else atomicAdd((uint32_t*)(hist + kk), 1u);
+                    } else {        // histograms too large for two planes: plane 1 only, each direction added
+                        if (ca) {
+                            if constexpr (W) put(run, k0 + m * kB, qlo, qhi);
+                            else atomicAdd((uint32_t*)(hist + k0 + m * kB), 1u);
+                        }
+                        if (cj) {
+                            if constexpr (W) put(run, k0 + mr * kB, qlo, qhi);
+                            else atomicAdd((uint32_t*)(hist + k0 + mr * kB), 1u);
                         }
                     }
                 }
-                // each wave drains after drain_at of its own possible increments (every candidate
-                // counted twice; the increments held in the lanes' run caches included)
-                if (bound > drain_at) {
-                    if constexpr (W) flush();
-                    const size_t ro = batched ? (size_t)cur_r : 0;
-                    drain(hc, hw, nbt, nm, reps, W, mirror, lane, kWave, a.out_cnt + ro * nbt,
-                          a.out_w + ro * 2 * nbt);
-                    bound = 0;
+                return false;
+            };
+            // ... and queued if so: entry number (lane + k) & 63 of the tile, apex point ia
+            auto visit = [&](const Apex<R>& A, const bool ca, const int ia, const int k, Run& run, const bool on)
+                             __attribute__((always_inline)) {
+                bool un = false;
+                if (on) un = visit1(A, ca, run);
+                if constexpr (RSD || !FP64) {
+                    const unsigned long long um = __ballot(un);
+                    if (um) {
+                        const int nu = __popcll(um);
+                        if (nq + nu > kWave) recheck();
+                        if (un) {
+                            const int at = nq + (int)__builtin_amdgcn_mbcnt_hi((unsigned)(um >> 32),
+                                                                              __builtin_amdgcn_mbcnt_lo((unsigned)um, 0u));
+                            queue[at] = make_int2(ia, jlist[(lane + k) & (kWave - 1)]);
+                        }
+                        nq += nu;
+                    }
+                }
+            };
+            auto rotate = [&]() __attribute__((always_inline)) {
+                ex = rot_lane(ex); ey = rot_lane(ey); ez = rot_lane(ez);
+                if constexpr (RSD) ed = rot_lane(ed);
+                if constexpr (W) ew = rot_lane(ew);
+                ec = rot_lane(ec);
+            };
+            auto entry_class = [&](uint32_t f) {
+                const int c = (f & 1u) ? nbm * kB : 0;
+                return BUF ? (c << 1) | (int)((f >> 1) & 1u) : c;
+            };
+            auto tile_done = [&](int nt) {
+                bound += (unsigned long long)nt * (BUF && planes == 1 ? 2u : 1u);
+                if constexpr (W) {
+                    if (r1.cn >= kRunMax * kCountOne) flush(r1);
+                    if (r2.cn >= kRunMax * kCountOne) flush(r2);
+                }
+                if (bound > look_at) look();
+            };
+
+            // ---- pairs inside the chunk
+            if (part == 0) n_cand += (unsigned long long)(n_i * (n_i - 1) / 2);
+            if (part == 0 && !chunk_buf) {
+                ex = v1 ? A1.x : -Real4<R>::far; ey = A1.y; ez = A1.z; ed = A1.d; ew = A1.w;
+                ec = entry_class(f1);
+                wave_sync();
+                jlist[lane] = ib + min(ai, n_i - 1);
+                wave_sync();
+                for (int k = 1; k <= half; ++k) {
+                    rotate();
+                    visit(A1, c1, ib + ai, k, r1, lane < (k < half ? group : half));
+                }
+                tile_done(n_i * (n_i - 1) / 2);
+            }
+
+            // ---- the other points of the half stencil
+            for (int r0 = 0; r0 < a.nrows; r0 += kWave) {
+                int js = 0, len = 0;
+                if (r0 + lane < a.nrows) {
+                    const Row rw = a.rows[r0 + lane];
+                    const int by = cy + rw.dy, bz = cz + rw.dz;
+                    const int bx0 = max(cx_first + rw.x0, 0), bx1 = min(cx_last + rw.x1, nx - 1);
+                    if (by >= 0 && by < ny && bz >= 0 && bz < nz && bx0 <= bx1) {
+                        const int rb = cb + (bz * ny + by) * nx;
+                        js = a.cell_start[rb + bx0];
+                        const int je = a.cell_start[rb + bx1 + 1];
+                        if (rw.dy == 0 && rw.dz == 0) js = max(js, ib + n_i);
+                        len = max(je - js, 0);
+                    }
+                }
+                int incl = len;
+                for (int off = 1; off < kWave; off <<= 1) {
+                    const int y = __shfl_up(incl, off, kWave);
+                    if (lane >= off) incl += y;
+                }
+                const int excl = incl - len;
+                const int total = lane_int(incl, kWave - 1);
+                const int tiles = (total + kWave - 1) / kWave;
+                const int t1 = (int)(((long long)tiles * (part + 1)) >> a.lg_parts);
+                int t = (int)(((long long)tiles * part) >> a.lg_parts);
+                for (; t < t1; ++t) {
+                    // the lane's entry: its point, from the row of this tile it falls into
+                    const int c0 = t * kWave, my = c0 + lane;
+                    const int nt = min(kWave, total - c0);
+                    const bool has = lane < nt;
+                    int j = ib;
+                    unsigned long long rows = __ballot(incl > c0 && excl < c0 + kWave && len > 0);
+                    while (rows) {
+                        const int r = (int)__builtin_ctzll(rows);
+                        rows &= rows - 1;
+                        const int e0 = lane_int(excl, r), j0 = lane_int(js, r);
+                        if (my >= e0) j = j0 + (my - e0);
+                    }
+                    if (!has) j = ib;
+                    n_cand += (unsigned long long)(n_i * nt);
+                    const uint32_t f = a.flags[j];
+                    if (chunk_buf && __ballot(has && !(f & 2u)) == 0) continue;
+                    const double4 P = a.pw[j];
+                    if constexpr (FP64) { ex = P.x; ey = P.y; ez = P.z; }
+                    else { ex = (float)(P.x - px); ey = (float)(P.y - py); ez = (float)(P.z - pz); }
+                    if constexpr (RSD) ed = (R)d_of(P);
+                    if constexpr (W) ew = ldexp(P.w, (f & 1u) ? sr : sd);
+                    ec = entry_class(f);
+                    if (!has) ex = -Real4<R>::far;
+                    wave_sync();
+                    jlist[lane] = j;
+                    wave_sync();
+                    for (int k = 0; k < half; ++k) {
+                        visit(A1, c1, ib + ai, k, r1, true);
+                        visit(A2, c2, ib + ai2, k, r2, true);
+                        rotate();
+                    }
+                    tile_done(n_i * nt);
                 }
             }
         }
     }
-    if constexpr (W) flush();
+    if (nq) recheck();
+    if constexpr (W) { flush(r1); flush(r2); }
     if (batched) {
-        if (cur_r >= 0)
-            drain(hc, hw, nbt, nm, reps, W, mirror, lane, kWave, a.out_cnt + (size_t)cur_r * nbt,
-                  a.out_w + (size_t)cur_r * 2 * nbt);
+        if (cur_r >= 0) drain(lane, kWave);
     } else {
         __syncthreads();
-        drain(hc, hw, nbt, nm, reps, W, mirror, tid, nthr, a.out_cnt, a.out_w);
+        drain(tid, nthr);
     }
 
-    // wave-reduce the statistics
-    for (int off = 32; off > 0; off >>= 1) {
-        st.cand += __shfl_down(st.cand, off, 64);
-        st.rechk += __shfl_down(st.rechk, off, 64);
-        st.over += __shfl_down(st.over, off, 64);
-    }
+    // statistics (candidates and rechecks are counted per wave, overflow pairs per lane), one atomic per
+    // work-group each
+    unsigned long long ov = n_over;
+    for (int off = 32; off > 0; off >>= 1) ov += __shfl_down(ov, off, 64);
+    __shared__ unsigned long long s_stat[3];
+    if (tid < 3) s_stat[tid] = 0;
+    __syncthreads();
     if (lane == 0) {
-        if (st.cand) atomicAdd(&a.out_stats[0], st.cand);
-        if (st.rechk) atomicAdd(&a.out_stats[1], st.rechk);
-        if (st.over) atomicAdd(&a.out_stats[2], st.over);
+        if (n_cand) atomicAdd(&s_stat[0], n_cand);
+        if (n_rechk) atomicAdd(&s_stat[1], n_rechk);
+        if (ov) atomicAdd(&s_stat[2], ov);
+    }
+    __syncthreads();
+    if (tid < 3 && s_stat[tid]) atomicAdd(&a.out_stats[copy + tid], s_stat[tid]);
+}
+
+// Sums the copies of the outputs and folds their two planes: counts [nreg][nbt] and 128-bit sums
+// [nreg][nbt][2] over ordered pairs, and the statistics.  Every work-group drains its histogram with
+// device-wide atomics, which run one after another where they meet (about 40 ns each): with one copy
+// the drains of a small catalogue's 2048 work-groups into 30 bins took 1.3 ms, longer than its pairs.
+// One wave per entry, one lane per copy.
+__global__ __launch_bounds__(256) void k_pair_reduce(const unsigned long long* __restrict__ in, int copies,
+                                                     int64_t copy_stride, int nreg, int nbt, int nm, int weighted,
+                                                     unsigned long long* __restrict__ out)
+{
+    const int lane = threadIdx.x & (kWave - 1);
+    const int64_t e = blockIdx.x * (int64_t)(blockDim.x / kWave) + threadIdx.x / kWave;
+    const int64_t ne = (int64_t)nreg * nbt;
+    const unsigned long long* c = in + (size_t)lane * (size_t)copy_stride;
+    if (e < ne) {
+        const int64_t r = e / nbt;
+        const int k = (int)(e % nbt);
+        const int km = k - k % nm + (nm - 1 - k % nm);
+        unsigned long long n = 0, lo = 0, hi = 0;
+        if (lane < copies) {
+            const unsigned long long* cc = c + r * 2 * nbt;
+            n = cc[k] + cc[km] + cc[nbt + k];
+            if (weighted) {
+                const unsigned long long* cw = c + ne * 2 + r * 4 * nbt;
+                add128(lo, hi, cw[2 * k], cw[2 * k + 1]);
+                add128(lo, hi, cw[2 * km], cw[2 * km + 1]);
+                add128(lo, hi, cw[2 * (nbt + k)], cw[2 * (nbt + k) + 1]);
+            }
+        }
+        for (int off = 32; off > 0; off >>= 1) {
+            n += __shfl_down(n, off, 64);
+            const unsigned long long l = __shfl_down(lo, off, 64), h = __shfl_down(hi, off, 64);
+            add128(lo, hi, l, h);
+        }
+        if (lane == 0) {
+            out[e] = n;
+            out[ne + 2 * e] = lo;
+            out[ne + 2 * e + 1] = hi;
+        }
+    } else if (e == ne) {
+        for (int q = 0; q < 4; ++q) {
+            unsigned long long v = lane < copies ? c[6 * ne + q] : 0;
+            for (int off = 32; off > 0; off >>= 1) v += __shfl_down(v, off, 64);
+            if (lane == 0) out[3 * ne + q] = v;
+        }
     }
 }
 
-template <bool FP64, bool RSD, bool W, bool LOGB, bool DUAL>
-static int occ_k(size_t lds, int wg)
+hipError_t launch_pair_reduce(const unsigned long long* in, int copies, int nreg, int nbt, int nm, bool weighted,
+                              unsigned long long* out, hipStream_t st)
 {
-    int nb = 0;
-    auto kern = k_pair2<FP64, RSD, W, LOGB, DUAL>;
-    if (lds > 64 * 1024 &&
-        hipFuncSetAttribute((const void*)kern, hipFuncAttributeMaxDynamicSharedMemorySize, (int)lds) != hipSuccess)
-        return 0;
-    if (hipOccupancyMaxActiveBlocksPerMultiprocessor(&nb, kern, wg, lds) != hipSuccess)
-        return 1;
-    return nb;
-}
-
-// Whether the weighted FP32 kernel runs with two apexes per lane: where the LDS histogram already limits
-// the resident work-groups to what the larger register file allows (many bins), else not.
-// GS_PAIR_DUAL=0 / 1 forces it off / on (tests, tuning).
-template <bool RSD, bool LOGB>
-static bool use_dual(size_t lds, int wg)
-{
-    const char* ev = getenv("GS_PAIR_DUAL");
-    if (ev && *ev) return atoi(ev) != 0;
-    return occ_k<false, RSD, true, LOGB, true>(lds, wg) >= occ_k<false, RSD, true, LOGB, false>(lds, wg);
-}
-
-template <bool FP64, bool RSD, bool W, bool LOGB>
-static hipError_t launch_t(const PairArgs& a, size_t lds, int nblocks, int wg, hipStream_t st)
-{
-    auto kern = k_pair2<FP64, RSD, W, LOGB, false>;
-    if constexpr (W && !FP64)
-        if (use_dual<RSD, LOGB>(lds, wg)) kern = k_pair2<FP64, RSD, W, LOGB, true>;
-    if (lds > 64 * 1024) {
-        hipError_t e = hipFuncSetAttribute((const void*)kern, hipFuncAttributeMaxDynamicSharedMemorySize, (int)lds);
-        if (e != hipSuccess) return e;
-    }
-    hipLaunchKernelGGL(kern, dim3(nblocks), dim3(wg), lds, st, a);
+    const int64_t ne = (int64_t)nreg * nbt;
+    const int64_t nblk = (ne + 1 + kWG / kWave - 1) / (kWG / kWave);
+    hipLaunchKernelGGL(k_pair_reduce, dim3((unsigned)nblk), dim3(kWG), 0, st, in, copies, pair_copy_words(nreg, nbt),
+                       nreg, nbt, nm, weighted ? 1 : 0, out);
     return hipGetLastError();
 }
 
-template <bool FP64, bool RSD, bool W, bool LOGB>
-static int occ_t(size_t lds, int wg)
-{
-    return occ_k<FP64, RSD, W, LOGB, false>(lds, wg);
-}
-
-// Runs F<FP64, RSD, W, LOGB>(args...) for the runtime flags.
-template <template <bool, bool, bool, bool> class F, class... Args>
-static auto dispatch(bool fp64, bool rsd, bool w, bool logb, Args... args)
-{
-#define GS_D4(A, B, C, D) \
-    if (fp64 == A && rsd == B && w == C && logb == D) return F<A, B, C, D>::run(args...);
-    GS_D4(true, true, true, true) GS_D4(true, true, true, false) GS_D4(true, true, false, true)
-    GS_D4(true, true, false, false) GS_D4(true, false, true, true) GS_D4(true, false, true, false)
-    GS_D4(true, false, false, true) GS_D4(true, false, false, false) GS_D4(false, true, true, true)
-    GS_D4(false, true, true, false) GS_D4(false, true, false, true) GS_D4(false, true, false, false)
-    GS_D4(false, false, true, true) GS_D4(false, false, true, false) GS_D4(false, false, false, true)
-#undef GS_D4
-    return F<false, false, false, false>::run(args...);
-}
-
-template <bool A, bool B, bool C, bool D>
-struct Launch {
-    static hipError_t run(const PairArgs& a, size_t lds, int nblocks, int wg, hipStream_t st)
+template <bool FP64, bool RSD, bool W, bool LOGB, bool BUF>
+struct Pair2 {
+    static hipError_t launch(const PairArgs& a, size_t lds, int nblocks, int wg, hipStream_t st)
     {
-        return launch_t<A, B, C, D>(a, lds, nblocks, wg, st);
+        auto kern = k_pair2<FP64, RSD, W, LOGB, BUF>;
+        if (lds > 64 * 1024) {
+            hipError_t e = hipFuncSetAttribute((const void*)kern, hipFuncAttributeMaxDynamicSharedMemorySize, (int)lds);
+            if (e != hipSuccess) return e;
+        }
+        hipLaunchKernelGGL(kern, dim3(nblocks), dim3(wg), lds, st, a);
+        return hipGetLastError();
+    }
+    static int occupancy(size_t lds, int wg)
+    {
+        int nb = 0;
+        auto kern = k_pair2<FP64, RSD, W, LOGB, BUF>;
+        if (lds > 64 * 1024 &&
+            hipFuncSetAttribute((const void*)kern, hipFuncAttributeMaxDynamicSharedMemorySize, (int)lds) != hipSuccess)
+            return 0;
+        if (hipOccupancyMaxActiveBlocksPerMultiprocessor(&nb, kern, wg, lds) != hipSuccess) return 1;
+        return nb;
     }
 };
-template <bool A, bool B, bool C, bool D>
-struct Occ {
-    static int run(size_t lds, int wg) { return occ_t<A, B, C, D>(lds, wg); }
-};
 
-hipError_t launch_pair2(const PairArgs& a, int nb, int nm, bool fp64, bool rsd, bool weighted, bool logb,
-                        int nblocks, int wg, hipStream_t st)
+// f(Pair2<...>{}) for the variant v
+template <bool... Done, class F>
+static auto with_variant(const PairVariant& v, F&& f)
 {
-    const size_t lds = pair2_lds_bytes(nb, rsd ? nm : 1, a.reps, fp64, weighted, a.nreg > 0, wg);
-    return dispatch<Launch>(fp64, rsd, weighted, logb, a, lds, nblocks, wg, st);
+    if constexpr (sizeof...(Done) == 5) {
+        return f(Pair2<Done...>{});
+    } else {
+        constexpr int k = sizeof...(Done);
+        const bool b = k == 0 ? v.fp64 : k == 1 ? v.nm >= 2 : k == 2 ? v.weighted : k == 3 ? v.logb : v.buf;
+        return b ? with_variant<Done..., true>(v, f) : with_variant<Done..., false>(v, f);
+    }
 }
 
-int pair2_occupancy(int nb, int nm, int reps, bool fp64, bool rsd, bool weighted, bool logb, bool batched, int wg)
+hipError_t launch_pair2(const PairArgs& a, const PairVariant& v, int nblocks, int wg, hipStream_t st)
 {
-    const size_t lds = pair2_lds_bytes(nb, rsd ? nm : 1, reps, fp64, weighted, batched, wg);
-    if (lds > 160 * 1024) return 0;
-    return dispatch<Occ>(fp64, rsd, weighted, logb, lds, wg);
+    const size_t lds = pair2_lds_bytes(v.nb, v.nm, v.buf ? a.planes : 1, a.reps, v.weighted, a.nreg > 0, wg);
+    return with_variant(v, [&](auto k) { return k.launch(a, lds, nblocks, wg, st); });
+}
+
+int pair2_occupancy(const PairVariant& v, int planes, int reps, bool batched, int wg)
+{
+    const size_t lds = pair2_lds_bytes(v.nb, v.nm, planes, reps, v.weighted, batched, wg);
+    if (lds > kPairLdsMax) return 0;
+    return with_variant(v, [&](auto k) { return k.occupancy(lds, wg); });
+}
+
+// ---------------------------------------------------------------- chunks
+// Descriptors of the pair kernels' chunks: {first point, points, x-row in its region, region}.
+__global__ __launch_bounds__(256) void k_chunks(const int32_t* __restrict__ row_chunk, int nrow,
+                                                const int32_t* __restrict__ cell_start, int nx,
+                                                const RegionDesc* __restrict__ regions,
+                                                const int32_t* __restrict__ row_base, int nreg, int group,
+                                                int4* __restrict__ out)
+{
+    const int n = row_chunk[nrow];
+    for (int c = blockIdx.x * blockDim.x + threadIdx.x; c < n; c += gridDim.x * blockDim.x) {
+        const int grow = upper_index(row_chunk, nrow, c);
+        int row = grow, r = 0, c0, dim = nx;
+        if (nreg > 0) {
+            r = upper_index(row_base, nreg, grow);
+            row = grow - regions[r].row_base;
+            dim = regions[r].dim[0];
+            c0 = regions[r].cell_base + row * dim;
+        } else {
+            c0 = row * dim;
+        }
+        const int i0 = cell_start[c0] + (c - row_chunk[grow]) * group;
+        out[c] = make_int4(i0, min(group, cell_start[c0 + dim] - i0), row, r);
+    }
+}
+
+hipError_t launch_chunks(const int32_t* row_chunk, int nrow, const int32_t* cell_start, int nx,
+                         const RegionDesc* regions, const int32_t* row_base, int nreg, int group, int64_t max_chunks,
+                         int4* out, hipStream_t st)
+{
+    int64_t nblk = (max_chunks + 255) / 256;
+    if (nblk > 4096) nblk = 4096;
+    if (nblk < 1) nblk = 1;
+    hipLaunchKernelGGL(k_chunks, dim3((unsigned)nblk), dim3(256), 0, st, row_chunk, nrow, cell_start, nx, regions,
+                       row_base, nreg, group, out);
+    return hipGetLastError();
 }
 
 }  // namespace gs

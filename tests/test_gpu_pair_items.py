@@ -1,0 +1,86 @@
+"""The pair kernel's work decomposition at its edges: chunk sizes, items per chunk, partial chunks and
+tiles, the drains of its packed weighted histogram, and the ranges outside the FP32 error bounds."""
+import numpy as np
+import pytest
+
+import oracle as O
+from gramsci_amd import catalog as C
+from gramsci_amd.engine import Engine
+
+pytestmark = pytest.mark.gpu
+
+
+@pytest.fixture(scope="module")
+def eng():
+    e = Engine(0)
+    yield e
+    e.close()
+
+
+def _check(eng, xyz, w, nd, p, buf=None):
+    ref = O.pcf2(xyz, w, nd, p, buf=buf)
+    for prec in ("fp32", "fp64"):
+        eng.set_catalogue(xyz, w, nd, buf)
+        r = eng.pcf2(p.rmin, p.rmax, p.nbins, p.nmu, p.log_bins, prec)
+        assert np.array_equal(r["cnt"], ref["cnt"]), prec
+        for k in ("wsum", "n2", "n3"):      # sums of at most n^2 rounded products, exact in fixed point
+            assert np.all(np.abs(r[k] - ref[k]) <= 1e-13 * max(np.abs(ref[k]).max(), 1e-300)), (prec, k)
+
+
+@pytest.mark.parametrize("group", ["16", "32", "64"])
+@pytest.mark.parametrize("parts", ["1", "8", "64"])
+@pytest.mark.parametrize("weighted,buffered,nmu", [(True, False, 6), (True, True, 5), (False, True, 1), (False, False, 4)])
+def test_groups_and_parts(eng, monkeypatch, group, parts, weighted, buffered, nmu):
+    monkeypatch.setenv("GS_PAIR_GROUP", group)
+    monkeypatch.setenv("GS_PAIR_PARTS", parts)
+    rng = np.random.default_rng(7)
+    # a dense cluster (long tiles), sparse rows (chunks cut into pieces) and single points
+    xyz = np.concatenate([C.clustered(1203, 40.0, 5), rng.uniform(0, 40.0, (805, 3)), rng.uniform(0, 400.0, (61, 3))])
+    w = np.exp(rng.normal(0, 0.3, len(xyz))) if weighted else None
+    buf = (rng.random(len(xyz)) < 0.4).astype(np.int32) if buffered else None
+    _check(eng, xyz, w, 1203, O.Params(0.5, 9.0, 5, nmu, True), buf)
+
+
+@pytest.mark.parametrize("n", [2, 15, 16, 17, 31, 33, 63, 64, 65, 127, 129])
+def test_chunk_edges(eng, monkeypatch, n):
+    # one x-row of n points: chunks of 16 / 32 / 64 and their remainders
+    rng = np.random.default_rng(n)
+    xyz = np.column_stack([np.sort(rng.uniform(0, 30.0, n)), rng.uniform(0, 1.0, n), rng.uniform(0, 1.0, n)])
+    w = rng.uniform(0.5, 2.0, n)
+    for group in ("16", "32", "64"):
+        monkeypatch.setenv("GS_PAIR_GROUP", group)
+        _check(eng, xyz, w, n // 2, O.Params(0.0, 12.0, 4, 3, False))
+
+
+@pytest.mark.parametrize("prec", ["fp32", "fp64"])
+def test_packed_histogram_drains(eng, prec):
+    # every pair in one bin: each work-group passes 2^20 increments of it, so the waves' scans drain it
+    # before the 22-bit counts run over; closed form n (n - 1), (sum w)^2 - sum w^2
+    n = 60000
+    rng = np.random.default_rng(3)
+    xyz = 100.0 + rng.uniform(0.0, 1.0, (n, 3))
+    w = rng.uniform(0.1, 1.0, n)
+    eng.set_catalogue(xyz, w, n)
+    r = eng.pcf2(0.0, 2.0, 1, 1, False, prec)
+    assert int(r["cnt"][0, 0, 0]) == n * (n - 1)
+    s, s2 = np.sum(w.astype(np.longdouble)), np.sum(w.astype(np.longdouble) ** 2)
+    exact = float(s * s - s2)
+    assert abs(r["wsum"][0, 0, 0] - exact) <= 1e-14 * exact
+
+
+@pytest.mark.parametrize("scale", [1e-40, 1e-12, 1e-7, 1e-3, 1e6, 1e9, 1e40])
+def test_scales_beyond_the_fp32_bounds(eng, scale):
+    # coordinates scaled by powers of ten: beyond the range of the FP32 mu estimate every pair is
+    # rechecked, and beyond that of its bin table the FP64 geometry runs
+    rng = np.random.default_rng(9)
+    xyz = (rng.uniform(0, 30.0, (700, 3)) - 7.0) * scale
+    _check(eng, xyz, None, 300, O.Params(1.0 * scale, 8.0 * scale, 4, 5, True))
+
+
+def test_cells_much_wider_than_rmax(eng):
+    # a few points in a box of 1e6 rmax: the grid's cells are widened to ~1e3 rmax and the FP32 guard
+    # bands with them
+    rng = np.random.default_rng(11)
+    a = rng.uniform(0, 1e6, (60, 3))
+    xyz = np.concatenate([a + rng.normal(0, 0.4, a.shape) for _ in range(6)])
+    _check(eng, xyz, None, 100, O.Params(0.1, 2.0, 4, 3, False))
