@@ -22,17 +22,6 @@ static int adjoint_impl(gs_ctx* c, const gs_params* p, const double* gN2, const 
     const bool rsd = nm >= 2, fp64 = p->precision == GS_FP64;
     CtxView v = view(c);
     const int64_t n = v.n_data + v.n_rand;
-    const int m = p->cell_div > 0 ? p->cell_div : default_cell_div(c, p->rmax, 2);
-    const int sx = pair_cell_sx();
-
-    (void)hipEventRecord(v.ev[0], v.stream);
-    double h;
-    if ((rc = ctx_build_grid(c, p->rmax, m, sx, &h)) || (rc = ctx_row_chunks(c))) return rc;
-    (void)hipEventRecord(v.ev[1], v.stream);
-    v = view(c);
-    const int mst = (int)std::ceil(p->rmax / h - 1e-12);
-    BinDesc B;
-    if ((rc = fill_bins(*p, (mst + 1) * h, ctx_xmax(c), v.wmax_d, v.wmax_r, B))) return rc;
     if (!(v.wsum_d > 0) && v.n_data > 0) return fail(GS_EINVAL, "data weights sum to zero");
     if (!(v.wsum_r > 0) && v.n_rand > 0) return fail(GS_EINVAL, "random weights sum to zero");
     const double inv_wd = v.n_data > 0 ? (double)(1.0L / v.wsum_d) : 0.0;
@@ -60,20 +49,44 @@ static int adjoint_impl(gs_ctx* c, const gs_params* p, const double* gN2, const 
                 half = false;
         }
     }
-    std::vector<Row> rows = half ? half_stencil(h, h / sx, p->rmax, mst) : full_stencil(h, h / sx, p->rmax, mst);
+    // the half-stencil kernel walks the pair kernel's grid and chunks, the full-stencil one its own
+    (void)hipEventRecord(v.ev[0], v.stream);
+    PairGrid q;
+    BinDesc B;
+    std::vector<Row> rows;
+    int mst = 1;
+    if (half) {
+        q = ctx_pair_grid(c, *p);
+        if ((rc = ctx_build_pair_grid(c, q)) || (rc = fill_pair_bins(*p, q, ctx_xmax(c), v.wmax_d, v.wmax_r, B))) return rc;
+        mst = q.mst;
+        half = !B.wide;     // beyond the FP32 geometry's range
+        rows = half_stencil(q.h, q.h / q.sx, p->rmax, mst);
+    }
+    if (!half) {
+        double h;
+        const int m = p->cell_div > 0 ? p->cell_div : default_cell_div(c, p->rmax, 2), sx = pair_cell_sx();
+        if ((rc = ctx_build_grid(c, p->rmax, m, sx, &h)) || (rc = ctx_row_chunks(c))) return rc;
+        mst = (int)std::ceil(p->rmax / h - 1e-12);
+        if ((rc = fill_bins(*p, (mst + 1) * h, ctx_xmax(c), v.wmax_d, v.wmax_r, B))) return rc;
+        rows = full_stencil(h, h / sx, p->rmax, mst);
+    }
+    if ((int)rows.size() > kMaxRows) return fail(GS_ELIMIT, "stencil too large");
+    (void)hipEventRecord(v.ev[1], v.stream);
+    v = view(c);
 
     GsExtra& X = *v.extra;
     const size_t g_off = ((sizeof(BinDesc) + 15) / 16) * 16;
     const size_t rows_off = g_off + ((size_t)nb * nm * 16 + 15) / 16 * 16;
     const int nblk_red = 256;
     if ((rc = X.params.reserve(rows_off + rows.size() * sizeof(Row) + 16)) || (rc = X.out.reserve(8)) ||
-        (rc = X.queue.reserve(16)) ||
+        (rc = X.queue.reserve(64 * kQueuePad)) ||
         (rc = X.dbl.reserve(2 * (size_t)n + 2 * nblk_red + 8 + 2 * (size_t)std::max<int64_t>(n, 1))))
         return rc;
     double* G = X.dbl.ptr;
     double* outd = out_dev ? out_dev : X.dbl.ptr + n;
     double* part = X.dbl.ptr + 2 * n;
-    unsigned long long* Gq = (unsigned long long*)(X.dbl.ptr + 2 * n + 2 * nblk_red + 8);   // [max(n, 1)][2]
+    unsigned long long* Glo = (unsigned long long*)(X.dbl.ptr + 2 * n + 2 * nblk_red + 8);  // [max(n, 1)] each
+    long long* Ghi = (long long*)Glo + std::max<int64_t>(n, 1);
     hipError_t e = hipMemcpyAsync(X.params.ptr, &B, sizeof(B), hipMemcpyHostToDevice, v.stream);
     if (e == hipSuccess)
         e = hipMemcpyAsync(X.params.ptr + g_off, gN2, (size_t)nb * nm * 8, hipMemcpyHostToDevice, v.stream);
@@ -83,45 +96,67 @@ static int adjoint_impl(gs_ctx* c, const gs_params* p, const double* gN2, const 
     if (e == hipSuccess && !rows.empty())
         e = hipMemcpyAsync(X.params.ptr + rows_off, rows.data(), rows.size() * sizeof(Row), hipMemcpyHostToDevice,
                            v.stream);
-    if (e == hipSuccess) e = hipMemsetAsync(X.queue.ptr, 0, 16 * sizeof(int32_t), v.stream);
+    if (e == hipSuccess) e = hipMemsetAsync(X.queue.ptr, 0, 64 * kQueuePad * sizeof(int32_t), v.stream);
     if (e == hipSuccess) e = hipMemsetAsync(X.out.ptr, 0, 8 * sizeof(unsigned long long), v.stream);
     if (e == hipSuccess) e = hipMemsetAsync(G, 0, (size_t)std::max<int64_t>(n, 1) * 8, v.stream);
-    if (e == hipSuccess && half) e = hipMemsetAsync(Gq, 0, (size_t)std::max<int64_t>(n, 1) * 16, v.stream);
+    if (e == hipSuccess && half) e = hipMemsetAsync(Glo, 0, (size_t)std::max<int64_t>(n, 1) * 16, v.stream);
     if (e != hipSuccess) return hip_fail(e, "adjoint parameter upload");
 
-    AdjArgs a{};
-    a.pw = v.pw;
-    a.ws = v.ws;
-    a.pl = v.pl;
-    a.flags = v.flags;
-    a.orig = v.orig;
-    a.cell_start = v.cell_start;
-    a.row_chunk = v.row_chunk;
-    a.rows = (const Row*)(X.params.ptr + rows_off);
-    a.bins = (const BinDesc*)X.params.ptr;
-    a.g2 = (const double*)(X.params.ptr + g_off);
-    a.g3 = a.g2 + nb * nm;
-    a.queue = X.queue.ptr;
-    a.G = G;
-    a.out_stats = X.out.ptr;
-    a.g = v.g;
-    a.g.m = mst;
-    a.nrows = (int)rows.size();
-    a.n_chunks = v.n_chunks;
-    a.inv_wd = inv_wd;
-    a.inv_wr = inv_wr;
-    a.Gq = Gq;
-    a.g_scale = std::ldexp(1.0, Fa);
-    a.w_scale = std::ldexp(1.0, Fb);
-    const int occ = half ? adjoint2h_occupancy(nb, nm, rsd) : adjoint2_occupancy(nb, nm, fp64, rsd);
-    int nblocks = std::max(1, std::min(v.n_cu * occ, std::max(v.n_chunks, 1)));
+    const double *g2 = (const double*)(X.params.ptr + g_off), *g3 = g2 + nb * nm;
     (void)hipEventRecord(v.ev[2], v.stream);
-    if (v.n_chunks > 0) {
-        e = half ? launch_adjoint2h(a, nb, nm, rsd, nblocks, v.stream)
-                 : launch_adjoint2(a, nb, nm, fp64, rsd, nblocks, v.stream);
+    if (half && n > 0) {
+        AdjHalfArgs a{};
+        a.pw = v.pw;
+        a.pl = v.pl;
+        a.flags = v.flags;
+        a.cell_start = v.cell_start;
+        a.chunks = v.chunks;
+        a.n_chunks_dev = v.row_chunk + (size_t)v.g.dim[1] * v.g.dim[2];
+        a.rows = (const Row*)(X.params.ptr + rows_off);
+        a.bins = (const BinDesc*)X.params.ptr;
+        a.queue = X.queue.ptr;
+        a.g = v.g;
+        a.g.m = mst;
+        a.nrows = (int)rows.size();
+        a.g2 = g2;
+        a.g3 = g3;
+        a.Glo = Glo;
+        a.Ghi = Ghi;
+        a.out_stats = X.out.ptr;
+        a.inv_wd = inv_wd;
+        a.inv_wr = inv_wr;
+        a.g_scale = std::ldexp(1.0, Fa);
+        a.w_scale = std::ldexp(1.0, Fb);
+        const bool logb = p->log_bins != 0;
+        const int waves = adjoint2h_occupancy(nb, nm, logb, v.has_buf) * (kWG / kWave);
+        e = launch_adjoint2h(a, nb, nm, logb, v.has_buf, walk_shape(a, q, n, kWG, waves, v.n_cu), v.stream);
         if (e != hipSuccess) return hip_fail(e, "adjoint kernel launch");
-        if (half && (e = launch_adj_fx(Gq, v.orig, n, F, G, v.stream)) != hipSuccess)
+        if ((e = launch_adj_fx(Glo, Ghi, v.orig, n, F, G, v.stream)) != hipSuccess)
             return hip_fail(e, "adjoint fixed-point conversion");
+    } else if (n > 0 && v.n_chunks > 0) {
+        AdjArgs a{};
+        a.pw = v.pw;
+        a.pl = v.pl;
+        a.flags = v.flags;
+        a.orig = v.orig;
+        a.cell_start = v.cell_start;
+        a.row_chunk = v.row_chunk;
+        a.rows = (const Row*)(X.params.ptr + rows_off);
+        a.bins = (const BinDesc*)X.params.ptr;
+        a.g2 = g2;
+        a.g3 = g3;
+        a.queue = X.queue.ptr;
+        a.G = G;
+        a.out_stats = X.out.ptr;
+        a.g = v.g;
+        a.g.m = mst;
+        a.nrows = (int)rows.size();
+        a.n_chunks = v.n_chunks;
+        a.inv_wd = inv_wd;
+        a.inv_wr = inv_wr;
+        const int nblocks = std::min(v.n_cu * adjoint2_occupancy(nb, nm, fp64, rsd), v.n_chunks);
+        e = launch_adjoint2(a, nb, nm, fp64, rsd, nblocks, v.stream);
+        if (e != hipSuccess) return hip_fail(e, "adjoint kernel launch");
     }
     (void)hipEventRecord(v.ev[3], v.stream);
     e = launch_adj_partials(G, v.w, n, v.n_data, inv_wd, inv_wr, part, nblk_red, v.stream);

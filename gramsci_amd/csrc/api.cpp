@@ -384,7 +384,6 @@ struct gs_ctx {
     int grid_sx = 1;
     DevBuf<int32_t> cell_of, cell_start, fill, chunk_nc, chunk_off, scan_tmp;
     DevBuf<double4> pw;
-    DevBuf<double> ws;          // sorted raw weights
     DevBuf<float4> pl;
     DevBuf<uint32_t> flags;
     DevBuf<int32_t> orig;
@@ -447,7 +446,7 @@ extern "C" int gs_destroy(gs_ctx* c)
     (void)hipStreamSynchronize(c->stream);
     c->xyz.release(); c->w.release(); c->buf.release();
     c->cell_of.release(); c->cell_start.release(); c->fill.release(); c->chunk_nc.release();
-    c->chunk_off.release(); c->chunks.release(); c->scan_tmp.release(); c->pw.release(); c->ws.release(); c->pl.release(); c->flags.release();
+    c->chunk_off.release(); c->chunks.release(); c->scan_tmp.release(); c->pw.release(); c->pl.release(); c->flags.release();
     c->orig.release();
     c->params.release(); c->out.release(); c->queue.release(); c->part.release(); c->wpart.release();
     extra_release(c->extra);
@@ -686,7 +685,7 @@ int grid_build_raw(const double* xyz, const double* w, const int32_t* buf, int64
     if (e == hipSuccess) e = exclusive_scan(b.fill, b.cell_start, ncell + 1, b.scan_tmp, st);
     if (e == hipSuccess) e = launch_fill_u32(b.fill, ncell + 1, 0u, st);
     if (e == hipSuccess)
-        e = launch_scatter(xyz, w, buf, n, n_data, g, b.cell_of, b.cell_start, b.fill, b.pw, b.ws, b.pl, b.flags, b.orig,
+        e = launch_scatter(xyz, w, buf, n, n_data, g, b.cell_of, b.cell_start, b.fill, b.pw, b.pl, b.flags, b.orig,
                            st);
     if (e != hipSuccess) return hip_fail(e, "grid build");
     *g_out = g;
@@ -707,7 +706,7 @@ hipError_t pair_chunks_raw(const GridDesc& g, int64_t n, int group, const GridBu
 static GridBufs grid_bufs(gs_ctx* c)
 {
     return GridBufs{c->cell_of.ptr, c->cell_start.ptr, c->fill.ptr, c->chunk_nc.ptr, c->chunk_off.ptr, c->scan_tmp.ptr,
-                    c->pw.ptr, c->ws.ptr, c->pl.ptr, c->flags.ptr, c->orig.ptr, c->chunks.ptr};
+                    c->pw.ptr, c->pl.ptr, c->flags.ptr, c->orig.ptr, c->chunks.ptr};
 }
 
 int build_grid(gs_ctx* c, double h, int sx)
@@ -719,7 +718,7 @@ int build_grid(gs_ctx* c, double h, int sx)
     if (ncell > (1 << 26)) return fail(GS_ELIMIT, "grid too large (%lld cells)", (long long)ncell);
     int rc;
     if ((rc = c->cell_of.reserve(n)) || (rc = c->cell_start.reserve(ncell + 1)) || (rc = c->fill.reserve(ncell + 1)) ||
-        (rc = c->scan_tmp.reserve(scan_scratch_size(ncell + 1))) || (rc = c->pw.reserve(n)) || (rc = c->ws.reserve(n)) ||
+        (rc = c->scan_tmp.reserve(scan_scratch_size(ncell + 1))) || (rc = c->pw.reserve(n)) ||
         (rc = c->pl.reserve(n)) || (rc = c->flags.reserve(n)) || (rc = c->orig.reserve(n)))
         return rc;
     GridDesc g;
@@ -749,6 +748,17 @@ static int build_chunks(gs_ctx* c, int group)
     if (e != hipSuccess) return hip_fail(e, "row chunks");
     c->chunk_group = group;
     return GS_OK;
+}
+
+PairGrid ctx_pair_grid(const gs_ctx* c, const gs_params& p)
+{
+    return pair_grid(c->n_data + c->n_rand, c->bbox, p.rmax, p.cell_div, (int64_t)1 << 24);
+}
+
+int ctx_build_pair_grid(gs_ctx* c, const PairGrid& q)
+{
+    int rc = build_grid(c, q.h, q.sx);
+    return rc ? rc : build_chunks(c, q.group);
 }
 
 int ctx_row_chunks(gs_ctx* c)
@@ -924,20 +934,28 @@ int pair2_shape(const PairVariant& v, PairShape* out)
     return GS_OK;
 }
 
-// Work split and launch of the pair kernel over one catalogue's chunks (a: the arrays and outputs).
-hipError_t pair_launch(PairArgs& a, const PairVariant& var, const PairShape& shape, const PairGrid& q, int64_t n,
-                       int n_cu, hipStream_t st)
+// Work split of a walk over one catalogue's chunks on work-groups of wg threads, `waves` waves per CU; returns
+// the number of work-groups.
+int walk_shape(WalkArgs& a, const PairGrid& q, int64_t n, int wg, int waves, int n_cu)
 {
     a.group = q.group;
     a.cap_cells = (float)q.cap_cells;
-    a.reps = shape.reps;
-    a.planes = shape.planes;
     a.lg_parts = pair_lg_parts(n, q);
     // no more work-groups than items could fill, a multiple of 8 (the same number on each XCD)
-    const int64_t wpg = shape.wg / kWave;
+    const int64_t wpg = wg / kWave;
     const int64_t items = max_chunks(n, (int64_t)a.g.dim[1] * a.g.dim[2], q.group) << a.lg_parts;
-    const int64_t nblocks = std::min<int64_t>((int64_t)n_cu * shape.waves / wpg, (items + wpg - 1) / wpg);
-    return launch_pair2(a, var, (int)((nblocks + 7) / 8 * 8), shape.wg, st);
+    const int64_t nblocks = std::min<int64_t>((int64_t)n_cu * waves / wpg, (items + wpg - 1) / wpg);
+    return (int)((nblocks + 7) / 8 * 8);
+}
+
+// Launch of the pair kernel over one catalogue's chunks (a: the arrays and outputs).
+hipError_t pair_launch(PairArgs& a, const PairVariant& var, const PairShape& shape, const PairGrid& q, int64_t n,
+                       int n_cu, hipStream_t st)
+{
+    a.reps = shape.reps;
+    a.planes = shape.planes;
+    const int nblocks = walk_shape(a, q, n, shape.wg, shape.waves, n_cu);
+    return launch_pair2(a, var, nblocks, shape.wg, st);
 }
 
 // Pair kernel outputs (counts [3][nb][nm], 128-bit class sums, statistics) -> the C ABI's outputs:
@@ -992,13 +1010,12 @@ extern "C" int gs_count_2pcf(gs_ctx* c, const gs_params* p, uint64_t* cnt, doubl
     const int nbt = 3 * nb * nm;
     const bool weighted = c->has_w;
     const int64_t n = c->n_data + c->n_rand;
-    const PairGrid q = pair_grid(n, c->bbox, p->rmax, p->cell_div, (int64_t)1 << 24);
+    const PairGrid q = ctx_pair_grid(c, *p);
     std::vector<Row> rows = half_stencil(q.h, q.h / q.sx, p->rmax, q.mst);
     if ((int)rows.size() > kMaxRows) return fail(GS_ELIMIT, "stencil too large");
 
     (void)hipEventRecord(c->ev[0], c->stream);
-    if ((rc = build_grid(c, q.h, q.sx))) return rc;
-    if ((rc = build_chunks(c, q.group))) return rc;
+    if ((rc = ctx_build_pair_grid(c, q))) return rc;
     (void)hipEventRecord(c->ev[1], c->stream);
 
     double xmax = 0;
@@ -1132,12 +1149,12 @@ CtxView view(gs_ctx* c)
     for (int k = 0; k < 6; ++k) v.bbox[k] = c->bbox[k];
     v.g = c->g;
     v.pw = c->pw.ptr;
-    v.ws = c->ws.ptr;
     v.flags = c->flags.ptr;
     v.orig = c->orig.ptr;
     v.cell_start = c->cell_start.ptr;
     v.pl = c->pl.ptr;
     v.row_chunk = c->chunk_off.ptr;
+    v.chunks = c->chunks.ptr;
     v.w = c->has_w ? c->w.ptr : nullptr;
     v.n_chunks = c->n_chunks;
     v.extra = &c->extra;

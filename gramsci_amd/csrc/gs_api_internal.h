@@ -60,7 +60,6 @@ struct GsBatch {
     DevBuf<unsigned char> big;           // 3PCF: device-memory neighbour lists
     DevBuf<unsigned char> d_regions, params;
     DevBuf<double4> pw;
-    DevBuf<double> ws;                   // sorted raw weights
     DevBuf<float4> pl;
     DevBuf<int4> chunks;                 // pair kernel: chunk descriptors
     DevBuf<uint32_t> flags;
@@ -108,12 +107,12 @@ struct CtxView {
     double bbox[6];
     GridDesc g;
     const double4* pw;
-    const double* ws;           // sorted raw weights
     const uint32_t* flags;
     const int32_t* orig;
     const int32_t* cell_start;
     const float4* pl;
     const int32_t* row_chunk;
+    const int4* chunks;
     const double* w;            // raw weights, original order (NULL for unit weights)
     int32_t n_chunks;
     GsExtra* extra;
@@ -127,14 +126,14 @@ int ctx_set_device(gs_ctx* c);
 int ctx_upload(gs_ctx* c, const double* xyz, const double* w, const int32_t* buf, int64_t n);
 double round11(double h);
 int ctx_build_grid(gs_ctx* c, double rmax, int m, int sx, double* h_out);
-// row chunks of kChunk points of the context's grid for the adjoint kernels: view().row_chunk, view().n_chunks
+// row chunks of kChunk points of the context's grid for the full-stencil adjoint kernel: view().row_chunk,
+// view().n_chunks
 int ctx_row_chunks(gs_ctx* c);
-// device buffers of a grid build (sizes: cell_of, pw, ws, pl, flags, orig n; cell_start, fill ncell + 1;
+// device buffers of a grid build (sizes: cell_of, pw, pl, flags, orig n; cell_start, fill ncell + 1;
 // scan_tmp scan_scratch_size(ncell + 1)) and of its chunks (chunk_nc, chunk_off rows + 1; chunks max_chunks)
 struct GridBufs {
     int32_t *cell_of, *cell_start, *fill, *chunk_nc, *chunk_off, *scan_tmp;
     double4* pw;
-    double* ws;
     float4* pl;
     uint32_t* flags;
     int32_t* orig;
@@ -170,6 +169,9 @@ struct PairShape {
 int pair2_shape(const PairVariant& v, PairShape* out);
 // log2 of the work items per chunk for n points on that grid
 int pair_lg_parts(int64_t n, const PairGrid& q);
+int walk_shape(WalkArgs& a, const PairGrid& q, int64_t n, int wg, int waves, int n_cu);
+PairGrid ctx_pair_grid(const gs_ctx* c, const gs_params& p);
+int ctx_build_pair_grid(gs_ctx* c, const PairGrid& q);
 hipError_t pair_launch(PairArgs& a, const PairVariant& var, const PairShape& shape, const PairGrid& q, int64_t n,
                        int n_cu, hipStream_t st);
 double choose_h_bbox(const double* bbox, double rmax, int m, int64_t max_cells, int sx);

@@ -187,6 +187,14 @@ __device__ __forceinline__ int next_item(int32_t* queue, int n, int xcd, int& tr
     return -1;
 }
 
+// v, in a way the compiler cannot see through: keeps what is computed from it inside a rarely run block
+// instead of in registers over the loop around it
+__device__ __forceinline__ int opaque(int v)
+{
+    asm volatile("" : "+v"(v));
+    return v;
+}
+
 // Work items [0, n) in 64 segments, 8 per XCD, each with a counter on a cache line of its own (device-wide
 // atomics on one line run one after another, about 40 ns each: measured).  A wave's first item is its own
 // slot of its home segment, taken without an atomic; later ones come from the segment's counter, and when
@@ -224,8 +232,9 @@ struct ItemQueue {
                 k = lo(seg) + slots(seg) + __builtin_amdgcn_readfirstlane(k);
                 if (k < lo(seg + 1)) return k;
             }
-            const int used = __hip_atomic_load(&counters[lane * kQueuePad], __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT);
-            const unsigned long long m = __ballot(used < lo(lane + 1) - lo(lane) - slots(lane));
+            const int s = opaque(lane);
+            const int used = __hip_atomic_load(&counters[s * kQueuePad], __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT);
+            const unsigned long long m = __ballot(used < lo(s + 1) - lo(s) - slots(s));
             if (!m) return -1;
             // the first such segment after this one, cyclically: the own XCD's come first
             const int sh = (seg + 1) & 63;

@@ -20,7 +20,7 @@ hipError_t exclusive_scan(const int32_t* in, int32_t* out, int64_t n, int32_t* s
 int64_t scan_scratch_size(int64_t n);
 hipError_t launch_scatter(const double* xyz, const double* w, const int32_t* buf, int64_t n, int64_t n_data,
                           const GridDesc& g, const int32_t* cell_of, const int32_t* start, int32_t* fill,
-                          double4* pw, double* ws, float4* pl, uint32_t* flags, int32_t* orig, hipStream_t st);
+                          double4* pw, float4* pl, uint32_t* flags, int32_t* orig, hipStream_t st);
 hipError_t launch_row_chunks(const int32_t* start, int nx, int nrow, int group, int32_t* nch, hipStream_t st);
 
 // batched regions (grid.hip)
@@ -30,7 +30,7 @@ hipError_t launch_cell_count_b(const double* xyz, int64_t n, const int32_t* off,
 hipError_t launch_scatter_b(const double* xyz, const double* w, const int32_t* buf, int64_t n, const int32_t* off,
                             int nreg, const RegionDesc* reg, double h, double hx, const int32_t* cell_of,
                             const int32_t* start,
-                            int32_t* fill, double4* pw, double* ws, float4* pl, uint32_t* flags, int32_t* orig,
+                            int32_t* fill, double4* pw, float4* pl, uint32_t* flags, int32_t* orig,
                             hipStream_t st);
 hipError_t launch_row_chunks_b(const int32_t* start, const RegionDesc* reg, const int32_t* row_base, int nreg,
                                int nrow_tot, int group, int32_t* nch, hipStream_t st);
@@ -41,33 +41,35 @@ hipError_t launch_region_flag(const float* xyz, int64_t n, const float* ext, int
 hipError_t launch_region_scatter(const float* xyz, int64_t n, const float* box, const int32_t* flag, const int32_t* pos,
                                  int32_t* idx, int32_t* buf, hipStream_t st);
 
-// Arguments of the persistent 2PCF pair kernel (pair2.hip).
-struct PairArgs {
+// The half-stencil walk of the pair and adjoint kernels (gs_pair_tiles.h).
+struct WalkArgs {
     const double4* pw;          // sorted points: x, y, z, raw weight
     const float4* pl;           // sorted: .w the cell x index
     const uint32_t* flags;      // sorted: bit0 random, bit1 never-apex
     const int32_t* cell_start;  // ncell+1
     const int4* chunks;         // chunk descriptors (launch_chunks)
+    const int32_t* n_chunks_dev;
     const Row* rows;            // half stencil
     const BinDesc* bins;        // device copy
     int32_t* queue;             // 64 work counters (dev::ItemQueue), zeroed before launch
+    GridDesc g;
+    int32_t nrows;
+    int32_t group;              // points per chunk: 16, 32 or 64
+    int32_t lg_parts;           // log2 of the work items per chunk
+    float cap_cells;            // largest extent of a chunk in x cells, less one
+    const RegionDesc* regions;  // batched regions (nreg > 0): per-region grids
+    int32_t nreg;
+};
+
+// Arguments of the persistent 2PCF pair kernel (pair2.hip).
+struct PairArgs : WalkArgs {
     unsigned long long* out_cnt;    // [2][3][nb][nm]: plane 0 counts for both directions, plane 1 for one
     unsigned long long* out_w;      // [2][3][nb][nm][2] 128-bit fixed point (lo, hi)
     unsigned long long* out_stats;  // [0] candidates, [1] rechecks, [2] overflow pairs
     int64_t copy_stride;        // words between the copies of the outputs (pair_copy_words)
     int32_t copies;             // power of two <= 64; work-group b adds to copy b mod copies
-    int32_t nrows;
-    GridDesc g;
-    const int32_t* n_chunks_dev;
-    int32_t group;              // points per chunk: 16, 32 or 64
-    int32_t lg_parts;           // log2 of the work items per chunk
-    float cap_cells;            // largest extent of a chunk in x cells, less one
     int32_t reps;               // LDS histogram replicas (power of two <= 32)
     int32_t planes;             // with buffer points: 2 if the LDS histogram has a plane per direction count
-    // batched regions (nreg > 0): per-region grids and outputs; each wave keeps a private
-    // histogram of its current region
-    const RegionDesc* regions;
-    int32_t nreg;
 };
 
 // One copy of the pair kernel's outputs: [nreg][2][nbt] counts, [nreg][2][nbt][2] sums, 4 statistics.
@@ -187,7 +189,6 @@ int quad4_occupancy(const QuadArgs& a, int nb, bool weighted);
 // Arguments of the persistent 2PCF adjoint kernel (adjoint.hip).
 struct AdjArgs {
     const double4* pw;
-    const double* ws;           // sorted raw weights alone
     const float4* pl;
     const uint32_t* flags;
     const int32_t* orig;
@@ -204,21 +205,28 @@ struct AdjArgs {
     int32_t nrows;
     int32_t n_chunks;
     double inv_wd, inv_wr;
-    // half-stencil FP32 kernel: per sorted point a 128-bit fixed-point sum [n][2] (lo, hi; zeroed before
-    // launch) of G * 2^F, with the dL/dN tables scaled by g_scale and the normalised weights by w_scale
-    // (g_scale * w_scale = 2^F)
-    unsigned long long* Gq;
-    double g_scale, w_scale;
+};
+// Arguments of the half-stencil FP32 adjoint kernel: per sorted point a fixed-point sum Ghi * 2^32 + Glo of
+// G * 2^F (zeroed before launch), with the dL/dN tables scaled by g_scale and the normalised weights by
+// w_scale (g_scale * w_scale = 2^F).
+struct AdjHalfArgs : WalkArgs {
+    const double* g2;           // dL/dN2 [nb][nm]
+    const double* g3;           // dL/dN3 [nb][nm]
+    unsigned long long* Glo;
+    long long* Ghi;
+    unsigned long long* out_stats;  // candidates, rechecks
+    double inv_wd, inv_wr, g_scale, w_scale;
 };
 size_t adjoint2_lds_bytes(int nb, int nm, bool fp64);
 hipError_t launch_adjoint2(const AdjArgs& a, int nb, int nm, bool fp64, bool rsd, int nblocks, hipStream_t st);
 int adjoint2_occupancy(int nb, int nm, bool fp64, bool rsd);
 // half-stencil FP32 adjoint (rows: half stencil): every unordered pair once, its term added to both ends
-size_t adjoint2h_lds_bytes(int nb, int nm);
-hipError_t launch_adjoint2h(const AdjArgs& a, int nb, int nm, bool rsd, int nblocks, hipStream_t st);
-int adjoint2h_occupancy(int nb, int nm, bool rsd);
-// G[orig[k]] = Gq[k] * 2^-F (the 128-bit sums as doubles, original order)
-hipError_t launch_adj_fx(const unsigned long long* Gq, const int32_t* orig, int64_t n, int F, double* G, hipStream_t st);
+size_t adjoint2h_lds_bytes(int nb, int nm, bool buf);
+hipError_t launch_adjoint2h(const AdjHalfArgs& a, int nb, int nm, bool logb, bool buf, int nblocks, hipStream_t st);
+int adjoint2h_occupancy(int nb, int nm, bool logb, bool buf);
+// G[orig[k]] = (Ghi[k] * 2^32 + Glo[k]) * 2^-F (the sums as doubles, original order)
+hipError_t launch_adj_fx(const unsigned long long* Glo, const long long* Ghi, const int32_t* orig, int64_t n, int F,
+                         double* G, hipStream_t st);
 hipError_t launch_adj_partials(const double* G, const double* w, int64_t n, int64_t n_data, double inv_wd,
                                double inv_wr, double* part, int nblk, hipStream_t st);
 hipError_t launch_adj_finish(const double* G, int64_t n, int64_t n_data, double s_d, double s_r, double inv_wd,

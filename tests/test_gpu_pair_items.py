@@ -84,3 +84,23 @@ def test_cells_much_wider_than_rmax(eng):
     a = rng.uniform(0, 1e6, (60, 3))
     xyz = np.concatenate([a + rng.normal(0, 0.4, a.shape) for _ in range(6)])
     _check(eng, xyz, None, 100, O.Params(0.1, 2.0, 4, 3, False))
+
+
+@pytest.mark.parametrize("group", ["16", "32", "64"])
+@pytest.mark.parametrize("parts", ["1", "16"])
+@pytest.mark.parametrize("buffered,nmu,log", [(False, 6, True), (True, 5, False), (True, 1, True)])
+def test_adjoint_groups_and_parts(eng, monkeypatch, group, parts, buffered, nmu, log):
+    monkeypatch.setenv("GS_PAIR_GROUP", group)
+    monkeypatch.setenv("GS_PAIR_PARTS", parts)
+    rng = np.random.default_rng(17)
+    # dense points (more than 64 tiles to a chunk, so that its sums are flushed within an item), sparse ones
+    xyz = np.concatenate([rng.uniform(10.0, 22.0, (4700, 3)), rng.uniform(0, 60.0, (301, 3))])
+    w = np.exp(rng.normal(0, 0.3, len(xyz)))
+    buf = (rng.random(len(xyz)) < 0.4).astype(np.int32) if buffered else None
+    p = O.Params(0.5 if log else 0.0, 12.0, 5, nmu, log)
+    g2, g3 = rng.normal(size=(2, 5, nmu))
+    ref = O.adjoint2(xyz, w, 2000, p, g2, g3, buf=buf)
+    eng.set_catalogue(xyz, w, 2000, buf)
+    got = eng.adjoint2(g2, g3, p.rmin, p.rmax, p.nbins, p.nmu, log)
+    # each term is rounded to 2^-50 of the largest; at most 5000 terms a point
+    assert np.max(np.abs(got - ref)) <= 1e-11 * np.max(np.abs(ref))
