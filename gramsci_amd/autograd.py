@@ -47,8 +47,7 @@ class WeightedXi(torch.autograd.Function):
         # derivatives non-finite; any other non-finite value is passed on, so the adjoint
         # returns NaN gradients as for a loss that depends on an undefined xi.
         zero = g == 0
-        g2 = torch.where(zero, torch.zeros_like(g), g / n3).cpu().numpy()
-        g3 = torch.where(zero, torch.zeros_like(g), -g * n2 / (n3 * n3)).cpu().numpy()
+        g2, g3 = torch.where(zero, torch.zeros_like(g), torch.stack((g / n3, -g * n2 / (n3 * n3)))).cpu().numpy()
         # the context may hold another catalogue since the forward pass
         if eng.generation != ctx.generation:
             eng.set_catalogue(ctx.xyz, wd, ctx.n_data, ctx.buf)

@@ -101,13 +101,22 @@ __global__ __launch_bounds__(kWG) void k_adjoint2(AdjArgs a)
         const int n_i = min(kChunk, re - i0);
         const int i = i0 + lane;
         const bool vi = lane < n_i;
-        const int cx_first = (int)a.pl[i0].w;
-        const int cx_last = (int)a.pl[i0 + n_i - 1].w;
+        const int cx_first = a.cell[i0].x;
+        const int cx_last = a.cell[i0 + n_i - 1].x;
 
+        // FP32: cell-local coordinates, and the x cell
+        auto local = [&](const double4& P, int cx, int ly, int lz) {
+            return make_float4((float)(P.x - (a.g.lo[0] + cx * a.g.hx)), (float)(P.y - (a.g.lo[1] + ly * a.g.h)),
+                               (float)(P.z - (a.g.lo[2] + lz * a.g.h)), (float)cx);
+        };
         double4 Pi = make_double4(0, 0, 0, 0);
         float4 Li = make_float4(0, 0, 0, 0);
         uint32_t fi = 2u;
-        if (vi) { Pi = a.pw[i]; Li = a.pl[i]; fi = a.flags[i]; }
+        if (vi) {
+            Pi = a.pw[i];
+            if constexpr (!FP64) Li = local(Pi, a.cell[i].x, cy, cz);
+            fi = a.flags[i];
+        }
         const int ri = fi & 1, ci = (fi & 2) ? 0 : 1;
         const float ax32 = (float)Pi.x, ay32 = (float)Pi.y, az32 = (float)Pi.z;
         double G = 0.0;
@@ -132,7 +141,7 @@ __global__ __launch_bounds__(kWG) void k_adjoint2(AdjArgs a)
                     if constexpr (FP64) {
                         tx[lane] = Pj.x; ty[lane] = Pj.y; tz[lane] = Pj.z;
                     } else {
-                        tl[lane] = a.pl[j];
+                        tl[lane] = local(Pj, a.cell[j].x, by, bz);
                     }
                     tw[lane] = (fj & 1u) ? -Pj.w * inv_wr : Pj.w * inv_wd;   // normalised weight
                     tf[lane] = fj;
@@ -391,10 +400,13 @@ __global__ __launch_bounds__(256) void k_adj_fx(const unsigned long long* __rest
     }
 }
 
-// per-block partial sums of wn*G over data (slot 0) and randoms (slot 1)
+// Per-block partial sums of wn*G over data (slot 0) and randoms (slot 1); the last block to finish adds them
+// up in double-double (more than the long double the host used) into part[2 gridDim.x ..] and hands the pair
+// kernel's counters to the host.  stats[2] is the blocks' ticket.
 __global__ __launch_bounds__(256) void k_adj_partials(const double* __restrict__ G, const double* __restrict__ w,
                                                       int64_t n, int64_t n_data, double inv_wd, double inv_wr,
-                                                      double* __restrict__ part)
+                                                      double* part, unsigned long long* stats,
+                                                      unsigned long long* host_stats)
 {
     __shared__ double sd[256], sr[256];
     double a = 0.0, b = 0.0;
@@ -417,12 +429,37 @@ __global__ __launch_bounds__(256) void k_adj_partials(const double* __restrict__
         part[2 * blockIdx.x] = sd[0];
         part[2 * blockIdx.x + 1] = sr[0];
     }
+    if (!last_block((unsigned*)&stats[2])) return;
+    // thread t < 64: partials t, t + 64, ... of both sums, then a tree; (hi, lo) stays exact to ~2^-104
+    double hi[2] = {0.0, 0.0}, lo[2] = {0.0, 0.0};
+    auto add = [&](int q, double h, double l) {
+        const double s = hi[q] + h, bb = s - hi[q];
+        const double err = (hi[q] - (s - bb)) + (h - bb);
+        hi[q] = s;
+        lo[q] += err + l;
+    };
+    if (threadIdx.x < 64) {
+        for (int k = threadIdx.x; k < (int)gridDim.x; k += 64)
+            for (int q = 0; q < 2; ++q) add(q, load_agent(&part[2 * k + q]), 0.0);
+        for (int off = 32; off > 0; off >>= 1)
+            for (int q = 0; q < 2; ++q) {
+                const double h = __shfl_down(hi[q], off, 64), l = __shfl_down(lo[q], off, 64);
+                add(q, h, l);
+            }
+        if (threadIdx.x == 0) {
+            // a non-finite sum has a NaN in lo: its hi alone is the result
+            for (int q = 0; q < 2; ++q) part[2 * gridDim.x + q] = isfinite(hi[q]) ? hi[q] + lo[q] : hi[q];
+            for (int q = 0; q < 2; ++q) host_stats[q] = load_agent(&stats[q]);
+        }
+    }
 }
 
+// sums: of wn*G over data and randoms
 __global__ __launch_bounds__(256) void k_adj_finish(const double* __restrict__ G, int64_t n, int64_t n_data,
-                                                    double s_d, double s_r, double inv_wd, double inv_wr,
+                                                    const double* __restrict__ sums, double inv_wd, double inv_wr,
                                                     double* __restrict__ out)
 {
+    const double s_d = sums[0], s_r = sums[1];
     for (int64_t k = blockIdx.x * (int64_t)blockDim.x + threadIdx.x; k < n; k += (int64_t)gridDim.x * blockDim.x)
         out[k] = k < n_data ? (G[k] - s_d) * inv_wd : -(G[k] + s_r) * inv_wr;
 }
@@ -507,18 +544,20 @@ int adjoint2_occupancy(int nb, int nm, bool fp64, bool rsd)
 }
 
 hipError_t launch_adj_partials(const double* G, const double* w, int64_t n, int64_t n_data, double inv_wd,
-                               double inv_wr, double* part, int nblk, hipStream_t st)
+                               double inv_wr, double* part, int nblk, unsigned long long* stats,
+                               unsigned long long* host_stats, hipStream_t st)
 {
-    hipLaunchKernelGGL(k_adj_partials, dim3(nblk), dim3(256), 0, st, G, w, n, n_data, inv_wd, inv_wr, part);
+    hipLaunchKernelGGL(k_adj_partials, dim3(nblk), dim3(256), 0, st, G, w, n, n_data, inv_wd, inv_wr, part, stats,
+                       host_stats);
     return hipGetLastError();
 }
 
-hipError_t launch_adj_finish(const double* G, int64_t n, int64_t n_data, double s_d, double s_r, double inv_wd,
+hipError_t launch_adj_finish(const double* G, int64_t n, int64_t n_data, const double* sums, double inv_wd,
                              double inv_wr, double* out, hipStream_t st)
 {
     int nblk = (int)std::min<int64_t>((n + 255) / 256, 65535);
     if (nblk < 1) nblk = 1;
-    hipLaunchKernelGGL(k_adj_finish, dim3(nblk), dim3(256), 0, st, G, n, n_data, s_d, s_r, inv_wd, inv_wr, out);
+    hipLaunchKernelGGL(k_adj_finish, dim3(nblk), dim3(256), 0, st, G, n, n_data, sums, inv_wd, inv_wr, out);
     return hipGetLastError();
 }
 

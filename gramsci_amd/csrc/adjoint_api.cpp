@@ -49,57 +49,61 @@ static int adjoint_impl(gs_ctx* c, const gs_params* p, const double* gN2, const 
                 half = false;
         }
     }
-    // the half-stencil kernel walks the pair kernel's grid and chunks, the full-stencil one its own
-    (void)hipEventRecord(v.ev[0], v.stream);
+    // The half-stencil kernel walks the pair kernel's grid, the full-stencil one its own.  Parameters (bins,
+    // dL/dN tables, stencil rows) go to the device in one copy from pinned memory; the counters come back
+    // through it, written by a kernel.
+    GsExtra& X = *v.extra;
+    HostBuf& H = ctx_host(c);
+    const size_t ng = (size_t)nb * nm, g_off = (sizeof(BinDesc) + 15) / 16 * 16, rows_off = g_off + (ng * 16 + 15) / 16 * 16;
+    const size_t stats_off = rows_off + kMaxRows * sizeof(Row);
+    double t64[kMaxBins + 2];
+    if ((rc = ctx_thresholds(c, *p, t64)) || (rc = H.reserve(stats_off + 16)) || (rc = X.params.reserve(stats_off)))
+        return rc;
+    BinDesc& B = *(BinDesc*)H.ptr;
     PairGrid q;
-    BinDesc B;
-    std::vector<Row> rows;
-    int mst = 1;
     if (half) {
         q = ctx_pair_grid(c, *p);
-        if ((rc = ctx_build_pair_grid(c, q)) || (rc = fill_pair_bins(*p, q, ctx_xmax(c), v.wmax_d, v.wmax_r, B))) return rc;
-        mst = q.mst;
+        if ((rc = fill_pair_bins(*p, t64, q, ctx_xmax(c), v.wmax_d, v.wmax_r, B))) return rc;
         half = !B.wide;     // beyond the FP32 geometry's range
-        rows = half_stencil(q.h, q.h / q.sx, p->rmax, mst);
     }
-    if (!half) {
+    const int nblk_red = 256;
+    const size_t n1 = (size_t)std::max<int64_t>(n, 1), queue_bytes = 64 * kQueuePad * sizeof(int32_t);
+    std::vector<Row> rows;
+    int mst;
+    unsigned char* z = nullptr;     // cleared: work counters, {candidates, rechecks, ticket}, fixed-point sums
+    (void)hipEventRecord(v.ev[0], v.stream);
+    if (half) {
+        mst = q.mst;
+        rows = half_stencil(q.h, q.h / q.sx, p->rmax, mst);
+        if ((rc = ctx_build_pair_grid(c, q, (queue_bytes + 256 + n1 * 16 + 255) / 256 * 256, &z))) return rc;
+    } else {
         double h;
         const int m = p->cell_div > 0 ? p->cell_div : default_cell_div(c, p->rmax, 2), sx = pair_cell_sx();
         if ((rc = ctx_build_grid(c, p->rmax, m, sx, &h)) || (rc = ctx_row_chunks(c))) return rc;
         mst = (int)std::ceil(p->rmax / h - 1e-12);
-        if ((rc = fill_bins(*p, (mst + 1) * h, ctx_xmax(c), v.wmax_d, v.wmax_r, B))) return rc;
+        if ((rc = fill_bins(*p, t64, (mst + 1) * h, ctx_xmax(c), v.wmax_d, v.wmax_r, B))) return rc;
         rows = full_stencil(h, h / sx, p->rmax, mst);
+        if ((rc = X.queue.reserve((queue_bytes + 256) / 4))) return rc;
+        z = (unsigned char*)X.queue.ptr;
     }
     if ((int)rows.size() > kMaxRows) return fail(GS_ELIMIT, "stencil too large");
-    (void)hipEventRecord(v.ev[1], v.stream);
+    if ((rc = X.dbl.reserve(2 * n1 + 2 * nblk_red + 8))) return rc;
     v = view(c);
-
-    GsExtra& X = *v.extra;
-    const size_t g_off = ((sizeof(BinDesc) + 15) / 16) * 16;
-    const size_t rows_off = g_off + ((size_t)nb * nm * 16 + 15) / 16 * 16;
-    const int nblk_red = 256;
-    if ((rc = X.params.reserve(rows_off + rows.size() * sizeof(Row) + 16)) || (rc = X.out.reserve(8)) ||
-        (rc = X.queue.reserve(64 * kQueuePad)) ||
-        (rc = X.dbl.reserve(2 * (size_t)n + 2 * nblk_red + 8 + 2 * (size_t)std::max<int64_t>(n, 1))))
-        return rc;
     double* G = X.dbl.ptr;
     double* outd = out_dev ? out_dev : X.dbl.ptr + n;
-    double* part = X.dbl.ptr + 2 * n;
-    unsigned long long* Glo = (unsigned long long*)(X.dbl.ptr + 2 * n + 2 * nblk_red + 8);  // [max(n, 1)] each
-    long long* Ghi = (long long*)Glo + std::max<int64_t>(n, 1);
-    hipError_t e = hipMemcpyAsync(X.params.ptr, &B, sizeof(B), hipMemcpyHostToDevice, v.stream);
-    if (e == hipSuccess)
-        e = hipMemcpyAsync(X.params.ptr + g_off, gN2, (size_t)nb * nm * 8, hipMemcpyHostToDevice, v.stream);
-    if (e == hipSuccess)
-        e = hipMemcpyAsync(X.params.ptr + g_off + (size_t)nb * nm * 8, gN3, (size_t)nb * nm * 8,
-                           hipMemcpyHostToDevice, v.stream);
-    if (e == hipSuccess && !rows.empty())
-        e = hipMemcpyAsync(X.params.ptr + rows_off, rows.data(), rows.size() * sizeof(Row), hipMemcpyHostToDevice,
-                           v.stream);
-    if (e == hipSuccess) e = hipMemsetAsync(X.queue.ptr, 0, 64 * kQueuePad * sizeof(int32_t), v.stream);
-    if (e == hipSuccess) e = hipMemsetAsync(X.out.ptr, 0, 8 * sizeof(unsigned long long), v.stream);
-    if (e == hipSuccess) e = hipMemsetAsync(G, 0, (size_t)std::max<int64_t>(n, 1) * 8, v.stream);
-    if (e == hipSuccess && half) e = hipMemsetAsync(Glo, 0, (size_t)std::max<int64_t>(n, 1) * 16, v.stream);
+    double* part = X.dbl.ptr + 2 * n1;
+    int32_t* queue = (int32_t*)z;
+    unsigned long long* stats = (unsigned long long*)(z + queue_bytes);
+    unsigned long long* Glo = (unsigned long long*)(z + queue_bytes + 256);     // half: [n1] each
+    long long* Ghi = (long long*)Glo + n1;
+    std::copy(gN2, gN2 + ng, (double*)(H.ptr + g_off));
+    std::copy(gN3, gN3 + ng, (double*)(H.ptr + g_off) + ng);
+    std::copy(rows.begin(), rows.end(), (Row*)(H.ptr + rows_off));
+    unsigned long long* const h_stats = (unsigned long long*)(H.ptr + stats_off);
+    hipError_t e = hipMemcpyAsync(X.params.ptr, H.ptr, rows_off + rows.size() * sizeof(Row), hipMemcpyHostToDevice,
+                                  v.stream);
+    if (e == hipSuccess && !half) e = launch_fill_u32(z, (int64_t)(queue_bytes + 256) / 4, 0u, v.stream);
+    if (e == hipSuccess && !half) e = launch_fill_u32(G, (int64_t)n1 * 2, 0u, v.stream);
     if (e != hipSuccess) return hip_fail(e, "adjoint parameter upload");
 
     const double *g2 = (const double*)(X.params.ptr + g_off), *g3 = g2 + nb * nm;
@@ -107,14 +111,12 @@ static int adjoint_impl(gs_ctx* c, const gs_params* p, const double* gN2, const 
     if (half && n > 0) {
         AdjHalfArgs a{};
         a.pw = v.pw;
-        a.pl = v.pl;
+        a.cell = v.cell;
         a.flags = v.flags;
         a.cell_start = v.cell_start;
-        a.chunks = v.chunks;
-        a.n_chunks_dev = v.row_chunk + (size_t)v.g.dim[1] * v.g.dim[2];
         a.rows = (const Row*)(X.params.ptr + rows_off);
         a.bins = (const BinDesc*)X.params.ptr;
-        a.queue = X.queue.ptr;
+        a.queue = queue;
         a.g = v.g;
         a.g.m = mst;
         a.nrows = (int)rows.size();
@@ -122,7 +124,7 @@ static int adjoint_impl(gs_ctx* c, const gs_params* p, const double* gN2, const 
         a.g3 = g3;
         a.Glo = Glo;
         a.Ghi = Ghi;
-        a.out_stats = X.out.ptr;
+        a.out_stats = stats;
         a.inv_wd = inv_wd;
         a.inv_wr = inv_wr;
         a.g_scale = std::ldexp(1.0, Fa);
@@ -136,7 +138,7 @@ static int adjoint_impl(gs_ctx* c, const gs_params* p, const double* gN2, const 
     } else if (n > 0 && v.n_chunks > 0) {
         AdjArgs a{};
         a.pw = v.pw;
-        a.pl = v.pl;
+        a.cell = v.cell;
         a.flags = v.flags;
         a.orig = v.orig;
         a.cell_start = v.cell_start;
@@ -145,9 +147,9 @@ static int adjoint_impl(gs_ctx* c, const gs_params* p, const double* gN2, const 
         a.bins = (const BinDesc*)X.params.ptr;
         a.g2 = g2;
         a.g3 = g3;
-        a.queue = X.queue.ptr;
+        a.queue = queue;
         a.G = G;
-        a.out_stats = X.out.ptr;
+        a.out_stats = stats;
         a.g = v.g;
         a.g.m = mst;
         a.nrows = (int)rows.size();
@@ -159,31 +161,22 @@ static int adjoint_impl(gs_ctx* c, const gs_params* p, const double* gN2, const 
         if (e != hipSuccess) return hip_fail(e, "adjoint kernel launch");
     }
     (void)hipEventRecord(v.ev[3], v.stream);
-    e = launch_adj_partials(G, v.w, n, v.n_data, inv_wd, inv_wr, part, nblk_red, v.stream);
-    std::vector<double> hp(2 * nblk_red);
-    unsigned long long hs[2] = {0, 0};
-    if (e == hipSuccess)
-        e = hipMemcpyAsync(hp.data(), part, hp.size() * 8, hipMemcpyDeviceToHost, v.stream);
-    if (e == hipSuccess) e = hipMemcpyAsync(hs, X.out.ptr, 16, hipMemcpyDeviceToHost, v.stream);
-    if (e == hipSuccess) e = hipStreamSynchronize(v.stream);
-    if (e != hipSuccess) return hip_fail(e, "adjoint kernel");
-    long double sd = 0, sr = 0;
-    for (int b = 0; b < nblk_red; ++b) { sd += hp[2 * b]; sr += hp[2 * b + 1]; }
-    e = launch_adj_finish(G, n, v.n_data, (double)sd, (double)sr, inv_wd, inv_wr, outd, v.stream);
+    e = launch_adj_partials(G, v.w, n, v.n_data, inv_wd, inv_wr, part, nblk_red, stats, h_stats, v.stream);
+    if (e == hipSuccess) e = launch_adj_finish(G, n, v.n_data, part + 2 * nblk_red, inv_wd, inv_wr, outd, v.stream);
     if (e == hipSuccess && out_host) e = hipMemcpyAsync(out_host, outd, (size_t)n * 8, hipMemcpyDeviceToHost, v.stream);
     if (e == hipSuccess) e = hipStreamSynchronize(v.stream);
-    if (e != hipSuccess) return hip_fail(e, "adjoint finish");
+    if (e != hipSuccess) return hip_fail(e, "adjoint kernel");
     if (st) {
         memset(st, 0, sizeof(*st));
         float ms_grid = 0, ms_count = 0;
-        (void)hipEventElapsedTime(&ms_grid, v.ev[0], v.ev[1]);
+        (void)hipEventElapsedTime(&ms_grid, v.ev[0], v.ev[2]);
         (void)hipEventElapsedTime(&ms_count, v.ev[2], v.ev[3]);
         st->ms_grid = ms_grid;
         st->ms_count = ms_count;
         st->ms_kernel_avg = ms_count;
-        st->n_candidates = hs[0];
-        st->n_evaluated = hs[0];
-        st->n_recheck = hs[1];
+        st->n_candidates = h_stats[0];
+        st->n_evaluated = h_stats[0];
+        st->n_recheck = h_stats[1];
         st->cell_div = mst;
     }
     return GS_OK;

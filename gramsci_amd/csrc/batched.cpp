@@ -35,10 +35,9 @@ void batch_release(GsBatch& b)
         pl.blob.release();
     }
     b.plans.clear();
-    b.d_off.release(); b.d_row_base.release(); b.cell_of.release(); b.count.release(); b.cell_start.release();
-    b.nch.release(); b.row_chunk.release(); b.scan_tmp.release(); b.queue.release(); b.orig.release();
-    b.d_regions.release(); b.params.release(); b.pw.release(); b.pl.release(); b.flags.release();
-    b.chunks.release();
+    b.d_off.release(); b.d_row_base.release(); b.rank.release(); b.count.release(); b.boff.release();
+    b.cell_start.release(); b.queue.release(); b.orig.release();
+    b.d_regions.release(); b.params.release(); b.pw.release(); b.cell.release(); b.flags.release();
     b.out.release();
     b.xyz.release(); b.w.release(); b.buf.release(); b.ovf.release(); b.big.release();
     b.valid = false;
@@ -110,7 +109,9 @@ static int get_plan(gs_ctx* c, const gs_params& p, const BatchTune& tu, int kind
     std::vector<Row> rows = kind == 3 ? full_stencil(h, hx, p.rmax, mst) : half_stencil(h, hx, p.rmax, mst);
     if ((int)rows.size() > kMaxRows) return fail(GS_ELIMIT, "stencil too large");
     BinDesc bins;
+    double t64[kMaxBins + 2];
     int rc;
+    if ((rc = ctx_thresholds(c, p, t64))) return rc;
     // pair kernel: chunk size for the regions' mean density and row length
     PairGrid q;
     if (kind == 2) {
@@ -126,8 +127,8 @@ static int get_plan(gs_ctx* c, const gs_params& p, const BatchTune& tu, int kind
         q.h = h;
         q.mst = mst;
         pair_group(q, (double)n / vol, len / vol, p.rmax);
-        if ((rc = fill_pair_bins(p, q, B.xmax, B.wmax_d, B.wmax_r, bins))) return rc;
-    } else if ((rc = fill_bins(p, 1.5 * p.rmax, B.xmax, B.wmax_d, B.wmax_r, bins))) {
+        if ((rc = fill_pair_bins(p, t64, q, B.xmax, B.wmax_d, B.wmax_r, bins))) return rc;
+    } else if ((rc = fill_bins(p, t64, 1.5 * p.rmax, B.xmax, B.wmax_d, B.wmax_r, bins))) {
         return rc;
     }
 
@@ -148,14 +149,12 @@ static int get_plan(gs_ctx* c, const gs_params& p, const BatchTune& tu, int kind
         nh = ta.ncfg * nm * 4;
     }
     const size_t nout = kind == 3 ? (size_t)nreg * 3 * nh + 8 : (size_t)nreg * 3 * nbt + 4 + (size_t)pair_copies(nreg, nbt) * pair_copy_words(nreg, nbt);
-    const int64_t nchunk = kind == 2 ? max_chunks(n, rows_tot, q.group) : 0;
-    const int64_t scan_n = std::max<int64_t>(cells + 1, rows_tot + 1);
+    const int64_t nblk_scan = cell_scan_blocks(cells);
     // captured graphs hold raw pointers to the shared work buffers: if any of
     // them has to grow, every existing plan is destroyed before reallocating
-    const bool grow = (size_t)n > B.cell_of.cap || (size_t)(cells + 1) > B.count.cap ||
-                      (size_t)(cells + 1) > B.cell_start.cap || (size_t)(rows_tot + 1) > B.nch.cap ||
-                      (size_t)(rows_tot + 1) > B.row_chunk.cap || (size_t)scan_scratch_size(scan_n) > B.scan_tmp.cap ||
-                      nout > B.out.cap || (size_t)nchunk > B.chunks.cap || (kind == 3 && (size_t)(2 * n + 3) > B.ovf.cap) || B.queue.cap < 32 + 64 * kQueuePad;
+    const bool grow = (size_t)n > B.rank.cap || (size_t)(2 * cells + 1) > B.count.cap ||
+                      (size_t)(cells + 1) > B.cell_start.cap || (size_t)nblk_scan > B.boff.cap || nout > B.out.cap ||
+                      (kind == 3 && (size_t)(2 * n + 3) > B.ovf.cap) || B.queue.cap < 32 + 64 * kQueuePad;
     if (grow) {
         for (auto& pl : B.plans) {
             if (pl.exec) (void)hipGraphExecDestroy(pl.exec);
@@ -164,13 +163,10 @@ static int get_plan(gs_ctx* c, const gs_params& p, const BatchTune& tu, int kind
         }
         B.plans.clear();
     }
-    if ((rc = B.cell_of.reserve(n)) || (rc = B.count.reserve(cells + 1)) || (rc = B.cell_start.reserve(cells + 1)) ||
-        (rc = B.nch.reserve(rows_tot + 1)) || (rc = B.row_chunk.reserve(rows_tot + 1)) ||
-        (rc = B.scan_tmp.reserve(scan_scratch_size(scan_n))) || (rc = B.queue.reserve(32 + 64 * kQueuePad)) ||
-        (kind == 3 && (rc = B.ovf.reserve(2 * n + 3))) ||
-        (rc = B.orig.reserve(n)) || (rc = B.pw.reserve(n)) || (rc = B.pl.reserve(n)) ||
-        (rc = B.flags.reserve(n)) || (rc = B.chunks.reserve(nchunk)) ||
-        (rc = B.out.reserve(nout)))
+    if ((rc = B.rank.reserve(n)) || (rc = B.count.reserve(2 * cells + 1)) || (rc = B.cell_start.reserve(cells + 1)) ||
+        (rc = B.boff.reserve(nblk_scan)) || (rc = B.queue.reserve(32 + 64 * kQueuePad)) ||
+        (kind == 3 && (rc = B.ovf.reserve(2 * n + 3))) || (rc = B.orig.reserve(n)) || (rc = B.pw.reserve(n)) ||
+        (rc = B.cell.reserve(n)) || (rc = B.flags.reserve(n)) || (rc = B.out.reserve(nout)))
         return rc;
     // per-plan parameter blob: regions, bins, stencil rows (kept for the plan's lifetime)
     const size_t reg_bytes = ((nreg * sizeof(RegionDesc) + 15) / 16) * 16;
@@ -202,10 +198,9 @@ static int get_plan(gs_ctx* c, const gs_params& p, const BatchTune& tu, int kind
 
     PairArgs a{};
     a.pw = B.pw.ptr;
-    a.pl = B.pl.ptr;
+    a.cell = B.cell.ptr;
     a.flags = B.flags.ptr;
     a.cell_start = B.cell_start.ptr;
-    a.chunks = B.chunks.ptr;
     a.rows = (const Row*)(pblob->ptr + rows_off);
     a.bins = (const BinDesc*)(pblob->ptr + bin_off);
     // outputs: the sum ([nreg][nbt] counts, [nreg][nbt][2] sums, statistics), then the copies it is made of
@@ -223,13 +218,32 @@ static int get_plan(gs_ctx* c, const gs_params& p, const BatchTune& tu, int kind
     a.g.m = mst;
     a.nrows = (int)rows.size();
     a.group = q.group;
-    a.cap_cells = (float)q.cap_cells;
+    a.n = (int32_t)n;
+    a.cap_cells = q.cap_cells;
     a.reps = 1;
     a.planes = 1;
     a.regions = d_reg;
-    a.n_chunks_dev = B.row_chunk.ptr + rows_tot;
+    a.row_base = (const int32_t*)(pblob->ptr + rb_off);
     a.nreg = nreg;
-    const int32_t* d_row_base = (const int32_t*)(pblob->ptr + rb_off);
+    GridArgs ga{};
+    ga.xyz = B.xyz.ptr;
+    ga.w = B.has_w ? B.w.ptr : nullptr;
+    ga.buf = B.has_buf ? B.buf.ptr : nullptr;
+    ga.n = n;
+    ga.ncell = cells;
+    ga.g = a.g;
+    ga.regions = d_reg;
+    ga.off = B.d_off.ptr;
+    ga.nreg = nreg;
+    ga.rank = B.rank.ptr;
+    ga.count = B.count.ptr;
+    ga.boff = B.boff.ptr;
+    ga.ticket = (unsigned*)B.queue.ptr + 28;
+    ga.pw = B.pw.ptr;
+    ga.cell = B.cell.ptr;
+    ga.flags = B.flags.ptr;
+    ga.orig = B.orig.ptr;
+    ga.cell_start = B.cell_start.ptr;
     // one histogram per wave: fewer planes and waves where it would not fit otherwise
     const PairVariant var{nb, nm, fp64 || (kind == 2 && bins.wide), weighted, p.log_bins != 0, B.has_buf};
     int pair_wg = kWG, pair_waves = 0;
@@ -315,28 +329,15 @@ static int get_plan(gs_ctx* c, const gs_params& p, const BatchTune& tu, int kind
                                   : (v.n_cu * occ + 7) / 8 * 8;
     if (kind == 3) ta1.batch = triplet_batch(n, nblocks);
 
-    // capture: clear, count sort into cells, scans, scatter, row chunks, pair or triplet kernel
+    // capture: clear, sort into cells, pair or triplet kernel
     e = hipStreamBeginCapture(v.stream, hipStreamCaptureModeThreadLocal);
-    if (e == hipSuccess) e = launch_fill_u32(B.count.ptr, cells + 1, 0, v.stream);
+    if (e == hipSuccess) e = launch_fill_u32(B.count.ptr, 2 * cells + 1, 0, v.stream);
     if (e == hipSuccess) e = launch_fill_u32(B.queue.ptr, 32 + 64 * kQueuePad, 0, v.stream);
     if (e == hipSuccess && nblocks2 > 0) e = launch_fill_u32(B.ovf.ptr, 1, 0, v.stream);
     if (e == hipSuccess && kind == 3) e = launch_fill_u32(B.ovf.ptr + n + 1, 2, 0, v.stream);
     if (e == hipSuccess) e = launch_fill_u32(B.out.ptr, (int64_t)nout * 2, 0, v.stream);
-    if (e == hipSuccess)
-        e = launch_cell_count_b(B.xyz.ptr, n, B.d_off.ptr, nreg, d_reg, h, hx, B.cell_of.ptr, B.count.ptr, v.stream);
-    if (e == hipSuccess) e = exclusive_scan(B.count.ptr, B.cell_start.ptr, cells + 1, B.scan_tmp.ptr, v.stream);
-    if (e == hipSuccess) e = launch_fill_u32(B.count.ptr, cells + 1, 0, v.stream);
-    if (e == hipSuccess)
-        e = launch_scatter_b(B.xyz.ptr, B.has_w ? B.w.ptr : nullptr, B.has_buf ? B.buf.ptr : nullptr, n, B.d_off.ptr,
-                             nreg, d_reg, h, hx, B.cell_of.ptr, B.cell_start.ptr,
-                             B.count.ptr, B.pw.ptr, B.pl.ptr, B.flags.ptr, B.orig.ptr, v.stream);
+    if (e == hipSuccess) e = launch_cell_sort(ga, v.stream);
     if (kind == 2) {
-        if (e == hipSuccess)
-            e = launch_row_chunks_b(B.cell_start.ptr, d_reg, d_row_base, nreg, (int)rows_tot, q.group, B.nch.ptr, v.stream);
-        if (e == hipSuccess) e = exclusive_scan(B.nch.ptr, B.row_chunk.ptr, rows_tot + 1, B.scan_tmp.ptr, v.stream);
-        if (e == hipSuccess)
-            e = launch_chunks(B.row_chunk.ptr, (int)rows_tot, B.cell_start.ptr, 0, d_reg, d_row_base, nreg, q.group,
-                              nchunk, B.chunks.ptr, v.stream);
         if (e == hipSuccess) e = launch_pair2(a, var, nblocks, pair_wg, v.stream);
         if (e == hipSuccess)
             e = launch_pair_reduce(a.out_cnt, a.copies, nreg, nbt, nm, weighted, B.out.ptr, v.stream);

@@ -1,115 +1,150 @@
-// grid.hip -- GPU cell grid: bounding box, counting sort of points by cell,
-// cell start offsets.  Replaces the kd-tree build (kdtree2.F90:611-1012) and
-// its r-ball queries: a pair kernel reads each neighbour cell row as one
-// contiguous range of the sorted points.
+// grid.hip -- what a catalogue goes through before its pairs are counted: the pass that takes it over
+// (copy, bounding box, weight statistics) and the GPU cell grid (counting sort of points by cell, cell
+// start offsets).  Replaces the kd-tree build (kdtree2.F90:611-1012) and its r-ball queries: a pair
+// kernel reads each neighbour cell row as one contiguous range of the sorted points.
+#include <algorithm>
+
+#include "gs_device.h"
 #include "gs_kernels.h"
 
 namespace gs {
 
-// ---------------------------------------------------------------- bounding box
-// Per-block min/max of the three coordinates; the host reduces the partials.
-__global__ __launch_bounds__(256) void k_bbox(const double* __restrict__ xyz, int64_t n,
-                                              double* __restrict__ part /*[gridDim][6]*/)
+using namespace dev;
+
+// ---------------------------------------------------------------- catalogue
+// One pass over a catalogue handed over: copies it (where src and dst differ) and reduces its bounding box,
+// the largest data and random weight and the first invalid weight.  The last block to finish reduces the
+// blocks' partials, so that one launch and one wait give the host everything (with k_wsum, where there
+// are weights); before, the copies, the check, the sums and the bounding box were seven launches and three
+// waits.  Bound by memory: each coordinate and weight is read and written once.
+// The thread count is a multiple of 3, so that every thread's coordinates share one axis.
+constexpr int kIngestThreads = 192;
+
+__device__ __forceinline__ double block_reduce_max(double v, double* red)
 {
-    __shared__ double red[6][256];
-    double mn[3] = {1e308, 1e308, 1e308}, mx[3] = {-1e308, -1e308, -1e308};
-    for (int64_t i = blockIdx.x * (int64_t)blockDim.x + threadIdx.x; i < n; i += (int64_t)gridDim.x * blockDim.x) {
-        for (int k = 0; k < 3; ++k) {
-            double v = xyz[3 * i + k];
-            mn[k] = fmin(mn[k], v);
-            mx[k] = fmax(mx[k], v);
-        }
-    }
-    for (int k = 0; k < 3; ++k) { red[k][threadIdx.x] = mn[k]; red[3 + k][threadIdx.x] = mx[k]; }
+    for (int off = 32; off > 0; off >>= 1) v = fmax(v, __shfl_down(v, off, 64));
     __syncthreads();
-    for (int s = 128; s > 0; s >>= 1) {
-        if (threadIdx.x < s) {
-            for (int k = 0; k < 3; ++k) {
-                red[k][threadIdx.x] = fmin(red[k][threadIdx.x], red[k][threadIdx.x + s]);
-                red[3 + k][threadIdx.x] = fmax(red[3 + k][threadIdx.x], red[3 + k][threadIdx.x + s]);
-            }
-        }
-        __syncthreads();
-    }
-    if (threadIdx.x < 6) part[blockIdx.x * 6 + threadIdx.x] = red[threadIdx.x][0];
-}
-
-// ---------------------------------------------------------------- weights
-// per-block maxima of the data weights (i < n_data) and of the random weights: part_max[2 * block + class]
-__global__ __launch_bounds__(256) void k_wcheck(const double* __restrict__ w, int64_t n, int64_t n_data,
-                                                double* __restrict__ part_max, unsigned long long* __restrict__ bad)
-{
-    __shared__ double red[2][256];
-    double mx[2] = {0.0, 0.0};
-    for (int64_t i = blockIdx.x * (int64_t)blockDim.x + threadIdx.x; i < n; i += (int64_t)gridDim.x * blockDim.x) {
-        const double v = w[i];
-        if (!(v >= 0.0) || !isfinite(v)) atomicMin(bad, (unsigned long long)i);
-        else if (i < n_data) mx[0] = fmax(mx[0], v);
-        else mx[1] = fmax(mx[1], v);
-    }
-    red[0][threadIdx.x] = mx[0];
-    red[1][threadIdx.x] = mx[1];
+    if ((threadIdx.x & 63) == 0) red[threadIdx.x >> 6] = v;
     __syncthreads();
-    for (int s = 128; s > 0; s >>= 1) {
-        if (threadIdx.x < s)
-            for (int q = 0; q < 2; ++q) red[q][threadIdx.x] = fmax(red[q][threadIdx.x], red[q][threadIdx.x + s]);
-        __syncthreads();
+    double r = red[0];
+    for (int k = 1; k < (int)(blockDim.x >> 6); ++k) r = fmax(r, red[k]);
+    return r;
+}
+
+__global__ __launch_bounds__(kIngestThreads) void k_ingest(const double* __restrict__ xyz, const double* __restrict__ w,
+                                                           const int32_t* __restrict__ buf, int64_t n, int64_t n_data,
+                                                           double* xyz_out, double* w_out, int32_t* buf_out,
+                                                           IngestScratch* sc, CatalogueStats* out)
+{
+    __shared__ double red[kIngestThreads / 64];
+    const int64_t t = blockIdx.x * (int64_t)blockDim.x + threadIdx.x, step = gridDim.x * (int64_t)blockDim.x;
+    const int axis = (int)(t % 3);
+    double mn = 1e308, mx = -1e308;
+    for (int64_t i = t; i < 3 * n; i += step) {
+        const double v = xyz[i];
+        if (xyz_out != xyz) xyz_out[i] = v;
+        mn = fmin(mn, v);
+        mx = fmax(mx, v);
     }
-    if (threadIdx.x < 2) part_max[2 * blockIdx.x + threadIdx.x] = red[threadIdx.x][0];
+    double wm[2] = {0.0, 0.0};
+    unsigned long long bad = ~0ull;
+    if (w)
+        for (int64_t i = t; i < n; i += step) {
+            const double v = w[i];
+            if (w_out != w) w_out[i] = v;
+            if (!(v >= 0.0) || !isfinite(v)) bad = bad < (unsigned long long)i ? bad : (unsigned long long)i;
+            else if (i < n_data) wm[0] = fmax(wm[0], v);
+            else wm[1] = fmax(wm[1], v);
+        }
+    if (buf && buf_out != buf)
+        for (int64_t i = t; i < n; i += step) buf_out[i] = buf[i];
+
+    IngestScratch& P = sc[blockIdx.x];
+    for (int k = 0; k < 3; ++k) {
+        const double hi = block_reduce_max(axis == k ? mx : -1e308, red);
+        const double lo = -block_reduce_max(axis == k ? -mn : -1e308, red);
+        if (threadIdx.x == 0) { P.v[k] = lo; P.v[3 + k] = hi; }
+    }
+    for (int q = 0; q < 2; ++q) {
+        const double m = block_reduce_max(wm[q], red);
+        if (threadIdx.x == 0) P.v[6 + q] = m;
+    }
+    // the index as a double: exact below 2^53
+    const double fb = -block_reduce_max(bad == ~0ull ? -1e308 : -(double)bad, red);
+    if (threadIdx.x == 0) P.v[8] = fb;
+
+    if (!last_block(&out->ticket)) return;
+    for (int q = 0; q < 9; ++q) {
+        const bool lowest = q < 3 || q == 8;
+        double v = -1e308;
+        for (int b = threadIdx.x; b < (int)gridDim.x; b += blockDim.x) {
+            const double x = load_agent(&sc[b].v[q]);
+            v = fmax(v, lowest ? -x : x);
+        }
+        v = block_reduce_max(v, red);
+        if (threadIdx.x == 0) out->v[q] = lowest ? -v : v;
+    }
+    // without weights there is no k_wsum to hand the statistics to the host
+    if (!w && threadIdx.x < 9 && threadIdx.x == 0)
+        for (int q = 0; q < 9; ++q) out->host->v[q] = out->v[q];
 }
 
-__device__ __forceinline__ void add128(unsigned long long& lo, unsigned long long& hi, unsigned long long l,
-                                       unsigned long long h)
+// Exact fixed-point sums of the data and the random weights (wsum_fixed at the scale of the largest weight),
+// then the statistics to the host.
+__global__ __launch_bounds__(256) void k_wsum(const double* __restrict__ w, int64_t n, int64_t n_data,
+                                              IngestScratch* sc, CatalogueStats* out)
 {
-    lo += l;
-    hi += h + (lo < l ? 1ull : 0ull);
-}
-
-__global__ __launch_bounds__(256) void k_wsum(const double* __restrict__ w, int64_t n, int64_t n_data, int k,
-                                              unsigned long long* __restrict__ part)
-{
-    __shared__ unsigned long long red[4][256];
+    __shared__ unsigned long long red[4][4];
+    const int k = wsum_scale(fmax(out->v[6], out->v[7]));
     unsigned long long a[4] = {0, 0, 0, 0};     // data lo, hi, randoms lo, hi
-    for (int64_t i = blockIdx.x * (int64_t)blockDim.x + threadIdx.x; i < n; i += (int64_t)gridDim.x * blockDim.x) {
-        uint64_t lo, hi;
-        wsum_fixed(w[i], k, lo, hi);
-        const int o = i < n_data ? 0 : 2;
-        add128(a[o], a[o + 1], lo, hi);
-    }
-    for (int q = 0; q < 4; ++q) red[q][threadIdx.x] = a[q];
-    __syncthreads();
-    for (int s = 128; s > 0; s >>= 1) {
-        if (threadIdx.x < s) {
-            const int t = threadIdx.x;
-            unsigned long long l0 = red[0][t], h0 = red[1][t], l1 = red[2][t], h1 = red[3][t];
-            add128(l0, h0, red[0][t + s], red[1][t + s]);
-            add128(l1, h1, red[2][t + s], red[3][t + s]);
-            red[0][t] = l0; red[1][t] = h0; red[2][t] = l1; red[3][t] = h1;
+    if (out->v[8] >= 1e308)                     // no invalid weight
+        for (int64_t i = blockIdx.x * (int64_t)blockDim.x + threadIdx.x; i < n; i += (int64_t)gridDim.x * blockDim.x) {
+            uint64_t lo, hi;
+            wsum_fixed(w[i], k, lo, hi);
+            const int o = i < n_data ? 0 : 2;
+            add128(a[o], a[o + 1], lo, hi);
         }
+    auto block_sum = [&]() {                    // the block's sum of a, in thread 0
+        for (int off = 32; off > 0; off >>= 1)
+            for (int q = 0; q < 4; q += 2) {
+                const unsigned long long l = __shfl_down(a[q], off, 64), h = __shfl_down(a[q + 1], off, 64);
+                add128(a[q], a[q + 1], l, h);
+            }
         __syncthreads();
+        if ((threadIdx.x & 63) == 0)
+            for (int q = 0; q < 4; ++q) red[threadIdx.x >> 6][q] = a[q];
+        __syncthreads();
+        if (threadIdx.x == 0)
+            for (int v = 1; v < 4; ++v)
+                for (int q = 0; q < 4; q += 2) add128(a[q], a[q + 1], red[v][q], red[v][q + 1]);
+    };
+    block_sum();
+    if (threadIdx.x == 0)
+        for (int q = 0; q < 4; ++q) sc[blockIdx.x].s[q] = a[q];
+    if (!last_block(&out->ticket)) return;
+    for (int q = 0; q < 4; ++q) a[q] = 0;
+    for (int b = threadIdx.x; b < (int)gridDim.x; b += blockDim.x)
+        for (int q = 0; q < 4; q += 2) add128(a[q], a[q + 1], load_agent(&sc[b].s[q]), load_agent(&sc[b].s[q + 1]));
+    block_sum();
+    if (threadIdx.x == 0) {
+        for (int q = 0; q < 4; ++q) out->host->s[q] = a[q];
+        for (int q = 0; q < 9; ++q) out->host->v[q] = out->v[q];
     }
-    if (threadIdx.x < 4) part[blockIdx.x * 4 + threadIdx.x] = red[threadIdx.x][0];
 }
 
-// ---------------------------------------------------------------- cell of point
-__device__ __forceinline__ int cell_coord(double v, double lo, double inv_h, int dim)
+hipError_t launch_ingest(const double* xyz, const double* w, const int32_t* buf, int64_t n, int64_t n_data,
+                         double* xyz_out, double* w_out, int32_t* buf_out, IngestScratch* scratch, CatalogueStats* stats,
+                         hipStream_t st)
 {
-    int c = (int)floor((v - lo) * inv_h);
-    return c < 0 ? 0 : (c >= dim ? dim - 1 : c);
-}
-
-__global__ __launch_bounds__(256) void k_cell_count(const double* __restrict__ xyz, int64_t n, GridDesc g,
-                                                    int32_t* __restrict__ cell_of, int32_t* __restrict__ count)
-{
-    const double inv_h = 1.0 / g.h, inv_hx = 1.0 / g.hx;
-    for (int64_t i = blockIdx.x * (int64_t)blockDim.x + threadIdx.x; i < n; i += (int64_t)gridDim.x * blockDim.x) {
-        int cx = cell_coord(xyz[3 * i + 0], g.lo[0], inv_hx, g.dim[0]);
-        int cy = cell_coord(xyz[3 * i + 1], g.lo[1], inv_h, g.dim[1]);
-        int cz = cell_coord(xyz[3 * i + 2], g.lo[2], inv_h, g.dim[2]);
-        int c = (cz * g.dim[1] + cy) * g.dim[0] + cx;
-        cell_of[i] = c;
-        atomicAdd(&count[c], 1);
+    const int nblk = (int)std::min<int64_t>(std::max<int64_t>((3 * n + 4 * kIngestThreads - 1) / (4 * kIngestThreads), 1),
+                                            kIngestBlocks);
+    hipLaunchKernelGGL(k_ingest, dim3(nblk), dim3(kIngestThreads), 0, st, xyz, w, buf, n, n_data, xyz_out, w_out, buf_out,
+                       scratch, stats);
+    if (w) {
+        const int wblk = (int)std::min<int64_t>(std::max<int64_t>((n + 1023) / 1024, 1), kIngestBlocks);
+        hipLaunchKernelGGL(k_wsum, dim3(wblk), dim3(256), 0, st, w_out, n, n_data, scratch, stats);
     }
+    return hipGetLastError();
 }
 
 // ---------------------------------------------------------------- exclusive scan
@@ -192,37 +227,150 @@ int64_t scan_scratch_size(int64_t n)
     return tot + 2;
 }
 
-// ---------------------------------------------------------------- scatter
-// Writes the points in cell order, a cell's data points before its randoms
-// (consecutive neighbours then mostly share a class).  Order inside a cell otherwise follows the atomic
-// slot order; every count and fixed-point sum computed from the sorted arrays
-// is independent of it.
-__global__ __launch_bounds__(256) void k_scatter(const double* __restrict__ xyz, const double* __restrict__ w,
-                                                 const int32_t* __restrict__ buf, int64_t n, int64_t n_data, GridDesc g,
-                                                 const int32_t* __restrict__ cell_of, const int32_t* __restrict__ start,
-                                                 int32_t* __restrict__ fill, double4* __restrict__ pw,
-                                                 float4* __restrict__ pl,
-                                                 uint32_t* __restrict__ flags, int32_t* __restrict__ orig, int pass)
+// ---------------------------------------------------------------- cells
+// Counting sort of the points into cells, a cell's data points before its randoms (consecutive neighbours
+// then mostly share a class), in three launches: the counts of data and randoms per cell, each point
+// keeping its rank in its count; the exclusive scan of the counts, by blocks, with the blocks' offsets
+// scanned by the last block; the scatter, which adds the offsets where it needs them and writes the final
+// cell starts beside.  The order inside a count follows the atomics' order; every count and fixed-point sum
+// computed from the sorted arrays is independent of it.  One grid, or one per region of a batch.
+constexpr int kCellScan = 2048;     // counts per block of the scan
+
+__device__ __forceinline__ int cell_coord(double v, double lo, double inv_h, int dim)
 {
-    const int nx = g.dim[0], ny = g.dim[1];
-    for (int64_t i = blockIdx.x * (int64_t)blockDim.x + threadIdx.x; i < n; i += (int64_t)gridDim.x * blockDim.x) {
-        if ((i >= n_data) != (pass == 1)) continue;    // pass 0: data points, pass 1: randoms
-        const int c = cell_of[i];
-        const int pos = start[c] + atomicAdd(&fill[c], 1);
-        const double x = xyz[3 * i], y = xyz[3 * i + 1], z = xyz[3 * i + 2];
-        const double wi = w ? w[i] : 1.0;
-        pw[pos] = make_double4(x, y, z, wi);
-        const int cx = c % nx, cy = (c / nx) % ny, cz = c / (nx * ny);
-        // cell-local FP32 coordinates; .w carries the cell's x index (exact in FP32)
-        pl[pos] = make_float4((float)(x - (g.lo[0] + cx * g.hx)), (float)(y - (g.lo[1] + cy * g.h)),
-                              (float)(z - (g.lo[2] + cz * g.h)), (float)cx);
-        const uint32_t f = (i >= n_data ? 1u : 0u) | ((buf && buf[i] == 1) ? 2u : 0u);
-        flags[pos] = f;
-        orig[pos] = (int32_t)i;
+    int c = (int)floor((v - lo) * inv_h);
+    return c < 0 ? 0 : (c >= dim ? dim - 1 : c);
+}
+
+__device__ __forceinline__ int region_of(const int32_t* off, int nreg, int64_t i)
+{
+    int lo = 0, hi = nreg - 1;
+    while (lo < hi) {
+        int mid = (lo + hi + 1) >> 1;
+        if (off[mid] <= i) lo = mid; else hi = mid - 1;
+    }
+    return lo;
+}
+
+struct PointCell {
+    int cx, row, cell;      // x cell and x-row (over all regions), cell
+    bool random;
+};
+
+__device__ __forceinline__ PointCell point_cell(const GridArgs& a, int64_t i)
+{
+    double lo[3] = {a.g.lo[0], a.g.lo[1], a.g.lo[2]};
+    int nx = a.g.dim[0], ny = a.g.dim[1], nz = a.g.dim[2], cell0 = 0, row0 = 0;
+    int64_t p0 = 0, nd = a.n_data;
+    if (a.nreg > 0) {
+        const RegionDesc& R = a.regions[region_of(a.off, a.nreg, i)];
+        for (int k = 0; k < 3; ++k) lo[k] = R.lo[k];
+        nx = R.dim[0]; ny = R.dim[1]; nz = R.dim[2];
+        cell0 = R.cell_base;
+        row0 = R.row_base;
+        p0 = R.pt_base;
+        nd = R.n_data;
+    }
+    const double inv_h = 1.0 / a.g.h, inv_hx = 1.0 / a.g.hx;
+    PointCell c;
+    c.cx = cell_coord(a.xyz[3 * i + 0], lo[0], inv_hx, nx);
+    const int cy = cell_coord(a.xyz[3 * i + 1], lo[1], inv_h, ny);
+    const int cz = cell_coord(a.xyz[3 * i + 2], lo[2], inv_h, nz);
+    const int row = cz * ny + cy;
+    c.row = row0 + row;
+    c.cell = cell0 + row * nx + c.cx;
+    c.random = i - p0 >= nd;
+    return c;
+}
+
+__global__ __launch_bounds__(256) void k_cell_rank(GridArgs a)
+{
+    for (int64_t i = blockIdx.x * (int64_t)blockDim.x + threadIdx.x; i < a.n; i += (int64_t)gridDim.x * blockDim.x) {
+        const PointCell c = point_cell(a, i);
+        a.rank[i] = atomicAdd(&a.count[2 * (int64_t)c.cell + (c.random ? 1 : 0)], 1);
     }
 }
 
-// Work chunks of the pair kernels: up to `group` consecutive points of one x-row of
+__global__ __launch_bounds__(256) void k_cell_scan(int32_t* __restrict__ v, int64_t n, int32_t* __restrict__ boff,
+                                                   unsigned* ticket)
+{
+    __shared__ int32_t wsum[4];
+    const int lane = threadIdx.x & 63, wv = threadIdx.x >> 6;
+    // exclusive prefix of x over the block's threads; *total: the block's sum
+    auto block_scan = [&](int x, int* total) {
+        int inc = x;
+        for (int off = 1; off < 64; off <<= 1) {
+            const int y = __shfl_up(inc, off, 64);
+            if (lane >= off) inc += y;
+        }
+        __syncthreads();
+        if (lane == 63) wsum[wv] = inc;
+        __syncthreads();
+        int pre = 0, all = 0;
+        for (int k = 0; k < 4; ++k) {
+            if (k < wv) pre += wsum[k];
+            all += wsum[k];
+        }
+        *total = all;
+        return pre + inc - x;
+    };
+    const int64_t base = (int64_t)blockIdx.x * kCellScan + threadIdx.x * 8;
+    int x[8], sum = 0, total;
+    for (int k = 0; k < 8; ++k) {
+        x[k] = base + k < n ? v[base + k] : 0;
+        sum += x[k];
+    }
+    int run = block_scan(sum, &total);
+    for (int k = 0; k < 8; ++k) {
+        if (base + k < n) v[base + k] = run;
+        run += x[k];
+    }
+    if (threadIdx.x == 0) __hip_atomic_store(&boff[blockIdx.x], total, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT);
+    if (!last_block(ticket)) return;
+    int carry = 0;
+    for (int b0 = 0; b0 < (int)gridDim.x; b0 += 256) {
+        const int b = b0 + threadIdx.x;
+        const int t = b < (int)gridDim.x ? load_agent(&boff[b]) : 0;
+        const int e = block_scan(t, &total);
+        if (b < (int)gridDim.x) boff[b] = carry + e;
+        carry += total;
+    }
+}
+
+__global__ __launch_bounds__(256) void k_cell_scatter(GridArgs a)
+{
+    const int64_t t = blockIdx.x * (int64_t)blockDim.x + threadIdx.x, step = gridDim.x * (int64_t)blockDim.x;
+    auto start = [&](int64_t k) { return a.count[k] + a.boff[k / kCellScan]; };
+    for (int64_t i = t; i < a.n; i += step) {
+        const PointCell c = point_cell(a, i);
+        const int pos = start(2 * (int64_t)c.cell + (c.random ? 1 : 0)) + a.rank[i];
+        a.pw[pos] = make_double4(a.xyz[3 * i], a.xyz[3 * i + 1], a.xyz[3 * i + 2], a.w ? a.w[i] : 1.0);
+        a.cell[pos] = make_int2(c.cx, c.row);
+        a.flags[pos] = (c.random ? 1u : 0u) | ((a.buf && a.buf[i] == 1) ? 2u : 0u);
+        a.orig[pos] = (int32_t)i;
+    }
+    for (int64_t c = t; c <= a.ncell; c += step) a.cell_start[c] = start(2 * c);
+}
+
+int64_t cell_scan_blocks(int64_t ncell) { return (2 * ncell + 1 + kCellScan - 1) / kCellScan; }
+
+static int blocks_for(int64_t n)
+{
+    int64_t b = (n + 255) / 256;
+    if (b > 65535) b = 65535;
+    return (int)(b < 1 ? 1 : b);
+}
+
+hipError_t launch_cell_sort(const GridArgs& a, hipStream_t st)
+{
+    hipLaunchKernelGGL(k_cell_rank, dim3(blocks_for(a.n)), dim3(256), 0, st, a);
+    hipLaunchKernelGGL(k_cell_scan, dim3((unsigned)cell_scan_blocks(a.ncell)), dim3(256), 0, st, a.count, 2 * a.ncell + 1,
+                       a.boff, a.ticket);
+    hipLaunchKernelGGL(k_cell_scatter, dim3(blocks_for(std::max<int64_t>(a.n, a.ncell + 1))), dim3(256), 0, st, a);
+    return hipGetLastError();
+}
+
+// Work chunks of the full-stencil adjoint kernel: up to `group` consecutive points of one x-row of
 // cells (fixed cy, cz).  nch[r] = chunks of row r; nch[nrow] = 0.
 __global__ __launch_bounds__(256) void k_row_chunks(const int32_t* __restrict__ start, int nx, int nrow, int group,
                                                     int32_t* __restrict__ nch)
@@ -236,129 +384,8 @@ __global__ __launch_bounds__(256) void k_row_chunks(const int32_t* __restrict__ 
 
 hipError_t launch_row_chunks(const int32_t* start, int nx, int nrow, int group, int32_t* nch, hipStream_t st)
 {
-    int nblk = (nrow + 256) / 256;
-    if (nblk > 65535) nblk = 65535;
-    hipLaunchKernelGGL(k_row_chunks, dim3(nblk), dim3(256), 0, st, start, nx, nrow, group, nch);
+    hipLaunchKernelGGL(k_row_chunks, dim3(blocks_for(nrow + 1)), dim3(256), 0, st, start, nx, nrow, group, nch);
     return hipGetLastError();
-}
-
-hipError_t launch_bbox(const double* xyz, int64_t n, double* part, int nblk, hipStream_t st)
-{
-    hipLaunchKernelGGL(k_bbox, dim3(nblk), dim3(256), 0, st, xyz, n, part);
-    return hipGetLastError();
-}
-
-hipError_t launch_wcheck(const double* w, int64_t n, int64_t n_data, double* part_max, unsigned long long* bad, int nblk,
-                         hipStream_t st)
-{
-    hipLaunchKernelGGL(k_wcheck, dim3(nblk), dim3(256), 0, st, w, n, n_data, part_max, bad);
-    return hipGetLastError();
-}
-
-hipError_t launch_wsum(const double* w, int64_t n, int64_t n_data, int k, unsigned long long* part, int nblk,
-                       hipStream_t st)
-{
-    hipLaunchKernelGGL(k_wsum, dim3(nblk), dim3(256), 0, st, w, n, n_data, k, part);
-    return hipGetLastError();
-}
-
-hipError_t launch_cell_count(const double* xyz, int64_t n, const GridDesc& g, int32_t* cell_of, int32_t* count,
-                             hipStream_t st)
-{
-    int nblk = (int)((n + 255) / 256);
-    if (nblk > 65535) nblk = 65535;
-    if (nblk < 1) nblk = 1;
-    hipLaunchKernelGGL(k_cell_count, dim3(nblk), dim3(256), 0, st, xyz, n, g, cell_of, count);
-    return hipGetLastError();
-}
-
-hipError_t launch_scatter(const double* xyz, const double* w, const int32_t* buf, int64_t n, int64_t n_data,
-                          const GridDesc& g, const int32_t* cell_of, const int32_t* start, int32_t* fill,
-                          double4* pw, float4* pl, uint32_t* flags, int32_t* orig, hipStream_t st)
-{
-    int nblk = (int)((n + 255) / 256);
-    if (nblk > 65535) nblk = 65535;
-    if (nblk < 1) nblk = 1;
-    // two passes on one stream: a cell's data points take its first slots, its randoms the rest
-    for (int pass = 0; pass < 2; ++pass)
-        hipLaunchKernelGGL(k_scatter, dim3(nblk), dim3(256), 0, st, xyz, w, buf, n, n_data, g, cell_of, start, fill,
-                           pw, pl, flags, orig, pass);
-    return hipGetLastError();
-}
-
-// ---------------------------------------------------------------- batched regions
-__device__ __forceinline__ int region_of(const int32_t* off, int nreg, int64_t i)
-{
-    int lo = 0, hi = nreg - 1;
-    while (lo < hi) {
-        int mid = (lo + hi + 1) >> 1;
-        if (off[mid] <= i) lo = mid; else hi = mid - 1;
-    }
-    return lo;
-}
-
-__global__ __launch_bounds__(256) void k_cell_count_b(const double* __restrict__ xyz, int64_t n,
-                                                      const int32_t* __restrict__ off, int nreg,
-                                                      const RegionDesc* __restrict__ reg, double h, double hx,
-                                                      int32_t* __restrict__ cell_of, int32_t* __restrict__ count)
-{
-    const double inv_h = 1.0 / h, inv_hx = 1.0 / hx;
-    for (int64_t i = blockIdx.x * (int64_t)blockDim.x + threadIdx.x; i < n; i += (int64_t)gridDim.x * blockDim.x) {
-        const RegionDesc R = reg[region_of(off, nreg, i)];
-        int cx = cell_coord(xyz[3 * i + 0], R.lo[0], inv_hx, R.dim[0]);
-        int cy = cell_coord(xyz[3 * i + 1], R.lo[1], inv_h, R.dim[1]);
-        int cz = cell_coord(xyz[3 * i + 2], R.lo[2], inv_h, R.dim[2]);
-        int c = R.cell_base + (cz * R.dim[1] + cy) * R.dim[0] + cx;
-        cell_of[i] = c;
-        atomicAdd(&count[c], 1);
-    }
-}
-
-__global__ __launch_bounds__(256) void k_scatter_b(const double* __restrict__ xyz, const double* __restrict__ w,
-                                                   const int32_t* __restrict__ buf, int64_t n,
-                                                   const int32_t* __restrict__ off, int nreg,
-                                                   const RegionDesc* __restrict__ reg, double h, double hx,
-                                                   const int32_t* __restrict__ cell_of,
-                                                   const int32_t* __restrict__ start, int32_t* __restrict__ fill,
-                                                   double4* __restrict__ pw,
-                                                   float4* __restrict__ pl, uint32_t* __restrict__ flags,
-                                                   int32_t* __restrict__ orig, int pass)
-{
-    for (int64_t i = blockIdx.x * (int64_t)blockDim.x + threadIdx.x; i < n; i += (int64_t)gridDim.x * blockDim.x) {
-        const int r = region_of(off, nreg, i);
-        const RegionDesc R = reg[r];
-        if (((i - R.pt_base) >= R.n_data) != (pass == 1)) continue;   // pass 0: data points, pass 1: randoms
-        const int c = cell_of[i];
-        const int pos = start[c] + atomicAdd(&fill[c], 1);
-        const double x = xyz[3 * i], y = xyz[3 * i + 1], z = xyz[3 * i + 2];
-        const double wi = w ? w[i] : 1.0;
-        pw[pos] = make_double4(x, y, z, wi);
-        const int lc = c - R.cell_base;
-        const int cx = lc % R.dim[0], cy = (lc / R.dim[0]) % R.dim[1], cz = lc / (R.dim[0] * R.dim[1]);
-        pl[pos] = make_float4((float)(x - (R.lo[0] + cx * hx)), (float)(y - (R.lo[1] + cy * h)),
-                              (float)(z - (R.lo[2] + cz * h)), (float)cx);
-        const uint32_t f = ((i - R.pt_base) >= R.n_data ? 1u : 0u) | ((buf && buf[i] == 1) ? 2u : 0u);
-        flags[pos] = f;
-        orig[pos] = (int32_t)i;
-    }
-}
-
-// chunks of each global x-row; nch[total_rows] = 0
-__global__ __launch_bounds__(256) void k_row_chunks_b(const int32_t* __restrict__ start,
-                                                      const RegionDesc* __restrict__ reg,
-                                                      const int32_t* __restrict__ row_base, int nreg, int nrow_tot,
-                                                      int group, int32_t* __restrict__ nch)
-{
-    for (int r = blockIdx.x * blockDim.x + threadIdx.x; r <= nrow_tot; r += gridDim.x * blockDim.x) {
-        int v = 0;
-        if (r < nrow_tot) {
-            const RegionDesc R = reg[region_of(row_base, nreg, r)];
-            const int lr = r - R.row_base;
-            const int c0 = R.cell_base + lr * R.dim[0];
-            v = (start[c0 + R.dim[0]] - start[c0] + group - 1) / group;
-        }
-        nch[r] = v;
-    }
 }
 
 __global__ __launch_bounds__(256) void k_fill_u32(uint32_t* __restrict__ p, int64_t n, uint32_t v)
@@ -367,47 +394,11 @@ __global__ __launch_bounds__(256) void k_fill_u32(uint32_t* __restrict__ p, int6
         p[i] = v;
 }
 
-static int blocks_for(int64_t n)
-{
-    int64_t b = (n + 255) / 256;
-    if (b > 65535) b = 65535;
-    return (int)(b < 1 ? 1 : b);
-}
-
 hipError_t launch_fill_u32(void* p, int64_t n, uint32_t v, hipStream_t st)
 {
     if (n <= 0) return hipSuccess;
-    hipLaunchKernelGGL(k_fill_u32, dim3(blocks_for(n)), dim3(256), 0, st, (uint32_t*)p, n, v);
-    return hipGetLastError();
-}
-
-hipError_t launch_cell_count_b(const double* xyz, int64_t n, const int32_t* off, int nreg, const RegionDesc* reg,
-                               double h, double hx, int32_t* cell_of, int32_t* count, hipStream_t st)
-{
-    hipLaunchKernelGGL(k_cell_count_b, dim3(blocks_for(n)), dim3(256), 0, st, xyz, n, off, nreg, reg, h, hx, cell_of,
-                       count);
-    return hipGetLastError();
-}
-
-hipError_t launch_scatter_b(const double* xyz, const double* w, const int32_t* buf, int64_t n, const int32_t* off,
-                            int nreg, const RegionDesc* reg, double h, double hx, const int32_t* cell_of,
-                            const int32_t* start,
-                            int32_t* fill, double4* pw, float4* pl, uint32_t* flags, int32_t* orig,
-                            hipStream_t st)
-{
-    for (int pass = 0; pass < 2; ++pass)
-        hipLaunchKernelGGL(k_scatter_b, dim3(blocks_for(n)), dim3(256), 0, st, xyz, w, buf, n, off, nreg, reg, h, hx,
-                           cell_of, start, fill, pw, pl, flags, orig, pass);
-    return hipGetLastError();
-}
-
-hipError_t launch_row_chunks_b(const int32_t* start, const RegionDesc* reg, const int32_t* row_base, int nreg,
-                               int nrow_tot, int group, int32_t* nch, hipStream_t st)
-{
-    hipLaunchKernelGGL(k_row_chunks_b, dim3(blocks_for(nrow_tot + 1)), dim3(256), 0, st, start, reg, row_base, nreg,
-                       nrow_tot, group, nch);
+    hipLaunchKernelGGL(k_fill_u32, dim3(std::min(blocks_for(n), 2048)), dim3(256), 0, st, (uint32_t*)p, n, v);
     return hipGetLastError();
 }
 
 }  // namespace gs
-

@@ -25,6 +25,14 @@ struct DevBuf {
     void release();
 };
 
+// Pinned host memory: parameters on their way to the device, results on their way back.
+struct HostBuf {
+    unsigned char* ptr = nullptr;
+    size_t cap = 0;
+    int reserve(size_t bytes);   // grows only; contents are not preserved
+    void release();
+};
+
 // Buffers owned by a context for the 3PCF/4PCF/adjoint/batched paths.
 struct GsExtra {
     DevBuf<unsigned char> params;
@@ -55,13 +63,12 @@ struct GsBatch {
     std::vector<double> wmr;             // per-region largest weight (1 for unit weights)
     std::vector<double> wmr_d, wmr_r;    // per-region largest data / random weight (1 for none)
     double wmax = 1.0, wmax_d = 1.0, wmax_r = 1.0, xmax = 0.0;
-    DevBuf<int32_t> d_off, d_row_base, cell_of, count, cell_start, nch, row_chunk, scan_tmp, queue, orig;
+    DevBuf<int32_t> d_off, d_row_base, rank, count, boff, cell_start, queue, orig;
     DevBuf<int32_t> ovf;                 // 3PCF: queued apexes of the second and the device-memory pass
     DevBuf<unsigned char> big;           // 3PCF: device-memory neighbour lists
     DevBuf<unsigned char> d_regions, params;
     DevBuf<double4> pw;
-    DevBuf<float4> pl;
-    DevBuf<int4> chunks;                 // pair kernel: chunk descriptors
+    DevBuf<int2> cell;
     DevBuf<uint32_t> flags;
     DevBuf<unsigned long long> out;
     DevBuf<double> xyz, w;               // the batch's catalogue, input order
@@ -110,42 +117,34 @@ struct CtxView {
     const uint32_t* flags;
     const int32_t* orig;
     const int32_t* cell_start;
-    const float4* pl;
+    const int2* cell;
     const int32_t* row_chunk;
     const int4* chunks;
     const double* w;            // raw weights, original order (NULL for unit weights)
     int32_t n_chunks;
     GsExtra* extra;
     GsBatch* batch;
-    const double* xyz;           // catalogue, original order
-    const int32_t* buf;
 };
 
 CtxView view(gs_ctx* c);
 int ctx_set_device(gs_ctx* c);
-int ctx_upload(gs_ctx* c, const double* xyz, const double* w, const int32_t* buf, int64_t n);
 double round11(double h);
 int ctx_build_grid(gs_ctx* c, double rmax, int m, int sx, double* h_out);
 // row chunks of kChunk points of the context's grid for the full-stencil adjoint kernel: view().row_chunk,
 // view().n_chunks
 int ctx_row_chunks(gs_ctx* c);
-// device buffers of a grid build (sizes: cell_of, pw, pl, flags, orig n; cell_start, fill ncell + 1;
-// scan_tmp scan_scratch_size(ncell + 1)) and of its chunks (chunk_nc, chunk_off rows + 1; chunks max_chunks)
-struct GridBufs {
-    int32_t *cell_of, *cell_start, *fill, *chunk_nc, *chunk_off, *scan_tmp;
-    double4* pw;
-    float4* pl;
-    uint32_t* flags;
-    int32_t* orig;
-    int4* chunks;
+// what a call needs to know of a catalogue
+struct CatalogueInfo {
+    double bbox[6] = {0, 0, 0, 0, 0, 0};
+    double wmax = 1.0, wmax_d = 1.0, wmax_r = 1.0;  // largest, data, random weight (1 where none is positive)
+    long double wsum_d = 0, wsum_r = 0;
 };
-int grid_build_raw(const double* xyz, const double* w, const int32_t* buf, int64_t n, int64_t n_data,
-                   const double* bbox, double h, int sx, const GridBufs& b, int64_t max_cells, GridDesc* g_out,
-                   hipStream_t st);
-// row chunks of `group` points and their descriptors; their number is left at b.chunk_off[rows]
-hipError_t pair_chunks_raw(const GridDesc& g, int64_t n, int group, const GridBufs& b, hipStream_t st);
-// most chunks of `group` points that n points in nrow x-rows can make
-inline int64_t max_chunks(int64_t n, int64_t nrow, int group) { return n / group + std::min(n, nrow) + 1; }
+// The pass over a catalogue in device memory (launch_ingest) and one wait: copies it to xyz_out, w_out, buf_out
+// (unless they are the same), refuses invalid weights and coordinates.
+int ctx_catalogue_info(gs_ctx* c, const double* xyz, const double* w, const int32_t* buf, int64_t n, int64_t n_data,
+                       double* xyz_out, double* w_out, int32_t* buf_out, IngestScratch* scratch, CatalogueInfo* out);
+// grid description for a bounding box with cell edges h (y, z) and h / sx (x); fails beyond max_cells
+int grid_desc(const double* bbox, double h, int sx, int64_t max_cells, GridDesc* out);
 
 // Grid and work decomposition of the pair kernel for a catalogue.
 struct PairGrid {
@@ -161,7 +160,7 @@ PairGrid pair_grid(int64_t n, const double* bbox, double rmax, int cell_div, int
 // volume in rows of length len_x
 void pair_group(PairGrid& q, double dens, double len_x, double rmax);
 // binning constants of the pair kernel on that grid
-int fill_pair_bins(const gs_params& p, const PairGrid& q, double xmax, double wmax_d, double wmax_r, BinDesc& B);
+int fill_pair_bins(const gs_params& p, const double* t64, const PairGrid& q, double xmax, double wmax_d, double wmax_r, BinDesc& B);
 // Launch shape of the pair kernel.
 struct PairShape {
     int planes = 1, reps = 1, wg = kWG, waves = 0;  // histogram planes and replicas, threads, waves per CU
@@ -171,7 +170,11 @@ int pair2_shape(const PairVariant& v, PairShape* out);
 int pair_lg_parts(int64_t n, const PairGrid& q);
 int walk_shape(WalkArgs& a, const PairGrid& q, int64_t n, int wg, int waves, int n_cu);
 PairGrid ctx_pair_grid(const gs_ctx* c, const gs_params& p);
-int ctx_build_pair_grid(gs_ctx* c, const PairGrid& q);
+// builds the grid (unless it is there) and clears `extra` bytes (a multiple of 256) at *cleared
+int ctx_build_pair_grid(gs_ctx* c, const PairGrid& q, size_t extra, unsigned char** cleared);
+// exact bin thresholds (gs_bin_thresholds), kept in the context for the last few parameter sets
+int ctx_thresholds(gs_ctx* c, const gs_params& p, double* t);
+HostBuf& ctx_host(gs_ctx* c);
 hipError_t pair_launch(PairArgs& a, const PairVariant& var, const PairShape& shape, const PairGrid& q, int64_t n,
                        int n_cu, hipStream_t st);
 double choose_h_bbox(const double* bbox, double rmax, int m, int64_t max_cells, int sx);
@@ -180,7 +183,7 @@ int apex_cell_sx();
 void combine2(const unsigned long long* h_out, int nb, int nm, const BinDesc& B, bool weighted, long double Wd,
               long double Wr, uint64_t* cnt, double* wsum, double* n2, double* n3, gs_stats* st);
 int check_params(const gs_params* p, int mode);
-int fill_bins(const gs_params& p, double rrel, double xmax, double wmax_d, double wmax_r, BinDesc& B);
+int fill_bins(const gs_params& p, const double* t64, double rrel, double xmax, double wmax_d, double wmax_r, BinDesc& B);
 // fixed-point scales (exponents F of 2^F): of one point's weight in a pair product, for the largest
 // weight wmax of its class (wmax * 2^F < 2^26); of a triple product for the largest weight wmax
 int fx_shift_point(double wmax);

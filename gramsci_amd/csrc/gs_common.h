@@ -80,7 +80,7 @@ struct RegionDesc {
 // 2^31 such integers fits in 128 bits, so the host loops and the device
 // reduction give identical sums in any order.  Relative to wmax, a weight
 // loses at most 2^-96 in the rounding.
-inline int wsum_scale(double wmax)
+__host__ __device__ inline int wsum_scale(double wmax)
 {
     int e = 0;
     if (wmax > 0) (void)frexp(wmax, &e);   // wmax < 2^e

@@ -244,5 +244,27 @@ struct ItemQueue {
     }
 };
 
+// true in every thread of the last block to call it; resets the counter.  What the blocks wrote before is
+// visible to it.
+__device__ __forceinline__ bool last_block(unsigned* ticket)
+{
+    __shared__ bool s_last;
+    __threadfence();
+    __syncthreads();
+    if (threadIdx.x == 0) {
+        s_last = atomicAdd(ticket, 1u) == gridDim.x - 1;
+        if (s_last) *ticket = 0;
+    }
+    __syncthreads();
+    if (s_last) __threadfence();
+    return s_last;
+}
+
+template <class T>
+__device__ __forceinline__ T load_agent(const T* p)
+{
+    return __hip_atomic_load(p, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT);
+}
+
 }  // namespace dev
 }  // namespace gs

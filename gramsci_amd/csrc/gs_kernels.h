@@ -6,34 +6,53 @@
 namespace gs {
 
 // grid.hip
-hipError_t launch_bbox(const double* xyz, int64_t n, double* part, int nblk, hipStream_t st);
-// weights: per-block maxima of the data and of the random weights (part_max[2 * block + class]) and
-// the first invalid (negative or non-finite) index (atomic min; *bad starts at ~0), then per-block
-// 128-bit fixed-point sums over data and randoms ([nblk][4]: data lo, hi, randoms lo, hi)
-hipError_t launch_wcheck(const double* w, int64_t n, int64_t n_data, double* part_max, unsigned long long* bad,
-                         int nblk, hipStream_t st);
-hipError_t launch_wsum(const double* w, int64_t n, int64_t n_data, int k, unsigned long long* part, int nblk,
-                       hipStream_t st);
-hipError_t launch_cell_count(const double* xyz, int64_t n, const GridDesc& g, int32_t* cell_of, int32_t* count,
-                             hipStream_t st);
+// What the pass over a new catalogue finds: v = bounding box (3 lowest, 3 highest), largest data and random
+// weight, index of the first invalid (negative or non-finite) weight (1e308: none); s = exact fixed-point
+// sums of the data and the random weights (lo, hi each).  Lives in device memory, with a pointer to the
+// pinned host copy that the last kernel fills in.
+struct CatalogueStats {
+    double v[9];
+    unsigned long long s[4];
+    unsigned ticket;            // blocks done (zero between launches)
+    CatalogueStats* host;
+};
+struct IngestScratch {          // one per block
+    double v[9];
+    unsigned long long s[4];
+};
+constexpr int kIngestBlocks = 1024;
+// copies xyz, w, buf (w, buf may be NULL) to xyz_out, w_out, buf_out (or nothing where they are the same) and
+// fills *stats and its host copy
+hipError_t launch_ingest(const double* xyz, const double* w, const int32_t* buf, int64_t n, int64_t n_data,
+                         double* xyz_out, double* w_out, int32_t* buf_out, IngestScratch* scratch, CatalogueStats* stats,
+                         hipStream_t st);
+
+// Counting sort of a catalogue (input order) into the cells of a grid, or of each region's grid.
+struct GridArgs {
+    const double *xyz, *w;
+    const int32_t* buf;
+    int64_t n, n_data, ncell;
+    GridDesc g;                 // lo, dim: single grid; h, hx
+    const RegionDesc* regions;  // batch (nreg > 0)
+    const int32_t* off;         // nreg+1 first point of each region
+    int32_t nreg;
+    int32_t* rank;              // [n] scratch
+    int32_t* count;             // [2 ncell + 1] scratch: data and randoms per cell, zero before
+    int32_t* boff;              // [cell_scan_blocks(ncell)] scratch
+    unsigned* ticket;           // zero before and after
+    // the sorted catalogue: point and raw weight, x cell and x-row (over all regions), flags, input index
+    double4* pw;
+    int2* cell;
+    uint32_t* flags;
+    int32_t *orig, *cell_start; // cell_start[ncell + 1]
+};
+int64_t cell_scan_blocks(int64_t ncell);
+hipError_t launch_cell_sort(const GridArgs& a, hipStream_t st);
+
 hipError_t exclusive_scan(const int32_t* in, int32_t* out, int64_t n, int32_t* scratch, hipStream_t st);
 int64_t scan_scratch_size(int64_t n);
-hipError_t launch_scatter(const double* xyz, const double* w, const int32_t* buf, int64_t n, int64_t n_data,
-                          const GridDesc& g, const int32_t* cell_of, const int32_t* start, int32_t* fill,
-                          double4* pw, float4* pl, uint32_t* flags, int32_t* orig, hipStream_t st);
 hipError_t launch_row_chunks(const int32_t* start, int nx, int nrow, int group, int32_t* nch, hipStream_t st);
-
-// batched regions (grid.hip)
 hipError_t launch_fill_u32(void* p, int64_t n, uint32_t v, hipStream_t st);
-hipError_t launch_cell_count_b(const double* xyz, int64_t n, const int32_t* off, int nreg, const RegionDesc* reg,
-                               double h, double hx, int32_t* cell_of, int32_t* count, hipStream_t st);
-hipError_t launch_scatter_b(const double* xyz, const double* w, const int32_t* buf, int64_t n, const int32_t* off,
-                            int nreg, const RegionDesc* reg, double h, double hx, const int32_t* cell_of,
-                            const int32_t* start,
-                            int32_t* fill, double4* pw, float4* pl, uint32_t* flags, int32_t* orig,
-                            hipStream_t st);
-hipError_t launch_row_chunks_b(const int32_t* start, const RegionDesc* reg, const int32_t* row_base, int nreg,
-                               int nrow_tot, int group, int32_t* nch, hipStream_t st);
 
 // domain decomposition (decompose.hip)
 hipError_t launch_region_box(const float* xyz, const int32_t* reg, int64_t n, int nreg, int32_t* keys, hipStream_t st);
@@ -44,20 +63,20 @@ hipError_t launch_region_scatter(const float* xyz, int64_t n, const float* box, 
 // The half-stencil walk of the pair and adjoint kernels (gs_pair_tiles.h).
 struct WalkArgs {
     const double4* pw;          // sorted points: x, y, z, raw weight
-    const float4* pl;           // sorted: .w the cell x index
+    const int2* cell;           // sorted: x cell, x-row of cells (over all regions)
     const uint32_t* flags;      // sorted: bit0 random, bit1 never-apex
     const int32_t* cell_start;  // ncell+1
-    const int4* chunks;         // chunk descriptors (launch_chunks)
-    const int32_t* n_chunks_dev;
     const Row* rows;            // half stencil
     const BinDesc* bins;        // device copy
     int32_t* queue;             // 64 work counters (dev::ItemQueue), zeroed before launch
     GridDesc g;
+    int32_t n;                  // points
     int32_t nrows;
     int32_t group;              // points per chunk: 16, 32 or 64
     int32_t lg_parts;           // log2 of the work items per chunk
-    float cap_cells;            // largest extent of a chunk in x cells, less one
+    int32_t cap_cells;          // largest extent of a piece of a chunk in x cells, less one
     const RegionDesc* regions;  // batched regions (nreg > 0): per-region grids
+    const int32_t* row_base;    // nreg+1 first x-row of each region
     int32_t nreg;
 };
 
@@ -189,7 +208,7 @@ int quad4_occupancy(const QuadArgs& a, int nb, bool weighted);
 // Arguments of the persistent 2PCF adjoint kernel (adjoint.hip).
 struct AdjArgs {
     const double4* pw;
-    const float4* pl;
+    const int2* cell;           // sorted: x cell, x-row
     const uint32_t* flags;
     const int32_t* orig;
     const int32_t* cell_start;
@@ -227,9 +246,11 @@ int adjoint2h_occupancy(int nb, int nm, bool logb, bool buf);
 // G[orig[k]] = (Ghi[k] * 2^32 + Glo[k]) * 2^-F (the sums as doubles, original order)
 hipError_t launch_adj_fx(const unsigned long long* Glo, const long long* Ghi, const int32_t* orig, int64_t n, int F,
                          double* G, hipStream_t st);
+// part: 2 nblk + 2; stats: the pair kernel's two counters and a zero ticket; host_stats: pinned host memory
 hipError_t launch_adj_partials(const double* G, const double* w, int64_t n, int64_t n_data, double inv_wd,
-                               double inv_wr, double* part, int nblk, hipStream_t st);
-hipError_t launch_adj_finish(const double* G, int64_t n, int64_t n_data, double s_d, double s_r, double inv_wd,
+                               double inv_wr, double* part, int nblk, unsigned long long* stats,
+                               unsigned long long* host_stats, hipStream_t st);
+hipError_t launch_adj_finish(const double* G, int64_t n, int64_t n_data, const double* sums, double inv_wd,
                              double inv_wr, double* out, hipStream_t st);
 
 // largest dynamic LDS of the pair kernel (160 KiB less its static part)
@@ -242,10 +263,5 @@ hipError_t launch_pair_reduce(const unsigned long long* in, int copies, int nreg
                               unsigned long long* out, hipStream_t st);
 // Work-groups of wg threads per CU the pair kernel can keep resident (0 if it cannot run).
 int pair2_occupancy(const PairVariant& v, int planes, int reps, bool batched, int wg);
-// Chunk descriptors {first point, points, x-row in its region, region} of the row chunks row_chunk[nrow + 1]
-// (regions and row_base for a batch; else one grid with nx cells per row); at most max_chunks of them.
-hipError_t launch_chunks(const int32_t* row_chunk, int nrow, const int32_t* cell_start, int nx,
-                         const RegionDesc* regions, const int32_t* row_base, int nreg, int group, int64_t max_chunks,
-                         int4* out, hipStream_t st);
 
 }  // namespace gs

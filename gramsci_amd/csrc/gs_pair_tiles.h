@@ -242,7 +242,7 @@ __device__ __forceinline__ void walk(const WalkArgs& a, Sink& sink, const BinDes
     const int ai = lane & (group - 1), ai2 = ai ^ half;     // the lane's apexes in the chunk
     const bool batched = a.nreg > 0;
     int nx = a.g.dim[0], ny = a.g.dim[1], nz = a.g.dim[2], cb = 0;
-    int cur_r = batched ? -1 : 0;
+    int row0 = 0, row1 = batched ? 0 : ny * nz;     // x-rows of the current region
 
     int nq = 0;
     auto recheck = [&]() {
@@ -271,35 +271,35 @@ __device__ __forceinline__ void walk(const WalkArgs& a, Sink& sink, const BinDes
         wave_sync();
     };
 
-    ItemQueue items(a.queue, *a.n_chunks_dev << a.lg_parts, nwv);
+    const int n_chunks = (int)(((long long)a.n + group - 1) / group);
+    ItemQueue items(a.queue, n_chunks << a.lg_parts, nwv);
     while (true) {
         const int item = items.next(lane, wv);
-        int4 ch = make_int4(0, 0, 0, 0);
-        if (item >= 0) ch = a.chunks[item >> a.lg_parts];
-        const int rg = batched && item >= 0 ? __builtin_amdgcn_readfirstlane(ch.w) : 0;
-        if (nq && (item < 0 || rg != cur_r)) recheck();
         if (item < 0) break;
-        if (batched && rg != cur_r) {
-            cur_r = rg;
-            const RegionDesc& rd = a.regions[rg];
-            nx = rd.dim[0]; ny = rd.dim[1]; nz = rd.dim[2];
-            cb = rd.cell_base;
-            sink.region(rg);
-        }
         const int part = item & ((1 << a.lg_parts) - 1);
-        const int row = __builtin_amdgcn_readfirstlane(ch.z);
-        const int cy = row % ny, cz = row / ny;
-        int ib = __builtin_amdgcn_readfirstlane(ch.x);
-        const int iend = ib + __builtin_amdgcn_readfirstlane(ch.y);
+        int ib = (item >> a.lg_parts) * group;
+        const int iend = (int)min((long long)a.n, (long long)ib + group);
 
-        // The FP32 error bounds hold for chunks of at most cap_cells + 1 cells in x: a longer one (few points
-        // in a long row) is taken in pieces [ib, ib + n_i).
+        // A chunk is taken in pieces [ib, ib + n_i) of one x-row and at most cap_cells + 1 cells in x, for which
+        // the FP32 error bounds hold.
         int n_i;
         for (; ib < iend; ib += n_i) {
-            const float cxl = ib + ai < iend ? a.pl[ib + ai].w : INFINITY;
-            const int cx_first = (int)__int_as_float(lane_int(__float_as_int(cxl), 0));
-            n_i = uniform(__popcll(lanes(lane < group && cxl - (float)cx_first <= a.cap_cells)));
-            const int cx_last = (int)__int_as_float(lane_int(__float_as_int(cxl), n_i - 1));
+            int2 cl = make_int2(0, -1);
+            if (ib + ai < iend) cl = a.cell[ib + ai];
+            const int cx_first = lane_int(cl.x, 0), grow = lane_int(cl.y, 0);
+            n_i = uniform(__popcll(lanes(lane < group && cl.y == grow && cl.x - cx_first <= a.cap_cells)));
+            const int cx_last = lane_int(cl.x, n_i - 1);
+            if (batched && (grow < row0 || grow >= row1)) {
+                if (nq) recheck();
+                const int rg = uniform(upper_index(a.row_base, a.nreg, grow));
+                const RegionDesc& rd = a.regions[rg];
+                nx = rd.dim[0]; ny = rd.dim[1]; nz = rd.dim[2];
+                cb = rd.cell_base;
+                row0 = rd.row_base;
+                row1 = row0 + ny * nz;
+                sink.region(rg);
+            }
+            const int cy = (grow - row0) % ny, cz = (grow - row0) / ny;
 
             // ---- the lane's apexes, relative to the chunk's middle point
             const bool v1 = ai < n_i, v2 = ai2 < n_i;
@@ -399,6 +399,7 @@ __device__ __forceinline__ void walk(const WalkArgs& a, Sink& sink, const BinDes
             sink.piece(ib, n_i);
         }
     }
+    if (nq) recheck();
 }
 
 }  // namespace dev

@@ -7,9 +7,9 @@
 // (theta(j->i) = -theta(i->j) exactly).
 //
 // Work decomposition.  Points are sorted by cell with x fastest, so an x-row
-// of cells (fixed cy, cz) is one contiguous range.  A chunk is up to `group`
-// (16, 32 or 64) consecutive points of one x-row; a work item is one of
-// `parts` equal shares of a chunk's candidates.  The wave reads the point
+// of cells (fixed cy, cz) is one contiguous range.  A chunk is `group` (16, 32
+// or 64) consecutive points, taken in pieces of one x-row; a work item is one
+// of `parts` equal shares of a chunk's candidates.  The wave reads the point
 // ranges of 64 stencil rows at once (one row per lane), numbers their points
 // by a prefix sum, and takes them in tiles of 64 that run across rows, so no
 // tile but the last is partial.  Every lane holds two apexes and one tile
@@ -477,43 +477,6 @@ int pair2_occupancy(const PairVariant& v, int planes, int reps, bool batched, in
     const size_t lds = pair2_lds_bytes(v.nb, v.nm, planes, reps, v.weighted, batched, wg);
     if (lds > kPairLdsMax) return 0;
     return with_variant(v, [&](auto k) { return k.occupancy(lds, wg); });
-}
-
-// ---------------------------------------------------------------- chunks
-// Descriptors of the pair kernels' chunks: {first point, points, x-row in its region, region}.
-__global__ __launch_bounds__(256) void k_chunks(const int32_t* __restrict__ row_chunk, int nrow,
-                                                const int32_t* __restrict__ cell_start, int nx,
-                                                const RegionDesc* __restrict__ regions,
-                                                const int32_t* __restrict__ row_base, int nreg, int group,
-                                                int4* __restrict__ out)
-{
-    const int n = row_chunk[nrow];
-    for (int c = blockIdx.x * blockDim.x + threadIdx.x; c < n; c += gridDim.x * blockDim.x) {
-        const int grow = upper_index(row_chunk, nrow, c);
-        int row = grow, r = 0, c0, dim = nx;
-        if (nreg > 0) {
-            r = upper_index(row_base, nreg, grow);
-            row = grow - regions[r].row_base;
-            dim = regions[r].dim[0];
-            c0 = regions[r].cell_base + row * dim;
-        } else {
-            c0 = row * dim;
-        }
-        const int i0 = cell_start[c0] + (c - row_chunk[grow]) * group;
-        out[c] = make_int4(i0, min(group, cell_start[c0 + dim] - i0), row, r);
-    }
-}
-
-hipError_t launch_chunks(const int32_t* row_chunk, int nrow, const int32_t* cell_start, int nx,
-                         const RegionDesc* regions, const int32_t* row_base, int nreg, int group, int64_t max_chunks,
-                         int4* out, hipStream_t st)
-{
-    int64_t nblk = (max_chunks + 255) / 256;
-    if (nblk > 4096) nblk = 4096;
-    if (nblk < 1) nblk = 1;
-    hipLaunchKernelGGL(k_chunks, dim3((unsigned)nblk), dim3(256), 0, st, row_chunk, nrow, cell_start, nx, regions,
-                       row_base, nreg, group, out);
-    return hipGetLastError();
 }
 
 }  // namespace gs

@@ -71,6 +71,7 @@ class Engine:
         nd = n if n_data is None else int(n_data)
         if nd < 0 or nd > n:
             raise ValueError("n_data out of range")
+        self.generation += 1        # also where the hand-over fails: the context then holds no catalogue
         if is_dev:
             import torch
             xyz = xyz.to(torch.float64).contiguous()
@@ -94,7 +95,6 @@ class Engine:
             L.check(self._lib.gs_set_catalogue(self._ctx, L.ptr(xyz), L.ptr(w), L.ptr(buf, ctypes.c_int32),
                                                nd, n - nd))
         self.n_data, self.n_rand = nd, n - nd
-        self.generation += 1
 
     def set_catalogue_batched(self, xyz, w, buf, off, ndata):
         """Independent regions: region r is points off[r]:off[r+1] (data first,
