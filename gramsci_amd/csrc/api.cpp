@@ -272,6 +272,37 @@ int fill_bins(const gs_params& p, const double* t64, double rrel, double xmax, d
     return GS_OK;
 }
 
+// Tables of the triplet kernel on the matrix cores; its header derives the error bound.  ok[b].y and rej_w bound
+// differences rounded to FP32: rounding is monotonic, so s >= hi implies s - lo >= hi - lo also when rounded.
+void fill_triplet_matrix(const gs_params& p, const double* t64, double h, double hx, TripMatrix& M)
+{
+    memset(&M, 0, sizeof(M));
+    const int nb = p.nbins, e = std::ilogb(p.rmax);
+    M.t_top = std::min(t64[nb], t64[nb + 1]);
+    M.inv_h = 1.0 / h;
+    M.inv_hx = 1.0 / hx;
+    M.scale = std::ldexp(1.0, -e);
+    const double r = std::ldexp(p.rmax, -e), err = std::ldexp(r * r, -18) * 1.01;
+    auto t = [&](int b) { return std::ldexp(t64[b], -2 * e); };
+    for (int b = 0; b < nb; ++b) {
+        const float lo = f_up(t(b) + err);
+        const float hi = f_down((b == nb - 1 ? std::min(t(nb), t(nb + 1)) : t(b + 1)) - err);
+        M.ok[b] = make_float2(lo, hi > lo ? hi - lo : 0.0f);
+    }
+    M.rej_lo = f_down(t(0) - err);
+    const float w = std::nextafter(f_up(t(nb + 1) + err) - M.rej_lo, INFINITY);
+    memcpy(&M.rej_w, &w, sizeof(w));
+    if (p.log_bins) {
+        const double inv = 1.0 / ((std::log10(p.rmax) - std::log10(p.rmin)) / nb);
+        M.ua = (float)(0.5 * std::log10(2.0) * inv);
+        M.ub = (float)((std::log10(2.0) * e - std::log10(p.rmin)) * inv);
+    } else {
+        const double inv = 1.0 / ((p.rmax - p.rmin) / nb);
+        M.ua = (float)std::ldexp(inv, e);
+        M.ub = (float)(-p.rmin * inv);
+    }
+}
+
 // fill_bins for the pair kernel.  A chunk's points lie within q.ext of its reference point per axis, so a
 // pair within rmax has coordinates (relative to that point) of at most q.ext and q.ext + rmax: rounding
 // both to FP32 and subtracting costs at most u (2 ext + 2 rmax) per component, u = 2^-24.

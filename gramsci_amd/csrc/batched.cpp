@@ -135,7 +135,9 @@ static int get_plan(gs_ctx* c, const gs_params& p, const BatchTune& tu, int kind
     // triplet kernel: configuration and find_normal tables, LDS plan
     std::vector<uint16_t> tab3;
     std::vector<uint8_t> ntab;
-    TripArgs ta{};
+    TripArgs ta{}, tm{};            // tm: the matrix kernel (as for a single catalogue)
+    bool mat = false;
+    std::vector<uint32_t> cfgb;
     int nh = 0;
     if (kind == 3) {
         tab3 = table3_hist(nb);
@@ -147,14 +149,20 @@ static int get_plan(gs_ctx* c, const gs_params& p, const BatchTune& tu, int kind
         ta.nrows = (int)rows.size();     // the LDS plan holds the stencil rows' table
         if ((rc = plan_triplet_lds(ta, nb, fp64, weighted))) return rc;
         nh = ta.ncfg * nm * 4;
+        tm = ta;
+        mat = nm == 1 && !fp64 && !weighted && plan_triplet_matrix(tm, nb, B.has_buf);
+        if (mat) cfgb = cfg_bins3(nb);
     }
-    const size_t nout = kind == 3 ? (size_t)nreg * 3 * nh + 8 : (size_t)nreg * 3 * nbt + 4 + (size_t)pair_copies(nreg, nbt) * pair_copy_words(nreg, nbt);
+    const int64_t words3 = triplet_copy_words((int64_t)nreg * nh);
+    const int copies3 = output_copies(words3);
+    constexpr int kQueueInts = 64 * kQueuePad;      // work counters of a pass; two passes at 32 and after
+    const size_t nout = kind == 3 ? (size_t)(1 + copies3) * words3 : (size_t)nreg * 3 * nbt + 4 + (size_t)pair_copies(nreg, nbt) * pair_copy_words(nreg, nbt);
     const int64_t nblk_scan = cell_scan_blocks(cells);
     // captured graphs hold raw pointers to the shared work buffers: if any of
     // them has to grow, every existing plan is destroyed before reallocating
     const bool grow = (size_t)n > B.rank.cap || (size_t)(2 * cells + 1) > B.count.cap ||
                       (size_t)(cells + 1) > B.cell_start.cap || (size_t)nblk_scan > B.boff.cap || nout > B.out.cap ||
-                      (kind == 3 && (size_t)(2 * n + 3) > B.ovf.cap) || B.queue.cap < 32 + 64 * kQueuePad;
+                      (kind == 3 && (size_t)(2 * n + 3) > B.ovf.cap) || B.queue.cap < 32 + 2 * kQueueInts;
     if (grow) {
         for (auto& pl : B.plans) {
             if (pl.exec) (void)hipGraphExecDestroy(pl.exec);
@@ -164,7 +172,7 @@ static int get_plan(gs_ctx* c, const gs_params& p, const BatchTune& tu, int kind
         B.plans.clear();
     }
     if ((rc = B.rank.reserve(n)) || (rc = B.count.reserve(2 * cells + 1)) || (rc = B.cell_start.reserve(cells + 1)) ||
-        (rc = B.boff.reserve(nblk_scan)) || (rc = B.queue.reserve(32 + 64 * kQueuePad)) ||
+        (rc = B.boff.reserve(nblk_scan)) || (rc = B.queue.reserve(32 + 2 * kQueueInts)) ||
         (kind == 3 && (rc = B.ovf.reserve(2 * n + 3))) || (rc = B.orig.reserve(n)) || (rc = B.pw.reserve(n)) ||
         (rc = B.cell.reserve(n)) || (rc = B.flags.reserve(n)) || (rc = B.out.reserve(nout)))
         return rc;
@@ -174,7 +182,9 @@ static int get_plan(gs_ctx* c, const gs_params& p, const BatchTune& tu, int kind
     const size_t rb_off = rows_off + ((rows.size() * sizeof(Row) + 15) / 16) * 16;
     const size_t tab_off = rb_off + (((nreg + 1) * sizeof(int32_t) + 15) / 16) * 16;
     const size_t ntab_off = tab_off + ((tab3.size() * 2 + 15) / 16) * 16;
-    const size_t blob = ntab_off + ntab.size() + 16;
+    const size_t mat_off = (ntab_off + ntab.size() + 15) / 16 * 16;
+    const size_t cfgb_off = mat_off + (mat ? (sizeof(TripMatrix) + 15) / 16 * 16 : 0);
+    const size_t blob = cfgb_off + cfgb.size() * 4 + 16;
     // each plan owns its blob so that graphs of several parameter sets can coexist
     B.plans.emplace_back();
     GsBatch::Plan& P = B.plans.back();
@@ -192,6 +202,13 @@ static int get_plan(gs_ctx* c, const gs_params& p, const BatchTune& tu, int kind
         e = hipMemcpyAsync(pblob->ptr + tab_off, tab3.data(), tab3.size() * 2, hipMemcpyHostToDevice, v.stream);
     if (e == hipSuccess && !ntab.empty())
         e = hipMemcpyAsync(pblob->ptr + ntab_off, ntab.data(), ntab.size(), hipMemcpyHostToDevice, v.stream);
+    TripMatrix tmat;
+    if (mat) {
+        fill_triplet_matrix(p, t64, h, hx, tmat);
+        if (e == hipSuccess) e = hipMemcpyAsync(pblob->ptr + mat_off, &tmat, sizeof(tmat), hipMemcpyHostToDevice, v.stream);
+        if (e == hipSuccess)
+            e = hipMemcpyAsync(pblob->ptr + cfgb_off, cfgb.data(), cfgb.size() * 4, hipMemcpyHostToDevice, v.stream);
+    }
     if (e == hipSuccess) e = hipStreamSynchronize(v.stream);
     if (e != hipSuccess) { pblob->release(); B.plans.pop_back(); return hip_fail(e, "batch upload"); }
     const RegionDesc* d_reg = (const RegionDesc*)pblob->ptr;
@@ -268,11 +285,14 @@ static int get_plan(gs_ctx* c, const gs_params& p, const BatchTune& tu, int kind
         ta.bins = (const BinDesc*)(pblob->ptr + bin_off);
         ta.cfg_tab = (const uint16_t*)(pblob->ptr + tab_off);
         ta.ntab = ntab.empty() ? nullptr : (const uint8_t*)(pblob->ptr + ntab_off);
-        ta.queue = B.queue.ptr;
+        ta.queue = B.queue.ptr + 32;
         ta.err = B.queue.ptr + 8;
-        ta.out_cnt = B.out.ptr;
-        ta.out_w = B.out.ptr + (size_t)nreg * nh;
-        ta.out_stats = B.out.ptr + (size_t)nreg * 3 * nh;
+        // the copies' sum, then the copies
+        ta.out_cnt = B.out.ptr + words3;
+        ta.out_w = ta.out_cnt + (size_t)nreg * nh;
+        ta.out_stats = ta.out_cnt + (size_t)nreg * 3 * nh;
+        ta.copies = copies3;
+        ta.copy_stride = words3;
         ta.g.h = h;
         ta.g.h32 = (float)h;
         ta.g.hx = hx;
@@ -283,14 +303,24 @@ static int get_plan(gs_ctx* c, const gs_params& p, const BatchTune& tu, int kind
         ta.equi = 0;
         ta.nreg = nreg;
         ta.regions = d_reg;
+        ta.matrix = (const TripMatrix*)(pblob->ptr + mat_off);
+        ta.cfg_bins = (const uint32_t*)(pblob->ptr + cfgb_off);
+        if (mat) {
+            const int reps = tm.reps, kmax = tm.kmax, buf = tm.buf;
+            tm = ta;
+            tm.reps = reps;
+            tm.kmax = kmax;
+            tm.buf = buf;
+        }
     }
     // 3PCF in two captured passes: the first with a neighbour list sized for twice the largest
     // mean neighbour count of any region's box (apexes with more neighbours are queued), the
     // second over the queued apexes with the largest list that fits (count read on the device).
     // Apexes with more neighbours than that are queued again (B.ovf[n+1] count, [n+2] largest
     // neighbour count, apexes from n+3) for a pass with device-memory lists after the replay.
-    TripArgs ta1 = ta, ta2 = ta;
-    int nblocks2 = 0;
+    TripArgs ta1 = mat ? tm : ta, ta2 = ta1;
+    int nblocks2 = 0, wg1 = 0;
+    bool wave = false;      // matrix kernel: one wave per apex
     if (kind == 3) {
         ta1.ovf_n = B.ovf.ptr + n + 1;
         ta1.ovf = B.ovf.ptr + n + 3;
@@ -305,34 +335,46 @@ static int get_plan(gs_ctx* c, const gs_params& p, const BatchTune& tu, int kind
             for (int k = 0; k < 3; ++k) vol *= std::max(B.bbox[6 * r + 3 + k] - B.bbox[6 * r + k], p.rmax);
             kmean = std::max(kmean, (double)(B.off[r + 1] - B.off[r]) * shell / vol);
         }
-        ta1.wg = tu.wg > 0 ? tu.wg : triplet_wg(kmean);
         const char* evl = getenv("GS_T3_KMAX_LDS");     // test override: a shorter second-pass list
-        if (evl && *evl) ta.kmax = ta1.kmax = ta2.kmax = std::max(64, std::min(ta.kmax, atoi(evl)));
-        int kmax1 = std::min(ta.kmax, std::max(128, (int)std::ceil(2.0 * kmean / 64.0) * 64));
+        if (evl && *evl) {
+            ta.kmax = std::max(64, std::min(ta.kmax, atoi(evl)));
+            ta1.kmax = ta2.kmax = mat ? std::max(64, std::min(ta1.kmax, atoi(evl) / 64 * 64)) : ta.kmax;
+        }
+        const int full = ta1.kmax;
+        int kmax1 = std::min(full, std::max(128, (int)std::ceil(2.0 * kmean / 64.0) * 64));
         const char* ev = getenv("GS_T3_KMAX");      // tuning override (unset or empty: automatic)
-        if (tu.kmax1 > 0) kmax1 = std::max(64, std::min(ta.kmax, tu.kmax1));
-        else if (ev && *ev) kmax1 = std::max(64, std::min(ta.kmax, atoi(ev)));
-        if (kmax1 < ta.kmax) {
+        if (tu.kmax1 > 0) kmax1 = std::max(64, std::min(full, tu.kmax1));
+        else if (ev && *ev) kmax1 = std::max(64, std::min(full, atoi(ev)));
+        if (mat) {
+            kmax1 = std::max(64, kmax1 / 64 * 64);
+            wave = triplet_matrix_team(ta1, nb, kmax1, tu.wg);
+            ta1.kmax = full;
+            wg1 = wave ? kWave : ta1.wg;
+        } else {
+            wg1 = ta1.wg = tu.wg > 0 ? tu.wg : triplet_wg(kmean);
+        }
+        if (kmax1 < full) {
             ta1.kmax = kmax1;
             ta1.ovf_n = B.ovf.ptr;
             ta1.ovf = B.ovf.ptr + 1;
             ta2.items = B.ovf.ptr + 1;
             ta2.n_items_dev = B.ovf.ptr;
-            ta2.queue = B.queue.ptr + 16;
-            ta2.wg = kWG;           // the apexes with the most neighbours, one per fetch
+            ta2.queue = ta.queue + kQueueInts;
+            ta2.wg = mat ? 2 * kWG : kWG;   // the apexes with the most neighbours, one per fetch
             ta2.batch = 1;
-            nblocks2 = v.n_cu * triplet3_occupancy(ta2, nb, fp64, weighted);
+            nblocks2 = v.n_cu * (mat ? triplet_matrix_occupancy(ta2, nb, false) : triplet3_occupancy(ta2, nb, fp64, weighted));
         }
     }
-    const int occ = kind == 3 ? triplet3_occupancy(ta1, nb, fp64, weighted) : pair_waves / (pair_wg / kWave);
+    const int occ = kind != 3 ? pair_waves / (pair_wg / kWave)
+                  : std::max(1, mat ? triplet_matrix_occupancy(ta1, nb, wave) : triplet3_occupancy(ta1, nb, fp64, weighted));
     const int nblocks = kind == 3 ? std::max(1, (int)std::min<int64_t>((int64_t)v.n_cu * occ, std::max<int64_t>(n, 1)))
                                   : (v.n_cu * occ + 7) / 8 * 8;
-    if (kind == 3) ta1.batch = triplet_batch(n, nblocks);
+    if (kind == 3) ta1.batch = std::max(triplet_batch(n, nblocks), wave ? 8 * ta1.wg / kWave : 1);
 
     // capture: clear, sort into cells, pair or triplet kernel
     e = hipStreamBeginCapture(v.stream, hipStreamCaptureModeThreadLocal);
     if (e == hipSuccess) e = launch_fill_u32(B.count.ptr, 2 * cells + 1, 0, v.stream);
-    if (e == hipSuccess) e = launch_fill_u32(B.queue.ptr, 32 + 64 * kQueuePad, 0, v.stream);
+    if (e == hipSuccess) e = launch_fill_u32(B.queue.ptr, 32 + 2 * kQueueInts, 0, v.stream);
     if (e == hipSuccess && nblocks2 > 0) e = launch_fill_u32(B.ovf.ptr, 1, 0, v.stream);
     if (e == hipSuccess && kind == 3) e = launch_fill_u32(B.ovf.ptr + n + 1, 2, 0, v.stream);
     if (e == hipSuccess) e = launch_fill_u32(B.out.ptr, (int64_t)nout * 2, 0, v.stream);
@@ -342,8 +384,13 @@ static int get_plan(gs_ctx* c, const gs_params& p, const BatchTune& tu, int kind
         if (e == hipSuccess)
             e = launch_pair_reduce(a.out_cnt, a.copies, nreg, nbt, nm, weighted, B.out.ptr, v.stream);
     } else if (e == hipSuccess && n > 0) {
-        e = launch_triplet3(ta1, nb, fp64, weighted, nblocks, v.stream);
-        if (e == hipSuccess && nblocks2 > 0) e = launch_triplet3(ta2, nb, fp64, weighted, nblocks2, v.stream);
+        e = mat ? launch_triplet_matrix(ta1, nb, wave, nblocks, v.stream)
+                : launch_triplet3(ta1, nb, fp64, weighted, nblocks, v.stream);
+        if (e == hipSuccess && nblocks2 > 0)
+            e = mat ? launch_triplet_matrix(ta2, nb, false, nblocks2, v.stream)
+                    : launch_triplet3(ta2, nb, fp64, weighted, nblocks2, v.stream);
+        if (e == hipSuccess)
+            e = launch_sum_copies(ta.out_cnt, copies3, words3, (int64_t)nreg * nh, (int64_t)nreg * nh, 8, B.out.ptr, v.stream);
     }
     hipGraph_t graph = nullptr;
     hipError_t e2 = hipStreamEndCapture(v.stream, &graph);
@@ -375,8 +422,8 @@ static int get_plan(gs_ctx* c, const gs_params& p, const BatchTune& tu, int kind
     P.kind = kind;
     P.nh = nh;
     if (kind == 3) {
-        P.kmax = ta.kmax;
-        P.wg1 = ta1.wg;
+        P.kmax = mat ? ta2.kmax : ta.kmax;
+        P.wg1 = wg1;
         P.kmax1 = ta1.kmax;
         P.t3 = ta;              // tables, outputs and regions of the device-memory pass
         P.t3_list = B.ovf.ptr + n + 3;
@@ -398,9 +445,17 @@ static int run_plan(gs_ctx* c, GsBatch::Plan& P, float* ms)
     if (e != hipSuccess) return hip_fail(e, "batched graph launch");
     if (P.kind == 3) {
         // apexes with more neighbours than any LDS list: lists in device memory (not captured)
-        int rc = triplet_glist_pass(P.t3, P.nb, P.fp64, P.weighted, P.t3_list, P.t3_cnt, B.queue.ptr + 24, B.big,
-                                    v.n_cu, v.stream, nullptr);
-        if (rc) return rc;
+        int32_t h[2] = {0, 0};
+        e = hipMemcpyAsync(h, P.t3_cnt, sizeof(h), hipMemcpyDeviceToHost, v.stream);
+        if (e == hipSuccess) e = hipStreamSynchronize(v.stream);
+        if (e != hipSuccess) return hip_fail(e, "3PCF queued apex count");
+        if (h[0] > 0) {
+            const int64_t ne = (int64_t)B.nreg * P.nh;
+            int rc = triplet_glist_pass(P.t3, P.nb, P.fp64, P.weighted, P.t3_list, h, P.t3.queue, B.big, v.n_cu, v.stream);
+            if (rc) return rc;
+            e = launch_sum_copies(P.t3.out_cnt, P.t3.copies, P.t3.copy_stride, ne, ne, 8, B.out.ptr, v.stream);
+            if (e != hipSuccess) return hip_fail(e, "3PCF device-memory pass");
+        }
     }
     (void)hipEventRecord(v.ev[3], v.stream);
     e = hipStreamSynchronize(v.stream);

@@ -41,6 +41,7 @@ struct GsExtra {
     DevBuf<double> dbl;
     DevBuf<int32_t> i32;
     DevBuf<unsigned char> big;      // device-memory neighbour lists of the last 3PCF/4PCF pass
+    DevBuf<unsigned char> big_zero; // 3PCF/4PCF: what a call clears (work counters, outputs)
 };
 void extra_release(GsExtra& x);
 
@@ -183,6 +184,7 @@ int apex_cell_sx();
 void combine2(const unsigned long long* h_out, int nb, int nm, const BinDesc& B, bool weighted, long double Wd,
               long double Wr, uint64_t* cnt, double* wsum, double* n2, double* n3, gs_stats* st);
 int check_params(const gs_params* p, int mode);
+void fill_triplet_matrix(const gs_params& p, const double* t64, double h, double hx, TripMatrix& M);
 int fill_bins(const gs_params& p, const double* t64, double rrel, double xmax, double wmax_d, double wmax_r, BinDesc& B);
 // fixed-point scales (exponents F of 2^F): of one point's weight in a pair product, for the largest
 // weight wmax of its class (wmax * 2^F < 2^26); of a triple product for the largest weight wmax
@@ -208,10 +210,15 @@ int triplet_wg(double kmean);
 // (GS_APEX_BATCH overrides)
 int triplet_batch(int64_t n, int nblocks);
 void combine3(const long double* S, int nq, long double Wd, long double Wr, bool with_n3, double* n2, double* n3);
-// last 3PCF pass over the apexes queued in d_list (count d_cnt[0], largest neighbour count d_cnt[1]),
-// with neighbour lists in device memory (pcf34.cpp); *n_apex (may be NULL) receives the count
-int triplet_glist_pass(const TripArgs& base, int nb, bool fp64, bool weighted, const int32_t* d_list,
-                       const int32_t* d_cnt, int32_t* d_queue, DevBuf<unsigned char>& scratch, int n_cu,
-                       hipStream_t st, int* n_apex);
+// The matrix triplet kernel (triplet_matrix.hip) for nb bins: whether it takes the call, the histogram replicas and
+// the longest list of a pass with one apex per work-group (a.reps, a.kmax); and its team and work-group size for
+// lists of kmax1 entries.  cfg_bins: the three bins of each configuration, a byte each.
+bool plan_triplet_matrix(TripArgs& a, int nb, bool buf);
+bool triplet_matrix_team(TripArgs& a, int nb, int kmax1, int wg);
+std::vector<uint32_t> cfg_bins3(int nb);
+// last 3PCF pass over the apexes queued in d_list (h: their count, positive, and the largest neighbour count),
+// with neighbour lists in device memory (pcf34.cpp); d_queue: an ItemQueue's counters
+int triplet_glist_pass(const TripArgs& base, int nb, bool fp64, bool weighted, const int32_t* d_list, const int32_t h[2],
+                       int32_t* d_queue, DevBuf<unsigned char>& scratch, int n_cu, hipStream_t st);
 
 }  // namespace gs

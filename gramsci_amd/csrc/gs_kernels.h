@@ -91,15 +91,16 @@ struct PairArgs : WalkArgs {
     int32_t planes;             // with buffer points: 2 if the LDS histogram has a plane per direction count
 };
 
-// One copy of the pair kernel's outputs: [nreg][2][nbt] counts, [nreg][2][nbt][2] sums, 4 statistics.
-inline int64_t pair_copy_words(int64_t nreg, int64_t nbt) { return 6 * nreg * nbt + 4; }
-// Copies of the outputs: as many as fit 1 MiB, at most 64.
-inline int pair_copies(int64_t nreg, int64_t nbt)
+// Copies of `words` words that fit 1 MiB, at most 64 (a power of two, at least 1).
+inline int output_copies(int64_t words)
 {
     int c = 1;
-    while (c < 64 && 2 * c * pair_copy_words(nreg, nbt) <= 131072) c *= 2;
+    while (c < 64 && 2 * c * words <= 131072) c *= 2;
     return c;
 }
+// One copy of the pair kernel's outputs: [nreg][2][nbt] counts, [nreg][2][nbt][2] sums, 4 statistics.
+inline int64_t pair_copy_words(int64_t nreg, int64_t nbt) { return 6 * nreg * nbt + 4; }
+inline int pair_copies(int64_t nreg, int64_t nbt) { return output_copies(pair_copy_words(nreg, nbt)); }
 
 // The pair kernel's variant: histogram, precision, unit or given weights, bins, buffer points or none.
 struct PairVariant {
@@ -118,11 +119,14 @@ struct TripArgs {
     const BinDesc* bins;
     const uint16_t* cfg_tab;    // [nb][nb][nb] -> 0-based configuration (unused when equi)
     const uint8_t* ntab;        // RSD: [nm][nm] 0-based find_normal bin of (mu(k1), mu(k2))
-    int32_t* queue;             // 8 work counters
+    int32_t* queue;             // work counters (ItemQueue)
     int32_t* err;               // set to 1 if an apex has more than kmax neighbours
-    unsigned long long* out_cnt;    // [ncfg][nm][4]
-    unsigned long long* out_w;      // [ncfg][nm][4][2]
-    unsigned long long* out_stats;  // candidates, rechecks, overflow, units, binned
+    // outputs, `copies` of them copy_words() apart; work-group b adds to copy b mod copies
+    unsigned long long* out_cnt;    // [nreg][ncfg][nm][4]
+    unsigned long long* out_w;      // [nreg][ncfg][nm][4][2]
+    unsigned long long* out_stats;  // candidates, rechecks, overflow, units, evaluated pairs
+    int64_t copy_stride;
+    int32_t copies;             // power of two <= 64
     GridDesc g;
     int32_t nrows;
     int32_t n_items;            // apexes (all points; buffer points are skipped)
@@ -153,7 +157,33 @@ struct TripArgs {
     int32_t* ovf_kmax;
     void* glist;
     int64_t glist_stride;
+    // triplet_matrix.hip: tables, and the three bins of each configuration (a byte each); buffer points present
+    const struct TripMatrix* matrix;
+    const uint32_t* cfg_bins;
+    int32_t buf;
 };
+// Tables of the matrix kernel (fill_triplet_matrix), for coordinates scaled by a power of two such that rmax is
+// in [1, 2): bin b is certain if 0 <= s - ok[b].x < ok[b].y (in FP32), a pair certainly not kept unless
+// 0 <= s - rej_lo < rej_w (as a float's bits).
+struct TripMatrix {
+    double scale;
+    double t_top;               // kept neighbours of an apex: t64[0] < s < t_top (beyond, up to t64[nb+1]: overflow)
+    double inv_h, inv_hx;       // 1 / cell edges
+    float2 ok[kMaxBins + 1];
+    float rej_lo;
+    uint32_t rej_w;
+    float ua, ub;
+};
+// teams: waves of a work-group that take an apex each, or 1
+size_t triplet_matrix_lds(const TripArgs& a, int nb, int teams);
+hipError_t launch_triplet_matrix(const TripArgs& a, int nb, bool wave, int nblocks, hipStream_t st);
+int triplet_matrix_occupancy(const TripArgs& a, int nb, bool wave);
+// One copy of the triplet kernel's outputs (nh histogram entries over all regions): counts, sums, 8 statistics.
+inline int64_t triplet_copy_words(int64_t nh) { return 3 * nh + 8; }
+// Sums the copies into out (device or pinned host memory): entries [0, nplain) as 64-bit integers, then nwide
+// two-word integers, then ntail 64-bit ones.
+hipError_t launch_sum_copies(const unsigned long long* in, int copies, int64_t stride, int64_t nplain, int64_t nwide,
+                             int64_t ntail, unsigned long long* out, hipStream_t st);
 // bytes per neighbour of a device-memory neighbour list (glist) of the triplet kernel
 size_t triplet3_glist_entry_bytes(const TripArgs& a, bool fp64, bool weighted);
 size_t triplet3_lds_bytes(const TripArgs& a, int nb, bool fp64, bool weighted);

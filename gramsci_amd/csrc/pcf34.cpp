@@ -24,6 +24,7 @@ void extra_release(GsExtra& x)
     x.dbl.release();
     x.i32.release();
     x.big.release();
+    x.big_zero.release();
 }
 
 // bintable for the 3PCF (gramsci.F90:1459-1474), 0-based configuration of a
@@ -165,21 +166,50 @@ int plan_triplet_lds(TripArgs& a, int nb, bool fp64, bool weighted)
     return GS_OK;
 }
 
-// The last pass of the 3PCF: apexes whose neighbours outnumber every LDS list were queued
-// (d_list, count d_cnt[0], largest neighbour count d_cnt[1]); they run here with their
-// neighbour lists in device memory, one list per work-group, and the histogram in global
-// memory.  Reads the count (synchronising the stream) and launches nothing if it is 0.
-// `base` carries the pass's tables and outputs; d_queue is 8 work counters it may clear.
-int triplet_glist_pass(const TripArgs& base, int nb, bool fp64, bool weighted, const int32_t* d_list,
-                       const int32_t* d_cnt, int32_t* d_queue, DevBuf<unsigned char>& scratch, int n_cu,
-                       hipStream_t st, int* n_apex)
+std::vector<uint32_t> cfg_bins3(int nb)
 {
-    int32_t h[2] = {0, 0};
-    hipError_t e = hipMemcpyAsync(h, d_cnt, sizeof(h), hipMemcpyDeviceToHost, st);
-    if (e == hipSuccess) e = hipStreamSynchronize(st);
-    if (e != hipSuccess) return hip_fail(e, "3PCF queued apex count");
-    if (n_apex) *n_apex = h[0];
-    if (h[0] <= 0) return GS_OK;
+    std::vector<uint32_t> t;
+    for (int i = 0; i < nb; ++i)
+        for (int j = i; j < nb; ++j)
+            for (int k = j; k < nb; ++k) t.push_back((uint32_t)(i | j << 8 | k << 16));
+    return t;
+}
+
+bool plan_triplet_matrix(TripArgs& a, int nb, bool buf)
+{
+    a.buf = buf ? 1 : 0;
+    a.reps = 2;
+    const size_t hist = (size_t)nb * nb * nb * 4 * (buf ? 3 : 1) * 4;
+    if (hist > 32 * 1024) return false;     // beyond: the general kernel, whose histogram holds configurations
+    // replicas up to 8 KiB: more of them leave the LDS room for fewer work-groups (200k + 400k points, 5 bins:
+    // 2, 4, 8 replicas 11.5, 11.5, 12.3 ms; 16 regions, 4 bins, buffer points: 3.4, 3.7, 4.2 ms)
+    while (a.reps < 16 && hist * a.reps * 2 <= 8 * 1024) a.reps *= 2;
+    a.kmax = 4096;
+    while (a.kmax > 64 && triplet_matrix_lds(a, nb, 1) > 150 * 1024) a.kmax -= 64;
+    return triplet_matrix_lds(a, nb, 1) <= 150 * 1024;
+}
+
+// One wave per apex while four lists fit the LDS beside each other often enough (up to 256 entries: 16 regions of 60k points,
+// lists of 128, 3.6 ms, with work-groups of 256 6.4 ms), a work-group beyond (lists of 512 entries: 11.5 against 20.6 ms).
+bool triplet_matrix_team(TripArgs& a, int nb, int kmax1, int wg)
+{
+    a.kmax = kmax1;
+    const char* ev = getenv("GS_T3_WG");        // tuning override (unset or empty: automatic)
+    if (ev && *ev && (atoi(ev) == 64 || atoi(ev) == 128 || atoi(ev) == 256)) wg = atoi(ev);
+    const bool wave = (wg > 0 ? wg == 64 : kmax1 <= 256) && triplet_matrix_lds(a, nb, kWG / kWave) <= 150 * 1024;
+    a.wg = wave ? kWG : (wg > 0 ? wg : (triplet_matrix_lds(a, nb, 1) > 40 * 1024 ? 512 : kWG));
+    return wave;
+}
+
+// The last pass of the 3PCF: apexes whose neighbours outnumber every LDS list were queued
+// (d_list); they run here with their
+// neighbour lists in device memory, one list per work-group, and the histogram in global
+// memory.  h is the count (positive) and the largest neighbour count.
+// `base` carries the pass's tables and outputs; d_queue is an ItemQueue's counters, which it clears.
+int triplet_glist_pass(const TripArgs& base, int nb, bool fp64, bool weighted, const int32_t* d_list, const int32_t h[2],
+                       int32_t* d_queue, DevBuf<unsigned char>& scratch, int n_cu, hipStream_t st)
+{
+    hipError_t e;
     TripArgs a = base;
     a.items = d_list;
     a.n_items = h[0];
@@ -207,7 +237,7 @@ int triplet_glist_pass(const TripArgs& base, int nb, bool fp64, bool weighted, c
     if (rc) return rc;
     a.glist = scratch.ptr;
     a.glist_stride = (int64_t)stride;
-    e = hipMemsetAsync(d_queue, 0, 8 * sizeof(int32_t), st);
+    e = launch_fill_u32(d_queue, 64 * kQueuePad, 0u, st);
     if (e == hipSuccess) e = launch_triplet3(a, nb, fp64, weighted, nblk, st);
     if (e != hipSuccess) return hip_fail(e, "3PCF device-memory pass");
     return GS_OK;
@@ -273,26 +303,41 @@ static int count3(gs_ctx* c, const gs_params* p, bool equi, uint64_t* cnt, doubl
     a.equi = equi ? 1 : 0;
     a.nrows = (int)rows.size();      // the LDS plan holds the stencil rows' table
     if ((rc = plan_triplet_lds(a, nb, fp64, weighted))) return rc;
+    // FP32 counts of unit weights without mu bins: third sides from the matrix cores (am); its passes are the
+    // general kernel's, which also takes the apexes whose lists fit no LDS
+    TripArgs am = a;
+    const bool mat = !equi && nm == 1 && !fp64 && !weighted && plan_triplet_matrix(am, nb, v.has_buf);
+    const std::vector<uint32_t> cfgb = mat ? cfg_bins3(nb) : std::vector<uint32_t>();
 
+    // Parameters in one copy from pinned memory.  One region to clear: the work counters of two passes, the error
+    // flag, the counts of queued apexes, and the outputs' copies; their sum goes to pinned memory.
     GsExtra& X = *v.extra;
-    const size_t tab_off = ((sizeof(BinDesc) + 15) / 16) * 16;
-    const size_t ntab_off = tab_off + ((tab.size() * 2 + 15) / 16) * 16;
-    const size_t rows_off = ntab_off + ((ntab.size() + 15) / 16) * 16;
-    const size_t nout = (size_t)nh + 2 * (size_t)nh + 8;
-    if ((rc = X.params.reserve(rows_off + rows.size() * sizeof(Row) + 16)) || (rc = X.out.reserve(nout)) ||
-        (rc = X.queue.reserve(16)))
+    HostBuf& H = ctx_host(c);
+    const size_t tab_off = (sizeof(BinDesc) + 15) / 16 * 16;
+    const size_t ntab_off = tab_off + (tab.size() * 2 + 15) / 16 * 16;
+    const size_t mat_off = ntab_off + (ntab.size() + 15) / 16 * 16;
+    const size_t cfgb_off = mat_off + (mat ? (sizeof(TripMatrix) + 15) / 16 * 16 : 0);
+    const size_t rows_off = cfgb_off + (cfgb.size() * 4 + 15) / 16 * 16;
+    const size_t blob = rows_off + rows.size() * sizeof(Row), res_off = (blob + 255) / 256 * 256;
+    const int64_t words = triplet_copy_words(nh);
+    const int copies = output_copies(words);
+    constexpr size_t kQueueInts = 64 * kQueuePad, kHeadInts = 2 * kQueueInts + 64;
+    const size_t clear = kHeadInts * 4 + (size_t)copies * words * 8;
+    if ((rc = X.params.reserve(blob)) || (rc = X.big_zero.reserve(clear)) || (rc = H.reserve(res_off + words * 8 + 16)))
         return rc;
-    hipError_t e = hipMemcpyAsync(X.params.ptr, &B, sizeof(B), hipMemcpyHostToDevice, v.stream);
-    if (e == hipSuccess && !tab.empty())
-        e = hipMemcpyAsync(X.params.ptr + tab_off, tab.data(), tab.size() * 2, hipMemcpyHostToDevice, v.stream);
-    if (e == hipSuccess && !ntab.empty())
-        e = hipMemcpyAsync(X.params.ptr + ntab_off, ntab.data(), ntab.size(), hipMemcpyHostToDevice, v.stream);
-    if (e == hipSuccess && !rows.empty())
-        e = hipMemcpyAsync(X.params.ptr + rows_off, rows.data(), rows.size() * sizeof(Row), hipMemcpyHostToDevice,
-                           v.stream);
-    if (e == hipSuccess) e = hipMemsetAsync(X.out.ptr, 0, nout * sizeof(unsigned long long), v.stream);
-    if (e == hipSuccess) e = hipMemsetAsync(X.queue.ptr, 0, 16 * sizeof(int32_t), v.stream);
+    *(BinDesc*)H.ptr = B;
+    std::copy(tab.begin(), tab.end(), (uint16_t*)(H.ptr + tab_off));
+    std::copy(ntab.begin(), ntab.end(), H.ptr + ntab_off);
+    std::copy(rows.begin(), rows.end(), (Row*)(H.ptr + rows_off));
+    if (mat) fill_triplet_matrix(*p, t64, v.g.h, v.g.hx, *(TripMatrix*)(H.ptr + mat_off));
+    std::copy(cfgb.begin(), cfgb.end(), (uint32_t*)(H.ptr + cfgb_off));
+    hipError_t e = hipMemcpyAsync(X.params.ptr, H.ptr, blob, hipMemcpyHostToDevice, v.stream);
+    if (e == hipSuccess) e = launch_fill_u32(X.big_zero.ptr, (int64_t)clear / 4, 0u, v.stream);
     if (e != hipSuccess) return hip_fail(e, "3PCF parameter upload");
+    int32_t* const head = (int32_t*)X.big_zero.ptr;
+    int32_t* const d_cnt2 = head + 2 * kQueueInts + 16;     // second-pass apexes
+    int32_t* const d_cnt3 = head + 2 * kQueueInts + 32;     // last-pass apexes, their largest neighbour count, the error flag
+    unsigned long long* const out = (unsigned long long*)(head + kHeadInts);
 
     a.pw = v.pw;
     a.flags = v.flags;
@@ -302,16 +347,27 @@ static int count3(gs_ctx* c, const gs_params* p, bool equi, uint64_t* cnt, doubl
     a.bins = (const BinDesc*)X.params.ptr;
     a.cfg_tab = tab.empty() ? nullptr : (const uint16_t*)(X.params.ptr + tab_off);
     a.ntab = ntab.empty() ? nullptr : (const uint8_t*)(X.params.ptr + ntab_off);
-    a.queue = X.queue.ptr;
-    a.err = X.queue.ptr + 8;
-    a.out_cnt = X.out.ptr;
-    a.out_w = X.out.ptr + nh;
-    a.out_stats = X.out.ptr + 3 * nh;
+    a.queue = head;
+    a.err = d_cnt3 + 2;
+    a.out_cnt = out;
+    a.out_w = out + nh;
+    a.out_stats = out + 3 * nh;
+    a.copies = copies;
+    a.copy_stride = words;
     a.g = v.g;
     a.g.m = mst;
     a.nrows = (int)rows.size();
     const int n = (int)(v.n_data + v.n_rand);
     a.n_items = n;
+    a.matrix = (const TripMatrix*)(X.params.ptr + mat_off);
+    a.cfg_bins = (const uint32_t*)(X.params.ptr + cfgb_off);
+    if (mat) {
+        const int reps = am.reps, kmax = am.kmax, buf = am.buf;
+        am = a;
+        am.reps = reps;
+        am.kmax = kmax;
+        am.buf = buf;
+    }
 
     // Two passes.  The neighbour list in LDS bounds the work-groups a CU can hold, so the
     // first pass sizes it for the 99.5th percentile of the neighbour counts of ~8192
@@ -320,18 +376,16 @@ static int count3(gs_ctx* c, const gs_params* p, bool equi, uint64_t* cnt, doubl
     // one pass, so the sums are those of one pass.
     // An apex whose neighbours outnumber even the second pass's list is queued once more, for a
     // last pass with its list in device memory (triplet_glist_pass): no neighbour count is refused.
-    const int kmax_full = a.kmax;
+    const int kmax_full = mat ? am.kmax : a.kmax;
     int kmax1 = kmax_full;
     const int nsample = std::min(n, 8192);
     const int stride = nsample > 0 ? n / nsample : 1;
-    // i32: [0] second-pass count, [1, n] second-pass apexes, [n+1] last-pass count, [n+2] its largest
-    // neighbour count, [n+3, 2n+2] last-pass apexes, then the sampled neighbour counts
-    if ((rc = X.i32.reserve(2 * (size_t)n + 3 + nsample))) return rc;
-    int32_t* d_list2 = X.i32.ptr + 1;
-    int32_t* d_cnt3 = X.i32.ptr + n + 1;
-    int32_t* d_list3 = X.i32.ptr + n + 3;
+    // i32: second-pass apexes, last-pass apexes, the sampled neighbour counts
+    if ((rc = X.i32.reserve(2 * (size_t)n + nsample))) return rc;
+    int32_t* d_list2 = X.i32.ptr;
+    int32_t* d_list3 = X.i32.ptr + n;
     if (nsample > 0) {
-        int32_t* d_cnt = X.i32.ptr + 2 * n + 3;
+        int32_t* d_cnt = X.i32.ptr + 2 * (size_t)n;
         std::vector<int32_t> kc(nsample);
         e = launch_nbr_count(a, stride, nsample, nm > 1 ? 0 : 1, d_cnt, v.stream);
         if (e == hipSuccess) e = hipMemcpyAsync(kc.data(), d_cnt, nsample * sizeof(int32_t), hipMemcpyDeviceToHost, v.stream);
@@ -356,63 +410,62 @@ static int count3(gs_ctx* c, const gs_params* p, bool equi, uint64_t* cnt, doubl
     {
         const char* ev = getenv("GS_T3_KMAX_LDS");  // test override: a shorter second-pass list
         if (ev && *ev) {
-            a.kmax = std::max(64, std::min(kmax_full, atoi(ev)));
-            kmax1 = std::min(kmax1, a.kmax);
+            a.kmax = std::max(64, std::min(a.kmax, atoi(ev)));
+            am.kmax = std::max(64, std::min(am.kmax, atoi(ev) / 64 * 64));
+            kmax1 = std::min(kmax1, mat ? am.kmax : a.kmax);
         }
     }
-    const bool two_pass = kmax1 < a.kmax;
+    if (mat) kmax1 = std::max(64, kmax1 / 64 * 64);
+    const bool two_pass = kmax1 < (mat ? am.kmax : a.kmax);
     (void)hipEventRecord(v.ev[2], v.stream);
     if (n > 0) {
-        e = hipMemsetAsync(X.i32.ptr, 0, sizeof(int32_t), v.stream);
-        if (e == hipSuccess) e = hipMemsetAsync(d_cnt3, 0, 2 * sizeof(int32_t), v.stream);
-        if (e != hipSuccess) return hip_fail(e, "3PCF overflow counters");
-        TripArgs a1 = a;
+        auto launch = [&](TripArgs& t, bool wave, int most) {
+            const int occ = mat ? triplet_matrix_occupancy(t, nb, wave) : triplet3_occupancy(t, nb, fp64, weighted);
+            const int teams = wave ? t.wg / kWave : 1;
+            const int nblk = std::max(1, std::min(v.n_cu * std::max(occ, 1), (most + teams - 1) / teams));
+            // a wave team's work-group takes several apexes a wave between barriers
+            if (t.batch == 0) t.batch = std::max(triplet_batch(n, nblk), wave ? 8 * teams : 1);
+            return mat ? launch_triplet_matrix(t, nb, wave, nblk, v.stream)
+                       : launch_triplet3(t, nb, fp64, weighted, nblk, v.stream);
+        };
+        TripArgs a1 = mat ? am : a;
+        bool wave = false;
         a1.ovf_kmax = d_cnt3 + 1;
-        if (two_pass) {
-            a1.kmax = kmax1;
-            a1.ovf = d_list2;
-            a1.ovf_n = X.i32.ptr;
-        } else {
-            a1.ovf = d_list3;
-            a1.ovf_n = d_cnt3;
-        }
-        const int occ = triplet3_occupancy(a1, nb, fp64, weighted);
-        const int nblk1 = std::max(1, std::min(v.n_cu * occ, n));
-        a1.batch = triplet_batch(n, nblk1);
-        e = launch_triplet3(a1, nb, fp64, weighted, nblk1, v.stream);
+        a1.ovf = two_pass ? d_list2 : d_list3;
+        a1.ovf_n = two_pass ? d_cnt2 : d_cnt3;
+        if (two_pass) a1.kmax = kmax1;
+        if (mat) wave = triplet_matrix_team(a1, nb, a1.kmax, 0);
+        e = launch(a1, wave, n);
         if (e != hipSuccess) return hip_fail(e, "3PCF kernel launch");
         if (two_pass) {
-            int32_t nov = 0;
-            e = hipMemcpyAsync(&nov, X.i32.ptr, sizeof(int32_t), hipMemcpyDeviceToHost, v.stream);
-            if (e == hipSuccess) e = hipStreamSynchronize(v.stream);
-            if (e != hipSuccess) return hip_fail(e, "3PCF first pass");
-            if (nov > 0) {
-                TripArgs a2 = a;
-                a2.items = d_list2;
-                a2.n_items = nov;
-                a2.wg = kWG;            // the apexes with the most neighbours, one per fetch
-                a2.batch = 1;
-                a2.ovf = d_list3;
-                a2.ovf_n = d_cnt3;
-                a2.ovf_kmax = d_cnt3 + 1;
-                e = hipMemsetAsync(X.queue.ptr, 0, 8 * sizeof(int32_t), v.stream);   // work counters only
-                const int occ2 = triplet3_occupancy(a2, nb, fp64, weighted);
-                if (e == hipSuccess)
-                    e = launch_triplet3(a2, nb, fp64, weighted, std::max(1, std::min(v.n_cu * occ2, nov)), v.stream);
-                if (e != hipSuccess) return hip_fail(e, "3PCF second pass");
-            }
+            // the second pass, over the apexes with the most neighbours, reads their number on the device
+            TripArgs a2 = mat ? am : a;
+            a2.items = d_list2;
+            a2.n_items_dev = d_cnt2;
+            a2.wg = mat ? 2 * kWG : kWG;
+            a2.batch = 1;
+            a2.queue = head + kQueueInts;
+            a2.ovf = d_list3;
+            a2.ovf_n = d_cnt3;
+            a2.ovf_kmax = d_cnt3 + 1;
+            e = launch(a2, false, n);
+            if (e != hipSuccess) return hip_fail(e, "3PCF second pass");
         }
-        if ((rc = triplet_glist_pass(a, nb, fp64, weighted, d_list3, d_cnt3, X.queue.ptr, X.big, v.n_cu, v.stream,
-                                     nullptr)))
-            return rc;
     }
-    (void)hipEventRecord(v.ev[3], v.stream);
-    std::vector<unsigned long long> h_out(nout);
-    e = hipMemcpyAsync(h_out.data(), X.out.ptr, nout * sizeof(unsigned long long), hipMemcpyDeviceToHost, v.stream);
+    // the sums of the copies and the counters to pinned memory; once more after a last pass
+    unsigned long long* const h_out = (unsigned long long*)(H.ptr + res_off);
+    int32_t* const h_cnt = (int32_t*)(h_out + words);
     int32_t err = 0;
-    if (e == hipSuccess) e = hipMemcpyAsync(&err, X.queue.ptr + 8, sizeof(int32_t), hipMemcpyDeviceToHost, v.stream);
-    if (e == hipSuccess) e = hipStreamSynchronize(v.stream);
-    if (e != hipSuccess) return hip_fail(e, "3PCF kernel");
+    for (int pass = 0;; ++pass) {
+        (void)hipEventRecord(v.ev[3], v.stream);
+        e = launch_sum_copies(out, copies, words, nh, nh, 8, h_out, v.stream);
+        if (e == hipSuccess) e = hipMemcpyAsync(h_cnt, d_cnt3, 3 * sizeof(int32_t), hipMemcpyDeviceToHost, v.stream);
+        if (e == hipSuccess) e = hipStreamSynchronize(v.stream);
+        if (e != hipSuccess) return hip_fail(e, "3PCF kernel");
+        err = h_cnt[2];
+        if (pass > 0 || h_cnt[0] <= 0) break;
+        if ((rc = triplet_glist_pass(a, nb, fp64, weighted, d_list3, h_cnt, head, X.big, v.n_cu, v.stream))) return rc;
+    }
     if (err) return fail(GS_EHIP, "3PCF: an apex's neighbour list overflowed with no later pass (internal error)");
 
     std::vector<long double> S(nh);
@@ -422,7 +475,7 @@ static int count3(gs_ctx* c, const gs_params* p, bool equi, uint64_t* cnt, doubl
         if (wsum) wsum[k] = (double)S[k];
     }
     combine3(S.data(), ncfg * nm, v.wsum_d, v.wsum_r, !(equi && nm > 1), n2, n3);
-    fill_stats(st, v.ev, h_out.data() + 3 * nh, mst);
+    fill_stats(st, v.ev, h_out + 3 * nh, mst);
     if (st) {
         st->n_evaluated = h_out[3 * nh + 4];
         st->n_binned = 0;           // the binned triplets are the counts' total

@@ -156,10 +156,14 @@ __global__ __launch_bounds__(kWG) void k_triplet3(TripArgs a)
     const bool batched = GEN && a.nreg > 0;
     int cur_r = batched ? -1 : 0;   // region whose histogram the LDS holds (work-group uniform)
 
+    // the work-group's copy of the outputs
+    const size_t copy = (size_t)(blockIdx.x & (unsigned)(a.copies - 1)) * (size_t)a.copy_stride;
+    unsigned long long *const out_cnt = a.out_cnt + copy, *const out_w = a.out_w + copy;
+
     // adds the LDS histogram to region r's output and clears it (all threads of the work-group)
     auto drain = [&](int r) {
-        unsigned long long* oc = a.out_cnt + (size_t)r * nh;
-        unsigned long long* ow = a.out_w + (size_t)r * 2 * nh;
+        unsigned long long* oc = out_cnt + (size_t)r * nh;
+        unsigned long long* ow = out_w + (size_t)r * 2 * nh;
         for (int k = tid; k < nh; k += nt) {
             unsigned long long sum = 0;
             for (int q = 0; q < reps; ++q) { sum += hc[k * reps + q]; hc[k * reps + q] = 0; }
@@ -179,24 +183,30 @@ __global__ __launch_bounds__(kWG) void k_triplet3(TripArgs a)
     unsigned long long units = 0, rechk = 0, over = 0, cand = 0;   // binned triplets: the histogram's total
     unsigned long long evals = 0;   // neighbour pairs whose third side this kernel evaluated
     unsigned long long bound = 0;   // u32 increments since the last drain (uniform)
-    const int xcd = blockIdx.x & 7;
-    int tried = 0;
-
+    // work items: batches of consecutive apexes, fetched by wave 0
     const int n_items = a.n_items_dev ? *a.n_items_dev : a.n_items;
     const int bsz = max(a.batch, 1);
-    int b_next = 0, b_end = 0;      // thread 0: the work-group's current batch of apexes
+    ItemQueue items(a.queue, (n_items + bsz - 1) / bsz, 1);
+    int b_next = 0, b_end = 0;      // the rest of the current batch (work-group uniform)
     while (true) {
         if (tid == 0) {
-            if (b_next >= b_end) b_next = next_items(a.queue, n_items, xcd, tried, bsz, b_end);
-            s_item = b_next;        // -1 at the end
-            if (b_next >= 0) ++b_next;
             s_k = 0;
             s_kall = 0;
             s_over = 0;
         }
+        const bool fetch = b_next >= b_end;
+        if (fetch && tid < kWave) {
+            const int b = items.next(lane, 0);
+            if (tid == 0) s_item = b;
+        }
         __syncthreads();
-        const int item = s_item;
-        if (item < 0) break;
+        if (fetch) {
+            const int b = s_item;
+            if (b < 0) break;
+            b_next = b * bsz;
+            b_end = min(n_items, b_next + bsz);
+        }
+        const int item = b_next++;
         const int apex = a.items ? a.items[item] : item;
         const uint32_t fa = a.flags[apex];
         if (fa & 2u) {          // buffer point: never an apex (gramsci.F90:476)
@@ -419,8 +429,8 @@ __global__ __launch_bounds__(kWG) void k_triplet3(TripArgs a)
                 }
             } else {
                 const size_t go = (size_t)cur_r * nh + hk;
-                atomicAdd(&a.out_cnt[go], (unsigned long long)mult);
-                if constexpr (W) glb_add128(&a.out_w[2 * go], qs, 0ull);
+                atomicAdd(&out_cnt[go], (unsigned long long)mult);
+                if constexpr (W) glb_add128(&out_w[2 * go], qs, 0ull);
             }
         };
         // the FP32 path calls update where the bin is known (the certain interval, or after the FP64
@@ -554,20 +564,49 @@ __global__ __launch_bounds__(kWG) void k_triplet3(TripArgs a)
     }
     __syncthreads();
     if (lh && cur_r >= 0) drain(cur_r);
+    // statistics: summed over the work-group, then added to its copy of the outputs
+    __shared__ unsigned long long s_stat[5];
+    if (tid < 5) s_stat[tid] = 0;
+    __syncthreads();
+    const unsigned long long st[5] = {cand, rechk, over, units, evals};
+    for (int q = 0; q < 5; ++q) {
+        unsigned long long v = st[q];
+        for (int off = 32; off > 0; off >>= 1) v += __shfl_down(v, off, 64);
+        if (lane == 0 && v) atomicAdd(&s_stat[q], v);
+    }
+    __syncthreads();
+    if (tid < 5 && s_stat[tid]) atomicAdd(&a.out_stats[copy + tid], s_stat[tid]);
+}
+
+// Sums the outputs' copies.  The work-groups add to them with device-wide atomics, which run one after another
+// where they meet (about 40 ns each); one wave per entry, one lane per copy.
+__global__ __launch_bounds__(256) void k_sum_copies(const unsigned long long* __restrict__ in, int copies, int64_t stride,
+                                                    int64_t nplain, int64_t nwide, int64_t ntail,
+                                                    unsigned long long* __restrict__ out)
+{
+    const int lane = threadIdx.x & (kWave - 1);
+    const int64_t e = blockIdx.x * (int64_t)(blockDim.x / kWave) + threadIdx.x / kWave;
+    if (e >= nplain + nwide + ntail) return;
+    const bool wide = e >= nplain && e < nplain + nwide;
+    const int64_t at = e < nplain ? e : (wide ? nplain + 2 * (e - nplain) : e + nwide);
+    const unsigned long long* c = in + (size_t)lane * (size_t)stride + at;
+    unsigned long long lo = lane < copies ? c[0] : 0, hi = wide && lane < copies ? c[1] : 0;
     for (int off = 32; off > 0; off >>= 1) {
-        units += __shfl_down(units, off, 64);
-        evals += __shfl_down(evals, off, 64);
-        rechk += __shfl_down(rechk, off, 64);
-        over += __shfl_down(over, off, 64);
-        cand += __shfl_down(cand, off, 64);
+        const unsigned long long l = __shfl_down(lo, off, 64), h = __shfl_down(hi, off, 64);
+        add128(lo, hi, l, h);
     }
     if (lane == 0) {
-        if (cand) atomicAdd(&a.out_stats[0], cand);
-        if (rechk) atomicAdd(&a.out_stats[1], rechk);
-        if (over) atomicAdd(&a.out_stats[2], over);
-        if (units) atomicAdd(&a.out_stats[3], units);
-        if (evals) atomicAdd(&a.out_stats[4], evals);
+        out[at] = lo;
+        if (wide) out[at + 1] = hi;
     }
+}
+
+hipError_t launch_sum_copies(const unsigned long long* in, int copies, int64_t stride, int64_t nplain, int64_t nwide,
+                             int64_t ntail, unsigned long long* out, hipStream_t st)
+{
+    const int64_t nblk = (nplain + nwide + ntail + kWG / kWave - 1) / (kWG / kWave);
+    hipLaunchKernelGGL(k_sum_copies, dim3((unsigned)nblk), dim3(kWG), 0, st, in, copies, stride, nplain, nwide, ntail, out);
+    return hipGetLastError();
 }
 
 using T3Kernel = void (*)(TripArgs);
