@@ -202,8 +202,11 @@ struct QuadArgs {
     const Row* rows;            // full stencil
     const BinDesc* bins;
     const uint16_t* cfg_tab;    // [nb]^4 -> 1-based perimeter configuration, 0 = not sorted
-    int32_t* queue;
+    int32_t* queue;             // work counters (ItemQueue)
     int32_t* err;
+    // outputs, `copies` of them copy_stride words apart; work-group b adds to copy b mod copies
+    int64_t copy_stride;
+    int32_t copies;             // power of two <= 64
     unsigned long long* out_cnt;    // [ncell][16]
     double* out_w;              // weighted: [ncell][16] quad products, [6][ncell][4] disc pair (tetra: triple) products
     unsigned long long* out_stats;
@@ -219,7 +222,9 @@ struct QuadArgs {
     int32_t* ovf;
     int32_t* ovf_n;
     const int32_t* items;
+    const int32_t* n_items_dev; // if set, the number of work items is read here
     int32_t batch;              // apexes taken per queue fetch (0: 1)
+    int32_t lds_w;              // weighted sums in LDS (else global atomics; device-memory lists: always those)
     // as for the triplet kernel: with ovf_kmax set, the largest neighbour count of a queued apex is
     // kept there; with glist set, each work-group keeps its apex's neighbour list (kmax entries, a
     // power of two) at glist + blockIdx.x * glist_stride bytes of device memory, with no link matrix
@@ -231,9 +236,11 @@ struct QuadArgs {
 // bytes per neighbour of a device-memory neighbour list (glist) of the quad kernel: x, y, z, w,
 // key, permutation, packed bin, and the sort's staging copy of x, y, z, w and the packed bin
 constexpr size_t kQuadGlistEntryBytes = 4 * 8 + 3 * 4 + 4 * 8 + 4;
-size_t quad4_lds_bytes(int nb, int ncell, int kmax, bool lds_hist, bool tetra, int nrows, bool glist = false);
-hipError_t launch_quad4(const QuadArgs& a, int nb, bool weighted, int nblocks, hipStream_t st);
-int quad4_occupancy(const QuadArgs& a, int nb, bool weighted);
+// kmax: 64, 128 or 256; wave: one wave per apex (kmax 64)
+size_t quad4_lds_bytes(const QuadArgs& a, int nb, bool weighted, bool wave);
+hipError_t launch_quad4(const QuadArgs& a, int nb, bool weighted, bool wave, int nblocks, hipStream_t st);
+int quad4_occupancy(const QuadArgs& a, int nb, bool weighted, bool wave);
+hipError_t launch_sum_copies_f64(const double* in, int copies, int64_t stride, int64_t n, double* out, hipStream_t st);
 
 // Arguments of the persistent 2PCF adjoint kernel (adjoint.hip).
 struct AdjArgs {

@@ -531,49 +531,60 @@ static int count4(gs_ctx* c, const gs_params* p, bool tetra, uint64_t* cnt, doub
     if ((rc = ctx_thresholds(c, *p, t64)) || (rc = fill_bins(*p, t64, 1.5 * p->rmax, ctx_xmax(c), v.wmax_d, v.wmax_r, B))) return rc;
     std::vector<uint16_t> tab = tetra ? std::vector<uint16_t>() : table4(nb);
 
-    // LDS plan of the second pass: the longest list (a power of two, 64..256, with its K x K link
-    // matrix) that fits gfx950's 160 KiB of LDS per work-group beside the tables and, where it
-    // fits in 16 KiB, the count histogram.  Apexes with more neighbours go to a last pass with
-    // device-memory lists, so no neighbour count is refused.
-    const size_t budget = 160 * 1024;
-    int kmax = 256;
-    static_assert(kWG >= 256, "the LDS-list sort of k_quad4 takes one thread per list entry");
-    bool lds_hist = (size_t)ncell * 64 <= 16 * 1024;
-    while (kmax > 64 && quad4_lds_bytes(nb, ncell, kmax, lds_hist, tetra, (int)rows.size()) > budget) kmax /= 2;
-    if (quad4_lds_bytes(nb, ncell, kmax, lds_hist, tetra, (int)rows.size()) > budget) {
-        lds_hist = false;
-        kmax = 256;
-        while (kmax > 64 && quad4_lds_bytes(nb, ncell, kmax, lds_hist, tetra, (int)rows.size()) > budget) kmax /= 2;
+    // LDS plan of the last LDS pass: the longest list (64, 128 or 256, with its K x K matrix of links and its masks)
+    // that fits gfx950's 160 KiB of LDS per work-group beside the tables and, where it fits in 16 KiB, the count
+    // histogram.  Apexes with more neighbours go to a last pass with device-memory lists, so no neighbour count is
+    // refused.
+    const size_t budget = 160 * 1024 - 256;     // less the kernel's static part
+    QuadArgs a{};
+    a.tetra = tetra ? 1 : 0;
+    a.ncell = ncell;
+    a.nrows = (int)rows.size();
+    a.lds_hist = (size_t)ncell * 64 <= 16 * 1024;
+    auto fits = [&]() { return quad4_lds_bytes(a, nb, weighted, false) <= budget; };
+    for (int pass = 0; pass < 2; ++pass) {
+        a.kmax = 256;
+        while (a.kmax > 64 && !fits()) a.kmax /= 2;
+        if (fits()) break;
+        a.lds_hist = 0;
     }
-    if (quad4_lds_bytes(nb, ncell, kmax, lds_hist, tetra, (int)rows.size()) > budget)
-        return fail(GS_ELIMIT, "4PCF tables do not fit in LDS");
+    if (!fits()) return fail(GS_ELIMIT, "4PCF tables do not fit in LDS");
     {
         const char* ev = getenv("GS_T4_KMAX_LDS");  // test override: a shorter second-pass list
         if (ev && *ev)
-            while (kmax > 64 && kmax > atoi(ev)) kmax /= 2;
+            while (a.kmax > 64 && a.kmax > atoi(ev)) a.kmax /= 2;
     }
+    const int kmax = a.kmax;
 
+    // As for the 3PCF: parameters in one copy, one region to clear (the work counters of the passes, the error flag
+    // and counts of queued apexes, the outputs' copies: up to 16 MiB of them, since weighted sums that do not fit
+    // LDS go there pair by pair).
     GsExtra& X = *v.extra;
-    const size_t tab_off = ((sizeof(BinDesc) + 15) / 16) * 16;
-    const size_t rows_off = tab_off + ((tab.size() * 2 + 15) / 16) * 16;
+    HostBuf& H = ctx_host(c);
+    const size_t tab_off = (sizeof(BinDesc) + 15) / 16 * 16;
+    const size_t rows_off = tab_off + (tab.size() * 2 + 15) / 16 * 16;
+    const size_t blob = rows_off + rows.size() * sizeof(Row), res_off = (blob + 255) / 256 * 256;
     const size_t ncnt = (size_t)ncell * 16;
-    const size_t nout = ncnt + 8;
     const size_t nw = weighted ? (size_t)ncell * 16 + (size_t)6 * ncell * 4 : 0;
-    if ((rc = X.params.reserve(rows_off + rows.size() * sizeof(Row) + 16)) || (rc = X.out.reserve(nout)) ||
-        (rc = X.queue.reserve(16)) || (rc = X.dbl.reserve(std::max<size_t>(nw, 1))))
+    const int64_t words = (int64_t)(ncnt + 8 + nw);
+    int copies = 1;
+    while (copies < 64 && 2 * copies * words <= (int64_t)2 << 20) copies *= 2;
+    constexpr int kPasses = 3;
+    constexpr size_t kQueueInts = 64 * kQueuePad, kHeadInts = kPasses * kQueueInts + 64;
+    const size_t clear = kHeadInts * 4 + (size_t)copies * words * 8;
+    if ((rc = X.params.reserve(blob)) || (rc = X.big_zero.reserve(clear)) || (rc = X.out.reserve(words)) ||
+        (rc = H.reserve(res_off + 64)))
         return rc;
-    hipError_t e = hipMemcpyAsync(X.params.ptr, &B, sizeof(B), hipMemcpyHostToDevice, v.stream);
-    if (e == hipSuccess && !tab.empty())
-        e = hipMemcpyAsync(X.params.ptr + tab_off, tab.data(), tab.size() * 2, hipMemcpyHostToDevice, v.stream);
-    if (e == hipSuccess && !rows.empty())
-        e = hipMemcpyAsync(X.params.ptr + rows_off, rows.data(), rows.size() * sizeof(Row), hipMemcpyHostToDevice,
-                           v.stream);
-    if (e == hipSuccess) e = hipMemsetAsync(X.out.ptr, 0, nout * sizeof(unsigned long long), v.stream);
-    if (e == hipSuccess && nw) e = hipMemsetAsync(X.dbl.ptr, 0, nw * sizeof(double), v.stream);
-    if (e == hipSuccess) e = hipMemsetAsync(X.queue.ptr, 0, 16 * sizeof(int32_t), v.stream);
+    *(BinDesc*)H.ptr = B;
+    std::copy(tab.begin(), tab.end(), (uint16_t*)(H.ptr + tab_off));
+    std::copy(rows.begin(), rows.end(), (Row*)(H.ptr + rows_off));
+    hipError_t e = hipMemcpyAsync(X.params.ptr, H.ptr, blob, hipMemcpyHostToDevice, v.stream);
+    if (e == hipSuccess) e = launch_fill_u32(X.big_zero.ptr, (int64_t)clear / 4, 0u, v.stream);
     if (e != hipSuccess) return hip_fail(e, "4PCF parameter upload");
+    int32_t* const head = (int32_t*)X.big_zero.ptr;
+    int32_t* const d_cnt = head + kPasses * kQueueInts;     // per pass 4: apexes queued for the next, their largest count
+    unsigned long long* const out = (unsigned long long*)(head + kHeadInts);
 
-    QuadArgs a{};
     a.pw = v.pw;
     a.flags = v.flags;
     a.orig = v.orig;
@@ -581,34 +592,29 @@ static int count4(gs_ctx* c, const gs_params* p, bool tetra, uint64_t* cnt, doub
     a.rows = (const Row*)(X.params.ptr + rows_off);
     a.bins = (const BinDesc*)X.params.ptr;
     a.cfg_tab = tab.empty() ? nullptr : (const uint16_t*)(X.params.ptr + tab_off);
-    a.queue = X.queue.ptr;
-    a.err = X.queue.ptr + 8;
-    a.out_cnt = X.out.ptr;
-    a.out_w = X.dbl.ptr;
-    a.out_stats = X.out.ptr + ncnt;
+    a.err = d_cnt + 4 * kPasses;
+    a.out_cnt = out;
+    a.out_stats = out + ncnt;
+    a.out_w = (double*)(out + ncnt + 8);
+    a.copies = copies;
+    a.copy_stride = words;
     a.g = v.g;
     a.g.m = mst;
-    a.nrows = (int)rows.size();
     a.n_items = (int)(v.n_data + v.n_rand);
-    a.ncell = ncell;
-    a.kmax = kmax;
-    a.lds_hist = lds_hist ? 1 : 0;
-    a.tetra = tetra ? 1 : 0;
-    // Two passes, as for the 3PCF: the first pass's neighbour list (and its K x K link matrix)
-    // is sized for the 99.5th percentile of ~8192 sampled neighbour counts (+5%, a power of two
-    // for the bitonic sort, at least 64 for the sort's staging area); apexes with more
-    // neighbours are queued for a second pass with the full list.
+    // Passes, each over the apexes whose neighbours outnumbered the list of the one before: one wave per apex (64
+    // neighbours), work-groups with a list for the 99.5th percentile of ~8192 sampled neighbour counts (+5%, a power
+    // of two), work-groups with the longest LDS list, and last work-groups with device-memory lists.  The waves take
+    // unit weights where at least a quarter of the sample fits them: kernels of 0.97 against 1.84 ms (50k + 100k
+    // points), 0.42 against 0.63 (27k + 54k, 4 bins); with weights the FP64 atomics of the quads
+    // bound both, and work-groups are as fast or faster (0.69 against 0.71, 0.39 against 0.49 ms).
     const int n = a.n_items;
     int kmax1 = kmax;
+    double short_lists = 0.0;
     const int nsample = std::min(n, 8192);
     const int stride = nsample > 0 ? n / nsample : 1;
-    // i32 as for the 3PCF: [0] second-pass count, [1, n] its apexes, [n+1] last-pass count, [n+2]
-    // its largest neighbour count, [n+3, 2n+2] its apexes, then the sampled neighbour counts
-    if ((rc = X.i32.reserve(2 * (size_t)n + 3 + nsample))) return rc;
-    int32_t* d_list2 = X.i32.ptr + 1;
-    int32_t* d_cnt3 = X.i32.ptr + n + 1;
-    int32_t* d_list3 = X.i32.ptr + n + 3;
-    if (nsample > 0 && kmax > 64) {
+    // i32: the lists of queued apexes, then the sampled neighbour counts
+    if ((rc = X.i32.reserve(kPasses * (size_t)n + nsample))) return rc;
+    if (nsample > 0) {
         TripArgs ts{};
         ts.pw = a.pw;
         ts.flags = a.flags;
@@ -617,16 +623,17 @@ static int count4(gs_ctx* c, const gs_params* p, bool tetra, uint64_t* cnt, doub
         ts.bins = a.bins;
         ts.g = a.g;
         ts.nrows = a.nrows;
-        int32_t* d_cnt = X.i32.ptr + 2 * n + 3;
+        int32_t* d_kc = X.i32.ptr + kPasses * (size_t)n;
         std::vector<int32_t> kc(nsample);
-        e = launch_nbr_count(ts, stride, nsample, 0, d_cnt, v.stream);
-        if (e == hipSuccess) e = hipMemcpyAsync(kc.data(), d_cnt, nsample * sizeof(int32_t), hipMemcpyDeviceToHost, v.stream);
+        e = launch_nbr_count(ts, stride, nsample, 0, d_kc, v.stream);
+        if (e == hipSuccess) e = hipMemcpyAsync(kc.data(), d_kc, nsample * sizeof(int32_t), hipMemcpyDeviceToHost, v.stream);
         if (e == hipSuccess) e = hipStreamSynchronize(v.stream);
         if (e != hipSuccess) return hip_fail(e, "4PCF neighbour sample");
         std::vector<int32_t> ks;
         for (int32_t k : kc)
             if (k >= 0) ks.push_back(k);
         if (!ks.empty()) {
+            short_lists = (double)std::count_if(ks.begin(), ks.end(), [](int32_t k) { return k <= 64; }) / ks.size();
             const size_t q = std::min(ks.size() - 1, (size_t)std::ceil(0.995 * (ks.size() - 1)));
             std::nth_element(ks.begin(), ks.begin() + q, ks.end());
             const double want = 1.05 * ks[q];
@@ -641,85 +648,85 @@ static int count4(gs_ctx* c, const gs_params* p, bool tetra, uint64_t* cnt, doub
             while (kmax1 < kmax && kmax1 < atoi(ev)) kmax1 *= 2;
         }
     }
-    const bool two_pass = kmax1 < kmax;
-    (void)hipEventRecord(v.ev[2], v.stream);
-    if (n > 0) {
-        e = hipMemsetAsync(X.i32.ptr, 0, sizeof(int32_t), v.stream);
-        if (e == hipSuccess) e = hipMemsetAsync(d_cnt3, 0, 2 * sizeof(int32_t), v.stream);
-        if (e != hipSuccess) return hip_fail(e, "4PCF overflow counters");
-        QuadArgs a1 = a;
-        a1.ovf_kmax = d_cnt3 + 1;
-        if (two_pass) {
-            a1.kmax = kmax1;
-            a1.ovf_n = X.i32.ptr;
-            a1.ovf = d_list2;
-        } else {
-            a1.ovf_n = d_cnt3;
-            a1.ovf = d_list3;
-        }
-        const int occ = quad4_occupancy(a1, nb, weighted);
-        const int nblk1 = std::max(1, std::min(v.n_cu * occ, n));
-        a1.batch = triplet_batch(n, nblk1);
-        e = launch_quad4(a1, nb, weighted, nblk1, v.stream);
-        if (e != hipSuccess) return hip_fail(e, "4PCF kernel launch");
-        if (two_pass) {
-            int32_t nov = 0;
-            e = hipMemcpyAsync(&nov, X.i32.ptr, sizeof(int32_t), hipMemcpyDeviceToHost, v.stream);
-            if (e == hipSuccess) e = hipStreamSynchronize(v.stream);
-            if (e != hipSuccess) return hip_fail(e, "4PCF first pass");
-            if (nov > 0) {
-                QuadArgs a2 = a;
-                a2.items = d_list2;
-                a2.n_items = nov;
-                a2.batch = 1;
-                a2.ovf = d_list3;
-                a2.ovf_n = d_cnt3;
-                a2.ovf_kmax = d_cnt3 + 1;
-                e = hipMemsetAsync(X.queue.ptr, 0, 8 * sizeof(int32_t), v.stream);   // work counters only
-                const int occ2 = quad4_occupancy(a2, nb, weighted);
-                if (e == hipSuccess)
-                    e = launch_quad4(a2, nb, weighted, std::max(1, std::min(v.n_cu * occ2, nov)), v.stream);
-                if (e != hipSuccess) return hip_fail(e, "4PCF second pass");
-            }
-        }
-        // last pass: the apexes whose neighbours outnumber the second pass's list, with their lists
-        // in device memory (one per work-group; no link matrix)
-        int32_t h3[2] = {0, 0};
-        e = hipMemcpyAsync(h3, d_cnt3, sizeof(h3), hipMemcpyDeviceToHost, v.stream);
-        if (e == hipSuccess) e = hipStreamSynchronize(v.stream);
-        if (e != hipSuccess) return hip_fail(e, "4PCF queued apex count");
-        if (h3[0] > 0) {
-            QuadArgs a3 = a;
-            a3.items = d_list3;
-            a3.n_items = h3[0];
-            a3.batch = 1;
-            a3.kmax = 64;
-            while (a3.kmax < h3[1]) a3.kmax *= 2;           // a power of two for the bitonic sort
-            const size_t gstride = (a3.kmax * kQuadGlistEntryBytes + 255) / 256 * 256;
-            a3.glist = (void*)d_list3;      // selects the device-memory variant for the occupancy query
-            const int occ3 = quad4_occupancy(a3, nb, weighted);
-            const size_t gbudget = (size_t)1 << 30;
-            const int nblk3 = (int)std::max<size_t>(1, std::min<size_t>({(size_t)h3[0], (size_t)v.n_cu * occ3,
-                                                                      gbudget / gstride}));
-            if ((rc = X.big.reserve((size_t)nblk3 * gstride))) return rc;
-            a3.glist = X.big.ptr;
-            a3.glist_stride = (int64_t)gstride;
-            e = hipMemsetAsync(X.queue.ptr, 0, 8 * sizeof(int32_t), v.stream);
-            if (e == hipSuccess) e = launch_quad4(a3, nb, weighted, nblk3, v.stream);
-            if (e != hipSuccess) return hip_fail(e, "4PCF device-memory pass");
-        }
+    // weighted sums in LDS where that leaves room for two work-groups
+    auto with_sums = [&](int km, bool wv) {
+        QuadArgs t = a;
+        t.kmax = km;
+        t.lds_w = weighted ? 1 : 0;
+        if (quad4_lds_bytes(t, nb, weighted, wv) > 80 * 1024) t.lds_w = 0;
+        return t;
+    };
+    bool wave = !weighted && short_lists >= 0.25;
+    {
+        const char* ev = getenv("GS_T4_WAVE");      // tuning override (unset or empty: automatic)
+        if (ev && *ev) wave = !weighted && *ev != '0';
     }
-    (void)hipEventRecord(v.ev[3], v.stream);
-    std::vector<unsigned long long> h_out(nout);
-    std::vector<double> h_w(nw);
-    e = hipMemcpyAsync(h_out.data(), X.out.ptr, nout * sizeof(unsigned long long), hipMemcpyDeviceToHost, v.stream);
-    if (e == hipSuccess && nw)
-        e = hipMemcpyAsync(h_w.data(), X.dbl.ptr, nw * sizeof(double), hipMemcpyDeviceToHost, v.stream);
-    int32_t err = 0;
-    if (e == hipSuccess) e = hipMemcpyAsync(&err, X.queue.ptr + 8, sizeof(int32_t), hipMemcpyDeviceToHost, v.stream);
-    if (e == hipSuccess) e = hipStreamSynchronize(v.stream);
-    if (e != hipSuccess) return hip_fail(e, "4PCF kernel");
-    if (err) return fail(GS_EHIP, "4PCF: an apex's neighbour list overflowed with no later pass (internal error)");
+    wave = wave && quad4_lds_bytes(with_sums(64, true), nb, weighted, true) <= budget;
+    (void)hipEventRecord(v.ev[2], v.stream);
+    struct Pass { bool wave; int kmax; };
+    std::vector<Pass> passes;
+    if (wave) passes.push_back({true, 64});
+    if (kmax1 < kmax && !(wave && kmax1 == 64)) passes.push_back({false, kmax1});
+    passes.push_back({false, kmax});
+    const int np = (int)passes.size();
+    for (int k = 0; k < np && n > 0; ++k) {
+        const bool wv = passes[k].wave;
+        QuadArgs t = with_sums(passes[k].kmax, wv);
+        t.queue = head + k * kQueueInts;
+        t.ovf = X.i32.ptr + (size_t)k * n;
+        t.ovf_n = d_cnt + 4 * k;
+        t.ovf_kmax = t.ovf_n + 1;
+        if (k > 0) {
+            // the number of apexes is read on the device
+            t.items = X.i32.ptr + (size_t)(k - 1) * n;
+            t.n_items_dev = d_cnt + 4 * (k - 1);
+        }
+        const int teams = wv ? kWG / kWave : 1;
+        const int occ = quad4_occupancy(t, nb, weighted, wv);
+        const int nblk = std::max(1, std::min(v.n_cu * occ, (n + teams - 1) / teams));
+        t.batch = k > 0 ? 1 : std::max(triplet_batch(n, nblk), wv ? 4 * teams : 1);
+        e = launch_quad4(t, nb, weighted, wv, nblk, v.stream);
+        if (e != hipSuccess) return hip_fail(e, "4PCF kernel launch");
+    }
+    // the copies' sum; once more after a last pass, over the apexes whose neighbours outnumber every LDS list, with
+    // their lists in device memory (one per work-group; no link matrix)
+    int32_t* const h_cnt = (int32_t*)(H.ptr + res_off);
+    int32_t* const last = d_cnt + 4 * (np - 1);
+    std::vector<unsigned long long> h_out(words);
+    for (int pass = 0;; ++pass) {
+        (void)hipEventRecord(v.ev[3], v.stream);
+        e = launch_sum_copies(out, copies, words, (int64_t)ncnt, 0, 8, X.out.ptr, v.stream);
+        if (e == hipSuccess)
+            e = launch_sum_copies_f64(a.out_w, copies, words, (int64_t)nw, (double*)(X.out.ptr + ncnt + 8), v.stream);
+        if (e == hipSuccess)
+            e = hipMemcpyAsync(h_out.data(), X.out.ptr, (size_t)words * 8, hipMemcpyDeviceToHost, v.stream);
+        if (e == hipSuccess) e = hipMemcpyAsync(h_cnt, last, 2 * sizeof(int32_t), hipMemcpyDeviceToHost, v.stream);
+        if (e == hipSuccess) e = hipMemcpyAsync(h_cnt + 2, a.err, sizeof(int32_t), hipMemcpyDeviceToHost, v.stream);
+        if (e == hipSuccess) e = hipStreamSynchronize(v.stream);
+        if (e != hipSuccess) return hip_fail(e, "4PCF kernel");
+        if (pass > 0 || h_cnt[0] <= 0) break;
+        QuadArgs a3 = a;
+        a3.items = X.i32.ptr + (size_t)(np - 1) * n;
+        a3.n_items = h_cnt[0];
+        a3.batch = 1;
+        a3.kmax = 64;
+        while (a3.kmax < h_cnt[1]) a3.kmax *= 2;        // a power of two for the bitonic sort
+        const size_t gstride = (a3.kmax * kQuadGlistEntryBytes + 255) / 256 * 256;
+        a3.glist = (void*)a3.items;             // selects the device-memory variant for the occupancy query
+        const int occ3 = quad4_occupancy(a3, nb, weighted, false);
+        const size_t gbudget = (size_t)1 << 30;
+        const int nblk3 = (int)std::max<size_t>(1, std::min<size_t>({(size_t)h_cnt[0], (size_t)v.n_cu * occ3,
+                                                                  gbudget / gstride}));
+        if ((rc = X.big.reserve((size_t)nblk3 * gstride))) return rc;
+        a3.glist = X.big.ptr;
+        a3.glist_stride = (int64_t)gstride;
+        a3.queue = head;
+        e = launch_fill_u32(head, kQueueInts, 0u, v.stream);
+        if (e == hipSuccess) e = launch_quad4(a3, nb, weighted, false, nblk3, v.stream);
+        if (e != hipSuccess) return hip_fail(e, "4PCF device-memory pass");
+    }
+    if (h_cnt[2]) return fail(GS_EHIP, "4PCF: an apex's neighbour list overflowed with no later pass (internal error)");
+    const double* const h_w = (const double*)(h_out.data() + ncnt + 8);
 
     if (cnt) memcpy(cnt, h_out.data(), ncnt * sizeof(uint64_t));
     // normalised weight of one point: +w/Wd (data) or -w/Wr (random) (gramsci.F90:1390-1391)

@@ -57,14 +57,6 @@ __host__ __device__ inline size_t team_bytes(int kmax, int nrows)
     return (size_t)kListWords * 4 * (kmax + 16) + ((size_t)nrows * 12 + 15) / 16 * 16;
 }
 
-// v, the same in all lanes, in scalar registers
-__device__ __forceinline__ int scalar(int v) { return __builtin_amdgcn_readfirstlane(v); }
-__device__ __forceinline__ double scalar(double v)
-{
-    const long long b = __double_as_longlong(v);
-    return __longlong_as_double((long long)(unsigned)scalar((int)b) | ((long long)scalar((int)(b >> 32)) << 32));
-}
-
 __device__ __forceinline__ void lds_count(uint32_t at)
 {
     __hip_atomic_fetch_add((lds_ptr<uint32_t>)at, 1u, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_WORKGROUP);
