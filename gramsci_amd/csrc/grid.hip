@@ -16,19 +16,25 @@ using namespace dev;
 // the largest data and random weight and the first invalid weight.  The last block to finish reduces the
 // blocks' partials, so that one launch and one wait give the host everything (with k_wsum, where there
 // are weights); before, the copies, the check, the sums and the bounding box were seven launches and three
-// waits.  Bound by memory: each coordinate and weight is read and written once.
+// waits.  Bound by memory where it is large (each coordinate and weight is read and written once: 600k points 32 us),
+// by the chain load, reduction, release, reduction where it is small (60k points 11 us; with one load in flight, a
+// reduction per quantity and a release by every wave 19).
 // The thread count is a multiple of 3, so that every thread's coordinates share one axis.
 constexpr int kIngestThreads = 192;
 
-__device__ __forceinline__ double block_reduce_max(double v, double* red)
+// the maxima of v over the block, in every thread of it; all nine at once, so that their shuffles overlap
+__device__ __forceinline__ void block_reduce_max(double (&v)[9], double (*red)[9])
 {
-    for (int off = 32; off > 0; off >>= 1) v = fmax(v, __shfl_down(v, off, 64));
+    for (int off = 32; off > 0; off >>= 1)
+        for (int q = 0; q < 9; ++q) v[q] = fmax(v[q], __shfl_down(v[q], off, 64));
     __syncthreads();
-    if ((threadIdx.x & 63) == 0) red[threadIdx.x >> 6] = v;
+    if ((threadIdx.x & 63) == 0)
+        for (int q = 0; q < 9; ++q) red[threadIdx.x >> 6][q] = v[q];
     __syncthreads();
-    double r = red[0];
-    for (int k = 1; k < (int)(blockDim.x >> 6); ++k) r = fmax(r, red[k]);
-    return r;
+    for (int q = 0; q < 9; ++q) {
+        v[q] = red[0][q];
+        for (int k = 1; k < kIngestThreads / 64; ++k) v[q] = fmax(v[q], red[k][q]);
+    }
 }
 
 __global__ __launch_bounds__(kIngestThreads) void k_ingest(const double* __restrict__ xyz, const double* __restrict__ w,
@@ -36,56 +42,63 @@ __global__ __launch_bounds__(kIngestThreads) void k_ingest(const double* __restr
                                                            double* xyz_out, double* w_out, int32_t* buf_out,
                                                            IngestScratch* sc, CatalogueStats* out)
 {
-    __shared__ double red[kIngestThreads / 64];
+    __shared__ double red[kIngestThreads / 64][9];
     const int64_t t = blockIdx.x * (int64_t)blockDim.x + threadIdx.x, step = gridDim.x * (int64_t)blockDim.x;
     const int axis = (int)(t % 3);
     double mn = 1e308, mx = -1e308;
-    for (int64_t i = t; i < 3 * n; i += step) {
-        const double v = xyz[i];
-        if (xyz_out != xyz) xyz_out[i] = v;
-        mn = fmin(mn, v);
-        mx = fmax(mx, v);
+    // four loads in flight: a store between them could change what they read, for all the compiler knows
+    for (int64_t i = t; i < 3 * n; i += 4 * step) {
+        double v[4];
+        for (int k = 0; k < 4; ++k) v[k] = i + k * step < 3 * n ? xyz[i + k * step] : 0.0;
+        for (int k = 0; k < 4; ++k)
+            if (i + k * step < 3 * n) {
+                if (xyz_out != xyz) xyz_out[i + k * step] = v[k];
+                mn = fmin(mn, v[k]);
+                mx = fmax(mx, v[k]);
+            }
     }
     double wm[2] = {0.0, 0.0};
     unsigned long long bad = ~0ull;
     if (w)
-        for (int64_t i = t; i < n; i += step) {
-            const double v = w[i];
-            if (w_out != w) w_out[i] = v;
-            if (!(v >= 0.0) || !isfinite(v)) bad = bad < (unsigned long long)i ? bad : (unsigned long long)i;
-            else if (i < n_data) wm[0] = fmax(wm[0], v);
-            else wm[1] = fmax(wm[1], v);
+        for (int64_t i = t; i < n; i += 4 * step) {
+            double v[4];
+            for (int k = 0; k < 4; ++k) v[k] = i + k * step < n ? w[i + k * step] : 0.0;
+            for (int k = 0; k < 4; ++k) {
+                const int64_t at = i + k * step;
+                if (at >= n) break;
+                if (w_out != w) w_out[at] = v[k];
+                if (!(v[k] >= 0.0) || !isfinite(v[k])) bad = bad < (unsigned long long)at ? bad : (unsigned long long)at;
+                else if (at < n_data) wm[0] = fmax(wm[0], v[k]);
+                else wm[1] = fmax(wm[1], v[k]);
+            }
         }
     if (buf && buf_out != buf)
         for (int64_t i = t; i < n; i += step) buf_out[i] = buf[i];
 
-    IngestScratch& P = sc[blockIdx.x];
+    // lowest values negated; the index of a bad weight as a double: exact below 2^53
+    double v[9];
     for (int k = 0; k < 3; ++k) {
-        const double hi = block_reduce_max(axis == k ? mx : -1e308, red);
-        const double lo = -block_reduce_max(axis == k ? -mn : -1e308, red);
-        if (threadIdx.x == 0) { P.v[k] = lo; P.v[3 + k] = hi; }
+        v[k] = axis == k ? -mn : -1e308;
+        v[3 + k] = axis == k ? mx : -1e308;
     }
-    for (int q = 0; q < 2; ++q) {
-        const double m = block_reduce_max(wm[q], red);
-        if (threadIdx.x == 0) P.v[6 + q] = m;
-    }
-    // the index as a double: exact below 2^53
-    const double fb = -block_reduce_max(bad == ~0ull ? -1e308 : -(double)bad, red);
-    if (threadIdx.x == 0) P.v[8] = fb;
-
+    v[6] = wm[0];
+    v[7] = wm[1];
+    v[8] = bad == ~0ull ? -1e308 : -(double)bad;
+    block_reduce_max(v, red);
+    if (threadIdx.x == 0)
+        for (int q = 0; q < 9; ++q) sc[blockIdx.x].v[q] = v[q];
     if (!last_block(&out->ticket)) return;
-    for (int q = 0; q < 9; ++q) {
-        const bool lowest = q < 3 || q == 8;
-        double v = -1e308;
-        for (int b = threadIdx.x; b < (int)gridDim.x; b += blockDim.x) {
-            const double x = load_agent(&sc[b].v[q]);
-            v = fmax(v, lowest ? -x : x);
-        }
-        v = block_reduce_max(v, red);
-        if (threadIdx.x == 0) out->v[q] = lowest ? -v : v;
+    for (int q = 0; q < 9; ++q) v[q] = -1e308;
+    for (int b = threadIdx.x; b < (int)gridDim.x; b += blockDim.x) {
+        double x[9];
+        for (int q = 0; q < 9; ++q) x[q] = load_agent(&sc[b].v[q]);
+        for (int q = 0; q < 9; ++q) v[q] = fmax(v[q], x[q]);
     }
+    block_reduce_max(v, red);
+    if (threadIdx.x == 0)
+        for (int q = 0; q < 9; ++q) out->v[q] = q < 3 || q == 8 ? -v[q] : v[q];
     // without weights there is no k_wsum to hand the statistics to the host
-    if (!w && threadIdx.x < 9 && threadIdx.x == 0)
+    if (!w && threadIdx.x == 0)
         for (int q = 0; q < 9; ++q) out->host->v[q] = out->v[q];
 }
 
@@ -136,7 +149,7 @@ hipError_t launch_ingest(const double* xyz, const double* w, const int32_t* buf,
                          double* xyz_out, double* w_out, int32_t* buf_out, IngestScratch* scratch, CatalogueStats* stats,
                          hipStream_t st)
 {
-    const int nblk = (int)std::min<int64_t>(std::max<int64_t>((3 * n + 4 * kIngestThreads - 1) / (4 * kIngestThreads), 1),
+    const int nblk = (int)std::min<int64_t>(std::max<int64_t>((3 * n + 12 * kIngestThreads - 1) / (12 * kIngestThreads), 1),
                                             kIngestBlocks);
     hipLaunchKernelGGL(k_ingest, dim3(nblk), dim3(kIngestThreads), 0, st, xyz, w, buf, n, n_data, xyz_out, w_out, buf_out,
                        scratch, stats);
@@ -234,7 +247,8 @@ int64_t scan_scratch_size(int64_t n)
 // scanned by the last block; the scatter, which adds the offsets where it needs them and writes the final
 // cell starts beside.  The order inside a count follows the atomics' order; every count and fixed-point sum
 // computed from the sorted arrays is independent of it.  One grid, or one per region of a batch.
-constexpr int kCellScan = 2048;     // counts per block of the scan
+// Scan: 1,000,001 counts 13 us (with scalar loads, blocks of 2048 and a release by every wave 70).
+constexpr int kCellScan = 4096;     // counts per block of the scan, 8 per thread
 
 __device__ __forceinline__ int cell_coord(double v, double lo, double inv_h, int dim)
 {
@@ -291,10 +305,11 @@ __global__ __launch_bounds__(256) void k_cell_rank(GridArgs a)
     }
 }
 
-__global__ __launch_bounds__(256) void k_cell_scan(int32_t* __restrict__ v, int64_t n, int32_t* __restrict__ boff,
+__global__ __launch_bounds__(kCellScan / 8) void k_cell_scan(int32_t* __restrict__ v, int64_t n, int32_t* __restrict__ boff,
                                                    unsigned* ticket)
 {
-    __shared__ int32_t wsum[4];
+    constexpr int kThreads = kCellScan / 8, kWaves = kThreads / 64;
+    __shared__ int32_t wsum[kWaves];
     const int lane = threadIdx.x & 63, wv = threadIdx.x >> 6;
     // exclusive prefix of x over the block's threads; *total: the block's sum
     auto block_scan = [&](int x, int* total) {
@@ -307,7 +322,7 @@ __global__ __launch_bounds__(256) void k_cell_scan(int32_t* __restrict__ v, int6
         if (lane == 63) wsum[wv] = inc;
         __syncthreads();
         int pre = 0, all = 0;
-        for (int k = 0; k < 4; ++k) {
+        for (int k = 0; k < kWaves; ++k) {
             if (k < wv) pre += wsum[k];
             all += wsum[k];
         }
@@ -315,20 +330,33 @@ __global__ __launch_bounds__(256) void k_cell_scan(int32_t* __restrict__ v, int6
         return pre + inc - x;
     };
     const int64_t base = (int64_t)blockIdx.x * kCellScan + threadIdx.x * 8;
-    int x[8], sum = 0, total;
-    for (int k = 0; k < 8; ++k) {
-        x[k] = base + k < n ? v[base + k] : 0;
-        sum += x[k];
+    int x[8] = {0, 0, 0, 0, 0, 0, 0, 0}, sum = 0, total;
+    const bool whole = base + 8 <= n;       // a thread's 8 counts in two 16-byte accesses
+    if (whole) {
+        *(int4*)x = *(const int4*)(v + base);
+        *(int4*)(x + 4) = *(const int4*)(v + base + 4);
+    } else {
+        for (int k = 0; k < 8; ++k)
+            if (base + k < n) x[k] = v[base + k];
     }
+    for (int k = 0; k < 8; ++k) sum += x[k];
     int run = block_scan(sum, &total);
     for (int k = 0; k < 8; ++k) {
-        if (base + k < n) v[base + k] = run;
-        run += x[k];
+        const int t = x[k];
+        x[k] = run;
+        run += t;
+    }
+    if (whole) {
+        *(int4*)(v + base) = *(const int4*)x;
+        *(int4*)(v + base + 4) = *(const int4*)(x + 4);
+    } else {
+        for (int k = 0; k < 8; ++k)
+            if (base + k < n) v[base + k] = x[k];
     }
     if (threadIdx.x == 0) __hip_atomic_store(&boff[blockIdx.x], total, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT);
     if (!last_block(ticket)) return;
     int carry = 0;
-    for (int b0 = 0; b0 < (int)gridDim.x; b0 += 256) {
+    for (int b0 = 0; b0 < (int)gridDim.x; b0 += kThreads) {
         const int b = b0 + threadIdx.x;
         const int t = b < (int)gridDim.x ? load_agent(&boff[b]) : 0;
         const int e = block_scan(t, &total);
@@ -364,7 +392,7 @@ static int blocks_for(int64_t n)
 hipError_t launch_cell_sort(const GridArgs& a, hipStream_t st)
 {
     hipLaunchKernelGGL(k_cell_rank, dim3(blocks_for(a.n)), dim3(256), 0, st, a);
-    hipLaunchKernelGGL(k_cell_scan, dim3((unsigned)cell_scan_blocks(a.ncell)), dim3(256), 0, st, a.count, 2 * a.ncell + 1,
+    hipLaunchKernelGGL(k_cell_scan, dim3((unsigned)cell_scan_blocks(a.ncell)), dim3(kCellScan / 8), 0, st, a.count, 2 * a.ncell + 1,
                        a.boff, a.ticket);
     hipLaunchKernelGGL(k_cell_scatter, dim3(blocks_for(std::max<int64_t>(a.n, a.ncell + 1))), dim3(256), 0, st, a);
     return hipGetLastError();
