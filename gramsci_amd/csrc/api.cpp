@@ -966,11 +966,17 @@ int pair2_shape(const PairVariant& v, PairShape* out)
         if (ev_wg && ev_wg != w) return;
         if (pair2_lds_bytes(v.nb, v.nm, planes, r, v.weighted, false, w) > kPairLdsMax) return;
         const int waves = pair2_occupancy(v, planes, r, false, w) * (w / kWave);
-        if (waves > s.waves || (waves == s.waves && planes == s.planes && r > s.reps && w == s.wg))
+        if (waves > s.waves || (waves == s.waves && planes == s.planes && r > s.reps))
             s = PairShape{planes, r, w, waves};
     };
+    // The most waves, then the most replicas, of work-groups of 256 threads; of 512 where those would have a single
+    // replica (1,800 weighted bins, 4M points: 256 threads and 1 replica 164 ms, 512 and 2 158 ms; 360 bins, 150k
+    // points: 1 to 8 replicas of either 0.40 ms; 144 bins, 9k points: 256 threads 0.039, 512 0.048 ms).  Sizes that
+    // do not fill the four SIMDs evenly only where there is no other (640 threads, 20 waves by the occupancy query,
+    // 232 ms).
     for (int planes = v.buf ? 2 : 1; planes >= 1 && s.waves == 0; --planes) {
-        for (int r = 1; r <= 32; r *= 2) consider(planes, r, 256);
+        for (int w = 256; w <= 512 && (w == 256 || s.reps == 1); w += 256)
+            for (int r = 1; r <= 32; r *= 2) consider(planes, r, w);
         if (s.waves < 16)
             for (int r = 1; r <= 32; r *= 2)
                 for (int w = 320; w <= 1024; w += 64) consider(planes, r, w);

@@ -264,6 +264,11 @@ static int get_plan(gs_ctx* c, const gs_params& p, const BatchTune& tu, int kind
     // one histogram per wave: fewer planes and waves where it would not fit otherwise
     const PairVariant var{nb, nm, fp64 || (kind == 2 && bins.wide), weighted, p.log_bins != 0, B.has_buf};
     int pair_wg = kWG, pair_waves = 0;
+    // the histograms that a batch takes: four, with a word per count and two per sum, in 64 KiB with their tables
+    if (kind == 2 && (size_t)nbt * (weighted ? 80 : 16) + 2064 + (fp64 ? 10240 : 0) > 64 * 1024) {
+        pblob->release(); B.plans.pop_back();
+        return fail(GS_ELIMIT, "per-wave histograms of %d bins do not fit in LDS", nbt);
+    }
     if (kind == 2) {
         for (a.planes = var.buf ? 2 : 1; a.planes >= 1 && pair_waves == 0; --a.planes)
             for (pair_wg = kWG; pair_wg >= kWave && pair_waves == 0; pair_wg /= 2)

@@ -291,10 +291,13 @@ hipError_t launch_adj_finish(const double* G, int64_t n, int64_t n_data, const d
                              double inv_wr, double* out, hipStream_t st);
 
 // largest dynamic LDS of the pair kernel (160 KiB less its static part)
-constexpr size_t kPairLdsMax = 160 * 1024 - 64;
+constexpr size_t kPairLdsMax = 160 * 1024 - 32;
 // Dynamic LDS bytes of the pair kernel for these parameters and work-group size wg (a multiple of 64, <= 1024).
 size_t pair2_lds_bytes(int nb, int nm, int planes, int reps, bool weighted, bool batched, int wg);
 hipError_t launch_pair2(const PairArgs& a, const PairVariant& v, int nblocks, int wg, hipStream_t st);
+// its unit-weight variants (pair2_unit.hip)
+hipError_t launch_pair2_unit(const PairArgs& a, const PairVariant& v, size_t lds, int nblocks, int wg, hipStream_t st);
+int pair2_unit_occupancy(const PairVariant& v, size_t lds, int wg);
 // copies -> [nreg][nbt] counts and [nreg][nbt][2] sums over ordered pairs, 4 statistics
 hipError_t launch_pair_reduce(const unsigned long long* in, int copies, int nreg, int nbt, int nm, bool weighted,
                               unsigned long long* out, hipStream_t st);

@@ -12,7 +12,9 @@ namespace gs {
 namespace dev {
 
 constexpr int kOkBytes = (kMaxBins + 1) * 8;    // bin table at the start of the LDS (fill_bin_table)
-constexpr int kQueue = 2 * kWave;               // pairs waiting to be re-evaluated, per wave
+// Pairs waiting to be re-evaluated, per wave: a wave less a few, plus one wave (a wave would fit but for the largest
+// histograms, which leave 1.2 KB)
+constexpr int kQueue = 2 * kWave - 8;
 constexpr int kListBytes = kQueue * 8 + kWave * 4;      // per wave: the queue, tile index list
 
 __device__ __forceinline__ float rsq(float x) { return __builtin_amdgcn_rsqf(x); }
@@ -134,7 +136,12 @@ __device__ __forceinline__ void fill_bin_table(unsigned char* smem, const BinDes
 {
     for (int k = tid; k <= B.nb; k += nthr) {
         if constexpr (FP64) ((double*)smem)[k] = B.t64[k];
-        else ((float2*)smem)[k] = k < B.nb ? make_float2(B.ok_lo[k], B.ok_hi[k]) : make_float2(INFINITY, -INFINITY);
+        else {
+            // start and width; a width of 0 is never certain.  s - lo rounds monotonically, so s >= hi gives a
+            // rounded difference of at least the rounded width
+            const bool some = k < B.nb && B.ok_hi[k] > B.ok_lo[k];
+            ((float2*)smem)[k] = some ? make_float2(B.ok_lo[k], B.ok_hi[k] - B.ok_lo[k]) : make_float2(INFINITY, 0.0f);
+        }
     }
 }
 
@@ -148,6 +155,7 @@ struct Binner {
     int nb;
     float ua, ub;
     R rej_lo, rej_hi, ms, hms;
+    uint32_t rej_w;                 // FP32: not rejected if 0 <= s - rej_lo < this (a float's bits)
     R l0, l1, l2;                   // mu: certain where |fract(t) - 1/2| <= l0 + l1 q + l2 q^2 (1/2 - error bound)
 
     __device__ __forceinline__ Binner(const BinDesc& B, const unsigned char* t)
@@ -155,6 +163,8 @@ struct Binner {
           rej_hi(FP64 ? (R)B.t64[B.nb + 1] : (R)B.rej_hi), ms((R)B.mu_scale), hms((R)(0.5 * B.mu_scale)), l0(0), l1(0),
           l2(0)
     {
+        // one unit above the rounded width, so that no s below rej_hi is rejected
+        rej_w = FP64 ? 0u : __float_as_uint(B.rej_hi - B.rej_lo) + 1u;
         // in a vector register: an FMA reads one scalar operand at most
         asm volatile("" : "+v"(ub));
     }
@@ -178,7 +188,12 @@ struct Binner {
             return fmaf(dz, dz, fmaf(dy, dy, dx * dx));
         }
     }
-    __device__ __forceinline__ bool rejected(R s) const { return !(s > rej_lo && s < rej_hi); }
+    __device__ __forceinline__ bool rejected(R s) const
+    {
+        // FP32: one comparison of the difference's bits, in which negative numbers are above all others
+        if constexpr (FP64) return !(s > rej_lo && s < rej_hi);
+        else return !(__float_as_uint(s - rej_lo) < rej_w);
+    }
     // bins of a pair that is not rejected
     __device__ __forceinline__ PairKind bins(const Pt<R>& A, R ed, R s, int& b, int& m) const
     {
@@ -194,7 +209,7 @@ struct Binner {
         } else {
             b = cvt_sat(bin_estimate(s, LOGB, ua, ub));
             const float2 ok = ((const float2*)table)[b];
-            safe = s >= ok.x && s < ok.y;
+            safe = __float_as_uint(s - ok.x) < __float_as_uint(ok.y);
         }
         m = 0;
         if constexpr (RSD) {
@@ -387,9 +402,9 @@ __device__ __forceinline__ void walk(const WalkArgs& a, Sink& sink, const BinDes
                         if constexpr (RSD || !FP64) {
                             if (lanes(u1 || u2)) {
                                 enqueue(u1, ib + ai, k);
-                                if (nq > kWave) recheck();
+                                if (nq > kQueue - kWave) recheck();
                                 enqueue(u2, ib + ai2, k);
-                                if (nq > kWave) recheck();
+                                if (nq > kQueue - kWave) recheck();
                             }
                         }
                     }

@@ -5,6 +5,7 @@ import pytest
 
 import oracle as O
 from gramsci_amd import catalog as C
+from gramsci_amd._lib import GsError
 from gramsci_amd.engine import Engine
 
 pytestmark = pytest.mark.gpu
@@ -104,3 +105,25 @@ def test_adjoint_groups_and_parts(eng, monkeypatch, group, parts, buffered, nmu,
     got = eng.adjoint2(g2, g3, p.rmin, p.rmax, p.nbins, p.nmu, log)
     # each term is rounded to 2^-50 of the largest; at most 5000 terms a point
     assert np.max(np.abs(got - ref)) <= 1e-11 * np.max(np.abs(ref))
+
+
+@pytest.mark.parametrize("nbins,nmu", [(127, 106), (106, 127), (116, 116)])
+def test_largest_histograms(eng, nbins, nmu):
+    # 40,386 and 40,368 counts: the whole LDS of a compute unit but 2 KB
+    rng = np.random.default_rng(8)
+    xyz = rng.uniform(0, 10.0, (500, 3)) + 3.0
+    _check(eng, xyz, None, 200, O.Params(0.5, 6.0, nbins, nmu, False))
+
+
+@pytest.mark.parametrize("weighted,fits", [(False, 3900), (True, 780)])
+def test_batched_histogram_limit(eng, weighted, fits):
+    # four histograms in 64 KiB: 3,966 counts, 793 with sums
+    rng = np.random.default_rng(9)
+    xyz = rng.uniform(0, 10.0, (400, 3)) + 3.0
+    w = rng.uniform(0.5, 2.0, 400) if weighted else None
+    eng.set_catalogue_batched(xyz, w, None, np.array([0, 150, 400]), np.array([70, 100]))
+    nm = fits // 3 // 13
+    out = eng.pcf2_batched(0.5, 6.0, 13, nm, False, "fp32", cell_div=2)
+    assert out["cnt"].sum() > 0
+    with pytest.raises(GsError, match="do not fit in LDS"):
+        eng.pcf2_batched(0.5, 6.0, 13, nm + 5, False, "fp32", cell_div=2)

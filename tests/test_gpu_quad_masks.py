@@ -79,3 +79,16 @@ def test_every_pass(eng, monkeypatch, tetra):
         r = _check(eng, xyz, w, 1200, p, tetra)
         for q in ("n_candidates", "n_units", "n_overflow"):
             assert r["stats"][q] == base["stats"][q], q
+
+
+def test_largest_tables(eng):
+    # 16 bins and cells of rmax / 16: the perimeter table and the stencil rows beside the shortest list
+    d, r = C.clustered(300, 20.0, 71), C.uniform(500, 20.0, 72)
+    xyz = np.concatenate([d, r])
+    w = C.lognormal_weights(len(xyz), 0.2, 73)
+    ref = O.pcf4(xyz, w, 300, O.Params(1.0, 6.0, 16, 1, False))
+    eng.set_catalogue(xyz, w, 300)
+    for div in (2, 16):
+        out = eng.pcf4(1.0, 6.0, 16, False, cell_div=div)
+        assert np.array_equal(out["cnt"], ref["cnt"]) and out["stats"]["n_units"] == ref["n_quads"], div
+        assert _close(out["n3"], ref["n3"]) and _close_disc(out["disc_r"], ref["disc_r"])
