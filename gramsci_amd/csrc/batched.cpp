@@ -356,7 +356,7 @@ static int get_plan(gs_ctx* c, const gs_params& p, const BatchTune& tu, int kind
             ta1.kmax = full;
             wg1 = wave ? kWave : ta1.wg;
         } else {
-            wg1 = ta1.wg = tu.wg > 0 ? tu.wg : triplet_wg(kmean);
+            wg1 = ta1.wg = tu.wg > 0 ? tu.wg : triplet_wg(nm > 1 ? kmean : 0.5 * kmean, nm > 1, weighted);
         }
         if (kmax1 < full) {
             ta1.kmax = kmax1;

@@ -205,7 +205,7 @@ std::vector<uint16_t> table3_hist(int nb);   // 4 * configuration, for the tripl
 std::vector<uint8_t> normal_table(int nm);
 int plan_triplet_lds(TripArgs& a, int nb, bool fp64, bool weighted);
 // threads per triplet work-group for a mean neighbour count kmean (GS_T3_WG overrides)
-int triplet_wg(double kmean);
+int triplet_wg(double list, bool rsd, bool weighted);
 // apexes per queue fetch for n work items over nblocks work-groups: about 128 fetches per work-group
 // (GS_APEX_BATCH overrides)
 int triplet_batch(int64_t n, int nblocks);

@@ -124,18 +124,19 @@ std::vector<uint8_t> normal_table(int nm)
 // LDS plan of the triplet kernel for a.ncfg/a.nm: histogram replicas and
 // neighbour capacity within 64 KiB; a histogram too large for LDS goes to
 // global atomics instead.
-int triplet_wg(double kmean)
+int triplet_wg(double list, bool rsd, bool weighted)
 {
     const char* ev = getenv("GS_T3_WG");        // tuning override (unset or empty: automatic)
     if (ev && *ev) {
         const int w = atoi(ev);
         if (w == 64 || w == 128 || w == 256) return w;
     }
-    // 256 threads per apex measured fastest also for short neighbour lists (64 batched regions,
-    // mean ~100 neighbours: 108 ms per pass with 256 threads, 153 ms with 64), once work items are
-    // fetched in batches; smaller work-groups stay available for other shapes
-    (void)kmean;
-    return 256;
+    // Measured over uniform catalogues, in ms for 64, 128 and 256 threads.  Lists of 16: mu bins and weights 0.81,
+    // 0.73, 1.12, mu bins alone 0.56, 0.69, 1.08, weights alone (32 neighbours) 0.74, 0.76, 1.12.  Lists of 64: 2.32,
+    // 1.70, 1.99; 1.33, 1.40, 1.66; 0.88, 0.79, 0.88.  Lists of 128: 2.48, 1.76, 1.74; 1.67, 1.22, 1.29; 0.84, 0.64,
+    // 0.63.  Lists of 256: 2.43, 1.58, 1.33 and so on.
+    if (list < 24.0 && !(rsd && weighted)) return 64;
+    return list < 120.0 ? 128 : 256;
 }
 
 int triplet_batch(int64_t n, int nblocks)
@@ -152,7 +153,9 @@ int plan_triplet_lds(TripArgs& a, int nb, bool fp64, bool weighted)
     auto lds = [&]() { return triplet3_lds_bytes(a, nb, fp64, weighted); };
     a.lds_hist = 1;
     a.reps = 1;
-    while (a.reps < 32 && nh * a.reps * 2 * 4 <= 16 * 1024) a.reps *= 2;
+    // replicas of the counts up to 4 KiB: the LDS is better spent on work-groups (100k + 200k points, 5 bins, 6 mu
+    // bins, 128 threads: 16 KiB of replicas 1.75 ms, 4 KiB 1.59)
+    while (a.reps < 32 && nh * a.reps * 2 * 4 <= 4 * 1024) a.reps *= 2;
     a.kmax = 4096;
     while (a.kmax > 512 && lds() > budget) a.kmax -= 256;
     while (a.reps > 1 && lds() > budget) a.reps /= 2;
@@ -396,7 +399,7 @@ static int count3(gs_ctx* c, const gs_params* p, bool equi, uint64_t* cnt, doubl
         for (int32_t k : kc)
             if (k >= 0) { ks.push_back(k); ksum += k; }
         if (!ks.empty()) {
-            a.wg = triplet_wg(ksum / (double)ks.size());
+            a.wg = triplet_wg(ksum / (double)ks.size(), nm > 1, weighted);
             const size_t q = std::min(ks.size() - 1, (size_t)std::ceil(0.995 * (ks.size() - 1)));
             std::nth_element(ks.begin(), ks.begin() + q, ks.end());
             const int k995 = ks[q];

@@ -128,7 +128,7 @@ __global__ __launch_bounds__(kWG) void k_triplet3(TripArgs a)
     if (W) p += (size_t)kmax * 8;
     int32_t* ol = (int32_t*)p;           // RSD or weighted: original index of each neighbour
 
-    __shared__ int s_item, s_k, s_over, s_ncand, s_kall;
+    __shared__ int s_item, s_k, s_ncand, s_kall;
 
     if (lh) {
         for (int k = tid; k < nh * reps; k += nt) hc[k] = 0;
@@ -192,7 +192,6 @@ __global__ __launch_bounds__(kWG) void k_triplet3(TripArgs a)
         if (tid == 0) {
             s_k = 0;
             s_kall = 0;
-            s_over = 0;
         }
         const bool fetch = b_next >= b_end;
         if (fetch && tid < kWave) {
@@ -276,58 +275,49 @@ __global__ __launch_bounds__(kWG) void k_triplet3(TripArgs a)
             if (tid == 0) s_ncand = run;
         }
         __syncthreads();
-        const int ncand = s_ncand;
-        int row = 0, row_beg = 0, row_end = a.nrows > 0 ? rw_len[0] : 0, j0 = a.nrows > 0 ? rw_js[0] : 0;
+        const int ncand = __builtin_amdgcn_readfirstlane(s_ncand);
+        // The kept neighbours' indices go to the list by ballots; the rest of a record (bin, mu bins, weight) is
+        // worked out below with a list entry per thread: here only one candidate in four is kept.
+        int kall = 0;
         {
-            for (int next = tid; next < ncand; next += nt) {
-                while (next >= row_end) {           // the row holding candidate number next
-                    ++row;
-                    row_beg = rw_off[row];
-                    row_end = row_beg + rw_len[row];
-                    j0 = rw_js[row] - row_beg;
+            int row = 0, row_end = a.nrows > 0 ? rw_len[0] : 0, j0 = a.nrows > 0 ? rw_js[0] : 0;
+            for (int base = 0; base < ncand; base += nt) {
+                const int next = base + tid;
+                bool kept = false, listed = false;
+                int j = 0;
+                if (next < ncand) {
+                    while (next >= row_end) {       // the row holding candidate number next
+                        ++row;
+                        const int row_beg = rw_off[row];
+                        row_end = row_beg + rw_len[row];
+                        j0 = rw_js[row] - row_beg;
+                    }
+                    j = j0 + next;
+                    ++cand;
+                    const double4 Pj = a.pw[j];
+                    const double s = exact_s(Pa.x, Pa.y, Pa.z, Pj.x, Pj.y, Pj.z);
+                    kept = s > t_lo && s < t_hi;
+                    if (kept && s >= t64[nb]) {     // the reference's out-of-range bin
+                        kept = false;
+                        ++over;
+                    }
+                    // SYM: every kept neighbour counts for the apex's C(k, 2) candidates; only those after the apex
+                    // in the visiting order (buffer points, then larger index) enter its list
+                    listed = kept && (!SYM || j > apex || (a.flags[j] & 2u));
                 }
-                const int j = j0 + next;
-                ++cand;
-                const double4 Pj = a.pw[j];
-                const double s = exact_s(Pa.x, Pa.y, Pa.z, Pj.x, Pj.y, Pj.z);
-                if (!(s > t_lo && s < t_hi)) continue;
-                const float sf = (float)s;
-                int b = (int)__builtin_amdgcn_fmed3f(bin_estimate(sf, LOGB, ua, ub), 0.0f, nbm1f);
-                while (b > 0 && s < t64[b]) --b;
-                while (b < nb && s >= t64[b + 1]) ++b;
-                if (b == nb) { ++over; continue; }
-                const uint32_t fj = a.flags[j];
-                if constexpr (SYM) {
-                    // every kept neighbour counts for the apex's C(k, 2) candidates; only those after the
-                    // apex in the visiting order (buffer points, then larger index) enter its list
-                    atomicAdd(&s_kall, 1);
-                    if (!((fj & 2u) || j > apex)) continue;
-                }
-                const int pos = atomicAdd(&s_k, 1);
-                if (pos >= kmax) { s_over = 1; continue; }
-                // whole bytes for the flags let the pair loop add and subtract them with byte selects
-                // (SDWA) instead of extracting bits
-                uint32_t pk = __umul24((uint32_t)b, 2u * (uint32_t)nb) | ((fj & 1u) << 24);
-                if constexpr (SYM) pk |= (fj & 2u) << 15;       // byte 2 = 1: buffer point (never an apex)
-                if (nm > 1) {
-                    int m, mr;
-                    exact_mu(Pa.x, Pa.y, Pa.z, Pj.x, Pj.y, Pj.z, ms, nm, m, mr);   // apex -> j
-                    pk |= (uint32_t)m << 16;
-                }
-                if (nm > 1 || W) ol[pos] = a.orig[j];
-                if constexpr (FP64) {
-                    rec64[pos] = make_double4(Pj.x, Pj.y, Pj.z, (double)pk);
-                } else {
-                    rec32[pos] = make_float4((float)(Pj.x - Pa.x), (float)(Pj.y - Pa.y), (float)(Pj.z - Pa.z),
-                                             __uint_as_float(pk));
-                }
-                jl[pos] = j;
-                if constexpr (W) wl[pos] = ldexp(Pj.w, shift);
+                const unsigned long long m = __builtin_amdgcn_ballot_w64(listed);
+                if constexpr (SYM) kall += (int)__popcll(__builtin_amdgcn_ballot_w64(kept));
+                int at = 0;
+                if (lane == 0 && m) at = atomicAdd(&s_k, (int)__popcll(m));
+                const int pos = __builtin_amdgcn_readfirstlane(at) +
+                                (int)__builtin_amdgcn_mbcnt_hi((uint32_t)(m >> 32), __builtin_amdgcn_mbcnt_lo((uint32_t)m, 0u));
+                if (listed && pos < kmax) jl[pos] = j;
             }
         }
+        if (SYM && lane == 0 && kall) atomicAdd(&s_kall, kall);
         __syncthreads();
         const int K = min(s_k, kmax);
-        if (s_over) {
+        if (s_k > kmax) {
             if (a.ovf) {
                 // left to a later pass with room for all its neighbours (s_k counted every one)
                 if (tid == 0) {
@@ -341,6 +331,33 @@ __global__ __launch_bounds__(kWG) void k_triplet3(TripArgs a)
             }
             if (tid == 0) atomicExch(a.err, 1);
         }
+        for (int pos = tid; pos < K; pos += nt) {
+            const int j = jl[pos];
+            const double4 Pj = a.pw[j];
+            const uint32_t fj = a.flags[j];
+            const double s = exact_s(Pa.x, Pa.y, Pa.z, Pj.x, Pj.y, Pj.z);
+            int b = (int)__builtin_amdgcn_fmed3f(bin_estimate((float)s, LOGB, ua, ub), 0.0f, nbm1f);
+            while (b > 0 && s < t64[b]) --b;
+            while (b < nb - 1 && s >= t64[b + 1]) ++b;
+            // whole bytes for the flags let the pair loop add and subtract them with byte selects
+            // (SDWA) instead of extracting bits
+            uint32_t pk = __umul24((uint32_t)b, 2u * (uint32_t)nb) | ((fj & 1u) << 24);
+            if constexpr (SYM) pk |= (fj & 2u) << 15;       // byte 2 = 1: buffer point (never an apex)
+            if (nm > 1) {
+                int m, mr;
+                exact_mu(Pa.x, Pa.y, Pa.z, Pj.x, Pj.y, Pj.z, ms, nm, m, mr);   // apex -> j
+                pk |= (uint32_t)m << 16;
+            }
+            if (nm > 1 || W) ol[pos] = a.orig[j];
+            if constexpr (FP64) {
+                rec64[pos] = make_double4(Pj.x, Pj.y, Pj.z, (double)pk);
+            } else {
+                rec32[pos] = make_float4((float)(Pj.x - Pa.x), (float)(Pj.y - Pa.y), (float)(Pj.z - Pa.z),
+                                         __uint_as_float(pk));
+            }
+            if constexpr (W) wl[pos] = ldexp(Pj.w, shift);
+        }
+        __syncthreads();
         // pair index: K <= 4096 in LDS, so P < 2^31; a device-memory list may hold more
         using pidx_t = std::conditional_t<GEN == 2, long long, int>;
         const pidx_t P = (pidx_t)K * (K - 1) / 2;
