@@ -373,7 +373,7 @@ static int count3(gs_ctx* c, const gs_params* p, bool equi, uint64_t* cnt, doubl
     }
 
     // Two passes.  The neighbour list in LDS bounds the work-groups a CU can hold, so the
-    // first pass sizes it for the 99.5th percentile of the neighbour counts of ~8192
+    // first pass sizes it for the 99.5th percentile of the neighbour counts of ~2048
     // sampled apexes (+5%) and hands every apex with more neighbours to a second pass over
     // just those apexes, with the largest list that fits.  An apex is counted in exactly
     // one pass, so the sums are those of one pass.
@@ -381,7 +381,7 @@ static int count3(gs_ctx* c, const gs_params* p, bool equi, uint64_t* cnt, doubl
     // last pass with its list in device memory (triplet_glist_pass): no neighbour count is refused.
     const int kmax_full = mat ? am.kmax : a.kmax;
     int kmax1 = kmax_full;
-    const int nsample = std::min(n, 8192);
+    const int nsample = std::min(n, 2048);
     const int stride = nsample > 0 ? n / nsample : 1;
     // i32: second-pass apexes, last-pass apexes, the sampled neighbour counts
     if ((rc = X.i32.reserve(2 * (size_t)n + nsample))) return rc;
@@ -605,7 +605,7 @@ static int count4(gs_ctx* c, const gs_params* p, bool tetra, uint64_t* cnt, doub
     a.g.m = mst;
     a.n_items = (int)(v.n_data + v.n_rand);
     // Passes, each over the apexes whose neighbours outnumbered the list of the one before: one wave per apex (64
-    // neighbours), work-groups with a list for the 99.5th percentile of ~8192 sampled neighbour counts (+5%, a power
+    // neighbours), work-groups with a list for the 99.5th percentile of ~2048 sampled neighbour counts (+5%, a power
     // of two), work-groups with the longest LDS list, and last work-groups with device-memory lists.  The waves take
     // unit weights where at least a quarter of the sample fits them: kernels of 0.97 against 1.84 ms (50k + 100k
     // points), 0.42 against 0.63 (27k + 54k, 4 bins); with weights the FP64 atomics of the quads
@@ -613,7 +613,7 @@ static int count4(gs_ctx* c, const gs_params* p, bool tetra, uint64_t* cnt, doub
     const int n = a.n_items;
     int kmax1 = kmax;
     double short_lists = 0.0;
-    const int nsample = std::min(n, 8192);
+    const int nsample = std::min(n, 2048);
     const int stride = nsample > 0 ? n / nsample : 1;
     // i32: the lists of queued apexes, then the sampled neighbour counts
     if ((rc = X.i32.reserve(kPasses * (size_t)n + nsample))) return rc;
