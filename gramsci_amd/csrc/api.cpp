@@ -272,8 +272,8 @@ int fill_bins(const gs_params& p, const double* t64, double rrel, double xmax, d
     return GS_OK;
 }
 
-// Tables of the triplet kernel on the matrix cores; its header derives the error bound.  ok[b].y and rej_w bound
-// differences rounded to FP32: rounding is monotonic, so s >= hi implies s - lo >= hi - lo also when rounded.
+// Tables of the triplet kernel on the matrix cores; its header derives the error bound.  ok[k].y bounds differences
+// rounded to FP32: rounding is monotonic, so s >= hi implies s - lo >= hi - lo also when rounded.
 void fill_triplet_matrix(const gs_params& p, const double* t64, double h, double hx, TripMatrix& M)
 {
     memset(&M, 0, sizeof(M));
@@ -284,22 +284,20 @@ void fill_triplet_matrix(const gs_params& p, const double* t64, double h, double
     M.scale = std::ldexp(1.0, -e);
     const double r = std::ldexp(p.rmax, -e), err = std::ldexp(r * r, -18) * 1.01;
     auto t = [&](int b) { return std::ldexp(t64[b], -2 * e); };
-    for (int b = 0; b < nb; ++b) {
-        const float lo = f_up(t(b) + err);
-        const float hi = f_down((b == nb - 1 ? std::min(t(nb), t(nb + 1)) : t(b + 1)) - err);
-        M.ok[b] = make_float2(lo, hi > lo ? hi - lo : 0.0f);
-    }
-    M.rej_lo = f_down(t(0) - err);
-    const float w = std::nextafter(f_up(t(nb + 1) + err) - M.rej_lo, INFINITY);
-    memcpy(&M.rej_w, &w, sizeof(w));
+    auto interval = [](float lo, float hi) { return make_float2(lo, hi > lo ? hi - lo : 0.0f); };
+    // a squared side is below 4 r^2 <= 16 but for its error and the padding (1e30)
+    M.ok[0] = interval(-16.0f, f_down(t(0) - err));
+    for (int b = 0; b < nb; ++b)
+        M.ok[b + 1] = interval(f_up(t(b) + err), f_down((b == nb - 1 ? std::min(t(nb), t(nb + 1)) : t(b + 1)) - err));
+    M.ok[nb + 1] = make_float2(f_up(t(nb + 1) + err), INFINITY);
     if (p.log_bins) {
         const double inv = 1.0 / ((std::log10(p.rmax) - std::log10(p.rmin)) / nb);
         M.ua = (float)(0.5 * std::log10(2.0) * inv);
-        M.ub = (float)((std::log10(2.0) * e - std::log10(p.rmin)) * inv);
+        M.ub = (float)((std::log10(2.0) * e - std::log10(p.rmin)) * inv + 1.0);
     } else {
         const double inv = 1.0 / ((p.rmax - p.rmin) / nb);
         M.ua = (float)std::ldexp(inv, e);
-        M.ub = (float)(-p.rmin * inv);
+        M.ub = (float)(-p.rmin * inv + 1.0);
     }
 }
 

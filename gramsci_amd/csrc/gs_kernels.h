@@ -163,15 +163,13 @@ struct TripArgs {
     int32_t buf;
 };
 // Tables of the matrix kernel (fill_triplet_matrix), for coordinates scaled by a power of two such that rmax is
-// in [1, 2): bin b is certain if 0 <= s - ok[b].x < ok[b].y (in FP32), a pair certainly not kept unless
-// 0 <= s - rej_lo < rej_w (as a float's bits).
+// in [1, 2): a squared side s is certainly in slot k (0: below the bins, nb + 1: above) if s - ok[k].x, as a
+// float's bits, is below those of ok[k].y; its slot is estimated by f(s) ua + ub, f = sqrt (linear) or log2 (log).
 struct TripMatrix {
     double scale;
     double t_top;               // kept neighbours of an apex: t64[0] < s < t_top (beyond, up to t64[nb+1]: overflow)
     double inv_h, inv_hx;       // 1 / cell edges
-    float2 ok[kMaxBins + 1];
-    float rej_lo;
-    uint32_t rej_w;
+    float2 ok[kMaxBins + 2];
     float ua, ub;
 };
 // teams: waves of a work-group that take an apex each, or 1

@@ -182,18 +182,18 @@ bool plan_triplet_matrix(TripArgs& a, int nb, bool buf)
 {
     a.buf = buf ? 1 : 0;
     a.reps = 2;
-    const size_t hist = (size_t)nb * nb * nb * 4 * (buf ? 3 : 1) * 4;
+    const size_t hist = (size_t)nb * nb * (nb + 2) * 4 * (buf ? 3 : 1) * 4;
     if (hist > 32 * 1024) return false;     // beyond: the general kernel, whose histogram holds configurations
-    // replicas up to 8 KiB: more of them leave the LDS room for fewer work-groups (200k + 400k points, 5 bins:
-    // 2, 4, 8 replicas 11.5, 11.5, 12.3 ms; 16 regions, 4 bins, buffer points: 3.4, 3.7, 4.2 ms)
-    while (a.reps < 16 && hist * a.reps * 2 <= 8 * 1024) a.reps *= 2;
+    // replicas up to 12 KiB: more of them leave the LDS room for fewer work-groups (200k + 400k points, 5 bins: 2, 4,
+    // 8 replicas 11.1, 11.0, 13.4 ms; 16 regions, 4 bins, buffer points: 2 replicas 3.2, 4 4.8 ms)
+    while (a.reps < 16 && hist * a.reps * 2 <= 12 * 1024) a.reps *= 2;
     a.kmax = 4096;
     while (a.kmax > 64 && triplet_matrix_lds(a, nb, 1) > 150 * 1024) a.kmax -= 64;
     return triplet_matrix_lds(a, nb, 1) <= 150 * 1024;
 }
 
-// One wave per apex while four lists fit the LDS beside each other often enough (up to 256 entries: 16 regions of 60k points,
-// lists of 128, 3.6 ms, with work-groups of 256 6.4 ms), a work-group beyond (lists of 512 entries: 11.5 against 20.6 ms).
+// One wave per apex while four lists leave the LDS room for several work-groups, up to 256 entries (16 regions of 60k
+// points, lists of 128: 3.6 ms, with work-groups of 256 6.4); a work-group beyond (lists of 512: 11.5 against 20.6 ms).
 bool triplet_matrix_team(TripArgs& a, int nb, int kmax1, int wg)
 {
     a.kmax = kmax1;

@@ -13,8 +13,10 @@
 //    A lane then holds four pairs of one u, and the vector ALU only bins them.  The blocks are those of the
 //    upper triangle, so less than 16 / K of the pairs are computed in vain.
 //  * A neighbour's bin, class (random or not) and buffer flag are one tag, its part of the histogram's byte
-//    offset: the histogram is [buffer vertices][class][bin of u][bin of v][third bin], folded to configurations
-//    only when it is added to the outputs, so a pair's slot is one addition and one shift-add.
+//    offset: the histogram is [buffer vertices][class][bin of u][bin of v][third side], folded to configurations
+//    only when it is added to the outputs, so a pair's slot is one addition and one shift-add.  Third sides below
+//    and above the bins are slots too, certain or not like a bin, so that one comparison tells the pairs that FP64
+//    has to decide; those below are counted (nobody reads them), those above left out.
 //
 // Error of the squared side, in units where rmax is in [1, 2) (coordinates are scaled by a power of two), with
 // u = 2^-24 and |x| <= rmax for every neighbour: rounding the coordinates moves it by at most 8 u rmax^2, |u|^2
@@ -28,9 +30,9 @@
 // lanes busy, then walks its blocks.  With one wave per apex no barrier is needed between these phases.
 //
 // Measured against the general kernel: 200k + 400k points, rmax 30 of box 500, 5 bins (19.3e9 third sides) 20.2 ->
-// 11.5 ms; 16 regions of 60k points, 4 bins, buffer points 6.4 -> 3.4 ms.  About 45 vector instructions per block
-// of 256 pairs' four steps (before: 44 per pair step), which still bound it: the matrix instruction takes the place
-// of 6 of them per step and the tags of 10.
+// 11.0 ms; 16 regions of 60k points, 4 bins, buffer points 6.4 -> 3.2 ms.  About 43 vector instructions per block, for
+// four pairs a lane (before: 44 per pair), which still bound it (80 % of the issue cycles), with the gather of the
+// neighbours a quarter of them.  Counting the sides above the bins too (their slots are hot) cost 2 ms.
 #include "gs_device.h"
 #include "gs_kernels.h"
 
@@ -66,8 +68,8 @@ __device__ __forceinline__ void lds_count(uint32_t at)
 
 size_t triplet_matrix_lds(const TripArgs& a, int nb, int teams)
 {
-    size_t b = ((size_t)nb * a.reps * 4 + 15) / 16 * 16 + kControlBytes;                    // certain intervals
-    b += ((size_t)nb * nb * nb * 4 * (a.buf ? 3 : 1) * a.reps * 4 + 15) / 16 * 16;          // histogram
+    size_t b = ((size_t)(nb + 2) * a.reps * 4 + 15) / 16 * 16 + kControlBytes;              // certain intervals
+    b += ((size_t)nb * nb * (nb + 2) * 4 * (a.buf ? 3 : 1) * a.reps * 4 + 15) / 16 * 16;    // histogram
     b += ((size_t)(nb + 2) * 8 + 15) / 16 * 16;                                             // t64
     return b + teams * team_bytes(a.kmax, a.nrows);
 }
@@ -78,7 +80,8 @@ __global__ __launch_bounds__(kMatrixMaxWG) void k_triplet_matrix(TripArgs a)
     extern __shared__ __align__(16) unsigned char smem[];
     const BinDesc& B = *a.bins;
     const TripMatrix& M = *a.matrix;
-    const int nb = B.nb, nb3 = nb * nb * nb, nf = a.buf ? 3 : 1;
+    // slots of a pair of bins: sides below, in, above the nb bins
+    const int nb = B.nb, ns = nb + 2, nb3 = nb * nb * ns, nf = a.buf ? 3 : 1;
     const int reps = a.reps, rsh = 31 - __clz(reps);
     const int kmax = a.kmax, stride = kmax + 16;    // 16 mod 64: the four rows of an operand fall on all banks
     const int tid = threadIdx.x, nt = blockDim.x, lane = tid & 63, nw = nt >> 6;
@@ -88,7 +91,7 @@ __global__ __launch_bounds__(kMatrixMaxWG) void k_triplet_matrix(TripArgs a)
     // The certain intervals lie at the start, as far apart as the histogram's slots (4 reps bytes, reps >= 2): one
     // shift of a bin gives both its interval's and its slot's offset.
     const unsigned sh = (unsigned)rsh + 2;
-    const uint32_t hist_off = (uint32_t)(((size_t)nb * reps * 4 + 15) / 16 * 16) + kControlBytes;
+    const uint32_t hist_off = (uint32_t)(((size_t)ns * reps * 4 + 15) / 16 * 16) + kControlBytes;
     int* const ctl = (int*)(smem + hist_off - kControlBytes);      // no static LDS: the intervals are at address 0
     int &s_item = ctl[0], &s_k = ctl[1], &s_kall = ctl[2], &s_ncand = ctl[3];
     unsigned long long* const s_stat = (unsigned long long*)(ctl + 4);
@@ -110,7 +113,7 @@ __global__ __launch_bounds__(kMatrixMaxWG) void k_triplet_matrix(TripArgs a)
     };
 
     for (int k = tid; k < nb3 * 4 * nf * reps; k += nt) hc[k] = 0;
-    for (int k = tid; k < nb; k += nt) *(float2*)(smem + ((uint32_t)k << sh)) = M.ok[k];
+    for (int k = tid; k < ns; k += nt) *(float2*)(smem + ((uint32_t)k << sh)) = M.ok[k];
     for (int k = tid; k < nb + 2; k += nt) t64[k] = B.t64[k];
     if (tid == 0) { s_k = 0; s_kall = 0; }
     __syncthreads();
@@ -122,8 +125,8 @@ __global__ __launch_bounds__(kMatrixMaxWG) void k_triplet_matrix(TripArgs a)
         for (int o = opaque(t); o < a.ncfg * 4; o += step) {
             const uint32_t ijk = a.cfg_bins[o >> 2];
             const int i = ijk & 255, j = (ijk >> 8) & 255, k = ijk >> 16;
-            const int at[6] = {(i * nb + j) * nb + k, (i * nb + k) * nb + j, (j * nb + i) * nb + k,
-                               (j * nb + k) * nb + i, (k * nb + i) * nb + j, (k * nb + j) * nb + i};
+            const int at[6] = {(i * nb + j) * ns + k + 1, (i * nb + k) * ns + j + 1, (j * nb + i) * ns + k + 1,
+                               (j * nb + k) * ns + i + 1, (k * nb + i) * ns + j + 1, (k * nb + j) * ns + i + 1};
             unsigned long long sum = 0;
             for (int f = 0; f < nf; ++f)
                 for (int q = 0; q < 6; ++q) {
@@ -137,8 +140,7 @@ __global__ __launch_bounds__(kMatrixMaxWG) void k_triplet_matrix(TripArgs a)
         }
     };
 
-    const float ua = M.ua, rej_lo = M.rej_lo, nbm1f = (float)(nb - 1);
-    const uint32_t rej_w = M.rej_w;
+    const float ua = M.ua, above = M.ok[nb + 1].x, topf = (float)(nb + 1);
     float ubv = M.ub;               // in a VGPR: an FMA reads at most one scalar operand
     asm volatile("" : "+v"(ubv));
     const double t_lo = scalar(B.t64[0]), t_hi = scalar(B.t64[nb + 1]), t_top = scalar(M.t_top);
@@ -261,7 +263,7 @@ __global__ __launch_bounds__(kMatrixMaxWG) void k_triplet_matrix(TripArgs a)
                 const double4 Pj = a.pw[j];
                 const uint32_t fj = a.flags[j];
                 const double s = exact_s(Pa.x, Pa.y, Pa.z, Pj.x, Pj.y, Pj.z);
-                int b = (int)__builtin_amdgcn_fmed3f(bin_estimate((float)(s * scale * scale), LOGB, ua, ubv), 0.0f, nbm1f);
+                int b = (int)__builtin_amdgcn_fmed3f(bin_estimate((float)(s * scale * scale), LOGB, ua, ubv), 1.0f, topf - 1.0f) - 1;
                 while (b > 0 && s < t64[b]) --b;
                 while (b < nb - 1 && s >= t64[b + 1]) ++b;
                 x = (float)((Pj.x - Pa.x) * scale);
@@ -269,7 +271,7 @@ __global__ __launch_bounds__(kMatrixMaxWG) void k_triplet_matrix(TripArgs a)
                 z = (float)((Pj.z - Pa.z) * scale);
                 n2 = (float)((double)x * x + (double)y * y + (double)z * z);
                 const int cls = nb3 * ((int)(fj & 1u) + (a.buf ? (int)(fj & 2u) * 2 : 0));
-                tag = ((uint32_t)(b * nb * nb + cls) << sh) | ((uint32_t)(b * nb + cls) << sh << 16);
+                tag = ((uint32_t)(b * nb * ns + cls) << sh) | ((uint32_t)(b * ns + cls) << sh << 16);
             }
             xs[k] = x;
             xs[stride + k] = y;
@@ -321,15 +323,14 @@ __global__ __launch_bounds__(kMatrixMaxWG) void k_triplet_matrix(TripArgs a)
                     uint32_t off[4];
                     float2v ok[4];
                     for (int i = 0; i < 4; ++i)
-                        off[i] = (uint32_t)(int)__builtin_amdgcn_fmed3f(bin_estimate(d[i], LOGB, ua, ubv), 0.0f, nbm1f) << sh;
+                        off[i] = (uint32_t)(int)__builtin_amdgcn_fmed3f(bin_estimate(d[i], LOGB, ua, ubv), 0.0f, topf) << sh;
                     for (int i = 0; i < 4; ++i) ok[i] = *(lds_ptr<float2v>)off[i];
                     unsigned long long unc[4];      // lanes to decide in FP64
                     for (int i = 0; i < 4; ++i) {
-                        // differences as unsigned: negative floats are above every bound
+                        // as unsigned: negative differences are above every bound
                         const bool sure = __float_as_uint(d[i] - ok[i].x) < __float_as_uint(ok[i].y);
-                        unc[i] = __builtin_amdgcn_ballot_w64(__float_as_uint(d[i] - rej_lo) < rej_w) &
-                                 ~__builtin_amdgcn_ballot_w64(sure);
-                        if (sure) lds_count(off[i] + tg[i] + tcur);
+                        unc[i] = ~__builtin_amdgcn_ballot_w64(sure);
+                        if (sure && d[i] < above) lds_count(off[i] + tg[i] + tcur);
                     }
                     if (unc[0] | unc[1] | unc[2] | unc[3]) {
                         const int l = opaque(lane), uj = ut * 16 + (l & 15), vj = vt * 16 + 4 * (l >> 4);
@@ -341,7 +342,7 @@ __global__ __launch_bounds__(kMatrixMaxWG) void k_triplet_matrix(TripArgs a)
                                 if (se > B.t64[0] && se < B.t64[opaque(nb) + 1]) {
                                     const int be = exact_bin(se, t64, nb);
                                     if (be == nb) ++over;
-                                    else lds_count(((uint32_t)be << sh) + tg[i] + tcur);
+                                    else lds_count(((uint32_t)(be + 1) << sh) + tg[i] + tcur);
                                 }
                             }
                     }
