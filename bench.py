@@ -40,8 +40,9 @@ METRIC = "binned pair/triplet evals/s on 1 MI355X: batched FP32+guard vs plain F
 # readings for a copy of known size) and VALU wave-instructions per dispatch (SQ_INSTS_VALU)
 PAIR_RMU_COUNTERS = os.path.join(ROOT, "profiles", "k_pair2_rmu_counters.json")
 # the sources the pair kernel's code object is built from: the profile records their hash
-PAIR_KERNEL_SOURCES = ["gramsci_amd/csrc/pair2.hip", "gramsci_amd/csrc/gs_device.h", "gramsci_amd/csrc/gs_common.h",
-                       "gramsci_amd/csrc/gs_kernels.h"]
+PAIR_KERNEL_SOURCES = ["gramsci_amd/csrc/pair2.hip", "gramsci_amd/csrc/gs_pair_kernel.h",
+                       "gramsci_amd/csrc/gs_pair_tiles.h", "gramsci_amd/csrc/gs_device.h",
+                       "gramsci_amd/csrc/gs_common.h", "gramsci_amd/csrc/gs_kernels.h"]
 FLOPS_PER_PAIR_RMU = 22      # 3 sub, 3 mul, 2 add for s; 3 mid adds, m.s (5), |m|^2 (5), 1 product
 PEAK_FP32 = 157.3e12         # MI355X FP32 vector, dense
 PEAK_FP64 = 78.6e12

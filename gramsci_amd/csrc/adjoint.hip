@@ -11,12 +11,12 @@
 //     dL/dw_k = (G_k - S_D)/Wd (data),   -(G_k + S_R)/Wr (randoms),
 // S_D = sum_{data} wn G, S_R = sum_{randoms} wn G.
 //
-// Two kernels enumerate the pairs as the pair kernel does (wave-level x-row
-// chunks, FP32 geometry with the same guard band and FP64 recheck, or plain
-// FP64): k_adjoint2 over the FULL stencil, so that every ordered pair is seen
-// from its apex's lane and G_k accumulates in an FP64 register without
-// atomics (FP64 precision, and non-finite dL/dN); k_adjoint2h (FP32) over the
-// half stencil, each unordered pair once, with exact fixed-point sums.
+// Two kernels: k_adjoint2 takes 64 points of one x-row per wave over the FULL
+// stencil (FP32 geometry with guard band and FP64 recheck, or plain FP64), so
+// that every ordered pair is seen from its apex's lane and G_k accumulates in
+// an FP64 register without atomics (FP64 precision, and non-finite dL/dN);
+// k_adjoint2h (FP32) walks the pair kernel's tiles over the half stencil, each
+// unordered pair once, with exact fixed-point sums.
 #include "gs_pair_tiles.h"
 #include "gs_kernels.h"
 
