@@ -364,7 +364,7 @@ def triplet_leg(steps, warmup, with_fp64=True):
            "roofline": {"bound": "valu", "achieved": E * 8 / (kms * 1e-3) / 1e12, "peak": PEAK_FP32 / 1e12,
                         "unit": "TFLOP/s", "frac": E * 8 / (kms * 1e-3) / PEAK_FP32, "flops_per_unit": 8,
                         "units": "evaluated neighbour pairs",
-                        "kernel": "k_triplet3 (FP32 + guard, two passes)"}}
+                        "kernel": "k_triplet_matrix (FP32 + guard, two passes)"}}
     if "fp64" in res:
         assert np.array_equal(res["fp64"][1]["cnt"], out["cnt"]), "3PCF fp32/fp64 counts differ"
         leg["fp64"] = {"value": res["fp64"][1]["stats"]["n_units"] / res["fp64"][0],

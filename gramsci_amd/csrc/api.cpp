@@ -348,8 +348,8 @@ int fill_pair_bins(const gs_params& p, const double* t64, const PairGrid& q, dou
 
 // Fixed-point scales 2^F of the weights and products.  Pairs: each weight is scaled by its
 // class's 2^F, below 2^26, so the largest pair product of every class stays below 2^52 (the
-// pair kernel rounds it to an integer with one FP64 addition of 2^52 and sums runs of up to
-// 33 in one 64-bit register) and each class sum is exact to 2^-52 of its own largest product.
+// pair kernel rounds it to an integer with one FP64 addition of 2^52 and sums a run, of some
+// hundreds at most, in one 64-bit register) and each class sum is exact to 2^-52 of its own largest product.
 // Triples: the largest triple product stays below 2^61.
 int fx_shift_point(double wmax)
 {

@@ -30,9 +30,9 @@
 // lanes busy, then walks its blocks.  With one wave per apex no barrier is needed between these phases.
 //
 // Measured against the general kernel: 200k + 400k points, rmax 30 of box 500, 5 bins (19.3e9 third sides) 20.2 ->
-// 11.0 ms; 16 regions of 60k points, 4 bins, buffer points 6.4 -> 3.2 ms.  About 43 vector instructions per block, for
-// four pairs a lane (before: 44 per pair), which still bound it (80 % of the issue cycles), with the gather of the
-// neighbours a quarter of them.  Counting the sides above the bins too (their slots are hot) cost 2 ms.
+// 11.0 ms; 16 regions of 60k points, 4 bins, buffer points 6.4 -> 3.2 ms.  63 vector instructions per block, the
+// neighbours' gather included, for four pairs a lane (before: 44 per pair), still bound it: 0.81 a CU-cycle, the
+// LDS busy half of the time.  Counting the sides above the bins too (their slots are hot) cost 2 ms.
 #include "gs_device.h"
 #include "gs_kernels.h"
 
