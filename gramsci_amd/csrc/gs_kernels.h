@@ -185,6 +185,7 @@ hipError_t launch_sum_copies(const unsigned long long* in, int copies, int64_t s
 // bytes per neighbour of a device-memory neighbour list (glist) of the triplet kernel
 size_t triplet3_glist_entry_bytes(const TripArgs& a, bool fp64, bool weighted);
 size_t triplet3_lds_bytes(const TripArgs& a, int nb, bool fp64, bool weighted);
+size_t triplet3_queue_bytes(const TripArgs& a, bool weighted);
 hipError_t launch_triplet3(const TripArgs& a, int nb, bool fp64, bool weighted, int nblocks, hipStream_t st);
 int triplet3_occupancy(const TripArgs& a, int nb, bool fp64, bool weighted);
 // neighbour counts of the apexes t * stride (t < nsample) of a single catalogue; -1 for buffer points

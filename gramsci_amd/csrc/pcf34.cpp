@@ -134,7 +134,8 @@ int triplet_wg(double list, bool rsd, bool weighted)
     // Measured over uniform catalogues, in ms for 64, 128 and 256 threads.  Lists of 16: mu bins and weights 0.81,
     // 0.73, 1.12, mu bins alone 0.56, 0.69, 1.08, weights alone (32 neighbours) 0.74, 0.76, 1.12.  Lists of 64: 2.32,
     // 1.70, 1.99; 1.33, 1.40, 1.66; 0.88, 0.79, 0.88.  Lists of 128: 2.48, 1.76, 1.74; 1.67, 1.22, 1.29; 0.84, 0.64,
-    // 0.63.  Lists of 256: 2.43, 1.58, 1.33 and so on.
+    // 0.63.  Lists of 256: 2.43, 1.58, 1.33 and so on.  (Before the kernel queued its pairs; since, mu bins and weights,
+    // lists of 110: 2.21, 1.70, 1.80.)
     if (list < 24.0 && !(rsd && weighted)) return 64;
     return list < 120.0 ? 128 : 256;
 }
@@ -150,12 +151,17 @@ int plan_triplet_lds(TripArgs& a, int nb, bool fp64, bool weighted)
 {
     const size_t nh = (size_t)a.ncfg * a.nm * 4;
     const size_t budget = 64 * 1024;
-    auto lds = [&]() { return triplet3_lds_bytes(a, nb, fp64, weighted); };
+    // (without the queues, and with bin tables at their largest: what fits does not depend on either)
+    const size_t tables = (size_t)(2 * (kMaxBins - nb)) * 8;
+    auto lds = [&]() {
+        return triplet3_lds_bytes(a, nb, fp64, weighted) - triplet3_queue_bytes(a, weighted) + tables;
+    };
     a.lds_hist = 1;
     a.reps = 1;
-    // replicas of the counts up to 4 KiB: the LDS is better spent on work-groups (100k + 200k points, 5 bins, 6 mu
-    // bins, 128 threads: 16 KiB of replicas 1.75 ms, 4 KiB 1.59)
-    while (a.reps < 32 && nh * a.reps * 2 * 4 <= 4 * 1024) a.reps *= 2;
+    // replicas up to 4 KiB: the LDS is better spent on work-groups (100k + 200k points, 5 bins, 6 mu bins, 128
+    // threads: 16 KiB of replicas 1.75 ms, 4 KiB 1.59; weights, 4 mu bins, 90k points: 4 KiB 1.71, 12 KiB 1.69, 24 KiB
+    // 2.13, and weights, equal sides, 117k points: 1.14, 1.47, 1.46)
+    while (a.reps < 32 && nh * a.reps * 2 * (weighted ? 16 : 4) <= 4 * 1024) a.reps *= 2;
     a.kmax = 4096;
     while (a.kmax > 512 && lds() > budget) a.kmax -= 256;
     while (a.reps > 1 && lds() > budget) a.reps /= 2;

@@ -32,10 +32,15 @@
 //      the pair kernel - instead of a binary search in a neighbour list.
 // The LDS histogram is added to one of up to 64 copies of the outputs at the end.
 //
-// What bounds it: vector instructions of the pairs (72 % of the issue cycles, unweighted without mu bins), not the
+// With weights, mu bins or equal sides an update is several times as long as the test of the third side, and 40 % of
+// the lanes would idle in it: the pairs with a binned third side go to a queue per wave, and 64 of them are
+// updated at once.  A weighted histogram has two planes instead of three arrays, and so two LDS atomics an update.
+//
+// What bounds it: vector instructions of the pairs (0.78 a CU-cycle with weights and mu bins, 86 % of the lanes
+// active), beside the LDS (65 % busy, nearly half of it bank conflicts of the histogram's atomics), not the
 // histogram's release: 64 queues and output copies alone gave 2.38 -> 2.25 ms with weights and 4 mu bins at 90k
-// points.  Records by list entry, work-groups by list length and fewer replicas took that call from 2.25 to
-// 2.06 ms, and one of 300k points with 6 mu bins from 2.05 to 1.59.
+// points.  Records by list entry, work-groups by list length and fewer replicas took that call to 2.06 ms, the
+// queue and the packed planes to 1.71; 117k weighted points, equal sides, FP64 geometry 1.42 -> 1.10.
 #include <type_traits>
 
 #include "gs_device.h"
@@ -44,6 +49,14 @@
 namespace gs {
 
 using namespace dev;
+
+namespace {
+constexpr int kPairQueue = 2 * kWave;           // entries of a wave's queue: fewer than a wave are left, one wave comes
+constexpr int kPackShift = 42;                  // packed sums: bits of q in the low plane, of q's sum below the count
+constexpr unsigned long long kPackMax = (1ull << 22) - 1;       // increments a packed histogram can hold
+// certain intervals and thresholds of nb bins
+__host__ __device__ constexpr size_t triplet3_bin_bytes(int nb) { return ((size_t)(2 * nb + 3) * 8 + 15) / 16 * 16; }
+}  // namespace
 
 size_t triplet3_glist_entry_bytes(const TripArgs& a, bool fp64, bool weighted)
 {
@@ -56,17 +69,27 @@ size_t triplet3_lds_bytes(const TripArgs& a, int nb, bool fp64, bool weighted)
     const size_t kmax = (size_t)a.kmax;
     size_t b = 0;
     if (a.lds_hist) {
-        b += (nh * a.reps * 4 + 15) / 16 * 16;                  // counts
-        if (weighted) b += nh * 16;                             // split fixed-point sums
+        if (weighted && !a.glist) {
+            b += nh * a.reps * 16;                              // counts and fixed-point sums, packed
+        } else {
+            b += (nh * a.reps * 4 + 15) / 16 * 16;              // counts
+            if (weighted) b += nh * 16;                         // split fixed-point sums
+        }
     }
-    b += ((size_t)(kMaxBins + 1) * 8);                          // ok_lo/ok_hi
-    b += ((size_t)(kMaxBins + 2) * 8 + 15) / 16 * 16;           // t64
+    b += triplet3_bin_bytes(nb);                                // ok_lo/ok_hi, t64
     b += ((size_t)nb * nb * nb * 2 + 15) / 16 * 16;             // config table (u16)
     if (a.nm > 1) b += ((size_t)a.nm * a.nm + 15) / 16 * 16;    // find_normal table (u8)
     b += ((size_t)a.nrows * 12 + 15) / 16 * 16;                 // stencil rows: first point, length, offset
     // neighbour list: coords + packed bin/class/mu, sorted index, weight, orig (in LDS unless glist)
     if (!a.glist) b += kmax * triplet3_glist_entry_bytes(a, fp64, weighted);
-    return b;
+    return b + triplet3_queue_bytes(a, weighted);
+}
+
+// The waves' queues of neighbour pairs whose third side has a bin (variants with weights, mu bins or equal sides)
+size_t triplet3_queue_bytes(const TripArgs& a, bool weighted)
+{
+    const bool q = !a.glist && (weighted || a.nm > 1 || a.equi);
+    return q ? (size_t)(a.wg > 0 ? a.wg : kWG) / kWave * kPairQueue * 4 : 0;
 }
 
 // record packing: bits 0..14 2 * bin * nb (0-based bin, pre-multiplied for the byte offset of the
@@ -81,8 +104,11 @@ size_t triplet3_lds_bytes(const TripArgs& a, int nb, bool fp64, bool weighted)
 // device memory (apexes with more neighbours than an LDS list holds).
 enum { kT3Rsd = 1, kT3Equi = 2 };
 
+// Six waves per SIMD (at most 80 registers, up to four of them spilled) for mu bins without weights: 300k
+// points, 6 mu bins 1.47 -> 1.40 ms, FP64 1.02 -> 0.96.  With weights ten would be spilled, for no gain.
 template <bool FP64, bool W, int MODE, int GEN, bool LOGB>
-__global__ __launch_bounds__(kWG) void k_triplet3(TripArgs a)
+__global__ __launch_bounds__(kWG) __attribute__((amdgpu_waves_per_eu((MODE & kT3Rsd) && !W ? 6 : 1)))
+void k_triplet3(TripArgs a)
 {
     extern __shared__ __align__(16) unsigned char smem[];
     const BinDesc& B = *a.bins;
@@ -99,6 +125,12 @@ __global__ __launch_bounds__(kWG) void k_triplet3(TripArgs a)
     // are not buffer points, by index, then buffer points", whose list keeps only the neighbours after
     // it.  (The RSD mode bins by the apex's mu values and visits every apex's pairs.)
     constexpr bool SYM = (MODE & kT3Rsd) == 0;
+    // Where an update is long, the pairs with a binned third side are queued and updated 64 at a time.
+    constexpr bool Q = (W || MODE != 0) && GEN != 2;
+    // Weighted LDS histograms hold two planes of 64 bits: lo += q mod 2^42, hi += (q >> 42) + 2^42 for every count.
+    // With q <= 2^61 a triangle (fx_shift3), 2^22 - 1 of them leave every field below its width.
+    constexpr bool PK = W && GEN != 2;
+    constexpr unsigned long long kDrain = PK ? kPackMax : (1ull << 31);
     const int tid = threadIdx.x;
     const int nt = blockDim.x;              // threads per work-group: 256, or 64 for short neighbour lists
     const int lane = tid & 63;
@@ -109,14 +141,19 @@ __global__ __launch_bounds__(kWG) void k_triplet3(TripArgs a)
     uint32_t* hc = (uint32_t*)p;
     unsigned long long* hw = nullptr;
     if (lh) {
-        p += ((size_t)nh * reps * 4 + 15) / 16 * 16;
-        hw = (unsigned long long*)p;
-        if (W) p += (size_t)nh * 16;
+        if constexpr (PK) {
+            hw = (unsigned long long*)p;
+            p += (size_t)nh * reps * 16;
+        } else {
+            p += ((size_t)nh * reps * 4 + 15) / 16 * 16;
+            hw = (unsigned long long*)p;
+            if (W) p += (size_t)nh * 16;
+        }
     }
+    unsigned long long* const hhi = hw + (PK && lh ? nh * reps : 0);    // PK: hw holds the low plane
     float2* okb = (float2*)p;
-    p += (size_t)(kMaxBins + 1) * 8;
-    double* t64 = (double*)p;
-    p += ((size_t)(kMaxBins + 2) * 8 + 15) / 16 * 16;
+    double* t64 = (double*)(okb + nb + 1);
+    p += triplet3_bin_bytes(nb);
     uint16_t* tab = (uint16_t*)p;
     p += ((size_t)nb * nb * nb * 2 + 15) / 16 * 16;
     uint8_t* ntab = (uint8_t*)p;
@@ -126,6 +163,8 @@ __global__ __launch_bounds__(kWG) void k_triplet3(TripArgs a)
     int32_t* rw_len = rw_js + a.nrows;
     int32_t* rw_off = rw_len + a.nrows;
     p += ((size_t)a.nrows * 12 + 15) / 16 * 16;
+    uint32_t* const queue = (uint32_t*)p + (tid >> 6) * kPairQueue;     // Q: this wave's
+    if (Q) p += (size_t)(nt / kWave) * kPairQueue * 4;
     // the neighbour list: in LDS, or (GEN 2) in this work-group's part of device memory
     if constexpr (GEN == 2) p = (unsigned char*)a.glist + (size_t)blockIdx.x * (size_t)a.glist_stride;
     float4* rec32 = (float4*)p;          // FP32: x, y, z relative to the apex, packed bin/class/mu
@@ -140,9 +179,13 @@ __global__ __launch_bounds__(kWG) void k_triplet3(TripArgs a)
     __shared__ int s_item, s_k, s_ncand, s_kall;
 
     if (lh) {
-        for (int k = tid; k < nh * reps; k += nt) hc[k] = 0;
-        if (W)
-            for (int k = tid; k < 2 * nh; k += nt) hw[k] = 0;
+        if constexpr (PK) {
+            for (int k = tid; k < 2 * nh * reps; k += nt) hw[k] = 0;
+        } else {
+            for (int k = tid; k < nh * reps; k += nt) hc[k] = 0;
+            if (W)
+                for (int k = tid; k < 2 * nh; k += nt) hw[k] = 0;
+        }
     }
     for (int k = tid; k < nb; k += nt) okb[k] = make_float2(B.ok_lo[k], B.ok_hi[k]);
     for (int k = tid; k < nb + 2; k += nt) t64[k] = B.t64[k];
@@ -175,6 +218,22 @@ __global__ __launch_bounds__(kWG) void k_triplet3(TripArgs a)
         unsigned long long* ow = out_w + (size_t)r * 2 * nh;
         for (int k = tid; k < nh; k += nt) {
             unsigned long long sum = 0;
+            if constexpr (PK) {
+                unsigned long long L = 0, H = 0;
+                for (int q = 0; q < reps; ++q) {
+                    const unsigned long long lo = hw[k * reps + q], hi = hhi[k * reps + q];
+                    if (!(lo | hi)) continue;
+                    hw[k * reps + q] = 0;
+                    hhi[k * reps + q] = 0;
+                    sum += hi >> kPackShift;
+                    const unsigned long long hs = hi & ((1ull << kPackShift) - 1);
+                    add128(L, H, lo, 0ull);
+                    add128(L, H, hs << kPackShift, hs >> (64 - kPackShift));
+                }
+                if (sum) atomicAdd(&oc[k], sum);
+                if (L | H) glb_add128(&ow[2 * k], L, H);
+                continue;
+            }
             for (int q = 0; q < reps; ++q) { sum += hc[k * reps + q]; hc[k * reps + q] = 0; }
             if (sum) atomicAdd(&oc[k], sum);
             if (W) {
@@ -404,7 +463,7 @@ __global__ __launch_bounds__(kWG) void k_triplet3(TripArgs a)
         };
         // histogram update of the triangle (apex, u, v) whose third side has bin b3
         auto update = [&](const USide& U, const int v, const uint32_t pu, const uint32_t pv, const int b3) {
-            if (equi && __umul24((uint32_t)b3, 2u * (uint32_t)nb) != (pu & 0x7fffu)) return;
+            if (!Q && equi && __umul24((uint32_t)b3, 2u * (uint32_t)nb) != (pu & 0x7fffu)) return;
             // the triple product in the reference's order, (w_i w_k1) w_k2 with k1 the neighbour of
             // smaller original index (gramsci.F90:482, :501), so that sums do not depend on the
             // order in which neighbours were gathered
@@ -447,7 +506,10 @@ __global__ __launch_bounds__(kWG) void k_triplet3(TripArgs a)
                                                : (ldexp(Wv, -shift) * ldexp(U.w, -shift)) * Wa);
                 }
             }
-            if (lh) {
+            if (PK && lh) {
+                atomicAdd(&hw[(hk << rsh) + rep], qs & ((1ull << kPackShift) - 1));
+                atomicAdd(&hhi[(hk << rsh) + rep], (qs >> kPackShift) + ((unsigned long long)mult << kPackShift));
+            } else if (lh) {
                 atomicAdd(&hc[(hk << rsh) + rep], mult);
                 if constexpr (W) {
                     atomicAdd(&hw[2 * hk], qs & 0xffffffffull);
@@ -502,9 +564,104 @@ __global__ __launch_bounds__(kWG) void k_triplet3(TripArgs a)
                 }
             }
         };
+        // the bin of the third side of (u, v), -1 where it has none or (equi) not the bin of the other two
+        auto third = [&](const int u, const int v) {
+            int b3 = -1;
+            uint32_t pu;
+            if constexpr (FP64) {
+                const double4 Ru = rec64[u], Rv = rec64[v];
+                pu = (uint32_t)Ru.w;
+                if (!equi || ((pu ^ (uint32_t)Rv.w) & 0x7fffu) == 0) {
+                    const double s = exact_s(Ru.x, Ru.y, Ru.z, Rv.x, Rv.y, Rv.z);
+                    if (s > t_lo && s < t_hi) {
+                        int b = (int)__builtin_amdgcn_fmed3f(bin_estimate((float)s, LOGB, ua, ubv), 0.0f, nbm1f);
+                        while (b > 0 && s < t64[b]) --b;
+                        while (b < nb && s >= t64[b + 1]) ++b;
+                        if (b == nb) ++over; else b3 = b;
+                    }
+                }
+            } else {
+                const float4 Ru = rec32[u], Rv = rec32[v];
+                pu = __float_as_uint(Ru.w);
+                const float dx = Rv.x - Ru.x, dy = Rv.y - Ru.y, dz = Rv.z - Ru.z;
+                const float s = fmaf(dz, dz, fmaf(dy, dy, dx * dx));
+                if ((!equi || ((pu ^ __float_as_uint(Rv.w)) & 0x7fffu) == 0) && s > rej_lo && s < rej_hi) {
+                    b3 = (int)__builtin_amdgcn_fmed3f(bin_estimate(s, LOGB, ua, ubv), 0.0f, nbm1f);
+                    const float2 ok = okb[b3];
+                    if (!((s >= ok.x) & (s < ok.y))) {
+                        ++rechk;
+                        b3 = -1;
+                        const double4 Pu = a.pw[jl[u]], Pv = a.pw[jl[v]];
+                        const double se = exact_s(Pu.x, Pu.y, Pu.z, Pv.x, Pv.y, Pv.z);
+                        if (se > t_lo && se < t_hi) {
+                            const int be = exact_bin(se, t64, nb);
+                            if (be == nb) ++over; else b3 = be;
+                        }
+                    }
+                }
+            }
+            if (equi && b3 >= 0 && __umul24((uint32_t)b3, 2u * (uint32_t)nb) != (pu & 0x7fffu)) b3 = -1;
+            return b3;
+        };
+        // updates the triangle of a queue entry: u, v (12 bits each: an LDS list has at most 4096 entries) and bin
+        auto queued = [&](const uint32_t e) {
+            const int u = (int)(e & 0xfffu), v = (int)((e >> 12) & 0xfffu);
+            const USide U = load_u(u);
+            uint32_t pu, pv;
+            if constexpr (FP64) { pu = (uint32_t)U.R.w; pv = (uint32_t)rec64[v].w; }
+            else { pu = __float_as_uint(U.R.w); pv = __float_as_uint(rec32[v].w); }
+            update(U, v, pu, pv, (int)(e >> 24));
+        };
         const int R = K / 2;
         const int wv = tid >> 6, ln = tid & 63, nw = nt >> 6;
-        if constexpr (GEN != 2) {
+        if constexpr (Q) {
+            // The flat schedule (below) with a uniform number of steps per wave.  A third to a half of the pairs have
+            // a binned third side (with equal sides few), and an update is three times as long as the test, so it
+            // runs for 64 queued pairs at once.  In pieces of 2^20 pairs, which a packed histogram can take.
+            const int P = K * (K - 1) / 2;
+            const int KK = max(K, 1), dq = nt / KK, dr = nt - dq * KK;
+            for (int p0 = 0; p0 < P; p0 += 1 << 20) {
+                const int p1 = min(P, p0 + (1 << 20));
+                const unsigned long long more = (unsigned long long)(p1 - p0) * (SYM ? 3 : 1);
+                if (lh && bound + more > kDrain) {
+                    __syncthreads();
+                    drain(cur_r);
+                    bound = 0;
+                    __syncthreads();
+                }
+                bound += more;
+                int qn = 0;
+                int r = (p0 + tid) / K, c = p0 + tid - r * K;
+                for (int base = p0 + __builtin_amdgcn_readfirstlane(wv) * kWave; base < p1; base += nt) {
+                    int b3 = -1, u = 0, v = 0;
+                    if (base + ln < p1) {
+                        const bool first = c < K - 1 - r;
+                        u = first ? r : K - 2 - r;
+                        v = first ? r + 1 + c : c;
+                        b3 = third(u, v);
+                    }
+                    c += dr;
+                    const bool carry = c >= K;
+                    c -= carry ? K : 0;
+                    r += dq + (carry ? 1 : 0);
+                    const unsigned long long m = __builtin_amdgcn_ballot_w64(b3 >= 0);
+                    if (b3 >= 0)
+                        queue[qn + (int)__builtin_amdgcn_mbcnt_hi((uint32_t)(m >> 32),
+                                                                  __builtin_amdgcn_mbcnt_lo((uint32_t)m, 0u))] =
+                            (uint32_t)u | ((uint32_t)v << 12) | ((uint32_t)b3 << 24);
+                    qn += (int)__popcll(m);
+                    if (qn >= kWave) {
+                        qn -= kWave;
+                        wave_sync();
+                        queued(queue[qn + ln]);
+                        wave_sync();
+                    }
+                }
+                wave_sync();
+                if (ln < qn) queued(queue[ln]);
+                wave_sync();
+            }
+        } else if constexpr (GEN != 2) {
             // Two schedules, chosen per apex (K is uniform in the work-group):
             //  * rows, when they keep at least 7/8 of the lanes busy: wave w takes folded rows (groups of
             //    G = 64 / K rows for K <= 64) w, w + nw, ...; its lanes take columns l, l + 64, ...
@@ -580,9 +737,10 @@ __global__ __launch_bounds__(kWG) void k_triplet3(TripArgs a)
                 }
             }
         }
-        bound += GEN == 2 ? (1ull << 31) + 1 : (unsigned long long)P * (SYM ? 3 : 1);   // LDS increments since the last drain
+        // LDS increments since the last drain (Q adds them, and drains, before its pairs)
+        if constexpr (!Q) bound += GEN == 2 ? (1ull << 31) + 1 : (unsigned long long)P * (SYM ? 3 : 1);
         __syncthreads();
-        if (lh && bound > (1ull << 31)) {
+        if (!Q && lh && bound > kDrain) {
             drain(cur_r);
             bound = 0;
             __syncthreads();

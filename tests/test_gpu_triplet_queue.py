@@ -1,0 +1,65 @@
+"""The general triplet kernel's queue of binned pairs and its packed weighted histogram: lists around a queue's
+length, every work-group size and mode, and lists so long that an apex's pairs are taken in pieces and the packed
+counts are drained within it.  Counts equal the oracle's exactly; sums are exact integers, equal between geometries
+and to those of the pass with lists in device memory, which has neither queue nor packed planes."""
+import numpy as np
+import pytest
+
+import oracle as O
+from gramsci_amd import catalog as C
+from gramsci_amd.engine import Engine
+
+pytestmark = pytest.mark.gpu
+
+
+@pytest.fixture(scope="module")
+def eng():
+    e = Engine(0)
+    yield e
+    e.close()
+
+
+def _close(a, b):
+    # 1e-12 of the largest entry: the oracle adds the signed class sums in another order (no entry without data points)
+    b = np.asarray(b).reshape(np.shape(a))
+    fin = np.isfinite(b)
+    return np.all(np.abs(a - b)[fin] <= 1e-12 * np.max(np.abs(b[fin]), initial=0.0))
+
+
+@pytest.mark.parametrize("team", ["64", "128", "256"])
+@pytest.mark.parametrize("nmu,weighted,equi", [(1, True, False), (3, False, False), (3, True, False), (1, False, True),
+                                               (1, True, True), (2, True, True)])
+@pytest.mark.parametrize("n", [1, 2, 3, 12, 13, 24, 65, 130])
+def test_list_lengths(eng, monkeypatch, team, nmu, weighted, equi, n):
+    monkeypatch.setenv("GS_T3_WG", team)
+    rng = np.random.default_rng(n)
+    xyz = rng.uniform(0, 4.0, (n, 3)) + 20.0
+    w = C.lognormal_weights(n, 0.4, 7) if weighted else None
+    for buf in (None, (rng.random(n) < 0.3).astype(np.int32)):
+        p = O.Params(0.5, 5.0, 3, nmu, buf is not None)
+        ref = (O.pcf3_equi if equi else O.pcf3)(xyz, np.ones(n) if w is None else w, n // 3, p, buf=buf)
+        eng.set_catalogue(xyz, w, n // 3, buf)
+        run = eng.pcf3_equi if equi else eng.pcf3
+        a, b = (run(p.rmin, p.rmax, p.nbins, nmu, p.log_bins, prec) for prec in ("fp32", "fp64"))
+        assert np.array_equal(a["cnt"], b["cnt"]) and np.array_equal(a["cnt"].reshape(ref["cnt"].shape), ref["cnt"])
+        if weighted:
+            assert np.array_equal(a["wsum"], b["wsum"])
+            assert _close(a["n2"], ref["n2"])
+
+
+@pytest.mark.parametrize("nmu,weighted", [(1, True), (2, True), (2, False)])
+def test_long_lists(eng, monkeypatch, nmu, weighted):
+    # 1,500 points within reach of each other in one bin: 1.1 million pairs an apex, more than a piece, and more than
+    # 2^22 increments of a bin within four apexes; equal weights make every term the largest
+    rng = np.random.default_rng(21)
+    xyz = rng.uniform(0, 1.0, (1500, 3)) + 5.0
+    w = np.ones(1500) if weighted else None
+    eng.set_catalogue(xyz, w, 500, None)
+    a = eng.pcf3(0.0, 2.0, 1, nmu, False, "fp32")
+    monkeypatch.setenv("GS_T3_KMAX", "64")
+    monkeypatch.setenv("GS_T3_KMAX_LDS", "64")
+    b = eng.pcf3(0.0, 2.0, 1, nmu, False, "fp32")
+    assert a["cnt"].sum() == 1500 * 1499 * 1498 // 2
+    assert np.array_equal(a["cnt"], b["cnt"])
+    if weighted:
+        assert np.array_equal(a["wsum"], b["wsum"])
