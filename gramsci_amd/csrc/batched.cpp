@@ -583,7 +583,9 @@ static int batch_tune(gs_ctx* c, const gs_params& p, int kind, BatchTune* out)
         if (kv.first == key) { *out = kv.second; return GS_OK; }
     BatchTune best{};
     float tbest = 1e30f;
-    GsBatch::Plan* pbest = nullptr;
+    // the best plan's launch parameters: the plan itself is gone when a later candidate's grid outgrew the shared
+    // buffers, and with it the trials of its list lengths were (16 regions: 3.7 ms in half of the processes, 3.1 else)
+    int wg_best = kWG, kmax1_best = 0, kmax_best = 0;
     const char* ev_log = getenv("GS_TUNE_LOG");      // diagnostics: each candidate's time on stderr
     const bool log = ev_log && *ev_log && *ev_log != '0';
     auto trial = [&](const BatchTune& t) -> int {
@@ -600,13 +602,14 @@ static int batch_tune(gs_ctx* c, const gs_params& p, int kind, BatchTune* out)
         if (log)
             fprintf(stderr, "[gs tune] %dPCF m %d sx %d wg %d kmax1 %d: %.3f ms\n", kind, P->m, P->sx, P->wg1,
                     P->kmax1, ms);
-        if (ms < tbest) { tbest = ms; best = t; }
+        if (ms < tbest) {
+            tbest = ms;
+            best = t;
+            wg_best = P->wg1;
+            kmax1_best = P->kmax1;
+            kmax_best = P->kmax;
+        }
         return GS_OK;
-    };
-    auto best_plan = [&]() -> GsBatch::Plan* {
-        for (auto& pl : B.plans)
-            if (pl.kind == kind && same_params(pl.p, p) && pl.tune == best) return &pl;
-        return nullptr;
     };
     int rc;
     for (int m = kind == 2 ? 2 : 1; m <= (kind == 2 ? 6 : 3); ++m) {
@@ -632,8 +635,7 @@ static int batch_tune(gs_ctx* c, const gs_params& p, int kind, BatchTune* out)
             if ((rc = trial(t))) return rc;
         }
         b0 = best;
-        pbest = best_plan();
-        const int wg_auto = pbest ? pbest->wg1 : kWG;
+        const int wg_auto = wg_best;
         for (int wg : {64, 128, 256}) {
             if (wg == wg_auto) continue;
             BatchTune t = b0;
@@ -641,15 +643,12 @@ static int batch_tune(gs_ctx* c, const gs_params& p, int kind, BatchTune* out)
             if ((rc = trial(t))) return rc;
         }
         b0 = best;
-        pbest = best_plan();
-        if (pbest) {
-            const int k1 = pbest->kmax1, kx = pbest->kmax;
-            for (int cand : {k1 / 2 / 64 * 64, std::min(kx, k1 * 2)}) {
-                if (cand < 64 || cand == k1) continue;
-                BatchTune t = b0;
-                t.kmax1 = cand;
-                if ((rc = trial(t))) return rc;
-            }
+        const int k1 = kmax1_best, kx = kmax_best;
+        for (int cand : {k1 / 2 / 64 * 64, std::min(kx, k1 * 2)}) {
+            if (cand < 64 || cand == k1) continue;
+            BatchTune t = b0;
+            t.kmax1 = cand;
+            if ((rc = trial(t))) return rc;
         }
     }
     // keep only the winner's plan among this parameter set's
