@@ -328,15 +328,15 @@ int fill_pair_bins(const gs_params& p, const double* t64, const PairGrid& q, dou
     const double ew = fp64 ? 0.0 : std::ldexp(2.0 * q.ext + 2.0 * r, -24) * 1.01;
     const double g = fp64 ? std::ldexp(r * r, -50) : s_guard(r * r, ew);
     const double a = std::sqrt(3.0) * q.ext * 1.001, b = a + r * 1.001;
-    B.mu_ab = (float)((a + b) * 1.001);
-    B.mu_k0 = (float)(ms * 2.0 * std::ldexp(1.0, -20));
-    B.mu_k1a = (float)(ms * 2.0 * 2.0 * std::sqrt(3.0) * ew);
-    B.mu_k1b = (float)(ms * 2.0 * u * (a + b));
-    B.mu_k2a = (float)(ms * 4.0 * 0.5 * (9.0 * u * b * b + g) * r * r);
-    B.mu_k2b = (float)(ms * 4.0 * 3.0 * ew * ew);
+    B.mu_ab = (a + b) * 1.001;
+    B.mu_k0 = ms * 2.0 * std::ldexp(1.0, -20);
+    B.mu_k1a = ms * 2.0 * 2.0 * std::sqrt(3.0) * ew;
+    B.mu_k1b = ms * 2.0 * u * (a + b);
+    B.mu_k2a = ms * 4.0 * 0.5 * (9.0 * u * b * b + g) * r * r;
+    B.mu_k2b = ms * 4.0 * 3.0 * ew * ew;
     const bool in_range = fp64 ? (r > 1e-30 && xmax < 1e30 && q.ext < 1e30)
                                : (r > 1e-5 && r < 1e8 && xmax < 1e8 && q.ext < 1e8);
-    if (!in_range) B.mu_k0 = 1.0f;
+    if (!in_range) B.mu_k0 = 1.0;
     // the kernel's bin table has one entry past the last bin: the estimate of a pair that is not yet
     // rejected must not go beyond it
     const double top = std::sqrt((double)B.rej_hi);

@@ -47,8 +47,9 @@ struct BinDesc {
     float   mu_ew, mu_em, mu_c;    // mu guard: dt = ms*(mu_ew/|sep| + mu_em/|mid| + mu_c)
     // mu guard of the pair kernel (fill_pair_bins): the error of t is at most k0 + k1 q + k2 q^2 with
     // k1 = mu_k1a Sx + mu_k1b (2 rho + 3 mu_ab), k2 = mu_k2a + mu_k2b Sx^2, Sx = 2 rho + mu_ab and rho
-    // the distance of the chunk's reference point from the origin
-    float   mu_k0, mu_k1a, mu_k1b, mu_k2a, mu_k2b, mu_ab;
+    // the distance of the chunk's reference point from the origin.  In FP64: mu_k2a goes as rmax^4, which leaves the
+    // range of a float below an rmax of 1e-8, and FP64 geometry is held to the bound down to 1e-30.
+    double  mu_k0, mu_k1a, mu_k1b, mu_k2a, mu_k2b, mu_ab;
     int32_t wide;                  // the FP32 guard bands are too wide for the bin table
     // weighted fixed point.  Pairs: each point's weight is scaled by 2^fx_sd (data) or 2^fx_sr
     // (randoms), so that every scaled weight of its class is below 2^26, and a pair contributes

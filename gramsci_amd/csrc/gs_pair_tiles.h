@@ -172,11 +172,11 @@ struct Binner {
     __device__ __forceinline__ void chunk(const BinDesc& B, double p2)
     {
         if constexpr (RSD) {
-            const float rho = (float)sqrt(p2) * 1.001f;
-            const float sx = 2.0f * rho + B.mu_ab;
-            l0 = (R)(0.5f - B.mu_k0);
-            l1 = (R)(-(B.mu_k1a * sx + B.mu_k1b * (2.0f * rho + 3.0f * B.mu_ab)));
-            l2 = (R)(-(B.mu_k2a + B.mu_k2b * sx * sx));
+            const R rho = (R)sqrt(p2) * (R)1.001, ab = (R)B.mu_ab;
+            const R sx = (R)2.0 * rho + ab;
+            l0 = (R)0.5 - (R)B.mu_k0;
+            l1 = -((R)B.mu_k1a * sx + (R)B.mu_k1b * ((R)2.0 * rho + (R)3.0 * ab));
+            l2 = -((R)B.mu_k2a + (R)B.mu_k2b * sx * sx);
         }
     }
     __device__ __forceinline__ R separation2(const Pt<R>& A, R ex, R ey, R ez) const
