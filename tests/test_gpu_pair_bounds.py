@@ -33,3 +33,32 @@ def test_midpoints_at_the_origin(eng, scale, eps):
     for prec in ("fp32", "fp64"):
         r = eng.pcf2(p.rmin, p.rmax, p.nbins, p.nmu, p.log_bins, prec)
         assert np.array_equal(r["cnt"], ref["cnt"]), prec
+
+
+@pytest.mark.parametrize("weighted,buffered,nmu", [(True, False, 4), (False, False, 1), (True, True, 3)])
+@pytest.mark.parametrize("share", [0.02, 0.5])
+def test_points_that_are_not_numbers(eng, weighted, buffered, nmu, share):
+    # a point with a NaN coordinate has no pairs, as in the reference's arithmetic (no comparison with NaN holds), and
+    # takes none from the points beside it in its chunk
+    rng = np.random.default_rng(5)
+    n = 3000
+    xyz = rng.uniform(0, 25.0, (n, 3))
+    w = rng.uniform(0.5, 2.0, n) if weighted else None
+    buf = (rng.random(n) < 0.3).astype(np.int32) if buffered else None
+    for axis in range(3):
+        bad = rng.random(n) < share
+        bad[:2] = False
+        x = xyz.copy()
+        x[bad, axis] = np.nan
+        g = ~bad
+        p = O.Params(0.5, 5.0, 4, nmu, False)
+        ref = O.pcf2(xyz[g], None if w is None else w[g], int(g[:1000].sum()), p, buf=None if buf is None else buf[g])
+        eng.set_catalogue(x, w, 1000, buf)
+        for prec in ("fp32", "fp64"):
+            r = eng.pcf2(p.rmin, p.rmax, p.nbins, p.nmu, p.log_bins, prec)
+            assert np.array_equal(r["cnt"], ref["cnt"]), (axis, prec)
+            assert np.allclose(r["wsum"], ref["wsum"], rtol=1e-12, atol=0.0)
+        if weighted:
+            # no pairs, no gradient but that of the normalisation: dL/dwn of such a point is 0
+            ga, gb = (eng.adjoint2(np.ones((4, nmu)), np.zeros((4, nmu)), 0.5, 5.0, 4, nmu, False, prec) for prec in ("fp32", "fp64"))
+            assert np.all(np.isfinite(ga)) and np.max(np.abs(ga - gb)) <= 1e-11 * np.max(np.abs(gb))
