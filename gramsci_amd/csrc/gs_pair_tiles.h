@@ -22,10 +22,10 @@ __device__ __forceinline__ double rsq(double x) { return __builtin_amdgcn_rsq(x)
 __device__ __forceinline__ float fract(float x) { return __builtin_amdgcn_fractf(x); }
 __device__ __forceinline__ double fract(double x) { return __builtin_amdgcn_fract(x); }
 
-// v truncated to an unsigned integer, 0 for a negative v (the conversion saturates)
-__device__ __forceinline__ int cvt_sat(float v)
+// v truncated to an unsigned integer, 0 for a negative v or NaN, 2^32 - 1 for one beyond it (the conversion saturates)
+__device__ __forceinline__ unsigned cvt_sat(float v)
 {
-    int r;
+    unsigned r;
     asm("v_cvt_u32_f32 %0, %1" : "=v"(r) : "v"(v));
     return r;
 }
@@ -199,7 +199,8 @@ struct Binner {
     {
         bool safe = true;
         if constexpr (FP64) {
-            b = min(cvt_sat(bin_estimate((float)s, LOGB, ua, ub)), nb - 1);
+            // as unsigned: s may be beyond a float's range, and its estimate 2^32 - 1
+            b = (int)min(cvt_sat(bin_estimate((float)s, LOGB, ua, ub)), (unsigned)(nb - 1));
             const double* t = (const double*)table;
             if (!(s >= t[b] && s < t[b + 1])) {
                 while (b > 0 && s < t[b]) --b;
@@ -207,7 +208,7 @@ struct Binner {
                 if (b == nb) return kPairOverflow;
             }
         } else {
-            b = cvt_sat(bin_estimate(s, LOGB, ua, ub));
+            b = (int)cvt_sat(bin_estimate(s, LOGB, ua, ub));
             const float2 ok = ((const float2*)table)[b];
             safe = __float_as_uint(s - ok.x) < __float_as_uint(ok.y);
         }

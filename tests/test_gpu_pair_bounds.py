@@ -62,3 +62,17 @@ def test_points_that_are_not_numbers(eng, weighted, buffered, nmu, share):
             # no pairs, no gradient but that of the normalisation: dL/dwn of such a point is 0
             ga, gb = (eng.adjoint2(np.ones((4, nmu)), np.zeros((4, nmu)), 0.5, 5.0, 4, nmu, False, prec) for prec in ("fp32", "fp64"))
             assert np.all(np.isfinite(ga)) and np.max(np.abs(ga - gb)) <= 1e-11 * np.max(np.abs(gb))
+
+
+@pytest.mark.parametrize("rmax", [1.7e19, 1.9e19, 3e25, 1e60])
+@pytest.mark.parametrize("log", [False, True])
+@pytest.mark.parametrize("nmu", [1, 5])
+def test_squared_distances_beyond_float(eng, rmax, log, nmu):
+    # above 1.8e19 no float holds a squared distance: the bin's estimate is infinite, and has to stay within the table
+    rng = np.random.default_rng(12)
+    xyz = rng.uniform(0, 3.0, (600, 3)) * rmax
+    p = O.Params(0.1 * rmax, rmax, 6, nmu, log)
+    ref = O.pcf2(xyz, None, 250, p)
+    eng.set_catalogue(xyz, None, 250)
+    for prec in ("fp32", "fp64"):
+        assert np.array_equal(eng.pcf2(p.rmin, p.rmax, 6, nmu, log, prec)["cnt"], ref["cnt"]), prec
