@@ -337,12 +337,14 @@ int fill_pair_bins(const gs_params& p, const double* t64, const PairGrid& q, dou
     const bool in_range = fp64 ? (r > 1e-30 && xmax < 1e30 && q.ext < 1e30)
                                : (r > 1e-5 && r < 1e8 && xmax < 1e8 && q.ext < 1e8);
     if (!in_range) B.mu_k0 = 1.0;
-    // the kernel's bin table has one entry past the last bin: the estimate of a pair that is not yet
-    // rejected must not go beyond it
-    const double top = std::sqrt((double)B.rej_hi);
-    const double est = p.log_bins ? (std::log10(top) - std::log10(p.rmin)) / (std::log10(r) - std::log10(p.rmin)) * p.nbins
-                                  : (top - p.rmin) / (r - p.rmin) * p.nbins;
-    B.wide = !(est < p.nbins + 0.9) || r > 1e8 || q.ext > 1e8;
+    // The kernel's bin table has one entry past the last bin: the estimate of a pair that is not yet rejected must
+    // not go beyond it.  The largest such s, the estimate with the kernel's rounded constants, and its error: the
+    // square root or logarithm and the FMA, 2^-21 of each term (in a narrow range of bins the terms are large and
+    // nearly cancel: 100 log bins in the last 1e-4 of rmax are estimated 0.23 too high).
+    const double top = (double)B.rej_hi + std::ldexp(std::fabs((double)B.rej_hi) + std::fabs((double)B.rej_lo), -22);
+    const double fs = p.log_bins ? std::log2(top) : std::sqrt(top), ua = B.ua, ub = B.ub;
+    const double err = std::ldexp(std::fabs(ua) * (std::fabs(fs) + (p.log_bins ? 1.0 : 0.0)) + std::fabs(ub), -21);
+    B.wide = !(ua * fs + ub + err < p.nbins + 0.9) || r > 1e8 || q.ext > 1e8;
     return GS_OK;
 }
 

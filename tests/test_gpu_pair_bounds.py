@@ -76,3 +76,25 @@ def test_squared_distances_beyond_float(eng, rmax, log, nmu):
     eng.set_catalogue(xyz, None, 250)
     for prec in ("fp32", "fp64"):
         assert np.array_equal(eng.pcf2(p.rmin, p.rmax, 6, nmu, log, prec)["cnt"], ref["cnt"]), prec
+
+
+@pytest.mark.parametrize("rel", [1e-2, 1e-3, 1.35e-4, 1.02e-4, 1e-5])
+@pytest.mark.parametrize("log", [False, True])
+@pytest.mark.parametrize("nbins,nmu", [(100, 1), (127, 1), (20, 6)])
+def test_narrow_ranges_of_bins(eng, rel, log, nbins, nmu):
+    # the FP32 estimate of a bin is off by a sizeable part of it, or by more: FP64 geometry takes over
+    rng = np.random.default_rng(14)
+    xyz = rng.uniform(0, 100.0, (3000, 3))
+    w = rng.uniform(0.5, 2.0, 3000)
+    p = O.Params(88.8 * (1.0 - rel), 88.8, nbins, nmu, log)
+    ref = O.pcf2(xyz, w, 1000, p)
+    eng.set_catalogue(xyz, w, 1000)
+    for prec in ("fp32", "fp64"):
+        r = eng.pcf2(p.rmin, p.rmax, nbins, nmu, log, prec)
+        assert np.array_equal(r["cnt"], ref["cnt"]) and r["stats"]["n_overflow"] == ref["overflow"], prec
+    g2, g3 = rng.normal(size=(2, nbins, nmu))
+    ref = O.adjoint2(xyz, w, 1000, p, g2, g3)
+    for prec in ("fp32", "fp64"):
+        got = eng.adjoint2(g2, g3, p.rmin, p.rmax, nbins, nmu, log, prec)
+        # terms rounded to 2^-50 of the largest, at most 3000 a point
+        assert np.max(np.abs(got - ref)) <= 1e-11 * np.max(np.abs(ref)), prec
