@@ -46,8 +46,9 @@ __device__ __forceinline__ int below(unsigned long long m)
     return (int)__builtin_amdgcn_mbcnt_hi((unsigned)(m >> 32), __builtin_amdgcn_mbcnt_lo((unsigned)m, 0u));
 }
 
-// far away in the geometry's precision: missing apexes and entries
-template <class R> constexpr R far_away() { return std::is_same<R, double>::value ? (R)1e150 : (R)1e18f; }
+// x of missing apexes (entries: negative), farther from every point than any rmax: FP32 geometry runs up to 1e8, FP64
+// as long as rmax^2 is finite (an infinite squared distance is rejected like any other)
+template <class R> constexpr R far_away() { return std::is_same<R, double>::value ? (R)INFINITY : (R)1e18f; }
 
 // A point in the kernel's geometry: FP32 relative to the chunk's reference point p, FP64 absolute.
 template <class R>

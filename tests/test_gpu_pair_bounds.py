@@ -98,3 +98,16 @@ def test_narrow_ranges_of_bins(eng, rel, log, nbins, nmu):
         got = eng.adjoint2(g2, g3, p.rmin, p.rmax, nbins, nmu, log, prec)
         # terms rounded to 2^-50 of the largest, at most 3000 a point
         assert np.max(np.abs(got - ref)) <= 1e-11 * np.max(np.abs(ref)), prec
+
+
+@pytest.mark.parametrize("rmax", [1e148, 1e150, 1e151, 1e153])
+@pytest.mark.parametrize("nmu", [1, 4])
+def test_largest_rmax(eng, rmax, nmu):
+    # up to the largest rmax with a finite square: the lanes without a point are beyond it
+    rng = np.random.default_rng(15)
+    xyz = rng.uniform(0, 3.0, (300, 3)) * rmax
+    p = O.Params(0.1 * rmax, rmax, 3, nmu, nmu > 1)
+    ref = O.pcf2(xyz, None, 100, p)
+    eng.set_catalogue(xyz, None, 100)
+    for prec in ("fp32", "fp64"):
+        assert np.array_equal(eng.pcf2(p.rmin, p.rmax, 3, nmu, p.log_bins, prec)["cnt"], ref["cnt"]), prec
