@@ -223,6 +223,7 @@ struct QuadArgs {
     const int32_t* items;
     const int32_t* n_items_dev; // if set, the number of work items is read here
     int32_t batch;              // apexes taken per queue fetch (0: 1)
+    int32_t bin_masks;          // a mask per bin and neighbour of the quads' last points, else one per neighbour
     int32_t lds_w;              // weighted sums in LDS (else global atomics; device-memory lists: always those)
     // as for the triplet kernel: with ovf_kmax set, the largest neighbour count of a queued apex is
     // kept there; with glist set, each work-group keeps its apex's neighbour list (kmax entries, a

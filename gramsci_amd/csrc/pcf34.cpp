@@ -540,10 +540,10 @@ static int count4(gs_ctx* c, const gs_params* p, bool tetra, uint64_t* cnt, doub
     if ((rc = ctx_thresholds(c, *p, t64)) || (rc = fill_bins(*p, t64, 1.5 * p->rmax, ctx_xmax(c), v.wmax_d, v.wmax_r, B))) return rc;
     std::vector<uint16_t> tab = tetra ? std::vector<uint16_t>() : table4(nb);
 
-    // LDS plan of the last LDS pass: the longest list (64, 128 or 256, with its K x K matrix of links and its masks)
-    // that fits gfx950's 160 KiB of LDS per work-group beside the tables and, where it fits in 16 KiB, the count
-    // histogram.  Apexes with more neighbours go to a last pass with device-memory lists, so no neighbour count is
-    // refused.
+    // LDS plan of the last LDS pass: the longest list (64, 128 or 256, with its K x K matrix of links and the fewest
+    // masks) that fits gfx950's 160 KiB of LDS per work-group beside the tables and, where it fits in 16 KiB, the count
+    // histogram: 256 up to 14 bins (tetrahedra: always), 128 above.  Apexes with more neighbours go to a last pass with
+    // device-memory lists, so no neighbour count is refused.
     const size_t budget = 160 * 1024 - 256;     // less the kernel's static part
     QuadArgs a{};
     a.tetra = tetra ? 1 : 0;
@@ -661,6 +661,10 @@ static int count4(gs_ctx* c, const gs_params* p, bool tetra, uint64_t* cnt, doub
     auto with_sums = [&](int km, bool wv) {
         QuadArgs t = a;
         t.kmax = km;
+        // a mask per bin where that fits the same list (6,000 points with 180 neighbours: 8 bins 3.7 ms, with one mask
+        // 5.3; 4 bins 4.3, 6.5); else one mask (10 bins 5.0 ms; lists of 128, and longer ones in device memory, 41)
+        t.bin_masks = tetra ? 0 : 1;
+        if (quad4_lds_bytes(t, nb, weighted, wv) > budget) t.bin_masks = 0;
         t.lds_w = weighted ? 1 : 0;
         if (quad4_lds_bytes(t, nb, weighted, wv) > 80 * 1024) t.lds_w = 0;
         return t;

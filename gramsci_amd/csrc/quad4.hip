@@ -43,7 +43,7 @@ using namespace dev;
 namespace {
 
 struct QuadLds {
-    size_t t64, tab, hist, sums, lists, team, total;
+    size_t t64, tab, hist, sums, lists, masks, rows, team, total;
 };
 
 // km: list entries (64, 128, 256); teams of a work-group; big: k_quad4_big, without lists
@@ -52,7 +52,7 @@ __host__ __device__ inline QuadLds quad_lds(const QuadArgs& a, int nb, bool weig
     QuadLds l;
     size_t b = 0;
     l.t64 = b;
-    b += ((size_t)(kMaxBins + 2) * 8 + 15) / 16 * 16;
+    b += ((size_t)(nb + 2) * 8 + 15) / 16 * 16;
     l.tab = b;
     if (!a.tetra) b += ((size_t)nb * nb * nb * nb * 2 + 15) / 16 * 16;      // perimeter table
     l.hist = b;
@@ -60,10 +60,14 @@ __host__ __device__ inline QuadLds quad_lds(const QuadArgs& a, int nb, bool weig
     l.sums = b;
     if (weighted && a.lds_w && !big) b += (size_t)a.ncell * 40 * 8;
     l.lists = b;
-    // coordinates, later the masks; weights; original index; sorted index; bins, random flags; links; stencil rows
-    const size_t nw = km / 64, masks = 8 * nw * (1 + nb);
-    l.team = big ? 0 : km * ((masks > 24 ? masks : 24) + (weighted ? 8 : 0) + 4 + 4 + 2) + (size_t)km * (km + 4);
-    l.team += ((size_t)a.nrows * 12 + 15) / 16 * 16;
+    // stencil rows (after the links where they are longer), then coordinates, beside them original and sorted index,
+    // later the masks; weights; bins, random flags; links
+    const size_t per = (size_t)km / 8 * (a.tetra ? 1 : 1 + (a.bin_masks ? nb : 1));
+    const size_t rows = ((size_t)a.nrows * 12 + 15) / 16 * 16;
+    l.masks = km * (per > 32 ? per : 32);
+    l.team = big ? 0 : l.masks + km * ((weighted ? 8 : 0) + 2) + (size_t)km * (km + 4);
+    l.rows = !big && rows <= (size_t)km * 24 ? 0 : l.team;
+    if (l.rows == l.team) l.team += rows;
     l.total = b + teams * l.team;
     return l;
 }
@@ -385,18 +389,20 @@ __global__ __launch_bounds__(kWG) void k_quad4_big(QuadArgs a)
 // are masks of NW 64-bit words:
 //   M[u]     the neighbours k > u linked to u (a kept side);
 //   T[b][v]  the neighbours k > v with b <= ind5 <= ind3 (ind5 the bin of their side to v, ind3 that of their side to
-//            the apex; tetra: ind5 = ind3 = b),
-// so that the k3 of all quads of a linked pair (u, v) are the bits of T[ind4][v] & M[u] (tetra: & T[ind4][u]).  They
+//            the apex),
+// so that the k3 of all quads of a linked pair (u, v) are the bits of T[ind4][v] & M[u].  Those are BIN's 1 + nb
+// masks a neighbour.  Without BIN there is one T[v], of 1 <= ind5 <= ind3, and ind5 >= ind4 is tested bit by bit; or
+// (tetra) T[v] alone, of ind5 = ind3 = ind2, the one bin of all sides, and the k3 are the bits of T[v] & T[u].  The masks
 // come from the rows of link bytes, four at a time: with bytes below 128, (x | 0x80) - y keeps bit 7 exactly where
 // x >= y, and a dot product of the bytes' bits packs them.  Sums of weighted quads go to LDS where they fit (a.lds_w).
-template <bool W, int NW, bool WAVE>
+template <bool W, int NW, bool WAVE, bool BIN>
 __global__ __launch_bounds__(kWG) void k_quad4(QuadArgs a)
 {
     static_assert(!WAVE || (NW == 1 && !W), "a wave holds one neighbour per lane");
     extern __shared__ __align__(16) unsigned char smem[];
     const BinDesc& B = *a.bins;
     const int nb = scalar(B.nb), nb2 = nb * nb, ncell = a.ncell;
-    const bool lh = a.lds_hist != 0, lw = W && a.lds_w != 0, tetra = a.tetra != 0;
+    const bool lh = a.lds_hist != 0, lw = W && a.lds_w != 0, tetra = !BIN && a.tetra != 0;
     const int tid = threadIdx.x, lane = tid & 63, wv = scalar(tid >> 6);
     constexpr int teams = WAVE ? kWG / kWave : 1, tn = WAVE ? kWave : kWG, KM = 64 * NW, LD = KM + 4;
     const int tl = WAVE ? lane : tid;
@@ -411,23 +417,23 @@ __global__ __launch_bounds__(kWG) void k_quad4(QuadArgs a)
     uint32_t* hc = (uint32_t*)(smem + l.hist);
     double* hw = (double*)(smem + l.sums);  // [ncell][16] products, [6][ncell][4] disc terms
     unsigned char* p = smem + l.lists + (WAVE ? wv : 0) * l.team;
-    double* xs = (double*)p;                // the sorted neighbours; from step 3b on the masks
+    int32_t* rw_js = (int32_t*)(p + l.rows);
+    int32_t* rw_len = rw_js + a.nrows;
+    int32_t* rw_off = rw_len + a.nrows;
+    double* xs = (double*)p;                // the sorted neighbours, their indices; from step 3b on the masks
     double* ys = xs + KM;
     double* zs = ys + KM;
-    unsigned long long* M = (unsigned long long*)p;     // [NW][KM]
-    unsigned long long* T = M + NW * KM;                // [nb][NW][KM]
-    p += (size_t)KM * max(24, 8 * NW * (1 + nb));
+    int32_t* key = (int32_t*)(zs + KM);
+    int32_t* jl = key + KM;
+    unsigned long long* M = (unsigned long long*)p;     // [NW][KM] (not tetra)
+    unsigned long long* T = M + (tetra ? 0 : NW * KM);  // [BIN: nb][NW][KM]
+    p += l.masks;
     double* ws = (double*)p;
     if (W) p += KM * 8;
-    int32_t* key = (int32_t*)p;
-    int32_t* jl = key + KM;
-    uint8_t* A = (uint8_t*)(jl + KM);       // bin + 1 of the apex's sides
+    uint8_t* A = (uint8_t*)p;               // bin + 1 of the apex's sides
     uint8_t* rnd = A + KM;                  // random points
     uint8_t* L = rnd + KM;                  // [KM][LD] bin + 1 of side (u, v), u < v; 0: not kept.  An odd number of
                                             // words a row: lanes reading a column fall on all banks
-    int32_t* rw_js = (int32_t*)(L + KM * LD);
-    int32_t* rw_len = rw_js + a.nrows;
-    int32_t* rw_off = rw_len + a.nrows;
 
     __shared__ int s_item, s_k, s_ncand;
     if (lh)
@@ -630,12 +636,16 @@ __global__ __launch_bounds__(kWG) void k_quad4(QuadArgs a)
                     return (((unsigned long long)hi << 32) | lo) & above;
                 };
                 constexpr uint32_t kHigh = 0x80808080u, kOne = 0x01010101u;
+                if (tetra) {
+                    const uint32_t bb = A[tl] * kOne;
+                    T[w * KM + tl] = mask_of([&](uint32_t x, uint32_t y) { return ~(((x ^ bb) | (y ^ bb)) + 0x7f7f7f7fu); });
+                    continue;
+                }
                 M[w * KM + tl] = mask_of([&](uint32_t x, uint32_t) { return x + 0x7f7f7f7fu; });
-                for (int b = 1; b <= nb; ++b) {
+                for (int b = 1; b <= (BIN ? nb : 1); ++b) {
                     const uint32_t bb = (uint32_t)b * kOne;
-                    T[((b - 1) * NW + w) * KM + tl] = tetra ? mask_of([&](uint32_t x, uint32_t y) {
-                        return ~(((x ^ bb) | (y ^ bb)) + 0x7f7f7f7fu);
-                    }) : mask_of([&](uint32_t x, uint32_t y) { return ((y | kHigh) - x) & ((x | kHigh) - bb); });
+                    T[((b - 1) * NW + w) * KM + tl] =
+                        mask_of([&](uint32_t x, uint32_t y) { return ((y | kHigh) - x) & ((x | kHigh) - bb); });
                 }
             }
         }
@@ -651,8 +661,8 @@ __global__ __launch_bounds__(kWG) void k_quad4(QuadArgs a)
                 if (ind4 && (!tetra || (ind2 == ind1 && ind4 == ind1))) {       // tetra: gramsci.F90:564-567
                     units += (unsigned)(K - 1 - v);
                     // perimeters that do not begin ind1 <= ind4 have no configuration (:701)
-                    const unsigned long long* Tv = T + (size_t)(ind4 - 1) * NW * KM;
-                    const unsigned long long* Mu = (tetra ? Tv : M) + u;
+                    const unsigned long long* Tv = T + (BIN ? (size_t)(ind4 - 1) * NW * KM : 0);
+                    const unsigned long long* Mu = (tetra ? T : M) + u;
                     if (ind4 >= ind1)
                         for (int w = NW == 1 ? 0 : (v + 1) >> 6; w < NW; ++w) {
                             unsigned long long m = Tv[w * KM + v] & Mu[w * KM];
@@ -660,6 +670,7 @@ __global__ __launch_bounds__(kWG) void k_quad4(QuadArgs a)
                                 const int k3 = 64 * w + (int)__builtin_ctzll(m);
                                 m &= m - 1;
                                 const int ind5 = L[v * LD + k3], ind6 = L[u * LD + k3], ind3 = A[k3];
+                                if (!BIN && ind5 < ind4) continue;
                                 const int r1 = rnd[u], r2 = rnd[v], r3 = rnd[k3];
                                 int cell = ind1 - 1;
                                 if (!tetra) {
@@ -723,13 +734,19 @@ __global__ __launch_bounds__(kWG) void k_quad4(QuadArgs a)
     if (tid < 5 && s_stat[tid]) atomicAdd(&a.out_stats[copy + tid], s_stat[tid]);
 }
 
+template <bool BIN>
+static void (*quad_kernel_lds(const QuadArgs& a, bool weighted, bool wave))(QuadArgs)
+{
+    if (wave) return k_quad4<false, 1, true, BIN>;      // unit weights
+    if (a.kmax <= 64) return weighted ? k_quad4<true, 1, false, BIN> : k_quad4<false, 1, false, BIN>;
+    if (a.kmax <= 128) return weighted ? k_quad4<true, 2, false, BIN> : k_quad4<false, 2, false, BIN>;
+    return weighted ? k_quad4<true, 4, false, BIN> : k_quad4<false, 4, false, BIN>;
+}
+
 static void (*quad_kernel(const QuadArgs& a, bool weighted, bool wave))(QuadArgs)
 {
     if (a.glist) return weighted ? k_quad4_big<true> : k_quad4_big<false>;
-    if (wave) return k_quad4<false, 1, true>;       // unit weights
-    if (a.kmax <= 64) return weighted ? k_quad4<true, 1, false> : k_quad4<false, 1, false>;
-    if (a.kmax <= 128) return weighted ? k_quad4<true, 2, false> : k_quad4<false, 2, false>;
-    return weighted ? k_quad4<true, 4, false> : k_quad4<false, 4, false>;
+    return a.bin_masks ? quad_kernel_lds<true>(a, weighted, wave) : quad_kernel_lds<false>(a, weighted, wave);
 }
 
 size_t quad4_lds_bytes(const QuadArgs& a, int nb, bool weighted, bool wave)

@@ -92,3 +92,16 @@ def test_largest_tables(eng):
         out = eng.pcf4(1.0, 6.0, 16, False, cell_div=div)
         assert np.array_equal(out["cnt"], ref["cnt"]) and out["stats"]["n_units"] == ref["n_quads"], div
         assert _close(out["n3"], ref["n3"]) and _close_disc(out["disc_r"], ref["disc_r"])
+
+
+@pytest.mark.parametrize("weighted", [False, True])
+@pytest.mark.parametrize("nbins,tetra", [(9, False), (10, False), (14, False), (16, False), (11, True), (40, True), (127, True)])
+@pytest.mark.parametrize("n", [60, 129, 200])
+def test_many_bins(eng, weighted, nbins, tetra, n):
+    # lists for which no mask per bin fits the LDS: one mask a neighbour, or (tetrahedra) always one, their bins so wide
+    # that the first few hold all sides
+    rng = np.random.default_rng(n + nbins)
+    xyz = rng.uniform(0, 4.0, (n, 3))
+    w = np.exp(rng.normal(0, 0.3, n)) if weighted else np.ones(n)
+    p = O.Params(0.5, 0.5 + 1.2 * nbins, nbins, 1, False) if tetra else O.Params(2.6, 7.0, nbins, 1, False)
+    _check(eng, xyz, w, n // 3, p, tetra)
