@@ -581,7 +581,7 @@ static int count4(gs_ctx* c, const gs_params* p, bool tetra, uint64_t* cnt, doub
     constexpr int kPasses = 3;
     constexpr size_t kQueueInts = 64 * kQueuePad, kHeadInts = kPasses * kQueueInts + 64;
     const size_t clear = kHeadInts * 4 + (size_t)copies * words * 8;
-    if ((rc = X.params.reserve(blob)) || (rc = X.big_zero.reserve(clear)) || (rc = X.out.reserve(words)) ||
+    if ((rc = X.params.reserve(blob)) || (rc = X.big_zero.reserve(clear)) || (copies > 1 && (rc = X.out.reserve(words))) ||
         (rc = H.reserve(res_off + 64)))
         return rc;
     *(BinDesc*)H.ptr = B;
@@ -619,6 +619,7 @@ static int count4(gs_ctx* c, const gs_params* p, bool tetra, uint64_t* cnt, doub
     const int n = a.n_items;
     int kmax1 = kmax;
     double short_lists = 0.0;
+    bool long_lists = false;        // a last pass is to be expected
     const int nsample = std::min(n, 2048);
     const int stride = nsample > 0 ? n / nsample : 1;
     // i32: the lists of queued apexes, then the sampled neighbour counts
@@ -646,6 +647,7 @@ static int count4(gs_ctx* c, const gs_params* p, bool tetra, uint64_t* cnt, doub
             const size_t q = std::min(ks.size() - 1, (size_t)std::ceil(0.995 * (ks.size() - 1)));
             std::nth_element(ks.begin(), ks.begin() + q, ks.end());
             const double want = 1.05 * ks[q];
+            long_lists = ks[q] > kmax;
             kmax1 = 64;
             while (kmax1 < kmax && kmax1 < want) kmax1 *= 2;
         }
@@ -701,23 +703,38 @@ static int count4(gs_ctx* c, const gs_params* p, bool tetra, uint64_t* cnt, doub
         e = launch_quad4(t, nb, weighted, wv, nblk, v.stream);
         if (e != hipSuccess) return hip_fail(e, "4PCF kernel launch");
     }
-    // the copies' sum; once more after a last pass, over the apexes whose neighbours outnumber every LDS list, with
-    // their lists in device memory (one per work-group; no link matrix)
+    (void)hipEventRecord(v.ev[3], v.stream);
+    // the host makes its buffer (16 bins: 127 MB, 20 ms) beside the last kernels to run
+    std::vector<unsigned long long> h_out;
+    if (!long_lists) h_out.resize(words);
     int32_t* const h_cnt = (int32_t*)(H.ptr + res_off);
     int32_t* const last = d_cnt + 4 * (np - 1);
-    std::vector<unsigned long long> h_out(words);
-    for (int pass = 0;; ++pass) {
-        (void)hipEventRecord(v.ev[3], v.stream);
-        e = launch_sum_copies(out, copies, words, (int64_t)ncnt, 0, 8, X.out.ptr, v.stream);
-        if (e == hipSuccess)
-            e = launch_sum_copies_f64(a.out_w, copies, words, (int64_t)nw, (double*)(X.out.ptr + ncnt + 8), v.stream);
-        if (e == hipSuccess)
-            e = hipMemcpyAsync(h_out.data(), X.out.ptr, (size_t)words * 8, hipMemcpyDeviceToHost, v.stream);
-        if (e == hipSuccess) e = hipMemcpyAsync(h_cnt, last, 2 * sizeof(int32_t), hipMemcpyDeviceToHost, v.stream);
-        if (e == hipSuccess) e = hipMemcpyAsync(h_cnt + 2, a.err, sizeof(int32_t), hipMemcpyDeviceToHost, v.stream);
-        if (e == hipSuccess) e = hipStreamSynchronize(v.stream);
-        if (e != hipSuccess) return hip_fail(e, "4PCF kernel");
-        if (pass > 0 || h_cnt[0] <= 0) break;
+    auto counters = [&]() {         // apexes left to a last pass, their largest neighbour count, the error flag
+        hipError_t r = hipMemcpyAsync(h_cnt, last, 2 * sizeof(int32_t), hipMemcpyDeviceToHost, v.stream);
+        if (r == hipSuccess) r = hipMemcpyAsync(h_cnt + 2, a.err, sizeof(int32_t), hipMemcpyDeviceToHost, v.stream);
+        return r;
+    };
+    auto results = [&]() {          // the copies' sum
+        h_out.resize(words);
+        hipError_t r = hipSuccess;
+        if (copies > 1) {
+            r = launch_sum_copies(out, copies, words, (int64_t)ncnt, 0, 8, X.out.ptr, v.stream);
+            if (r == hipSuccess)
+                r = launch_sum_copies_f64(a.out_w, copies, words, (int64_t)nw, (double*)(X.out.ptr + ncnt + 8), v.stream);
+        }
+        if (r == hipSuccess)
+            r = hipMemcpyAsync(h_out.data(), copies > 1 ? X.out.ptr : out, (size_t)words * 8, hipMemcpyDeviceToHost, v.stream);
+        return r;
+    };
+    // one wait for both where there are copies; a large result (16 bins: 30 ms) is fetched once, when it is complete
+    e = counters();
+    if (e == hipSuccess && copies > 1) e = results();
+    if (e == hipSuccess) e = hipStreamSynchronize(v.stream);
+    if (e != hipSuccess) return hip_fail(e, "4PCF kernel");
+    const bool big = h_cnt[0] > 0;
+    if (big) {
+        // a last pass, over the apexes whose neighbours outnumber every LDS list, with their lists in device memory
+        // (one per work-group; no link matrix)
         QuadArgs a3 = a;
         a3.items = X.i32.ptr + (size_t)(np - 1) * n;
         a3.n_items = h_cnt[0];
@@ -737,7 +754,12 @@ static int count4(gs_ctx* c, const gs_params* p, bool tetra, uint64_t* cnt, doub
         e = launch_fill_u32(head, kQueueInts, 0u, v.stream);
         if (e == hipSuccess) e = launch_quad4(a3, nb, weighted, false, nblk3, v.stream);
         if (e != hipSuccess) return hip_fail(e, "4PCF device-memory pass");
+        (void)hipEventRecord(v.ev[3], v.stream);
+        e = counters();
     }
+    if (e == hipSuccess && (big || copies == 1)) e = results();
+    if (e == hipSuccess) e = hipStreamSynchronize(v.stream);
+    if (e != hipSuccess) return hip_fail(e, "4PCF kernel");
     if (h_cnt[2]) return fail(GS_EHIP, "4PCF: an apex's neighbour list overflowed with no later pass (internal error)");
     const double* const h_w = (const double*)(h_out.data() + ncnt + 8);
 
