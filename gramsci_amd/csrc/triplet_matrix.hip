@@ -49,8 +49,9 @@ constexpr int kMatrixMaxWG = 512;
 constexpr int kControlBytes = 64;       // work item, list counters, statistics
 constexpr int kListWords = 6;           // per list entry: x, y, z, |.|^2, its two tags (16 bits each), sorted index
 
-// LDS by byte address.  The kernel's LDS is all dynamic, so the array starts at address 0; through the array's name
-// the compiler adds that zero to every address it forms.
+// LDS by byte address.  The kernel's LDS is all dynamic, so the array starts at address 0 (the launch refuses a kernel
+// with static LDS, which a helper could bring with it); through the array's name the compiler adds that zero to every
+// address it forms.
 template <class T>
 using lds_ptr = __attribute__((address_space(3))) T*;
 
@@ -437,8 +438,12 @@ hipError_t launch_triplet_matrix(const TripArgs& a, int nb, bool wave, int nbloc
 {
     const size_t lds = triplet_matrix_lds(a, nb, wave ? a.wg / kWave : 1);
     return with_matrix(a.log_bins != 0, wave, a.nreg > 0, [&](auto kern) {
+        hipFuncAttributes at;
+        hipError_t e = hipFuncGetAttributes(&at, (const void*)kern);
+        if (e != hipSuccess) return e;
+        if (at.sharedSizeBytes != 0) return hipErrorInvalidDeviceFunction;
         if (lds > 64 * 1024) {
-            hipError_t e = hipFuncSetAttribute((const void*)kern, hipFuncAttributeMaxDynamicSharedMemorySize, (int)lds);
+            e = hipFuncSetAttribute((const void*)kern, hipFuncAttributeMaxDynamicSharedMemorySize, (int)lds);
             if (e != hipSuccess) return e;
         }
         hipLaunchKernelGGL(kern, dim3(nblocks), dim3(a.wg), lds, st, a);
