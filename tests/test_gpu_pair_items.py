@@ -127,3 +127,46 @@ def test_batched_histogram_limit(eng, weighted, fits):
     assert out["cnt"].sum() > 0
     with pytest.raises(GsError, match="do not fit in LDS"):
         eng.pcf2_batched(0.5, 6.0, 13, nm + 5, False, "fp32", cell_div=2)
+
+
+@pytest.mark.parametrize("prec", ["fp32", "fp64"])
+@pytest.mark.parametrize("buffered", [False, True])
+def test_packed_counts_beyond_their_width(eng, monkeypatch, prec, buffered):
+    # one replica and 1,024 threads a work-group, at most two of those on a compute unit: the pairs of one bin average
+    # more than 2^22 a histogram, the width of a packed count, so without the scans some count would run over
+    import torch
+    monkeypatch.setenv("GS_PAIR_REPS", "1")
+    monkeypatch.setenv("GS_PAIR_WG", "1024")
+    groups = 2 * torch.cuda.get_device_properties(0).multi_processor_count
+    n = 90000
+    rng = np.random.default_rng(4)
+    xyz = 100.0 + rng.uniform(0.0, 1.0, (n, 3))
+    w = rng.uniform(0.1, 1.0, n)
+    buf = (rng.random(n) < 0.02).astype(np.int32) if buffered else None
+    k = 0 if buf is None else int(buf.sum())
+    assert (n - k) * (n - k - 1) // 2 > groups * 2 ** 22 * 1.5
+    eng.set_catalogue(xyz, w, n, buf)
+    r = eng.pcf2(0.0, 2.0, 1, 1, False, prec)
+    assert int(r["cnt"][0, 0, 0]) == (n - k) * (n - 1)
+    wl = w.astype(np.longdouble)
+    apex = wl if buf is None else wl[buf == 0]
+    exact = float(np.sum(apex) * np.sum(wl) - np.sum(apex ** 2))
+    # each product is rounded to 2^-52 of the largest, one: 1e-16 of the mean product of 0.3 in the end
+    assert abs(r["wsum"][0, 0, 0] - exact) <= 1e-14 * exact
+
+
+def test_packed_counts_of_waves_beyond_their_width(eng):
+    # a batch has a histogram for every wave, at most 32 on a compute unit
+    import torch
+    waves = 32 * torch.cuda.get_device_properties(0).multi_processor_count
+    n = 280000
+    assert n * (n - 1) // 2 > waves * 2 ** 22 * 1.1
+    rng = np.random.default_rng(5)
+    xyz = 100.0 + rng.uniform(0.0, 1.0, (n, 3))
+    w = rng.uniform(0.1, 1.0, n)
+    eng.set_catalogue_batched(xyz, w, None, np.array([0, n]), np.array([n]))
+    r = eng.pcf2_batched(0.0, 2.0, 1, 1, False, cell_div=2)
+    assert int(r["cnt"][0, 0, 0, 0]) == n * (n - 1)
+    s, s2 = np.sum(w.astype(np.longdouble)), np.sum(w.astype(np.longdouble) ** 2)
+    exact = float(s * s - s2)
+    assert abs(r["wsum"][0, 0, 0, 0] - exact) <= 1e-14 * exact

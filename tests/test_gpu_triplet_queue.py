@@ -63,3 +63,32 @@ def test_long_lists(eng, monkeypatch, nmu, weighted):
     assert np.array_equal(a["cnt"], b["cnt"])
     if weighted:
         assert np.array_equal(a["wsum"], b["wsum"])
+
+
+@pytest.mark.parametrize("prec", ["fp32", "fp64"])
+@pytest.mark.parametrize("batched", [False, True])
+def test_packed_counts_beyond_their_width(eng, prec, batched):
+    # 2,000 points within reach of each other, every side in the first of 6 bins: a histogram of 224 entries has one
+    # replica, and lists of 28 bytes an entry (FP64: 44) leave the LDS of a compute unit room for two work-groups (FP64:
+    # one), so that the triangles, counted three times, average more than 2^22 a histogram: without the drains some
+    # packed count would run over
+    import torch
+    groups = 2 * torch.cuda.get_device_properties(0).multi_processor_count
+    n = 2000
+    assert n * (n - 1) * (n - 2) // 2 > groups * 2 ** 22 * 1.5
+    rng = np.random.default_rng(22)
+    xyz = rng.uniform(0, 1.0, (n, 3)) + 5.0
+    w = rng.uniform(0.5, 1.0, n)
+    if batched:
+        eng.set_catalogue_batched(xyz, w, None, np.array([0, n]), np.array([n]))
+        a = eng.pcf3_batched(0.0, 12.0, 6, 1, False, prec, cell_div=2)
+        cnt, wsum = a["cnt"][0, :, 0], a["wsum"][0, :, 0]
+    else:
+        eng.set_catalogue(xyz, w, n)
+        a = eng.pcf3(0.0, 12.0, 6, 1, False, prec)
+        cnt, wsum = a["cnt"], a["wsum"]
+    assert cnt[0, 0] == n * (n - 1) * (n - 2) // 2 and cnt.sum() == cnt[0, 0]
+    p1, p2, p3 = (np.sum(w.astype(np.longdouble) ** k) for k in (1, 2, 3))
+    exact = float((p1 ** 3 - 3 * p1 * p2 + 2 * p3) / 2)
+    # each product is rounded down to 2^-60 of the largest, and twice in FP64 before: 4e-16 of it
+    assert abs(wsum[0, 0] - exact) <= 2e-15 * exact
