@@ -69,10 +69,8 @@ void DevBuf<T>::release()
 template struct DevBuf<double>;
 template struct DevBuf<int32_t>;
 template struct DevBuf<double4>;
-template struct DevBuf<float4>;
 template struct DevBuf<unsigned long long>;
 template struct DevBuf<unsigned char>;
-template struct DevBuf<int64_t>;
 template struct DevBuf<float>;
 template struct DevBuf<int2>;
 template struct DevBuf<unsigned>;
@@ -454,7 +452,6 @@ struct gs_ctx {
     bool row_chunks_valid = false;
     // launch scratch: one region that a launch clears (work counters, output copies, cell counts), parameters
     DevBuf<unsigned char> zero, params;
-    DevBuf<unsigned long long> out;
     HostBuf host;               // parameters and results in flight
     // catalogue hand-over: statistics, and a ring of pinned pieces for catalogues in host memory
     DevBuf<CatalogueStats> stats;
@@ -535,7 +532,7 @@ extern "C" int gs_destroy(gs_ctx* c)
     c->xyz.release(); c->w.release(); c->buf.release();
     c->rank.release(); c->boff.release(); c->cell_start.release(); c->chunk_nc.release(); c->chunk_off.release();
     c->scan_tmp.release(); c->ticket.release(); c->pw.release(); c->cell.release(); c->flags.release();
-    c->orig.release(); c->zero.release(); c->params.release(); c->out.release(); c->host.release();
+    c->orig.release(); c->zero.release(); c->params.release(); c->host.release();
     c->stats.release(); c->ingest.release(); c->stats_host.release(); c->ring.release();
     for (auto& ev : c->ring_ev)
         if (ev) (void)hipEventDestroy(ev);

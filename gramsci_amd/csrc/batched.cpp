@@ -35,9 +35,9 @@ void batch_release(GsBatch& b)
         pl.blob.release();
     }
     b.plans.clear();
-    b.d_off.release(); b.d_row_base.release(); b.rank.release(); b.count.release(); b.boff.release();
+    b.d_off.release(); b.rank.release(); b.count.release(); b.boff.release();
     b.cell_start.release(); b.queue.release(); b.orig.release();
-    b.d_regions.release(); b.params.release(); b.pw.release(); b.cell.release(); b.flags.release();
+    b.pw.release(); b.cell.release(); b.flags.release();
     b.out.release();
     b.xyz.release(); b.w.release(); b.buf.release(); b.ovf.release(); b.big.release();
     b.valid = false;

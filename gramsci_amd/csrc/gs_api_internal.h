@@ -64,10 +64,9 @@ struct GsBatch {
     std::vector<double> wmr;             // per-region largest weight (1 for unit weights)
     std::vector<double> wmr_d, wmr_r;    // per-region largest data / random weight (1 for none)
     double wmax = 1.0, wmax_d = 1.0, wmax_r = 1.0, xmax = 0.0;
-    DevBuf<int32_t> d_off, d_row_base, rank, count, boff, cell_start, queue, orig;
+    DevBuf<int32_t> d_off, rank, count, boff, cell_start, queue, orig;
     DevBuf<int32_t> ovf;                 // 3PCF: queued apexes of the second and the device-memory pass
     DevBuf<unsigned char> big;           // 3PCF: device-memory neighbour lists
-    DevBuf<unsigned char> d_regions, params;
     DevBuf<double4> pw;
     DevBuf<int2> cell;
     DevBuf<uint32_t> flags;
@@ -120,7 +119,6 @@ struct CtxView {
     const int32_t* cell_start;
     const int2* cell;
     const int32_t* row_chunk;
-    const int4* chunks;
     const double* w;            // raw weights, original order (NULL for unit weights)
     int32_t n_chunks;
     GsExtra* extra;

@@ -28,7 +28,6 @@ struct HistSink {
     const PairArgs& a;
     unsigned char* hist;        // this wave's histogram
     int lane, nm, nbt, nbm, planes, nent, hi_off, rep_off;
-    bool batched;
     int cur_r;
     int sd, sr;                 // fixed-point scales of data and random weights (batched: the region's)
     // the work-group's copy of the outputs: [2][nbt] counts and [2][nbt][2] sums of the current region
@@ -242,7 +241,6 @@ __global__ __launch_bounds__(1024) void k_pair2(PairArgs a)
     sink.nent = sink.planes * sink.nbt * a.reps;                // words of one plane of the histogram
     sink.hi_off = sink.nent * 8;
     sink.rep_off = (lane & (a.reps - 1)) * sink.planes * sink.nbt * sink.kB;
-    sink.batched = batched;
     sink.cur_r = batched ? -1 : 0;
     sink.sd = B.fx_sd;
     sink.sr = B.fx_sr;
