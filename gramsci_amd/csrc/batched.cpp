@@ -43,6 +43,12 @@ void batch_release(GsBatch& b)
     b.valid = false;
 }
 
+// Histogram entries (3 nbins nmu) of a batched 2PCF
+static int batch_max_entries(bool fp64, bool weighted)
+{
+    return weighted ? (fp64 ? 665 : 793) : (fp64 ? 3327 : 3967);
+}
+
 static std::string plan_key(const gs_params& p, int kind)
 {
     char k[160];
@@ -264,8 +270,9 @@ static int get_plan(gs_ctx* c, const gs_params& p, const BatchTune& tu, int kind
     // one histogram per wave: fewer planes and waves where it would not fit otherwise
     const PairVariant var{nb, nm, fp64 || (kind == 2 && bins.wide), weighted, p.log_bins != 0, B.has_buf};
     int pair_wg = kWG, pair_waves = 0;
-    // the histograms that a batch takes: four, with a word per count and two per sum, in 64 KiB with their tables
-    if (kind == 2 && (size_t)nbt * (weighted ? 80 : 16) + 2064 + (fp64 ? 10240 : 0) > 64 * 1024) {
+    // A batch's limit on histogram entries is part of its interface: the LDS (a histogram for every wave) would hold
+    // more, and a work-group's fewer waves be slower.
+    if (kind == 2 && nbt > batch_max_entries(fp64, weighted)) {
         pblob->release(); B.plans.pop_back();
         return fail(GS_ELIMIT, "per-wave histograms of %d bins do not fit in LDS", nbt);
     }
