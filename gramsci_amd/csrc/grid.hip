@@ -286,10 +286,20 @@ __device__ __forceinline__ PointCell point_cell(const GridArgs& a, int64_t i)
         nd = R.n_data;
     }
     const double inv_h = 1.0 / a.g.h, inv_hx = 1.0 / a.g.hx;
+    const double x = a.xyz[3 * i + 0], y = a.xyz[3 * i + 1], z = a.xyz[3 * i + 2];
     PointCell c;
-    c.cx = cell_coord(a.xyz[3 * i + 0], lo[0], inv_hx, nx);
-    const int cy = cell_coord(a.xyz[3 * i + 1], lo[1], inv_h, ny);
-    const int cz = cell_coord(a.xyz[3 * i + 2], lo[2], inv_h, nz);
+    if (x != x || y != y || z != z) {
+        // A point that is not a number has no pairs.  It goes behind all cells, to an x-row of its own, so that no
+        // chunk of points has its coordinates relative to it.  (A single grid: regions have no such points.)
+        c.cx = 0;
+        c.row = ny * nz;
+        c.cell = (int)a.ncell;
+        c.random = false;
+        return c;
+    }
+    c.cx = cell_coord(x, lo[0], inv_hx, nx);
+    const int cy = cell_coord(y, lo[1], inv_h, ny);
+    const int cz = cell_coord(z, lo[2], inv_h, nz);
     const int row = cz * ny + cy;
     c.row = row0 + row;
     c.cell = cell0 + row * nx + c.cx;

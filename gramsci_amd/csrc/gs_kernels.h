@@ -37,7 +37,7 @@ struct GridArgs {
     const int32_t* off;         // nreg+1 first point of each region
     int32_t nreg;
     int32_t* rank;              // [n] scratch
-    int32_t* count;             // [2 ncell + 1] scratch: data and randoms per cell, zero before
+    int32_t* count;             // [2 ncell + 1] scratch: data and randoms per cell, points in none; zero before
     int32_t* boff;              // [cell_scan_blocks(ncell)] scratch
     unsigned* ticket;           // zero before and after
     // the sorted catalogue: point and raw weight, x cell and x-row (over all regions), flags, input index

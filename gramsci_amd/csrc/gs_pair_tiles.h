@@ -318,8 +318,7 @@ __device__ __forceinline__ void walk(const WalkArgs& a, Sink& sink, const BinDes
             }
             const int cy = (grow - row0) % ny, cz = (grow - row0) / ny;
 
-            // ---- the lane's apexes, relative to the chunk's middle point, or where that has a coordinate that is no
-            // number (which would reach every apex) to its first point without one
+            // ---- the lane's apexes, relative to the chunk's middle point
             const bool v1 = ai < n_i, v2 = ai2 < n_i;
             Pt<R> A1, A2;
             Ref ref;
@@ -329,9 +328,7 @@ __device__ __forceinline__ void walk(const WalkArgs& a, Sink& sink, const BinDes
                 uint32_t f1 = 2u, f2 = 2u;
                 if (v1) { P1 = a.pw[ib + ai]; f1 = a.flags[ib + ai]; }
                 if (v2) { P2 = a.pw[ib + ai2]; f2 = a.flags[ib + ai2]; }
-                const unsigned long long num = lanes(lane < n_i && P1.x == P1.x && P1.y == P1.y && P1.z == P1.z);
-                const int mid = n_i >> 1;
-                ref.set(P1, num == 0 || (num >> mid & 1) ? mid : uniform((int)__builtin_ctzll(num)));
+                ref.set(P1, n_i >> 1);
                 A1 = ref.point<R>(P1);
                 A2 = ref.point<R>(P2);
                 if (!v1) A1.x = far_away<R>();

@@ -111,3 +111,24 @@ def test_largest_rmax(eng, rmax, nmu):
     eng.set_catalogue(xyz, None, 100)
     for prec in ("fp32", "fp64"):
         assert np.array_equal(eng.pcf2(p.rmin, p.rmax, 3, nmu, p.log_bins, prec)["cnt"], ref["cnt"]), prec
+
+
+@pytest.mark.parametrize("weighted", [False, True])
+def test_triplets_and_quads_beside_points_that_are_not_numbers(eng, weighted):
+    rng = np.random.default_rng(6)
+    n = 700
+    xyz = rng.uniform(0, 12.0, (n, 3))
+    w = rng.uniform(0.5, 2.0, n) if weighted else None
+    bad = rng.random(n) < 0.2
+    x = xyz.copy()
+    x[bad, rng.integers(0, 3, int(bad.sum()))] = np.nan
+    g = ~bad
+    wg = np.ones(int(g.sum())) if w is None else w[g]
+    nd = int(g[:250].sum())
+    eng.set_catalogue(x, w, 250)
+    for nmu in (1, 3):
+        ref = O.pcf3(xyz[g], wg, nd, O.Params(0.5, 3.0, 3, nmu, False))
+        for prec in ("fp32", "fp64"):
+            assert np.array_equal(eng.pcf3(0.5, 3.0, 3, nmu, False, prec)["cnt"], ref["cnt"]), (nmu, prec)
+    ref = O.pcf4(xyz[g], wg, nd, O.Params(0.5, 3.0, 2, 1, False))
+    assert np.array_equal(eng.pcf4(0.5, 3.0, 2)["cnt"], ref["cnt"])
