@@ -135,7 +135,7 @@ struct RowTable {
 template <bool FP64>
 __device__ __forceinline__ void fill_bin_table(unsigned char* smem, const BinDesc& B, int tid, int nthr)
 {
-    for (int k = tid; k <= kMaxBins; k += nthr) {
+    for (int k = tid; k <= B.nb; k += nthr) {
         if constexpr (FP64) ((double*)smem)[k] = B.t64[k];
         else {
             // start and width; a width of 0 is never certain.  s - lo rounds monotonically, so s >= hi gives a
