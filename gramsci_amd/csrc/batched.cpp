@@ -381,7 +381,7 @@ static int get_plan(gs_ctx* c, const gs_params& p, const BatchTune& tu, int kind
                   : std::max(1, mat ? triplet_matrix_occupancy(ta1, nb, wave) : triplet3_occupancy(ta1, nb, fp64, weighted));
     const int nblocks = kind == 3 ? std::max(1, (int)std::min<int64_t>((int64_t)v.n_cu * occ, std::max<int64_t>(n, 1)))
                                   : (v.n_cu * occ + 7) / 8 * 8;
-    if (kind == 3) ta1.batch = std::max(triplet_batch(n, nblocks), wave ? 8 * ta1.wg / kWave : 1);
+    if (kind == 3) ta1.batch = triplet_batch(n, nblocks, wave ? ta1.wg / kWave : 1);
 
     // capture: clear, sort into cells, pair or triplet kernel
     e = hipStreamBeginCapture(v.stream, hipStreamCaptureModeThreadLocal);

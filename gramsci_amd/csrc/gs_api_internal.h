@@ -204,9 +204,9 @@ std::vector<uint8_t> normal_table(int nm);
 int plan_triplet_lds(TripArgs& a, int nb, bool fp64, bool weighted);
 // threads per triplet work-group for a mean neighbour count kmean (GS_T3_WG overrides)
 int triplet_wg(double list, bool rsd, bool weighted);
-// apexes per queue fetch for n work items over nblocks work-groups: about 128 fetches per work-group
-// (GS_APEX_BATCH overrides)
-int triplet_batch(int64_t n, int nblocks);
+// apexes per queue fetch for n work items over nblocks work-groups of `teams` teams: about 128 fetches per
+// work-group (GS_APEX_BATCH overrides)
+int triplet_batch(int64_t n, int nblocks, int teams);
 void combine3(const long double* S, int nq, long double Wd, long double Wr, bool with_n3, double* n2, double* n3);
 // The matrix triplet kernel (triplet_matrix.hip) for nb bins: whether it takes the call, the histogram replicas and
 // the longest list of a pass with one apex per work-group (a.reps, a.kmax); and its team and work-group size for
