@@ -169,6 +169,7 @@ __device__ __forceinline__ int next_item(int32_t* queue, int n, int xcd, int& tr
 
 // v, the same in all lanes, in scalar registers
 __device__ __forceinline__ int scalar(int v) { return __builtin_amdgcn_readfirstlane(v); }
+__device__ __forceinline__ float scalar(float v) { return __int_as_float(scalar(__float_as_int(v))); }
 __device__ __forceinline__ double scalar(double v)
 {
     const long long b = __double_as_longlong(v);

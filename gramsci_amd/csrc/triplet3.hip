@@ -107,7 +107,8 @@ enum { kT3Rsd = 1, kT3Equi = 2 };
 // Six waves per SIMD (at most 80 registers, up to four of them spilled) for mu bins without weights: 300k
 // points, 6 mu bins 1.47 -> 1.40 ms, FP64 1.02 -> 0.96.  With weights ten would be spilled, for no gain.
 template <bool FP64, bool W, int MODE, int GEN, bool LOGB>
-__global__ __launch_bounds__(kWG) __attribute__((amdgpu_waves_per_eu((MODE & kT3Rsd) && !W ? 6 : 1)))
+__global__ __launch_bounds__(kWG) __attribute__((amdgpu_waves_per_eu(
+    ((MODE & kT3Rsd) ? !W : W && GEN != 2) ? 6 : 1)))
 void k_triplet3(TripArgs a)
 {
     extern __shared__ __align__(16) unsigned char smem[];
@@ -564,12 +565,16 @@ void k_triplet3(TripArgs a)
                 }
             }
         };
-        // the bin of the third side of (u, v), -1 where it has none or (equi) not the bin of the other two
-        auto third = [&](const int u, const int v) {
+        auto record = [&](const int u) {
+            if constexpr (FP64) return rec64[u];
+            else return rec32[u];
+        };
+        // the bin of the third side of (u, v), u with record Ru, -1 where it has none or (equi) not the bin of the other two
+        auto third = [&](const rec_t& Ru, const int u, const int v) {
             int b3 = -1;
             uint32_t pu;
             if constexpr (FP64) {
-                const double4 Ru = rec64[u], Rv = rec64[v];
+                const double4 Rv = rec64[v];
                 pu = (uint32_t)Ru.w;
                 if (!equi || ((pu ^ (uint32_t)Rv.w) & 0x7fffu) == 0) {
                     const double s = exact_s(Ru.x, Ru.y, Ru.z, Rv.x, Rv.y, Rv.z);
@@ -581,7 +586,7 @@ void k_triplet3(TripArgs a)
                     }
                 }
             } else {
-                const float4 Ru = rec32[u], Rv = rec32[v];
+                const float4 Rv = rec32[v];
                 pu = __float_as_uint(Ru.w);
                 const float dx = Rv.x - Ru.x, dy = Rv.y - Ru.y, dz = Rv.z - Ru.z;
                 const float s = fmaf(dz, dz, fmaf(dy, dy, dx * dx));
@@ -615,14 +620,16 @@ void k_triplet3(TripArgs a)
         const int R = K / 2;
         const int wv = tid >> 6, ln = tid & 63, nw = nt >> 6;
         if constexpr (Q) {
-            // The flat schedule (below) with a uniform number of steps per wave.  A third to a half of the pairs have
-            // a binned third side (with equal sides few), and an update is three times as long as the test, so it
-            // runs for 64 queued pairs at once.  In pieces of 2^20 pairs, which a packed histogram can take.
+            // A third to a half of the pairs have a binned third side (with equal sides few), and an update is three
+            // times as long as the test, so it runs for 64 queued pairs at once.  The schedules below with a uniform
+            // number of steps per wave, by rows the record of a row's u in scalar registers: lists beyond 448 entries,
+            // whose rows leave few lanes idle (6,000 points with 2,000 neighbours, 3 mu bins: flat 14.4, by rows 13.0
+            // ms).  In pieces of 2^20 pairs, which a packed histogram can take.
             const int P = K * (K - 1) / 2;
-            const int KK = max(K, 1), dq = nt / KK, dr = nt - dq * KK;
-            for (int p0 = 0; p0 < P; p0 += 1 << 20) {
-                const int p1 = min(P, p0 + (1 << 20));
-                const unsigned long long more = (unsigned long long)(p1 - p0) * (SYM ? 3 : 1);
+            const bool by_rows = K > 448;
+            int qn = 0;
+            auto piece = [&](const int pairs) {         // room for another piece's counts
+                const unsigned long long more = (unsigned long long)pairs * (SYM ? 3 : 1);
                 if (lh && bound + more > kDrain) {
                     __syncthreads();
                     drain(cur_r);
@@ -630,36 +637,68 @@ void k_triplet3(TripArgs a)
                     __syncthreads();
                 }
                 bound += more;
-                int qn = 0;
-                int r = (p0 + tid) / K, c = p0 + tid - r * K;
-                for (int base = p0 + __builtin_amdgcn_readfirstlane(wv) * kWave; base < p1; base += nt) {
-                    int b3 = -1, u = 0, v = 0;
-                    if (base + ln < p1) {
-                        const bool first = c < K - 1 - r;
-                        u = first ? r : K - 2 - r;
-                        v = first ? r + 1 + c : c;
-                        b3 = third(u, v);
-                    }
-                    c += dr;
-                    const bool carry = c >= K;
-                    c -= carry ? K : 0;
-                    r += dq + (carry ? 1 : 0);
-                    const unsigned long long m = __builtin_amdgcn_ballot_w64(b3 >= 0);
-                    if (b3 >= 0)
-                        queue[qn + (int)__builtin_amdgcn_mbcnt_hi((uint32_t)(m >> 32),
-                                                                  __builtin_amdgcn_mbcnt_lo((uint32_t)m, 0u))] =
-                            (uint32_t)u | ((uint32_t)v << 12) | ((uint32_t)b3 << 24);
-                    qn += (int)__popcll(m);
-                    if (qn >= kWave) {
-                        qn -= kWave;
-                        wave_sync();
-                        queued(queue[qn + ln]);
-                        wave_sync();
-                    }
+            };
+            auto push = [&](const int b3, const int u, const int v) {
+                const unsigned long long m = __builtin_amdgcn_ballot_w64(b3 >= 0);
+                if (b3 >= 0)
+                    queue[qn + (int)__builtin_amdgcn_mbcnt_hi((uint32_t)(m >> 32),
+                                                              __builtin_amdgcn_mbcnt_lo((uint32_t)m, 0u))] =
+                        (uint32_t)u | ((uint32_t)v << 12) | ((uint32_t)b3 << 24);
+                qn += (int)__popcll(m);
+                if (qn >= kWave) {
+                    qn -= kWave;
+                    wave_sync();
+                    queued(queue[qn + ln]);
+                    wave_sync();
                 }
+            };
+            auto finish = [&]() {
                 wave_sync();
                 if (ln < qn) queued(queue[ln]);
                 wave_sync();
+                qn = 0;
+            };
+            if (by_rows) {
+                const int rows = max(nw, (1 << 20) / K / nw * nw);
+                for (int b0 = 0; b0 < R; b0 += rows) {
+                    const int b1 = min(R, b0 + rows);
+                    piece((b1 - b0) * K);
+                    for (int r = b0 + __builtin_amdgcn_readfirstlane(wv); r < b1; r += nw)
+                        for (int u = r;; u = K - 2 - r) {
+                            rec_t Ru = record(u);       // the same in all lanes
+                            Ru.x = scalar(Ru.x); Ru.y = scalar(Ru.y); Ru.z = scalar(Ru.z); Ru.w = scalar(Ru.w);
+                            for (int v0 = u + 1; v0 < K; v0 += kWave) {
+                                const int v = v0 + ln;
+                                int b3 = -1;
+                                if (v < K) b3 = third(Ru, u, v);
+                                push(b3, u, v);
+                            }
+                            if (u != r || K - 2 - r == r) break;    // both rows done; an even K's last is one
+                        }
+                    finish();
+                }
+            } else {
+                const int KK = max(K, 1), dq = nt / KK, dr = nt - dq * KK;
+                for (int p0 = 0; p0 < P; p0 += 1 << 20) {
+                    const int p1 = min(P, p0 + (1 << 20));
+                    piece(p1 - p0);
+                    int r = (p0 + tid) / K, c = p0 + tid - r * K;
+                    for (int base = p0 + __builtin_amdgcn_readfirstlane(wv) * kWave; base < p1; base += nt) {
+                        int b3 = -1, u = 0, v = 0;
+                        if (base + ln < p1) {
+                            const bool first = c < K - 1 - r;
+                            u = first ? r : K - 2 - r;
+                            v = first ? r + 1 + c : c;
+                            b3 = third(record(u), u, v);
+                        }
+                        c += dr;
+                        const bool carry = c >= K;
+                        c -= carry ? K : 0;
+                        r += dq + (carry ? 1 : 0);
+                        push(b3, u, v);
+                    }
+                    finish();
+                }
             }
         } else if constexpr (GEN != 2) {
             // Two schedules, chosen per apex (K is uniform in the work-group):

@@ -92,3 +92,21 @@ def test_packed_counts_beyond_their_width(eng, prec, batched):
     exact = float((p1 ** 3 - 3 * p1 * p2 + 2 * p3) / 2)
     # each product is rounded down to 2^-60 of the largest, and twice in FP64 before: 4e-16 of it
     assert abs(wsum[0, 0] - exact) <= 2e-15 * exact
+
+
+@pytest.mark.parametrize("prec", ["fp32", "fp64"])
+@pytest.mark.parametrize("nmu,weighted,equi", [(1, True, False), (3, False, False), (2, True, False), (1, False, True)])
+@pytest.mark.parametrize("n", [449, 450, 451, 577, 900])
+def test_lists_by_rows(eng, prec, nmu, weighted, equi, n):
+    # n points within reach of each other: every apex has n - 1 neighbours (isotropic: those after it), on both sides of
+    # the 448 entries from which the pairs go to the waves by rows
+    rng = np.random.default_rng(n)
+    xyz = rng.uniform(0, 4.0, (n, 3)) + 20.0
+    w = C.lognormal_weights(n, 0.4, 7) if weighted else None
+    p = O.Params(2.0, 8.0, 3, nmu, False)
+    ref = (O.pcf3_equi if equi else O.pcf3)(xyz, np.ones(n) if w is None else w, n // 3, p)
+    eng.set_catalogue(xyz, w, n // 3)
+    a = (eng.pcf3_equi if equi else eng.pcf3)(p.rmin, p.rmax, p.nbins, nmu, False, prec)
+    assert np.array_equal(a["cnt"].reshape(ref["cnt"].shape), ref["cnt"])
+    if weighted:
+        assert _close(a["n2"], ref["n2"])
