@@ -202,6 +202,8 @@ std::vector<uint16_t> table3(int nb);
 std::vector<uint16_t> table3_hist(int nb);   // 4 * configuration, for the triplet kernel
 std::vector<uint8_t> normal_table(int nm);
 int plan_triplet_lds(TripArgs& a, int nb, bool fp64, bool weighted);
+// more histogram replicas of a weighted pass with `occ` work-groups per compute unit
+void triplet_replicas(TripArgs& a, int nb, bool fp64, int occ);
 // threads per triplet work-group for a mean neighbour count kmean (GS_T3_WG overrides)
 int triplet_wg(double list, bool rsd, bool weighted);
 // apexes per queue fetch for n work items over nblocks work-groups of `teams` teams: about 128 fetches per
