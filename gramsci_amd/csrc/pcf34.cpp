@@ -292,6 +292,29 @@ void combine3(const long double* S, int nq, long double Wd, long double Wr, bool
     }
 }
 
+// The kept-neighbour counts of nsample apexes (none: of buffer points) spread over n, in d_out (2 nsample).  *gather: the
+// apexes have so many candidates that finding the neighbours is the work, as where a few outlying points widen the
+// cells (a box of 20 with one point at 5,000, 30,000 points, 150 neighbours: matrix kernel 1.75 ms, general kernel 1.35;
+// 4,000 points, 40 neighbours: 0.051 and 0.073).
+static int sample_neighbours(const TripArgs& a, int n, int nsample, int after_only, int32_t* d_out, hipStream_t st,
+                             std::vector<int32_t>& ks, bool* gather)
+{
+    if (nsample <= 0) return GS_OK;
+    std::vector<int32_t> h(2 * (size_t)nsample);
+    hipError_t e = launch_nbr_count(a, n / nsample, nsample, after_only, d_out, st);
+    if (e == hipSuccess) e = hipMemcpyAsync(h.data(), d_out, h.size() * sizeof(int32_t), hipMemcpyDeviceToHost, st);
+    if (e == hipSuccess) e = hipStreamSynchronize(st);
+    if (e != hipSuccess) return hip_fail(e, "neighbour sample");
+    double cand = 0.0;
+    for (int t = 0; t < nsample; ++t)
+        if (h[t] >= 0) {
+            ks.push_back(h[t]);
+            cand += h[nsample + t];
+        }
+    *gather = cand > 8192.0 * (double)ks.size();
+    return GS_OK;
+}
+
 // Shared body of gs_count_3pcf (all configurations) and gs_count_3pcf_equi.
 static int count3(gs_ctx* c, const gs_params* p, bool equi, uint64_t* cnt, double* wsum, double* n2, double* n3,
                   gs_stats* st)
@@ -333,7 +356,7 @@ static int count3(gs_ctx* c, const gs_params* p, bool equi, uint64_t* cnt, doubl
     // FP32 counts of unit weights without mu bins: third sides from the matrix cores (am); its passes are the
     // general kernel's, which also takes the apexes whose lists fit no LDS
     TripArgs am = a;
-    const bool mat = !equi && nm == 1 && !fp64 && !weighted && plan_triplet_matrix(am, nb, v.has_buf);
+    bool mat = !equi && nm == 1 && !fp64 && !weighted && plan_triplet_matrix(am, nb, v.has_buf);
     const std::vector<uint32_t> cfgb = mat ? cfg_bins3(nb) : std::vector<uint32_t>();
 
     // Parameters in one copy from pinned memory.  One region to clear: the work counters of two passes, the error
@@ -403,25 +426,21 @@ static int count3(gs_ctx* c, const gs_params* p, bool equi, uint64_t* cnt, doubl
     // one pass, so the sums are those of one pass.
     // An apex whose neighbours outnumber even the second pass's list is queued once more, for a
     // last pass with its list in device memory (triplet_glist_pass): no neighbour count is refused.
-    const int kmax_full = mat ? am.kmax : a.kmax;
-    int kmax1 = kmax_full;
+    // Without a matrix kernel where the gather is the work: its lists leave fewer waves than the general kernel's.
     const int nsample = std::min(n, 2048);
-    const int stride = nsample > 0 ? n / nsample : 1;
-    // i32: second-pass apexes, last-pass apexes, the sampled neighbour counts
-    if ((rc = X.i32.reserve(2 * (size_t)n + nsample))) return rc;
+    // i32: second-pass apexes, last-pass apexes, the sample
+    if ((rc = X.i32.reserve(2 * (size_t)n + 2 * nsample))) return rc;
     int32_t* d_list2 = X.i32.ptr;
     int32_t* d_list3 = X.i32.ptr + n;
+    std::vector<int32_t> ks;
+    bool gather = false;
+    if ((rc = sample_neighbours(a, n, nsample, nm > 1 ? 0 : 1, X.i32.ptr + 2 * (size_t)n, v.stream, ks, &gather))) return rc;
+    if (gather) mat = false;
+    const int kmax_full = mat ? am.kmax : a.kmax;
+    int kmax1 = kmax_full;
     if (nsample > 0) {
-        int32_t* d_cnt = X.i32.ptr + 2 * (size_t)n;
-        std::vector<int32_t> kc(nsample);
-        e = launch_nbr_count(a, stride, nsample, nm > 1 ? 0 : 1, d_cnt, v.stream);
-        if (e == hipSuccess) e = hipMemcpyAsync(kc.data(), d_cnt, nsample * sizeof(int32_t), hipMemcpyDeviceToHost, v.stream);
-        if (e == hipSuccess) e = hipStreamSynchronize(v.stream);
-        if (e != hipSuccess) return hip_fail(e, "3PCF neighbour sample");
-        std::vector<int32_t> ks;
         double ksum = 0.0;
-        for (int32_t k : kc)
-            if (k >= 0) { ks.push_back(k); ksum += k; }
+        for (int32_t k : ks) ksum += k;
         if (!ks.empty()) {
             a.wg = triplet_wg(ksum / (double)ks.size(), nm > 1, weighted);
             const size_t q = std::min(ks.size() - 1, (size_t)std::ceil(0.995 * (ks.size() - 1)));
@@ -640,9 +659,9 @@ static int count4(gs_ctx* c, const gs_params* p, bool tetra, uint64_t* cnt, doub
     double short_lists = 0.0;
     bool long_lists = false;        // a last pass is to be expected
     const int nsample = std::min(n, 2048);
-    const int stride = nsample > 0 ? n / nsample : 1;
-    // i32: the lists of queued apexes, then the sampled neighbour counts
-    if ((rc = X.i32.reserve(kPasses * (size_t)n + nsample))) return rc;
+    bool gather = false;
+    // i32: the lists of queued apexes, then the sample
+    if ((rc = X.i32.reserve(kPasses * (size_t)n + 2 * nsample))) return rc;
     if (nsample > 0) {
         TripArgs ts{};
         ts.pw = a.pw;
@@ -652,15 +671,8 @@ static int count4(gs_ctx* c, const gs_params* p, bool tetra, uint64_t* cnt, doub
         ts.bins = a.bins;
         ts.g = a.g;
         ts.nrows = a.nrows;
-        int32_t* d_kc = X.i32.ptr + kPasses * (size_t)n;
-        std::vector<int32_t> kc(nsample);
-        e = launch_nbr_count(ts, stride, nsample, 0, d_kc, v.stream);
-        if (e == hipSuccess) e = hipMemcpyAsync(kc.data(), d_kc, nsample * sizeof(int32_t), hipMemcpyDeviceToHost, v.stream);
-        if (e == hipSuccess) e = hipStreamSynchronize(v.stream);
-        if (e != hipSuccess) return hip_fail(e, "4PCF neighbour sample");
         std::vector<int32_t> ks;
-        for (int32_t k : kc)
-            if (k >= 0) ks.push_back(k);
+        if ((rc = sample_neighbours(ts, n, nsample, 0, X.i32.ptr + kPasses * (size_t)n, v.stream, ks, &gather))) return rc;
         if (!ks.empty()) {
             short_lists = (double)std::count_if(ks.begin(), ks.end(), [](int32_t k) { return k <= 64; }) / ks.size();
             const size_t q = std::min(ks.size() - 1, (size_t)std::ceil(0.995 * (ks.size() - 1)));
@@ -678,7 +690,8 @@ static int count4(gs_ctx* c, const gs_params* p, bool tetra, uint64_t* cnt, doub
             while (kmax1 < kmax && kmax1 < atoi(ev)) kmax1 *= 2;
         }
     }
-    // weighted sums in LDS where that leaves room for two work-groups
+    // weighted sums in LDS where that leaves room for two work-groups, and the gather (30,000 candidates an apex: 2.3 ms,
+    // with sums in global memory 1.3) is not the work
     auto with_sums = [&](int km, bool wv) {
         QuadArgs t = a;
         t.kmax = km;
@@ -686,7 +699,7 @@ static int count4(gs_ctx* c, const gs_params* p, bool tetra, uint64_t* cnt, doub
         // 5.3; 4 bins 4.3, 6.5); else one mask (10 bins 5.0 ms; lists of 128, and longer ones in device memory, 41)
         t.bin_masks = tetra ? 0 : 1;
         if (quad4_lds_bytes(t, nb, weighted, wv) > budget) t.bin_masks = 0;
-        t.lds_w = weighted ? 1 : 0;
+        t.lds_w = weighted && !gather ? 1 : 0;
         if (quad4_lds_bytes(t, nb, weighted, wv) > 80 * 1024) t.lds_w = 0;
         return t;
     };

@@ -887,7 +887,7 @@ __global__ __launch_bounds__(256) void k_nbr_count(TripArgs a, int stride, int n
     if (t >= nsample) return;
     const int apex = t * stride;
     if (a.flags[apex] & 2u) {
-        if (lane == 0) out[t] = -1;
+        if (lane == 0) { out[t] = -1; out[nsample + t] = 0; }
         return;
     }
     const BinDesc& B = *a.bins;
@@ -898,7 +898,7 @@ __global__ __launch_bounds__(256) void k_nbr_count(TripArgs a, int stride, int n
     const int cx = min(max((int)floor((Pa.x - a.g.lo[0]) * inv_hx), 0), nx - 1);
     const int cy = min(max((int)floor((Pa.y - a.g.lo[1]) * inv_h), 0), ny - 1);
     const int cz = min(max((int)floor((Pa.z - a.g.lo[2]) * inv_h), 0), nz - 1);
-    int cnt = 0;
+    int cnt = 0, cand = 0;
     for (int r = 0; r < a.nrows; ++r) {
         const Row rw = a.rows[r];
         const int by = cy + rw.dy, bz = cz + rw.dz;
@@ -907,6 +907,7 @@ __global__ __launch_bounds__(256) void k_nbr_count(TripArgs a, int stride, int n
         if (bx0 > bx1) continue;
         const int rb = (bz * ny + by) * nx;
         const int js = a.cell_start[rb + bx0], je = a.cell_start[rb + bx1 + 1];
+        cand += je - js;
         for (int j = js + lane; j < je; j += 64) {
             const double4 Pj = a.pw[j];
             const double s = exact_s(Pa.x, Pa.y, Pa.z, Pj.x, Pj.y, Pj.z);
@@ -914,7 +915,7 @@ __global__ __launch_bounds__(256) void k_nbr_count(TripArgs a, int stride, int n
         }
     }
     for (int off = 32; off > 0; off >>= 1) cnt += __shfl_down(cnt, off, 64);
-    if (lane == 0) out[t] = cnt;
+    if (lane == 0) { out[t] = cnt; out[nsample + t] = cand; }
 }
 
 hipError_t launch_nbr_count(const TripArgs& a, int stride, int nsample, int after_only, int32_t* out, hipStream_t st)

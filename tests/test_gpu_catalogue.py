@@ -85,3 +85,25 @@ def test_wide_grid_of_empty_cells(eng):
     t = [cKDTree(xyz[:400]), cKDTree(xyz[400:])]
     cc = [int(t[i].count_neighbors(t[j], 12.0)) for i, j in ((0, 0), (0, 1), (1, 1))]
     assert [int(v) for v in r["cnt"].reshape(-1)] == [cc[0] - 400, 2 * cc[1], cc[2] - 400]
+
+
+def test_outlying_point_widens_the_cells(eng):
+    # one point far away widens the cells until most points are an apex's candidates: triangles of unit weights leave the
+    # matrix kernel, four-point sums the LDS; counts are those without that point
+    rng = np.random.default_rng(5)
+    n = 12000
+    x = rng.uniform(0, 20.0, (n, 3))
+    w = rng.uniform(0.5, 2.0, n)
+    far = np.concatenate([x, [[5000.0, 5000.0, 5000.0]]])
+    got = []
+    for xyz, weights in ((x, w), (far, np.append(w, 1.0))):
+        eng.set_catalogue(xyz, None, 3000)
+        r3 = eng.pcf3(0.2, 1.2, 4)
+        eng.set_catalogue(xyz, weights, 3000)
+        r3w, r4w = eng.pcf3(0.2, 1.2, 4), eng.pcf4(0.3, 0.9, 3)
+        got.append((r3, r3w, r4w))
+    a, b = got
+    for k in range(3):
+        assert a[k]["cnt"].sum() > 0 and np.array_equal(a[k]["cnt"], b[k]["cnt"]), k
+        assert b[k]["stats"]["n_candidates"] > 8192 * n
+    assert np.array_equal(a[1]["wsum"], b[1]["wsum"])
