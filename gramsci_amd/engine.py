@@ -71,7 +71,9 @@ class Engine:
         nd = n if n_data is None else int(n_data)
         if nd < 0 or nd > n:
             raise ValueError("n_data out of range")
-        self.generation += 1        # also where the hand-over fails: the context then holds no catalogue
+        # also where the hand-over fails: the context then holds no catalogue
+        self.generation += 1
+        self.n_data = self.n_rand = 0
         if is_dev:
             import torch
             xyz = xyz.to(torch.float64).contiguous()

@@ -107,3 +107,16 @@ def test_outlying_point_widens_the_cells(eng):
         assert a[k]["cnt"].sum() > 0 and np.array_equal(a[k]["cnt"], b[k]["cnt"]), k
         assert b[k]["stats"]["n_candidates"] > 8192 * n
     assert np.array_equal(a[1]["wsum"], b[1]["wsum"])
+
+
+def test_engine_knows_that_a_failed_hand_over_left_nothing(eng):
+    import torch
+    x = np.random.default_rng(2).uniform(0, 9.0, (50, 3))
+    eng.set_catalogue(x, np.ones(50), 20)
+    with pytest.raises(GsError):
+        eng.set_catalogue(x, -np.ones(50), 20)
+    assert (eng.n_data, eng.n_rand) == (0, 0)
+    g = np.ones((2, 1))
+    assert eng.adjoint2(g, g, 0.0, 5.0, 2).size == 0
+    with pytest.raises(ValueError):         # an output for 50 points would stay as it was
+        eng.adjoint2(g, g, 0.0, 5.0, 2, out=torch.empty(50, dtype=torch.float64, device="cuda"))
