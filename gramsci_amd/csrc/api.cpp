@@ -613,7 +613,10 @@ static int ingest(gs_ctx* c, const double* d_xyz, const double* d_w, const int32
 
 static int check_catalogue(gs_ctx* c, const double* xyz, int64_t n_data, int64_t n_rand)
 {
-    if (!c || (!xyz && n_data + n_rand > 0)) return fail(GS_EINVAL, "NULL context or coordinates");
+    if (!c) return fail(GS_EINVAL, "NULL context or coordinates");
+    c->n_data = c->n_rand = 0;      // no catalogue stays behind a failure
+    c->grid_valid = false;
+    if (!xyz && n_data + n_rand > 0) return fail(GS_EINVAL, "NULL context or coordinates");
     if (n_data < 0 || n_rand < 0 || n_data + n_rand > (int64_t)INT32_MAX - 1024)
         return fail(GS_EINVAL, "bad catalogue size (n_data=%lld n_rand=%lld)", (long long)n_data, (long long)n_rand);
     return set_device(c);
@@ -650,8 +653,6 @@ extern "C" int gs_set_catalogue(gs_ctx* c, const double* xyz, const double* w, c
     int rc = check_catalogue(c, xyz, n_data, n_rand);
     if (rc) return rc;
     const int64_t n = n_data + n_rand;
-    c->n_data = c->n_rand = 0;
-    c->grid_valid = false;
     if ((rc = c->xyz.reserve(3 * n)) || (w && (rc = c->w.reserve(n))) || (buf && (rc = c->buf.reserve(n)))) return rc;
     if ((rc = upload(c, c->xyz.ptr, xyz, 3 * n * sizeof(double))) || (w && (rc = upload(c, c->w.ptr, w, n * sizeof(double)))) ||
         (buf && (rc = upload(c, c->buf.ptr, buf, n * sizeof(int32_t)))))
@@ -665,8 +666,6 @@ extern "C" int gs_set_catalogue_device(gs_ctx* c, const double* d_xyz, const dou
     int rc = check_catalogue(c, d_xyz, n_data, n_rand);
     if (rc) return rc;
     const int64_t n = n_data + n_rand;
-    c->n_data = c->n_rand = 0;
-    c->grid_valid = false;
     if ((rc = c->xyz.reserve(3 * n)) || (d_w && (rc = c->w.reserve(n))) || (d_buf && (rc = c->buf.reserve(n)))) return rc;
     return ingest(c, d_xyz, d_w, d_buf, n_data, n_rand);
 }

@@ -71,15 +71,13 @@ class Engine:
         nd = n if n_data is None else int(n_data)
         if nd < 0 or nd > n:
             raise ValueError("n_data out of range")
-        # also where the hand-over fails: the context then holds no catalogue
-        self.generation += 1
-        self.n_data = self.n_rand = 0
         if is_dev:
             import torch
             xyz = xyz.to(torch.float64).contiguous()
             w = None if w is None else w.to(torch.float64).contiguous()
             buf = None if buf is None else buf.to(torch.int32).contiguous()
             torch.cuda.current_stream().synchronize()
+            self._drop_catalogue()
             L.check(self._lib.gs_set_catalogue_device(
                 self._ctx, ctypes.c_void_p(xyz.data_ptr()),
                 None if w is None else ctypes.c_void_p(w.data_ptr()),
@@ -94,9 +92,15 @@ class Engine:
                 raise ValueError("w must be (n,)")
             if buf is not None and buf.shape != (n,):
                 raise ValueError("buf must be (n,)")
+            self._drop_catalogue()
             L.check(self._lib.gs_set_catalogue(self._ctx, L.ptr(xyz), L.ptr(w), L.ptr(buf, ctypes.c_int32),
                                                nd, n - nd))
         self.n_data, self.n_rand = nd, n - nd
+
+    def _drop_catalogue(self):
+        # before a hand-over: where it fails, the context holds no catalogue
+        self.generation += 1
+        self.n_data = self.n_rand = 0
 
     def set_catalogue_batched(self, xyz, w, buf, off, ndata):
         """Independent regions: region r is points off[r]:off[r+1] (data first,

@@ -120,3 +120,9 @@ def test_engine_knows_that_a_failed_hand_over_left_nothing(eng):
     assert eng.adjoint2(g, g, 0.0, 5.0, 2).size == 0
     with pytest.raises(ValueError):         # an output for 50 points would stay as it was
         eng.adjoint2(g, g, 0.0, 5.0, 2, out=torch.empty(50, dtype=torch.float64, device="cuda"))
+    # arguments that never reach the context leave its catalogue and the engine's sizes alone
+    eng.set_catalogue(x, None, 20)
+    with pytest.raises(ValueError):
+        eng.set_catalogue(x, np.ones(49), 20)
+    assert (eng.n_data, eng.n_rand) == (20, 30)
+    assert eng.adjoint2(g, g, 0.0, 5.0, 2).size == 50
