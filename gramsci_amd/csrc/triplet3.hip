@@ -105,7 +105,8 @@ size_t triplet3_queue_bytes(const TripArgs& a, bool weighted)
 enum { kT3Rsd = 1, kT3Equi = 2 };
 
 // Six waves per SIMD (at most 80 registers, up to four of them spilled) for mu bins without weights: 300k
-// points, 6 mu bins 1.47 -> 1.40 ms, FP64 1.02 -> 0.96.  With weights ten would be spilled, for no gain.
+// points, 6 mu bins 1.47 -> 1.40 ms, FP64 1.02 -> 0.96.  With both ten would be spilled, for no gain.  Weights without mu
+// bins stay within 80 by it, from 81 to 84.
 template <bool FP64, bool W, int MODE, int GEN, bool LOGB>
 __global__ __launch_bounds__(kWG) __attribute__((amdgpu_waves_per_eu(
     ((MODE & kT3Rsd) ? !W : W && GEN != 2) ? 6 : 1)))

@@ -170,3 +170,13 @@ def test_packed_counts_of_waves_beyond_their_width(eng):
     s, s2 = np.sum(w.astype(np.longdouble)), np.sum(w.astype(np.longdouble) ** 2)
     exact = float(s * s - s2)
     assert abs(r["wsum"][0, 0, 0, 0] - exact) <= 1e-14 * exact
+
+
+def test_largest_weighted_histograms(eng):
+    # 10,098 entries of 16 bytes fill the LDS; one bin more is refused
+    rng = np.random.default_rng(10)
+    xyz = rng.uniform(0, 10.0, (400, 3)) + 3.0
+    w = rng.uniform(0.5, 2.0, 400)
+    _check(eng, xyz, w, 150, O.Params(0.5, 6.0, 33, 102, False))
+    with pytest.raises(GsError, match="does not fit in LDS"):
+        eng.pcf2(0.5, 6.0, 99, 35, False)
